@@ -292,9 +292,9 @@ static int gemm64(omx_ctx ctx, bool trA, bool trB, int m, int n, int k, double a
 static int gemm64_lower(omx_ctx ctx, int n, int k, double alpha, const double *A, int64_t lda, const double *B,
                         int64_t ldb, double beta, double *C, int64_t ldc) {
     if (n <= 0 || k <= 0) return OMX_OK;
-    ctx->gemm_sym = true;
+    ctx->gemm_sym = 1;
     const int rc = launch_gemm(ctx, OMX_PREC_F64, OMX_F64, false, true, n, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
-    ctx->gemm_sym = false;
+    ctx->gemm_sym = 0;
     return rc;
 }
 

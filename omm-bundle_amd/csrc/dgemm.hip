@@ -1,0 +1,426 @@
+// FP64 products C := alpha * sum_p op(A_p) op(B_p) + beta0*C0 + beta*C on the FP64 matrix cores, with the
+// operands loaded straight into LDS, for every m, n, k and every leading dimension up to 2^20 (NPAIR = 2:
+// calc_G's two products back to back along K).
+//
+// Staging.  K is taken in slices of 16.  An operand whose row index is contiguous (A 'n', B 't') lands
+// k-major: ROWS doubles per k-row, 128 / ROWS k-rows per wave load.  One whose k is contiguous (A 't',
+// B 'n') lands row-major: 16 k values (128 bytes) per row, 8 rows per wave load, logical 16-byte chunk c
+// of row r at physical chunk c ^ ((r >> 1) & 7).  A wave load is one buffer_load_dwordx4 ... lds, 16 bytes
+// per lane, lane l landing at byte 16*l.  The descriptors are rebased at every slice, so a lane's byte
+// offset is the same for every slice, and they end exactly where the matrix ends: the hardware's range
+// check is per dword, so anything past the last element arrives as zero and an odd size, an odd leading
+// dimension or an 8-byte aligned operand needs no other path.  Rows past m or n inside the matrix only
+// feed results that are not stored.  k past the end of a k-contiguous row would be the next row's
+// values; the last slice clears those in LDS before they are read.
+//
+// What bounds it: the FP64 matrix core (64 cycles per 16x16x4 step and SIMD), except where the result has
+// fewer tiles than the chip has CUs; there it is the serial chain of slices of one tile, and below that
+// the launch.  Before, only m, n % 128 == 0 with k % 16 == 0 took this path and everything else was staged
+// through registers in 128x128 tiles: 54 x 54 x 108 22 us (now 5.5), 432 x 432 x 864 about 35 us (16),
+// 1458 x 1458 x 2916 340 us (236), 4394 x 4394 x 8788 5.84 ms (5.17), gradient of 2662 x 5324 2.96 ms (2.32).
+//
+// Tiles.  Three tile sizes with the same K chain per element (K in order, so the results do not depend
+// on the tile): 128x128 (8 waves of 32x64, two stages), 64x64 (4 waves of 32x32, three stages) and 32x32
+// (4 waves of 16x16, two stages of four slices: a lone tile's slice takes 0.16 us, with one-slice stages
+// 0.34 us, because the barrier and the first LDS read are paid once per stage).  Stage s+NST-1 is issued while stage s feeds the MFMAs, one barrier
+// per slice; waves whose sub-tile lies outside the result (or, for a symmetric product, above the
+// diagonal) take part in the loads and barriers only.
+#include <algorithm>
+
+#include "omx_internal.h"
+#include "omx_mfma.h"
+
+namespace omx {
+
+constexpr int DK = 16;  // K slice
+
+// Byte offset of lane `lane` of wave load `ins` of an operand tile (ROWS rows x DK) from the slice's
+// descriptor base.  KC: k contiguous.
+template <int ROWS, bool KC>
+__device__ inline int dl_voff(int ins, int lane, int ld) {
+    if constexpr (KC) {
+        const int r = ins * 8 + (lane >> 3);
+        return 8 * (r * ld + 2 * ((lane & 7) ^ dl_swz(r)));
+    } else {
+        constexpr int LPR = ROWS / 2;  // lanes per k-row
+        return 8 * ((ins * (64 / LPR) + lane / LPR) * ld + 2 * (lane % LPR));
+    }
+}
+// The element (row r, k kk) of a staged tile; dl_at: its place in a k-contiguous one.
+__device__ inline int dl_at(int r, int kk) { return r * DK + (((kk >> 1) ^ dl_swz(r)) << 1) + (kk & 1); }
+template <int ROWS, bool KC>
+__device__ inline double dl_elem(const double *t, int r, int kk) {
+    return t[KC ? dl_at(r, kk) : kk * ROWS + r];
+}
+// Start of an operand tile (row i0, k 0), and the bytes from there to the end of the operand (extent rows
+// x k, leading dimension ld).
+template <bool KC>
+__device__ inline const char *dl_base(const double *P, int i0, int64_t ld) {
+    return (const char *)(P + (KC ? (int64_t)i0 * ld : i0));
+}
+template <bool KC>
+__device__ inline int64_t dl_left(int extent, int k, int i0, int64_t ld) {
+    return 8 * (KC ? (int64_t)(extent - 1 - i0) * ld + k : (int64_t)(k - 1) * ld + (extent - i0));
+}
+
+// EXACT: m, n are multiples of the tile and k of the slice, so nothing needs the descriptors' end, a
+// cleared tail or guarded stores; the 128x128 tile is faster without them (8192 x 8192 x 16384 Gram 29.8
+// against 29.9 ms, gradient 60.4 against 61.6 ms).
+template <class CF, bool TRA, bool TRB, int NPAIR, bool EXACT>
+__global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int k, double alpha,
+                                                               const double *__restrict__ A1,
+                                                               const double *__restrict__ A2, int64_t lda,
+                                                               const double *__restrict__ B1,
+                                                               const double *__restrict__ B2, int64_t ldb,
+                                                               double beta0, const double *__restrict__ C0,
+                                                               double beta, double *__restrict__ C, int64_t ldc,
+                                                               int sym, int tbase, int nsplit, int sps,
+                                                               double *__restrict__ partial,
+                                                               const int *__restrict__ mask) {
+    constexpr int BM = CF::BM, BN = CF::BN, NST = CF::NST, NW = CF::WGM * CF::WGN;
+    constexpr int INS = DK * (BM + BN) / 128, LPW = INS / NW, U = CF::U;
+    constexpr int SLICE = DK * (BM + BN), STAGE = U * SLICE;
+    constexpr bool KCA = TRA, KCB = !TRB;
+    static_assert(LPW * NW == INS && BM == BN && NW % 2 == 0, "each wave loads one operand");
+    __shared__ __align__(16) double smem[NST * STAGE];
+    if (mask && !*mask) return;  // system masked off (grouped solver; whole workgroup, before any barrier)
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave / CF::WGN, wn = wave % CF::WGN;
+    // tile w of the launch's tile order and the part z of K it takes
+    const int w = tbase + (int)blockIdx.x / nsplit, z = (int)blockIdx.x % nsplit;
+    int tm, tn;
+    if (sym)
+        tile_of_lower(w, (m + BM - 1) / BM, tm, tn);
+    else
+        tile_of(w, (m + BM - 1) / BM, (n + BN - 1) / BN, tm, tn);
+    const int i0 = tm * BM, j0 = tn * BN;
+    const int wi = i0 + wm * CF::WM, wj = j0 + wn * CF::WN;
+    const bool live = wi < m && wj < n && !(sym && wj > wi + CF::WM - 1);
+    const int nsl = (k + DK - 1) / DK;  // slices of one product
+    const int sb = z * sps, ns = min(NPAIR * nsl, sb + sps) - sb;
+
+    d4v acc[CF::FBM][CF::FBN];
+#pragma unroll
+    for (int a = 0; a < CF::FBM; ++a)
+#pragma unroll
+        for (int b = 0; b < CF::FBN; ++b) acc[a][b] = d4v{0, 0, 0, 0};
+    // The first half of the waves loads A, the second half B.  Slices are issued in order: the wave's
+    // descriptor advances by one slice each time, and starts over at the second product of a pair.
+    const bool on_b = wave >= NW / 2;
+    const int ins0 = (on_b ? wave - NW / 2 : wave) * LPW;
+    int voff[LPW];
+#pragma unroll
+    for (int q = 0; q < LPW; ++q)
+        voff[q] = on_b ? dl_voff<BN, KCB>(ins0 + q, lane, (int)ldb) : dl_voff<BM, KCA>(ins0 + q, lane, (int)lda);
+    const int64_t step = 8 * (on_b ? (KCB ? DK : DK * ldb) : (KCA ? DK : DK * lda));
+    const int64_t all = on_b ? dl_left<KCB>(n, k, j0, ldb) : dl_left<KCA>(m, k, i0, lda);
+    const char *const first = on_b ? dl_base<KCB>(B1, j0, ldb) : dl_base<KCA>(A1, i0, lda);
+    const char *const second = on_b ? dl_base<KCB>(B2, j0, ldb) : dl_base<KCA>(A2, i0, lda);
+    const int sb_in = NPAIR == 2 && sb >= nsl ? sb - nsl : sb;
+    const char *pos = (NPAIR == 2 && sb >= nsl ? second : first) + sb_in * step;
+    int64_t left = all - sb_in * step;
+    // slice (of this part) where the second product starts; the last slice of each product if it is partial
+    const int sw = nsl - sb, t1 = k % DK ? sw - 1 : -1, t2 = NPAIR == 2 && k % DK ? sw + nsl - 1 : -1;
+    auto issue = [&](int s) {  // the U slices of stage s
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int sl = s * U + u;
+            if (U > 1 && sl >= ns) break;
+            double *st = smem + (s % NST) * STAGE + u * SLICE + wave * LPW * 128;
+            if (NPAIR == 2 && sl == sw) {
+                pos = second;
+                left = all;
+            }
+            const __amdgpu_buffer_rsrc_t r = raw_rsrc(pos, EXACT || (uint32_t)((uint64_t)left >> 31) ? 0x7ffffff8 : (int)left);
+            pos += step;
+            left -= step;
+#pragma unroll
+            for (int q = 0; q < LPW; ++q) {
+                const int vo = voff[q];  // (a local: see k_bgemm_tn)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(st + q * 128), 16, vo, 0, 0, 0);
+            }
+        }
+    };
+    const int li = lane & 15, lk = lane >> 4;
+    // one slice: the fragments of k step ks + 4 are read before the MFMAs of step ks
+    auto slice = [&](const double *As, const double *Bs) {
+        double a[2][CF::FBM], b[2][CF::FBN];
+        auto frag = [&](int ks, double (&fa)[CF::FBM], double (&fb)[CF::FBN]) {
+            const int kk = ks + lk;
+#pragma unroll
+            for (int f = 0; f < CF::FBM; ++f) fa[f] = dl_elem<BM, KCA>(As, wm * CF::WM + f * 16 + li, kk);
+#pragma unroll
+            for (int f = 0; f < CF::FBN; ++f) fb[f] = dl_elem<BN, KCB>(Bs, wn * CF::WN + f * 16 + li, kk);
+        };
+        frag(0, a[0], b[0]);
+#pragma unroll
+        for (int ks = 0; ks < DK; ks += 4) {
+            const int cur = (ks / 4) & 1;
+            if (ks + 4 < DK) frag(ks + 4, a[cur ^ 1], b[cur ^ 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int fm = 0; fm < CF::FBM; ++fm)
+#pragma unroll
+                for (int fn = 0; fn < CF::FBN; ++fn)  // (b, a): the result's columns run along i
+                    acc[fm][fn] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[cur][fn], a[cur][fm], acc[fm][fn], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    const int nst = (ns + U - 1) / U, nfull = ns / U;  // stages, and those with all their slices
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+        if (s < nst) issue(s);
+    auto march = [&](auto work) {  // waves outside the result only load, clear and wait
+        for (int s = 0; s < nst; ++s) {
+            // this wave's loads of stage s have landed (the NST - 2 later stages stay in flight)
+            if (NST > 2 && s + NST - 2 < nfull)
+                __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt(LPW * U * (NST - 2)));
+            else
+                __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt(0));
+            wg_barrier();  // everyone's have; stage s-1 is no longer read
+            if (s + NST - 1 < nst) issue(s + NST - 1);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int sl = s * U + u;
+                if (U > 1 && sl >= ns) break;
+                double *As = smem + (s % NST) * STAGE + u * SLICE, *Bs = As + DK * BM;
+                if (!EXACT && (KCA || KCB) && (sl == t1 || (NPAIR == 2 && sl == t2))) {  // k-contiguous rows end at k
+                    if (KCA)
+                        for (int e = t; e < BM * DK; e += CF::NT)
+                            if (e % DK >= k % DK) As[dl_at(e / DK, e % DK)] = 0.0;
+                    if (KCB)
+                        for (int e = t; e < BN * DK; e += CF::NT)
+                            if (e % DK >= k % DK) Bs[dl_at(e / DK, e % DK)] = 0.0;
+                    wg_barrier();
+                }
+                if (decltype(work)::value) slice(As, Bs);
+            }
+        }
+    };
+    if (!live) {
+        march(std::false_type{});
+        return;
+    }
+    march(std::true_type{});
+    const int lq = lane >> 4;
+    if (partial) {  // a K part of a split tile: the raw sums, reduced in part order later
+        double *pt = partial + (int64_t)blockIdx.x * (BM * BN);
+#pragma unroll
+        for (int fm = 0; fm < CF::FBM; ++fm)
+#pragma unroll
+            for (int fn = 0; fn < CF::FBN; ++fn)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    pt[(wm * CF::WM + fm * 16 + li) + (wn * CF::WN + fn * 16 + lq + 4 * v) * BM] = acc[fm][fn][v];
+        return;
+    }
+#pragma unroll
+    for (int fm = 0; fm < CF::FBM; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < CF::FBN; ++fn) {
+            const int i = wi + fm * 16 + li;
+            if (!EXACT && i >= m) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int j = wj + fn * 16 + lq + 4 * v;
+                if ((!EXACT && j >= n) || (sym && j > i)) continue;
+                double r = alpha * acc[fm][fn][v];
+                if (C0) r += beta0 * C0[(int64_t)i + (int64_t)j * ldc];
+                if (beta != 0.0) r += beta * C[(int64_t)i + (int64_t)j * ldc];
+                C[(int64_t)i + (int64_t)j * ldc] = r;
+                if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = r;
+            }
+        }
+}
+
+// C tile := alpha * (sum of its nsplit K parts, in part order) + beta0*C0 + beta*C for the tiles tbase..
+// of the launch's tile order (blockIdx.x: tile, blockIdx.y: a 1024-element slice of it).
+template <int BM, int BN>
+__global__ __launch_bounds__(256) void k_dl_split_reduce(int m, int n, int sym, int tbase, int nsplit,
+                                                         const double *__restrict__ partial, double alpha,
+                                                         double beta0, const double *__restrict__ C0, double beta,
+                                                         double *__restrict__ C, int64_t ldc) {
+    int tm, tn;
+    if (sym)
+        tile_of_lower(tbase + (int)blockIdx.x, (m + BM - 1) / BM, tm, tn);
+    else
+        tile_of(tbase + (int)blockIdx.x, (m + BM - 1) / BM, (n + BN - 1) / BN, tm, tn);
+    const double *pt = partial + (int64_t)blockIdx.x * nsplit * (BM * BN);
+    const int e0 = blockIdx.y * 1024;
+    for (int e = e0 + threadIdx.x; e < e0 + 1024; e += 256) {
+        const int i = tm * BM + e % BM, j = tn * BN + e / BM;
+        if (i >= m || j >= n || (sym && j > i)) continue;  // (parts above the diagonal are not written)
+        double sum = 0.0;
+        for (int zz = 0; zz < nsplit; ++zz) sum += pt[(int64_t)zz * (BM * BN) + e];
+        const int64_t off = (int64_t)i + (int64_t)j * ldc;
+        double r = alpha * sum;
+        if (C0) r += beta0 * C0[off];
+        if (beta != 0.0) r += beta * C[off];
+        C[off] = r;
+        if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = r;
+    }
+}
+
+template <int BM_, int BN_, int WGM_, int WGN_, int MINW_, int NST_, int U_>
+struct DlCfg {
+    static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, MINW = MINW_, U = U_;
+    static constexpr int NT = 64 * WGM * WGN, WM = BM / WGM, WN = BN / WGN, FBM = WM / 16, FBN = WN / 16;
+};
+typedef DlCfg<128, 128, 4, 2, 4, 2, 1> Dl128;
+typedef DlCfg<64, 64, 2, 2, 2, 3, 1> Dl64;
+typedef DlCfg<32, 32, 2, 2, 2, 2, 4> Dl32;
+
+static int tiles_of(int m, int n, int b, bool sym) {
+    const int tm = (m + b - 1) / b, tn = (n + b - 1) / b;
+    return sym ? tm * (tm + 1) / 2 : tm * tn;
+}
+
+// Time of a product by tile and by the parts K is split into, in microseconds: rounds of workgroups over
+// the CUs (workgroups that share a CU share its matrix cores) times the slices of a part, plus what a launch,
+// a round and the reduction of the parts cost.  The constants are a least-squares fit to 60 shapes (54 x 54
+// x 108 to 4394 x 4394 x 8788, Grams, symmetric Grams and pairs; every tile and 1 to 12 parts): 11 % rms, and
+// the choices they lead to are within 1.6 % of the fastest of all on average.
+// A symmetric product in 128x128 tiles whose last round of resident workgroups (two per CU) is not full:
+// the parts along K that each tile of that round is split into (1: it is not split).  Only for orders
+// that are multiples of 128; elsewhere the symmetric form adds exactly as the full product does.
+static int dl_tail_parts(omx_ctx ctx, int m, int tiles, bool sym, int nsl) {
+    const int slots = 2 * ctx->num_cus, rest = tiles % slots;
+    if (!sym || m % 128 || ctx->launch_mask || tiles < slots || !rest) return 1;
+    int parts = std::max(1, std::min(16, slots / rest));
+    while (parts > 1 && nsl % parts) --parts;
+    return parts;
+}
+static const int kDlEdge[3] = {128, 64, 32};
+static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int splits) {
+    const double slice[3] = {1.90, 0.515, 0.172};  // a CU's time for one 16-wide slice of a tile
+    const double alone[3] = {2.15, 0.69, 0.172};   // the same with a single workgroup on the CU
+    const int units = tiles_of(m, n, kDlEdge[q], sym) * splits, rounds = (units + ctx->num_cus - 1) / ctx->num_cus;
+    const int sps = (nsl + splits - 1) / splits;
+    const int tail = dl_tail_parts(ctx, q == 0 && splits == 1 ? m : 1, units, sym, nsl);
+    if (tail > 1) {
+        const int whole = units / (2 * ctx->num_cus) * 2;  // two workgroups of every round share a CU
+        return 9.8 + 0.55 * whole + slice[q] * (whole * sps + 2.0 * sps / tail);
+    }
+    return 4.5 + 0.55 * rounds + std::max(slice[q] * rounds, alone[q]) * sps +
+           (splits > 1 ? 5.3 + 8e-6 * (splits + 1) * m * n / 4.9 : 0.0);
+}
+static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, double *cost = nullptr) {
+    int best = 0;
+    double c = 0.0;
+    for (int q = 0; q < 3; ++q) {
+        const double t = dl_cost(ctx, q, sym, m, n, nsl, splits);
+        if (!q || t < c) {
+            best = q;
+            c = t;
+        }
+    }
+    if (cost) *cost = c;
+    return best;
+}
+
+// The number of parts with the least time; for a square result that of the full and the symmetric form
+// together, so that both add the same parts.
+int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl) {
+    if (ctx->launch_mask) return 1;
+    int best = 1;
+    double cost = 0.0;
+    for (int s : {1, 2, 3, 4, 5, 6, 8, 12}) {
+        if (s > 1 && nsl < 2 * s) break;
+        double t, u = 0.0;
+        dl_tile(ctx, false, m, n, nsl, s, &t);
+        if (m == n) dl_tile(ctx, true, m, n, nsl, s, &u);
+        if (s == 1 || t + u < cost) {
+            best = s;
+            cost = t + u;
+        }
+    }
+    return best;
+}
+
+template <class CF, bool TRA, bool TRB, int NPAIR>
+static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int k, double alpha, const double *A1,
+                    const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
+                    const double *C0, double beta, double *C, int64_t ldc) {
+    const int tiles = tiles_of(m, n, CF::BM, sym != 0);
+    const int nsl = NPAIR * ((k + DK - 1) / DK);
+    int whole = tiles, rest = 0, rsplit = 1;
+    if (splits > 1) {
+        whole = 0;
+        rest = tiles;
+        rsplit = splits;
+    } else if (CF::BM == 128 && (rsplit = dl_tail_parts(ctx, m, tiles, sym != 0, nsl)) > 1) {
+        rest = tiles % (2 * ctx->num_cus);
+        whole = tiles - rest;
+        sps = nsl / rsplit;
+    }
+    auto launch = [&](int grid, int tbase, int parts, int per, double *partial, const int *mask) {
+        if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
+            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, CF::BM == 128>), dim3(grid), dim3(CF::NT), 0, ctx->stream,
+                               m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, sym, tbase, parts, per,
+                               partial, mask);
+        else
+            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, false>), dim3(grid), dim3(CF::NT), 0, ctx->stream, m, n,
+                               k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, sym, tbase, parts, per,
+                               partial, mask);
+    };
+    if (whole) launch(whole, 0, 1, nsl, nullptr, ctx->launch_mask);
+    if (rest) {
+        int rc = ensure_ws(ctx, sizeof(double) * (size_t)rest * rsplit * CF::BM * CF::BN);
+        if (rc) return rc;
+        launch(rest * rsplit, whole, rsplit, sps, (double *)ctx->ws, nullptr);
+        hipLaunchKernelGGL((k_dl_split_reduce<CF::BM, CF::BN>), dim3(rest, CF::BM * CF::BN / 1024), dim3(256), 0,
+                           ctx->stream, m, n, sym, whole, rsplit, (const double *)ctx->ws, alpha, beta0, C0, beta, C,
+                           ldc);
+    }
+    OMX_CHECK_HIP(hipGetLastError());
+    return OMX_OK;
+}
+
+template <bool TRA, bool TRB, int NPAIR>
+static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const double *A1, const double *A2, int64_t lda,
+                   const double *B1, const double *B2, int64_t ldb, double beta0, const double *C0, double beta,
+                   double *C, int64_t ldc) {
+    const int sym = (m == n && NPAIR == 1 && !TRA && TRB) ? ctx->gemm_sym : 0;
+    const int nsl = NPAIR * ((k + DK - 1) / DK);
+    int splits = dgemm_k_splits(ctx, m, n, nsl);
+    const int sps = (nsl + splits - 1) / splits;
+    splits = (nsl + sps - 1) / sps;
+    const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM;
+    const int tile = dl_tile(ctx, sym != 0, m, n, nsl, splits);
+    hipEvent_t ev;
+    prof_begin(ctx, cls, &ev);
+    prof_work(ctx, cls, 2.0 * (sym ? sym_area(m, kDlEdge[tile]) : (double)m * n) * (double)NPAIR * k,
+              sizeof(double) * ((double)NPAIR * ((double)m * k + (double)k * n) +
+                                (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
+    int rc;
+#define OMX_DL_RUN(CF) \
+    run_tile<CF, TRA, TRB, NPAIR>(ctx, sym, splits, sps, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc)
+    if (tile == 0)
+        rc = OMX_DL_RUN(Dl128);
+    else if (tile == 1)
+        rc = OMX_DL_RUN(Dl64);
+    else
+        rc = OMX_DL_RUN(Dl32);
+#undef OMX_DL_RUN
+    prof_end(ctx, cls, ev);
+    if (!rc && sym == 2) ctx->gemm_sym = 3;  // the upper triangle is written too
+    return rc;
+}
+
+int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const double *A1,
+                 const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
+                 const double *C0, double beta, double *C, int64_t ldc) {
+    if (m <= 0 || n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20))  // 32-bit lane offsets
+        return OMX_ERR_UNSUPPORTED;
+    if (npair == 2)
+        return run_ops<false, false, 2>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
+    if (!trA && !trB)
+        return run_ops<false, false, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
+    if (!trA && trB)
+        return run_ops<false, true, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
+    if (trA && !trB)
+        return run_ops<true, false, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
+    return run_ops<true, true, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
+}
+
+}  // namespace omx

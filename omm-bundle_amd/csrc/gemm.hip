@@ -22,12 +22,9 @@
 #include <type_traits>
 
 #include "omx_internal.h"
+#include "omx_mfma.h"
 
 namespace omx {
-
-typedef double d4v __attribute__((ext_vector_type(4)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef __bf16 bf8v __attribute__((ext_vector_type(8)));
 
 // ---------------------------------------------------------------------------------------------
 // Precision traits: K slice, LDS element type, accumulator type and result lane layout.
@@ -394,250 +391,6 @@ __global__ void k_splitk_reduce(int m, int n, int splits, const AT *__restrict__
 
 static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
-// Output area (elements) of the lower-triangle tiles of an n x n product with bm x bm tiles: the
-// flop count of a symmetric product is 2*k times this (the MFMA work actually issued).
-static double sym_area(int n, int bm) {
-    double area = 0.0;
-    for (int a = 0; a * bm < n; ++a) area += (double)std::min(bm, n - a * bm) * std::min(n, (a + 1) * bm);
-    return area;
-}
-
-// ---------------------------------------------------------------------------------------------
-// FP64 products with direct-to-LDS staging (configuration 7): C := alpha*sum_p A_p*op(B_p) + beta0*C0
-// + beta*C over NPAIR products back to back along K (the Gram: NPAIR = 1, op 't'; calc_G's pair:
-// NPAIR = 2, op 'n'; single 'n','n' products: NPAIR = 1, op 'n').  A is m x k with the row index
-// contiguous, so every k-row of a 128-wide tile is 1 KB, which one wave moves with one
-// buffer_load_dwordx4 ... lds (16 bytes per lane, lane l landing at byte 16*l of the destination)
-// straight into the k-major LDS tile.  The descriptors are rebased at each slice, so the lanes'
-// byte offsets are small and fixed; the buffer form keeps the compiler's LDS waits counted (see
-// k_bgemm_tn), and the fragments of k step ks + 4 are read before the MFMAs of step ks.
-//   B 't' (n x k, row index contiguous): the same k-major rows.
-//   B 'n' (k x n, k contiguous): a j-major tile, one 128-byte row of 16 k values per column j, 8
-//   columns per wave load.  Logical 16-byte chunk c of column j is stored at physical chunk
-//   c ^ ((j >> 1) & 7).  A fragment read takes one k of 16 columns, 8 bytes at the same place in
-//   16 different 16-byte chunks, so it spans at most 8 of the 16-byte bank groups: two-way bank
-//   conflicts that no placement of whole chunks avoids (measured: conflict cycles on 40 % of the
-//   LDS-active cycles with this swizzle and with c ^ (j & 7); none on the 't' path).
-// No staging registers and no LDS write instructions; two LDS stages, the loads of slice s+1 in
-// flight while slice s feeds the MFMAs.  Tiles, waves and the MFMA chain per element are those of
-// the staged kernel with Cfg5, so the results are bitwise the same.  Requires m, n % 128 == 0,
-// k % 16 == 0, even leading dimensions and 16-byte aligned operands.
-// ---------------------------------------------------------------------------------------------
-typedef __attribute__((address_space(3))) void lds_void;
-// s_waitcnt immediate (gfx9 encoding): vmcnt(vm), expcnt and lgkmcnt left at their maxima
-constexpr int waitcnt_vmcnt(int vm) { return (vm & 0xF) | ((vm >> 4) << 14) | (7 << 4) | (0xF << 8); }
-__device__ inline int dl_swz(int j) { return (j >> 1) & 7; }
-// Raw (unstrided) buffer descriptor over `bytes` bytes from p, for the buffer loads into LDS of
-// the direct-to-LDS products; word 3 is gfx9's for 32-bit data without swizzling.  Reads at or
-// past `bytes` return zero instead of touching memory.
-template <typename T>
-__device__ inline __amdgpu_buffer_rsrc_t raw_rsrc(const T *p, int bytes = 0x7fffffff) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(p), (short)0, bytes, 0x00020000);
-}
-
-template <class CF, bool TRB, int NPAIR>
-__global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int k, double alpha,
-                                                               const double *__restrict__ A1,
-                                                               const double *__restrict__ A2, int64_t lda,
-                                                               const double *__restrict__ B1,
-                                                               const double *__restrict__ B2, int64_t ldb,
-                                                               double beta0, const double *__restrict__ C0,
-                                                               double beta, double *__restrict__ C, int64_t ldc,
-                                                               int sym, int tbase, int nsplit,
-                                                               double *__restrict__ partial,
-                                                               const int *__restrict__ mask) {
-    static_assert(CF::BM == 128 && CF::BN == 128, "one 1 KB row per wave load");
-    if (mask && !*mask) return;  // system masked off (grouped solver; whole workgroup, before any barrier)
-    constexpr int BK = Prec<OMX_PREC_F64>::BK, NW = CF::WGM * CF::WGN, INS = 2 * BK, LPW = INS / NW;
-    constexpr int STAGE = INS * 128;  // doubles: A rows (BK x 128), then B (BK x 128 or 128 x BK)
-    static_assert(LPW * NW == INS, "loads per wave");
-    __shared__ double smem[2 * STAGE];
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int wm = wave / CF::WGN, wn = wave % CF::WGN;
-    // tile w of the launch's tile order and, with nsplit > 1, the part z of K it takes
-    const int w = tbase + (int)blockIdx.x / nsplit, z = (int)blockIdx.x % nsplit;
-    int tm, tn;
-    if (sym)
-        tile_of_lower(w, m / 128, tm, tn);
-    else
-        tile_of(w, m / 128, n / 128, tm, tn);
-    const int i0 = tm * 128, j0 = tn * 128;
-    d4v acc[CF::FBM][CF::FBN];
-#pragma unroll
-    for (int a = 0; a < CF::FBM; ++a)
-#pragma unroll
-        for (int b = 0; b < CF::FBN; ++b) acc[a][b] = d4v{0, 0, 0, 0};
-    const int kpart = NPAIR * k / nsplit, s0 = z * (kpart / BK);  // this part's first slice
-    // Each lane's byte offset from its slice's descriptor base (A + i0 + kl*lda; B 't': B + j0 +
-    // kl*ldb; B 'n': B + j0*ldb + kl), the same for every slice.
-    const int uwave = __builtin_amdgcn_readfirstlane(wave);
-    int voff[LPW];
-#pragma unroll
-    for (int q = 0; q < LPW; ++q) {
-        const int ins = uwave * LPW + q;  // < BK: row k of A; else the B part
-        if (ins < BK) {
-            voff[q] = 8 * (2 * lane + ins * (int)lda);
-        } else if (TRB) {
-            voff[q] = 8 * (2 * lane + (ins - BK) * (int)ldb);
-        } else {
-            const int j = (ins - BK) * 8 + (lane >> 3);  // column of the tile
-            const int c = (lane & 7) ^ dl_swz(j);         // logical chunk this lane holds
-            voff[q] = 8 * (j * (int)ldb + 2 * c);
-        }
-    }
-    auto issue = [&](int s) {
-        double *st = smem + (s & 1) * STAGE;
-        int kl = (s0 + s) * BK;
-        const double *A = A1, *B = B1;
-        if (NPAIR == 2 && kl >= k) {
-            A = A2;
-            B = B2;
-            kl -= k;
-        }
-        const __amdgpu_buffer_rsrc_t ra = raw_rsrc(A + i0 + (int64_t)kl * lda);
-        const __amdgpu_buffer_rsrc_t rb = raw_rsrc(TRB ? B + j0 + (int64_t)kl * ldb : B + (int64_t)j0 * ldb + kl);
-#pragma unroll
-        for (int q = 0; q < LPW; ++q) {
-            const int ins = uwave * LPW + q;
-            const int vo = voff[q];  // (a local: see k_bgemm_tn)
-            if (ins < BK)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_void *)(st + ins * 128), 16, vo, 0, 0, 0);
-            else
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void *)(st + ins * 128), 16, vo, 0, 0, 0);
-        }
-    };
-    const int li = lane & 15, lk = lane >> 4;
-    const int ns = kpart / BK;
-    issue(0);
-    for (int s = 0; s < ns; ++s) {
-        __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt(0));  // this wave's rows of slice s have landed
-        __syncthreads();                               // everyone's have; slice s-1 is no longer read
-        if (s + 1 < ns) issue(s + 1);
-        const double *As = smem + (s & 1) * STAGE, *Bs = As + BK * 128;
-        // the fragments of k step ks + 4 are read before the MFMAs of step ks
-        double a[2][CF::FBM], b[2][CF::FBN];
-        auto frag = [&](int ks, double (&fa)[CF::FBM], double (&fb)[CF::FBN]) {
-#pragma unroll
-            for (int f = 0; f < CF::FBM; ++f) fa[f] = As[(ks + lk) * 128 + wm * CF::WM + f * 16 + li];
-#pragma unroll
-            for (int f = 0; f < CF::FBN; ++f) {
-                const int j = wn * CF::WN + f * 16 + li, kk = ks + lk;
-                fb[f] = TRB ? Bs[kk * 128 + j] : Bs[j * BK + ((kk >> 1) ^ dl_swz(j)) * 2 + (kk & 1)];
-            }
-        };
-        frag(0, a[0], b[0]);
-#pragma unroll
-        for (int ks = 0; ks < BK; ks += 4) {
-            const int cur = (ks / 4) & 1;
-            if (ks + 4 < BK) frag(ks + 4, a[cur ^ 1], b[cur ^ 1]);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int fm = 0; fm < CF::FBM; ++fm)
-#pragma unroll
-                for (int fn = 0; fn < CF::FBN; ++fn)
-                    acc[fm][fn] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[cur][fm], b[cur][fn], acc[fm][fn], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    const int lq = lane >> 4;
-    if (partial) {  // a K part of a split tile: the raw sums, reduced in part order later
-        double *pt = partial + (int64_t)blockIdx.x * (128 * 128);
-#pragma unroll
-        for (int fm = 0; fm < CF::FBM; ++fm)
-#pragma unroll
-            for (int fn = 0; fn < CF::FBN; ++fn)
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    pt[(wm * CF::WM + fm * 16 + Prec<OMX_PREC_F64>::out_row(lq, v)) +
-                       (wn * CF::WN + fn * 16 + li) * 128] = acc[fm][fn][v];
-        return;
-    }
-#pragma unroll
-    for (int fm = 0; fm < CF::FBM; ++fm)
-#pragma unroll
-        for (int fn = 0; fn < CF::FBN; ++fn) {
-            const int j = j0 + wn * CF::WN + fn * 16 + li;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = i0 + wm * CF::WM + fm * 16 + Prec<OMX_PREC_F64>::out_row(lq, v);
-                double r = alpha * acc[fm][fn][v];
-                if (C0) r += beta0 * C0[(int64_t)i + (int64_t)j * ldc];
-                if (beta != 0.0) r += beta * C[(int64_t)i + (int64_t)j * ldc];
-                C[(int64_t)i + (int64_t)j * ldc] = r;
-            }
-        }
-}
-
-// C tile := alpha * (sum of its nsplit K parts, in part order) + beta0*C0 + beta*C for the split
-// tiles tbase.. of a symmetric product's lower-triangle order (blockIdx.x: tile, blockIdx.y: a
-// 1024-element slice of it).
-__global__ __launch_bounds__(256) void k_dl_split_reduce(int n, int tbase, int nsplit, const double *__restrict__ partial,
-                                                         double alpha, double beta0, const double *__restrict__ C0,
-                                                         double beta, double *__restrict__ C, int64_t ldc) {
-    int tm, tn;
-    tile_of_lower(tbase + (int)blockIdx.x, n / 128, tm, tn);
-    const double *pt = partial + (int64_t)blockIdx.x * nsplit * (128 * 128);
-    const int e0 = blockIdx.y * 1024;
-    for (int e = e0 + threadIdx.x; e < e0 + 1024; e += 256) {
-        double sum = 0.0;
-        for (int zz = 0; zz < nsplit; ++zz) sum += pt[(int64_t)zz * (128 * 128) + e];
-        const int64_t off = (int64_t)(tm * 128 + e % 128) + (int64_t)(tn * 128 + e / 128) * ldc;
-        double r = alpha * sum;
-        if (C0) r += beta0 * C0[off];
-        if (beta != 0.0) r += beta * C[off];
-        C[off] = r;
-    }
-}
-
-// Launches configuration 7 when the product qualifies; returns OMX_ERR_UNSUPPORTED otherwise.
-// A symmetric product's tiles that do not fill a whole round of resident workgroups (two per CU)
-// are split along K over up to 16 workgroups each and reduced in part order, so the round that
-// would hold only them costs a fraction of a tile.
-template <bool TRB, int NPAIR>
-static int run_dgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const double *A1, const double *A2,
-                        int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0, const double *C0,
-                        double beta, double *C, int64_t ldc) {
-    typedef Cfg5 CF;
-    const bool sym = ctx->gemm_sym && m == n && NPAIR == 1;
-    const int tiles = sym ? (m / 128) * (m / 128 + 1) / 2 : (m / 128) * (n / 128);
-    if (m <= 0 || n <= 0 || k <= 0 || m % 128 || n % 128 || k % Prec<OMX_PREC_F64>::BK || lda % 2 || ldb % 2 ||
-        !aligned16(A1) || !aligned16(A2) || !aligned16(B1) || !aligned16(B2) || tiles < 2 * ctx->num_cus ||
-        lda > (1 << 20) || ldb > (1 << 20))  // 32-bit lane offsets from the slice descriptors
-        return OMX_ERR_UNSUPPORTED;
-    const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM;
-    hipEvent_t ev;
-    prof_begin(ctx, cls, &ev);
-    prof_work(ctx, cls, 2.0 * (sym ? sym_area(m, 128) : (double)m * n) * (double)NPAIR * k,
-              sizeof(double) * ((double)NPAIR * ((double)m * k + (double)k * n) +
-                                (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
-    const int slots = 2 * ctx->num_cus;
-    const int whole = sym ? tiles / slots * slots : tiles, rest = tiles - whole;
-    int nsplit = 1;
-    if (rest > 0 && !ctx->launch_mask) {  // masked (grouped, captured) launches use no workspace
-        nsplit = std::max(1, std::min(16, slots / rest));
-        while (nsplit > 1 && (k / Prec<OMX_PREC_F64>::BK) % nsplit) --nsplit;
-    }
-    if (rest > 0 && nsplit > 1) {
-        int rc = ensure_ws(ctx, sizeof(double) * (size_t)rest * nsplit * 128 * 128);
-        if (rc) return rc;
-        hipLaunchKernelGGL((k_dgemm_dl<CF, TRB, NPAIR>), dim3(whole), dim3(CF::NT), 0, ctx->stream, m, n, k, alpha, A1,
-                           A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, (int)sym, 0, 1, (double *)nullptr,
-                           (const int *)nullptr);
-        hipLaunchKernelGGL((k_dgemm_dl<CF, TRB, NPAIR>), dim3(rest * nsplit), dim3(CF::NT), 0, ctx->stream, m, n, k,
-                           alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, (int)sym, whole, nsplit,
-                           (double *)ctx->ws, (const int *)nullptr);
-        hipLaunchKernelGGL(k_dl_split_reduce, dim3(rest, 128 * 128 / 1024), dim3(256), 0, ctx->stream, m, whole, nsplit,
-                           (const double *)ctx->ws, alpha, beta0, C0, beta, C, ldc);
-    } else {
-        hipLaunchKernelGGL((k_dgemm_dl<CF, TRB, NPAIR>), dim3(tiles), dim3(CF::NT), 0, ctx->stream, m, n, k, alpha, A1,
-                           A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, (int)sym, 0, 1, (double *)nullptr,
-                           ctx->launch_mask);
-    }
-    prof_end(ctx, cls, ev);
-    OMX_CHECK_HIP(hipGetLastError());
-    return OMX_OK;
-}
-
 // ---------------------------------------------------------------------------------------------
 // FP32 Gram C := alpha*A*B^T + beta0*C0 + beta*C with direct-to-LDS staging (configuration 7 on
 // FP32 storage): A (m x k) and B (n x k) with the row index contiguous, 128x128 tiles, 8 waves of
@@ -789,7 +542,9 @@ static int run_cfg(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1,
     // Split K when the tile count cannot fill the chip (aim for >= 2 workgroups per CU).
     int splits = 1;
     const int target = 2 * ctx->num_cus;
-    if (tiles < target && !ctx->launch_mask) {
+    if constexpr (PREC == OMX_PREC_F64) {
+        splits = dgemm_k_splits(ctx, m, n, (ktot + BK - 1) / BK);  // as the direct-to-LDS kernel splits
+    } else if (tiles < target && !ctx->launch_mask) {
         int max_splits = std::max(1, ktot / (4 * BK));
         splits = std::min(max_splits, (target + tiles - 1) / tiles);
         splits = std::max(1, std::min(splits, 64));
@@ -836,12 +591,12 @@ static int run_cfg(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1,
 template <typename TS, int PREC, bool TRA, bool TRB, int NPAIR>
 struct CfgSet {
     static constexpr bool f64 = (PREC == OMX_PREC_F64) && !TRA;
-    static constexpr bool dl = f64 && std::is_same<TS, double>::value;
+    static constexpr bool dl = (PREC == OMX_PREC_F64) && std::is_same<TS, double>::value;
     static constexpr bool lowp = (PREC != OMX_PREC_F64) && std::is_same<TS, float>::value && !TRA && (TRB || NPAIR == 2);
     static constexpr bool sdl = lowp && PREC == OMX_PREC_F32 && TRB && NPAIR == 1;
     static std::vector<int> ids() {
-        if (dl) return {7, 0, 1, 2, 3, 5, 6};
-        if (f64) return {0, 1, 2, 3, 5, 6};
+        if (dl && f64) return {7, 0, 1, 2, 3, 5, 6};
+        if (dl) return {7, 0};
         if (sdl) return {7, 0, 4};
         if (lowp) return {0, 4};
         return {0};
@@ -855,9 +610,10 @@ static int run_cfg_id(int id, omx_ctx ctx, int m, int n, int k, double alpha, co
     typedef CfgSet<TS, PREC, TRA, TRB, NPAIR> CS;
     if constexpr (CS::dl) {
         if (id == 7) {
-            int rc = run_dgemm_dl<TRB, NPAIR>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
+            int rc = launch_dgemm(ctx, TRA, TRB, NPAIR, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C,
+                                  ldc);
             if (rc != OMX_ERR_UNSUPPORTED) return rc;
-            id = 5;  // the staged kernel with the same tiles covers every other shape
+            id = 5;  // the staged kernel (5 tiles; 0 with A transposed) for leading dimensions beyond 2^20
         }
     }
     if constexpr (CS::f64) {
@@ -926,6 +682,7 @@ static int tuned_cfg(omx_ctx ctx, int m, int n, int k, const TS *A1, const TS *A
     OMX_CHECK_HIP(hipEventCreate(&e0));
     OMX_CHECK_HIP(hipEventCreate(&e1));
     const bool prof = ctx->prof_on;
+    const int sym = ctx->gemm_sym;
     ctx->prof_on = false;
     int best = ids[0], rc = OMX_OK;
     float best_ms = 0.0f;
@@ -935,6 +692,7 @@ static int tuned_cfg(omx_ctx ctx, int m, int n, int k, const TS *A1, const TS *A
             (void)hipEventRecord(e0, ctx->stream);
             rc = run_cfg_id<TS, PREC, TRA, TRB, NPAIR>(id, ctx, m, n, k, 1.0, A1, A2, lda, B1, B2, ldb, 0.0, nullptr,
                                                        0.0, tmp, std::max(m, 1));
+            ctx->gemm_sym = sym;
             (void)hipEventRecord(e1, ctx->stream);
             (void)hipEventSynchronize(e1);
             (void)hipEventElapsedTime(&ms, e0, e1);
@@ -964,7 +722,7 @@ static int run_gemm(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1
     // staging where it applies (bitwise the same); the FP32 Gram's direct-to-LDS kernel where it
     // applies; 0 otherwise
     typedef CfgSet<TS, PREC, TRA, TRB, NPAIR> CS;
-    int id = (CS::dl || CS::sdl) ? 7 : CS::f64 ? 5 : 0;
+    int id = (CS::dl || CS::sdl) ? 7 : 0;
     if (ctx->gemm_cfg >= 0) {
         id = ctx->gemm_cfg;  // forced (omx_gemm_set_tile); a configuration that does not apply falls back to 0
     } else if (ctx->autotune) {
@@ -1419,8 +1177,15 @@ int launch_gemm_pair(omx_ctx ctx, int prec, int dt, int m, int n, int k, double 
     const int bk = (prec == OMX_PREC_F64)   ? Prec<OMX_PREC_F64>::BK
                    : (prec == OMX_PREC_F32) ? Prec<OMX_PREC_F32>::BK
                                             : Prec<OMX_PREC_BF16>::BK;
-    // The pair boundary must fall on a K-slice boundary; otherwise the caller runs separate passes.
-    if (k % bk != 0) return OMX_ERR_UNSUPPORTED;
+    // The pair boundary must fall on a K-slice boundary of the staged kernels (the direct-to-LDS FP64
+    // kernel pads each product's last slice); otherwise the caller runs separate passes.
+    if (k % bk != 0) {
+        if (dt == OMX_F64 && prec == OMX_PREC_F64 && (ctx->gemm_cfg < 0 || ctx->gemm_cfg == 7))
+            return launch_dgemm(ctx, false, false, 2, m, n, k, alpha, (const double *)A1, (const double *)A2, lda,
+                                (const double *)B1, (const double *)B2, ldb, beta0, (const double *)C0, beta,
+                                (double *)C, ldc);
+        return OMX_ERR_UNSUPPORTED;
+    }
     if (dt == OMX_F64) {
         const double *a1 = (const double *)A1, *a2 = (const double *)A2, *b1 = (const double *)B1,
                      *b2 = (const double *)B2, *c0 = (const double *)C0;
@@ -1477,10 +1242,11 @@ __global__ __launch_bounds__(256) void k_sym_mirror(int n, TS *__restrict__ C, i
 // triangle is then mirrored, so C is exactly symmetric.
 int launch_gemm_sym(omx_ctx ctx, int prec, int dt, int n, int k, double alpha, const void *A, int64_t lda,
                     const void *B, int64_t ldb, void *C, int64_t ldc) {
-    ctx->gemm_sym = true;
+    ctx->gemm_sym = 2;
     int rc = launch_gemm(ctx, prec, dt, false, true, n, n, k, alpha, A, lda, B, ldb, 0.0, C, ldc);
-    ctx->gemm_sym = false;
-    if (rc) return rc;
+    const bool whole = ctx->gemm_sym == 3;  // the product wrote the upper triangle too
+    ctx->gemm_sym = 0;
+    if (rc || whole) return rc;
     const int nt = (n + 63) / 64;
     const unsigned grid = (unsigned)(nt * (nt + 1) / 2);
     if (dt == OMX_F64)

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_bf16.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <map>
@@ -74,7 +75,9 @@ struct omx_ctx_s {
     double prof_bytes[OMX_K_COUNT] = {0};  // algorithmic (minimum) HBM bytes of the timed launches
     int num_cus = 256;
     int gemm_cfg = -1;    // forced GEMM tile configuration (-1: chosen by shape)
-    bool gemm_sym = false;  // set by omx_gemm_sym around its product: lower-triangle tiles only
+    // Set around a product known to be symmetric: 1 = only the lower triangle is wanted, 2 = both
+    // triangles.  A kernel that writes both sets 3 (no mirror pass needed).
+    int gemm_sym = 0;
     omx_spmm_shape_s spmm_shape;  // forced SpMM launch shape (when spmm_forced)
     bool spmm_forced = false;
     bool spmm_stencil = false;  // lattice operators use the 2.5-D stencil SpMM (omx_spmm_stencil)
@@ -177,14 +180,16 @@ inline bool valid_op(char op) { return op == 'n' || op == 'N' || is_trans(op); }
 // Scalar readback: copy `n` doubles from ctx->d_scalars to ctx->h_scalars and wait.
 int read_scalars(omx_ctx ctx, int n);
 
+// Position of workgroup id w among T when each XCD (ids are dealt round-robin over 8) takes a contiguous
+// band of T / 8 positions, the first T mod 8 bands one more: a bijection of 0..T-1 for every T.
+__device__ inline int xcd_band(int w, int T) { return (w & 7) * (T >> 3) + min(w & 7, T & 7) + (w >> 3); }
+
 // Tile index for workgroup id w of a tiles_m x tiles_n product: workgroup ids are dealt
 // round-robin over the 8 XCDs, so each XCD is given a contiguous band of tiles; inside a band
 // the tiles go in groups of 8 tile rows, column by column, so operand panels are shared in one
 // XCD's L2.
 __device__ inline void tile_of(int w, int tiles_m, int tiles_n, int &tm, int &tn) {
-    int T = tiles_m * tiles_n;
-    int t = w;
-    if ((T & 7) == 0) t = (w & 7) * (T >> 3) + (w >> 3);
+    const int t = xcd_band(w, tiles_m * tiles_n);
     constexpr int GM = 8;
     int group = t / (GM * tiles_n);
     int first_m = group * GM;
@@ -198,9 +203,7 @@ __device__ inline void tile_of(int w, int tiles_m, int tiles_n, int &tm, int &tn
 // XCDs as tile_of does and enumerated by tile rows (products known to be symmetric compute only
 // these and mirror them).
 __device__ inline void tile_of_lower(int w, int nt, int &tm, int &tn) {
-    const int T = nt * (nt + 1) / 2;
-    int t = w;
-    if ((T & 7) == 0) t = (w & 7) * (T >> 3) + (w >> 3);
+    const int t = xcd_band(w, nt * (nt + 1) / 2);
     int r = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
     while (r > 0 && r * (r + 1) / 2 > t) --r;
     while ((r + 1) * (r + 2) / 2 <= t) ++r;
@@ -208,9 +211,25 @@ __device__ inline void tile_of_lower(int w, int nt, int &tm, int &tn) {
     tn = t - r * (r + 1) / 2;
 }
 
+// Output area (elements) of the lower-triangle tiles of an n x n product with bm x bm tiles: the
+// flop count of a symmetric product is 2*k times this (the MFMA work actually issued).
+inline double sym_area(int n, int bm) {
+    double area = 0.0;
+    for (int a = 0; a * bm < n; ++a) area += (double)std::min(bm, n - a * bm) * std::min(n, (a + 1) * bm);
+    return area;
+}
+
 // Launch helpers implemented in the .hip files.
 int launch_gemm(omx_ctx ctx, int prec, int dt, bool trA, bool trB, int m, int n, int k, double alpha,
                 const void *A, int64_t lda, const void *B, int64_t ldb, double beta, void *C, int64_t ldc);
+// FP64 products of dgemm.hip (npair = 2: alpha*(A1*B1 + A2*B2), 'n','n'); OMX_ERR_UNSUPPORTED (nothing
+// launched) for leading dimensions beyond 2^20.
+int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const double *A1,
+                 const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
+                 const double *C0, double beta, double *C, int64_t ldc);
+// Parts K is split into for an FP64 product of nsl slices of 16; a function of the shape alone, so that
+// every tile configuration and the symmetric form add in the same order.
+int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl);
 // C := alpha*A*B^T known to be symmetric (n x n, 'n','t' operands of k columns): the lower-triangle
 // tiles where the kernels allow it, then a mirror of the lower triangle onto the upper (both honour
 // ctx->launch_mask).

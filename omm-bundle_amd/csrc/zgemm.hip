@@ -462,10 +462,10 @@ __global__ __launch_bounds__(256) void k_herm_mirror(int n, typename ZPrec<R>::c
 template <typename R>
 static int zgemm_herm_r(omx_ctx ctx, int n, int k, double alpha, const void *A, int64_t lda, const void *B,
                         int64_t ldb, void *C, int64_t ldc, int nbatch, const ZBatch &bat, bool allow_split) {
-    ctx->gemm_sym = true;
+    ctx->gemm_sym = 2;
     int rc = run_zgemm<R, false, false, true, true, 1>(ctx, n, n, k, alpha, A, A, lda, B, B, ldb, 0.0, nullptr, 0.0,
                                                        C, ldc, nbatch, bat, allow_split);
-    ctx->gemm_sym = false;
+    ctx->gemm_sym = 0;
     if (rc) return rc;
     const int nt = (n + 31) / 32;
     hipLaunchKernelGGL(k_herm_mirror<R>, dim3(nt * (nt + 1) / 2, nbatch), dim3(256), 0, ctx->stream, n,
