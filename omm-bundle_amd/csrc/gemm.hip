@@ -734,7 +734,9 @@ static int run_gemm(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1
 }
 
 // ---------------------------------------------------------------------------------------------
-// BF16 products of FP32 matrices through k-contiguous BF16 copies.
+// BF16 products of FP32 matrices through k-contiguous BF16 copies, for every m, n, k (k is padded with
+// zeros to whole slices: 5488 x 5488 x 10976 2.03 -> 0.72 ms, 250 x 250 x 500 44 -> 16 us, against the
+// staged kernel, which reads and rounds the FP32 operands again for every tile).
 //
 // The operands are first rounded to BF16 (round to nearest even, the same rounding as the
 // staging conversion of k_gemm) into k-contiguous panels: op(A) as At[kk + i*K] and op(B) as
@@ -747,73 +749,78 @@ static int run_gemm(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1
 
 constexpr int BG_T = 64;  // conversion tile (rows x cols)
 
-// Destinations of one operand's conversion: BgLay<L>::term[q] (1 = hi = bf16(a), 2 = mid =
-// bf16(a - hi), 3 = lo = bf16(a - hi - mid), each difference taken exactly in the source
-// precision) goes to p[q], q < BgLay<L>::n.  For FP32 sources hi + mid + lo is the value exactly;
-// hi + mid keeps about 16 significant bits.  Layouts: 0 = BF16; 1, 2 = BF16x3 A and B; 3, 4 =
-// BF16x6 A and B (the k blocks of the panel product, in order).
-struct BgDst {
-    __bf16 *p[6];
-};
-template <int L>
-struct BgLay;
+// The terms each k block of a panel holds, A's and B's (1 = hi = bf16(a), 2 = mid = bf16(a - hi), 3 = lo =
+// bf16(a - hi - mid), each difference taken exactly in the source precision).  For FP32 sources hi +
+// mid + lo is the value exactly; hi + mid keeps about 16 significant bits.  NS = 1: BF16; 2: BF16x3;
+// 3: BF16x6 (the term products in order, smallest first).
+template <int NS>
+struct BgTerms;
 template <>
-struct BgLay<0> {
+struct BgTerms<1> {
     static constexpr int n = 1;
-    __device__ static constexpr int term(int) { return 1; }
+    static constexpr int of[2][1] = {{1}, {1}};
 };
 template <>
-struct BgLay<1> {
+struct BgTerms<2> {
     static constexpr int n = 3;
-    __device__ static constexpr int term(int q) { return q == 2 ? 2 : 1; }  // hi hi mid
+    static constexpr int of[2][3] = {{1, 1, 2}, {1, 2, 1}};
 };
 template <>
-struct BgLay<2> {
-    static constexpr int n = 3;
-    __device__ static constexpr int term(int q) { return q == 1 ? 2 : 1; }  // hi mid hi
-};
-template <>
-struct BgLay<3> {
+struct BgTerms<3> {
     static constexpr int n = 6;
-    __device__ static constexpr int term(int q) { return q == 1 ? 3 : (q == 2 || q == 4) ? 2 : 1; }  // 1 3 2 1 2 1
-};
-template <>
-struct BgLay<4> {
-    static constexpr int n = 6;
-    __device__ static constexpr int term(int q) { return q == 0 ? 3 : (q == 2 || q == 3) ? 2 : 1; }  // 3 1 2 2 1 1
+    static constexpr int of[2][6] = {{1, 3, 2, 1, 2, 1}, {3, 1, 2, 2, 1, 1}};
 };
 
-// dst terms of src (rows x cols, ld lds, FP32 or FP64), each rounded once from the stored value:
-// TRANS: element (r, c) goes to dst[c + r*ldd], else to dst[r + c*ldd].  One 64 x 64 tile per
-// workgroup: 16-byte loads along r, and 16-byte stores of 8 BF16 along the destination's
-// contiguous index (through an LDS transpose for TRANS).  Edges and unaligned operands take
-// element-wise paths.
-template <bool TRANS, typename TS, int L>
-__global__ __launch_bounds__(256) void k_to_bf16(int rows, int cols, const TS *__restrict__ src, int64_t lds,
-                                                 BgDst dst, int64_t ldd) {
-    constexpr int ND = BgLay<L>::n;
+// One operand's conversion: src (rows x cols, ld lds) into the panel at dst, whose rows (ld ldd) hold
+// the k blocks of length kp one after another.  trans: element (r, c) goes to dst[c + r*ldd] (k runs
+// along the columns), else to dst[r + c*ldd] (k runs along the rows).
+struct BgJob {
+    const void *src;
+    int64_t lds;
+    __bf16 *dst;
+    int rows, cols, trans, side;  // side: 0 = A, 1 = B
+    int first, nbx;               // first workgroup and workgroups along the rows
+};
+struct BgJobs {
+    BgJob j[4];
+    int n, kp;
+    int64_t ldd;
+};
+
+// All conversions of a product in one launch (a launch each costs 2-3 us, as much as a small product),
+// each value rounded once from the stored one.  One 64 x 64 tile per workgroup: 16-byte loads along
+// the rows, and 16-byte stores of 8 BF16 along k (through an LDS transpose for trans); k is padded with
+// zeros up to kp (a multiple of 64, so every store is whole and aligned).  Edges and unaligned operands
+// load element by element.
+template <typename TS, int NS>
+__global__ __launch_bounds__(256) void k_to_bf16(BgJobs jobs) {
+    typedef BgTerms<NS> TT;
     constexpr int VEC = 16 / sizeof(TS);  // elements per 16-byte load
-    const int t = threadIdx.x;
-    const int r0 = blockIdx.x * BG_T, c0 = blockIdx.y * BG_T;
-    const bool vld = (lds % VEC) == 0 && ((uintptr_t)src & 15) == 0;
-    bool vst = (ldd % 8) == 0;
-#pragma unroll
-    for (int q = 0; q < ND; ++q) vst = vst && ((uintptr_t)dst.p[q] & 15) == 0;
+    __shared__ TS tile[BG_T][BG_T + 1];   // [c][r]
+    int q = 0;
+    while (q + 1 < jobs.n && (int)blockIdx.x >= jobs.j[q + 1].first) ++q;
+    const BgJob job = jobs.j[q];
+    const int t = threadIdx.x, w = blockIdx.x - job.first, kp = jobs.kp, rows = job.rows, cols = job.cols;
+    const int64_t ldd = jobs.ldd;
+    const TS *src = (const TS *)job.src;
+    const int r0 = (w % job.nbx) * BG_T, c0 = (w / job.nbx) * BG_T;
+    const bool vld = (job.lds % VEC) == 0 && ((uintptr_t)src & 15) == 0;
     auto load = [&](int gr, int gc, int count, TS *x) {  // x[0..count) = src(gr.., gc), zero outside
-        const TS *p = src + (int64_t)gr + (int64_t)gc * lds;
+        const TS *p = src + (int64_t)gr + (int64_t)gc * job.lds;
         if (vld && gc < cols && gr + count <= rows) {
 #pragma unroll
             for (int e = 0; e < count; e += VEC) {
                 typedef TS vec_t __attribute__((ext_vector_type(VEC)));
                 const vec_t v = *reinterpret_cast<const vec_t *>(p + e);
 #pragma unroll
-                for (int q = 0; q < VEC; ++q) x[e + q] = v[q];
+                for (int h = 0; h < VEC; ++h) x[e + h] = v[h];
             }
         } else {
+#pragma unroll
             for (int e = 0; e < count; ++e) x[e] = (gc < cols && gr + e < rows) ? p[e] : (TS)0;
         }
     };
-    auto store8 = [&](const TS *x, int64_t off, int avail) {  // the terms of 8 values to every destination
+    auto store8 = [&](const TS *x, int64_t off) {  // the terms of 8 values to every k block
         bf8v t1, t2, t3;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -825,19 +832,13 @@ __global__ __launch_bounds__(256) void k_to_bf16(int rows, int cols, const TS *_
             t3[e] = (__bf16)(r1 - (TS)md);
         }
 #pragma unroll
-        for (int q = 0; q < ND; ++q) {
-            const int tq = BgLay<L>::term(q);
-            const bf8v v = tq == 1 ? t1 : (tq == 2 ? t2 : t3);
-            if (vst && avail >= 8) {
-                *reinterpret_cast<bf8v *>(dst.p[q] + off) = v;
-            } else {
-                for (int e = 0; e < 8 && e < avail; ++e) dst.p[q][off + e] = v[e];
-            }
+        for (int b = 0; b < TT::n; ++b) {
+            const int tb = job.side ? TT::of[1][b] : TT::of[0][b];
+            *reinterpret_cast<bf8v *>(job.dst + off + (int64_t)b * kp) = tb == 1 ? t1 : (tb == 2 ? t2 : t3);
         }
     };
-    if constexpr (TRANS) {
-        __shared__ TS tile[BG_T][BG_T + 1];  // [c][r]
-        constexpr int VPC = BG_T / VEC;      // load vectors per tile column
+    if (job.trans) {
+        constexpr int VPC = BG_T / VEC;  // load vectors per tile column
         for (int v = t; v < BG_T * VPC; v += 256) {
             const int c = v / VPC, rv = (v % VPC) * VEC;
             TS x[VEC];
@@ -848,21 +849,19 @@ __global__ __launch_bounds__(256) void k_to_bf16(int rows, int cols, const TS *_
         __syncthreads();
         for (int u = t; u < BG_T * (BG_T / 8); u += 256) {
             const int r = u / (BG_T / 8), c8 = (u % (BG_T / 8)) * 8;
-            const int gr = r0 + r, gc = c0 + c8;
-            if (gr >= rows || gc >= cols) continue;
+            if (r0 + r >= rows || c0 + c8 >= kp) continue;
             TS x[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] = tile[c8 + e][r];
-            store8(x, (int64_t)gc + (int64_t)gr * ldd, cols - gc);
+            store8(x, (int64_t)(c0 + c8) + (int64_t)(r0 + r) * ldd);
         }
     } else {
         for (int u = t; u < BG_T * (BG_T / 8); u += 256) {
             const int c = u / (BG_T / 8), r8 = (u % (BG_T / 8)) * 8;
-            const int gr = r0 + r8, gc = c0 + c;
-            if (gr >= rows || gc >= cols) continue;
+            if (r0 + r8 >= kp || c0 + c >= cols) continue;
             TS x[8];
-            load(gr, gc, 8, x);
-            store8(x, (int64_t)gr + (int64_t)gc * ldd, rows - gr);
+            load(r0 + r8, c0 + c, 8, x);
+            store8(x, (int64_t)(r0 + r8) + (int64_t)(c0 + c) * ldd);
         }
     }
 }
@@ -931,7 +930,8 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_bgemm_tn(int m, int n, int
                                                      const __bf16 *__restrict__ At, int64_t lda,
                                                      const __bf16 *__restrict__ Bt, int64_t ldb, double beta0,
                                                      const TO *__restrict__ C0, double beta, TO *__restrict__ C,
-                                                     int64_t ldc, int sym) {
+                                                     int64_t ldc, int sym, int kps,
+                                                     float *__restrict__ partial) {
     constexpr int BK = Prec<OMX_PREC_BF16>::BK;
     constexpr int NW = CF::WGM * CF::WGN;
     constexpr int INS = (CF::BM + CF::BN) / 8;  // wave loads per slice, 8 rows each
@@ -972,9 +972,10 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_bgemm_tn(int m, int n, int
         else
             voff[q] = 2 * (int)(min(rr - CF::BM, n - 1 - j0) * ldb + (p ^ bg_swz(rr - CF::BM)) * 8);
     }
+    const int s0 = blockIdx.z * kps, nslices = min(K / BK - s0, kps);  // this part of K, in slices
     auto issue = [&](int s) {
         __bf16 *st = smem + (s & 1) * STAGE;
-        const int kb = 2 * s * BK;
+        const int kb = 2 * (s0 + s) * BK;
 #pragma unroll
         for (int q = 0; q < LPW; ++q) {
             const int ins = uwave * LPW + q;
@@ -989,7 +990,6 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_bgemm_tn(int m, int n, int
         }
     };
 
-    const int nslices = K / BK;
     if (nslices > 0) issue(0);
     for (int s = 0; s < nslices; ++s) {
         __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt(0));  // this wave's rows of slice s have landed
@@ -1010,6 +1010,10 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_bgemm_tn(int m, int n, int
             for (int v = 0; v < 4; ++v) {
                 const int i = i0 + wm * CF::WM + fm * 16 + Prec<OMX_PREC_BF16>::out_row(lq, v);
                 if (i >= m) continue;
+                if (partial) {  // a part of K: reduced in part order later
+                    partial[(int64_t)blockIdx.z * m * n + (int64_t)i + (int64_t)j * m] = acc[fm][fn][v];
+                    continue;
+                }
                 double r = alpha * (double)acc[fm][fn][v];
                 if (C0) r += beta0 * (double)C0[(int64_t)i + (int64_t)j * ldc];
                 if (beta != 0.0) r += beta * (double)C[(int64_t)i + (int64_t)j * ldc];
@@ -1026,32 +1030,41 @@ struct BgTerm {
     bool trans;  // true: X is stored K x extent (already k-contiguous)
 };
 
-template <typename TS, int L>
-static void bg_convert_l(omx_ctx ctx, const BgTerm &tm, int extent, int K, const BgDst &dst, int64_t ldd) {
-    const TS *X = (const TS *)tm.X;
-    if (tm.trans) {
-        // X is K x extent with k contiguous: same layout, dst[kk + e*ldd]
-        dim3 grid((K + BG_T - 1) / BG_T, (extent + BG_T - 1) / BG_T);
-        hipLaunchKernelGGL((k_to_bf16<false, TS, L>), grid, dim3(256), 0, ctx->stream, K, extent, X, tm.ldx, dst, ldd);
-    } else {
-        // X is extent x K: transpose so that dst[kk + e*ldd] = X(e, kk)
-        dim3 grid((extent + BG_T - 1) / BG_T, (K + BG_T - 1) / BG_T);
-        hipLaunchKernelGGL((k_to_bf16<true, TS, L>), grid, dim3(256), 0, ctx->stream, extent, K, X, tm.ldx, dst, ldd);
-    }
+// The job of one operand (extent x k as a panel): the columns of X hold k where X is transposed.
+static void bg_job(BgJobs &jobs, int &grid, const BgTerm &tm, int extent, int k, int side, __bf16 *dst) {
+    BgJob &j = jobs.j[jobs.n++];
+    j = BgJob{tm.X, tm.ldx, dst, tm.trans ? k : extent, tm.trans ? extent : k, !tm.trans, side, grid, 0};
+    const int along_r = tm.trans ? jobs.kp : extent, along_c = tm.trans ? extent : jobs.kp;
+    j.nbx = (along_r + BG_T - 1) / BG_T;
+    grid += j.nbx * ((along_c + BG_T - 1) / BG_T);
 }
 
-// Converts one operand into the panel blocks of layout `lay` (see BgLay).
-template <typename TS>
-static int bg_convert(omx_ctx ctx, const BgTerm &tm, int extent, int K, const BgDst &dst, int64_t ldd, int lay) {
-    switch (lay) {
-        case 0: bg_convert_l<TS, 0>(ctx, tm, extent, K, dst, ldd); break;
-        case 1: bg_convert_l<TS, 1>(ctx, tm, extent, K, dst, ldd); break;
-        case 2: bg_convert_l<TS, 2>(ctx, tm, extent, K, dst, ldd); break;
-        case 3: bg_convert_l<TS, 3>(ctx, tm, extent, K, dst, ldd); break;
-        default: bg_convert_l<TS, 4>(ctx, tm, extent, K, dst, ldd); break;
-    }
-    OMX_CHECK_HIP(hipGetLastError());
-    return OMX_OK;
+// Tile (256: 8 waves of 128x64, 128: 4 waves of 64x64, two workgroups per CU) and the parts K is split
+// into: the least of rounds of workgroups over the CUs times the 64-wide slices of a part, plus the
+// reduction of the parts.  Slice times (us) measured on Grams and gradients of 2662 to 5488 states, alone
+// with one workgroup on a CU; over 34 products of 54 to 5488 states the choice is within 3 % of the
+// fastest of both tiles and 1 to 8 parts on average.  A 256 tile moves half the bytes per operation, a 128
+// tile leaves less of the chip idle in the last round: 4394 states 0.46 ms against 0.53, 5488 0.89
+// against 0.72.  The choice depends on the full product's shape alone, so a symmetric product adds as the
+// full one does.
+static void bg_shape(omx_ctx ctx, int m, int n, int slices, int &tile, int &splits) {
+    const int edge[2] = {256, 128};
+    const double slice[2] = {1.75, 0.565}, alone[2] = {1.75, 0.77};
+    double cost = 0.0;
+    tile = 0;
+    for (int q = 0; q < 2; ++q)
+        for (int s : {1, 2, 3, 4, 6, 8}) {
+            if (s > 1 && slices < 2 * s) break;
+            const int64_t tiles = (int64_t)((m + edge[q] - 1) / edge[q]) * ((n + edge[q] - 1) / edge[q]) * s;
+            const int64_t rounds = (tiles + ctx->num_cus - 1) / ctx->num_cus;
+            const double c = std::max(slice[q] * rounds, alone[q]) * ((slices + s - 1) / s) +
+                             (s > 1 ? 3.5 + 4e-6 * (s + 1) * m * n / 4.5 : 0.0);
+            if (!tile || c < cost) {
+                tile = edge[q];
+                splits = s;
+                cost = c;
+            }
+        }
 }
 
 // C := alpha * sum_t op(A_t) op(B_t) + beta0*C0 + beta*C for nterm products of inner size k on
@@ -1064,42 +1077,61 @@ template <typename TS>
 static int bgemm_panels(omx_ctx ctx, int m, int n, int k, int nterm, const BgTerm *A, const BgTerm *B, int nsplit,
                         double alpha, double beta0, const TS *C0, double beta, TS *C, int64_t ldc) {
     constexpr int BK = Prec<OMX_PREC_BF16>::BK;
-    if (ctx->launch_mask || k % BK != 0 || m < 256 || n < 256 || k < 4 * BK) return OMX_ERR_UNSUPPORTED;
-    // k blocks per product term and the conversion layouts of A and B (BgLay)
-    static const int nblk[3] = {1, 3, 6}, lay_a[3] = {0, 1, 3}, lay_b[3] = {0, 2, 4};
+    if (ctx->launch_mask) return OMX_ERR_UNSUPPORTED;
+    // the split products run in FP32 outside these shapes; BF16 takes any
+    if (nsplit > 1 && (k % BK != 0 || m < 256 || n < 256 || k < 4 * BK)) return OMX_ERR_UNSUPPORTED;
+    const int kp = (k + BK - 1) / BK * BK;  // each k block of a panel ends in zeros up to a whole slice
+    static const int nblk[3] = {1, 3, 6};  // k blocks per product term
     OMX_REQUIRE(nsplit >= 1 && nsplit <= 3, "bf16 panels: split %d", nsplit);
     const int reps = nblk[nsplit - 1];
-    const int64_t K = (int64_t)k * nterm * reps;
+    const int64_t K = (int64_t)kp * nterm * reps;
     if ((int64_t)Cfg4::BM * K * (int64_t)sizeof(__bf16) >= (1LL << 31)) return OMX_ERR_UNSUPPORTED;  // 32-bit offsets
     const size_t bytes_a = sizeof(__bf16) * (size_t)K * m, bytes_b = sizeof(__bf16) * (size_t)K * n;
-    int rc = ensure_ws(ctx, bytes_a + bytes_b + 256);
+    int tile, splits;
+    bg_shape(ctx, m, n, (int)(K / BK), tile, splits);
+    const int kps = ((int)(K / BK) + splits - 1) / splits;
+    splits = ((int)(K / BK) + kps - 1) / kps;
+    const size_t panels = (bytes_a + 255) / 256 * 256 + (bytes_b + 255) / 256 * 256;
+    int rc = ensure_ws(ctx, panels + (splits > 1 ? sizeof(float) * (size_t)splits * m * n : 0));
     if (rc) return rc;
+    float *partial = splits > 1 ? (float *)((char *)ctx->ws + panels) : nullptr;
     __bf16 *At = (__bf16 *)ctx->ws;
     __bf16 *Bt = (__bf16 *)((char *)ctx->ws + ((bytes_a + 255) / 256) * 256);
     const bool sym = ctx->gemm_sym && m == n && nterm == 1;  // lower-triangle tiles of a symmetric product
     hipEvent_t ev;
     prof_begin(ctx, nterm == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM, &ev);
     prof_work(ctx, nterm == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM,
-              2.0 * (sym ? sym_area(m, Cfg4::BM) : (double)m * n) * (double)k * nterm,
+              2.0 * (sym ? sym_area(m, tile) : (double)m * n) * (double)k * nterm,
               sizeof(TS) * (nterm * ((double)m * k + (double)k * n) + (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0))));
     // Rows of At are m panels of length K (ld K), rows of Bt n of length K; product term tt takes
     // the K range [tt*reps*k, (tt+1)*reps*k), block b of it holding the A and B terms of pair b.
-    for (int tt = 0; tt < nterm && !rc; ++tt) {
-        const int64_t kb = (int64_t)tt * reps * k;
-        BgDst da{}, db{};
-        for (int b = 0; b < reps; ++b) {
-            da.p[b] = At + kb + (int64_t)b * k;
-            db.p[b] = Bt + kb + (int64_t)b * k;
-        }
-        rc = bg_convert<TS>(ctx, A[tt], m, k, da, K, lay_a[nsplit - 1]);
-        if (!rc) rc = bg_convert<TS>(ctx, B[tt], n, k, db, K, lay_b[nsplit - 1]);
+    BgJobs jobs{};
+    jobs.kp = kp;
+    jobs.ldd = K;
+    int cgrid = 0;
+    for (int tt = 0; tt < nterm; ++tt) {
+        bg_job(jobs, cgrid, A[tt], m, k, 0, At + (int64_t)tt * reps * kp);
+        bg_job(jobs, cgrid, B[tt], n, k, 1, Bt + (int64_t)tt * reps * kp);
     }
-    if (!rc) {
-        typedef Cfg4 CF;
-        const int tm = (m + CF::BM - 1) / CF::BM;
-        const int tiles = sym ? tm * (tm + 1) / 2 : tm * ((n + CF::BN - 1) / CF::BN);
-        hipLaunchKernelGGL((k_bgemm_tn<CF, TS>), dim3(tiles), dim3(CF::NT), 0, ctx->stream, m, n, (int)K, alpha, At, K,
-                           Bt, K, beta0, C0, beta, C, ldc, (int)sym);
+    if (nsplit == 1)
+        hipLaunchKernelGGL((k_to_bf16<TS, 1>), dim3(cgrid), dim3(256), 0, ctx->stream, jobs);
+    else if (nsplit == 2)
+        hipLaunchKernelGGL((k_to_bf16<TS, 2>), dim3(cgrid), dim3(256), 0, ctx->stream, jobs);
+    else
+        hipLaunchKernelGGL((k_to_bf16<TS, 3>), dim3(cgrid), dim3(256), 0, ctx->stream, jobs);
+    {
+        const int tm = (m + tile - 1) / tile, tn = (n + tile - 1) / tile;
+        const dim3 grid(sym ? tm * (tm + 1) / 2 : tm * tn, 1, splits);
+        if (tile == 256)
+            hipLaunchKernelGGL((k_bgemm_tn<Cfg4, TS>), grid, dim3(Cfg4::NT), 0, ctx->stream, m, n, (int)K, alpha, At, K,
+                               Bt, K, beta0, C0, beta, C, ldc, (int)sym, kps, partial);
+        else
+            hipLaunchKernelGGL((k_bgemm_tn<Cfg0, TS>), grid, dim3(Cfg0::NT), 0, ctx->stream, m, n, (int)K, alpha, At, K,
+                               Bt, K, beta0, C0, beta, C, ldc, (int)sym, kps, partial);
+        // (a symmetric product's elements above its tiles are not written: the mirror overwrites them)
+        if (partial)
+            hipLaunchKernelGGL((k_splitk_reduce<TS, float>), dim3((int)std::min<int64_t>(((int64_t)m * n + 255) / 256, 8192)),
+                               dim3(256), 0, ctx->stream, m, n, splits, partial, alpha, beta0, C0, beta, C, ldc);
         rc = hipGetLastError() == hipSuccess ? OMX_OK : OMX_ERR_HIP;
         if (rc) set_error("bf16 panel GEMM launch failed");
     }
