@@ -333,7 +333,7 @@ static int *flag(omx_zbatch b, int which) { return b->active + which * b->nsys; 
 enum { F_ACTIVE = 0, F_FAIL, F_CONT, F_GRAD, F_ICG, F_CONV, F_NFAIL, F_COUNT };
 
 // G = 4HC - 2SW*HC - 2HW*SC for the systems with mask[s] (calc_G, omm_ops.F90:17-39): one pair
-// launch, or three passes when no is not a multiple of the K slice.  T: double2 or Cx<float>.
+// launch, or three passes for complex64 when no is not a multiple of 8.  T: double2 or Cx<float>.
 template <typename T>
 static int batch_calc_G(omx_zbatch b, const int *mask) {
     omx_ctx ctx = b->ctx;

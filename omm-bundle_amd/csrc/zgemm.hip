@@ -4,18 +4,18 @@
 // mm_zmultiply products (MatrixSwitch/src/MatrixSwitch.F90:1395-1726, 'ref' semantics of
 // MatrixSwitch_mm_multiply.F90:85-185) for the k-point solves.
 //
-// Storage is the Fortran complex layout: (re, im) interleaved, column-major.  A workgroup of 4
-// wave64s owns a BM x BN tile of C; operand slices are staged through LDS as separate real and
-// imaginary k-major planes (conjugation is applied while staging, by negating the imaginary
-// plane), and each 16x16 output block keeps a real and an imaginary accumulator:
-//     acc_re += a_re*b_re - a_im*b_im,    acc_im += a_re*b_im + a_im*b_re,
-// four real MFMAs per block and k step.  K slices are double-buffered; split-K with an
-// in-order reduction covers shapes with too few tiles; the pair mode (two contractions back to
-// back over one K range) gives calc_G in one launch.  Tile ids are XCD-remapped as in the real
-// kernel.
+// Storage is the Fortran complex layout: (re, im) interleaved, column-major.  Each 16x16 output block
+// keeps a real and an imaginary accumulator, four real MFMAs per block and k step:
+//     acc_re += a_re*b_re - a_im*b_im,    acc_im += a_re*b_im + a_im*b_re.
+// k_zgemm_dl (operands straight into LDS) takes every product with leading dimensions up to 2^20; past
+// that k_zgemm stages
+// through registers into real and imaginary k-major LDS planes (conjugation negates the imaginary plane).
+// K slices are double-buffered in both; split-K with an in-order reduction covers shapes with too few
+// tiles; the pair mode (two contractions back to back over one K range) gives calc_G in one launch.
 #include <algorithm>
 
 #include "omx_internal.h"
+#include "omx_mfma.h"
 
 namespace omx {
 
@@ -302,11 +302,366 @@ __global__ void k_zsplitk_reduce(int m, int n, int splits, const R *__restrict__
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Direct-to-LDS products, for every m, n, k and leading dimensions up to 2^20.
+//
+// The operands stay interleaved (re, im) in LDS: an element is read whole (16 or 8 bytes), and the signs
+// that conjugation and the real part need are put on A's values in registers.  K is taken in slices of
+// 128 bytes of elements (8 complex128, 16 complex64), loaded with buffer_load_dwordx4 ... lds through
+// descriptors that end where the operand ends (dwords past it arrive as zero); a row-contiguous operand
+// lands k-major, a k-contiguous one in 128-byte rows whose 16-byte chunks are swizzled by row, and the
+// last slice of such a row is cleared past k.  Tiles: 64x64 (4 waves of 32x32, two stages: a third stage
+// leaves room for one workgroup fewer per CU and costs 2-4 %) and 32x32 (4 waves of 16x16, two stages of
+// four slices); the K chain per element does not depend on the tile.
+// What bounds it: the matrix cores (a 64x64 complex tile moves as few bytes per operation as a real
+// 128x128 one), or, where the tiles do not fill the chip, the serial chain of slices of one tile.  The
+// register-staged kernel below ran 64x128 tiles only: the 2000 x 2000 x 4000 complex128 Hermitian Gram
+// took 1.60 ms (now 1.09), the full Gram 2.24 (1.85, 69 TF/s), 16 Grams of 128 x 128 x 256 on 32 workgroups
+// 92 us (now 19).
+// ---------------------------------------------------------------------------------------------
+template <typename R>
+struct ZGeo {
+    static constexpr int ES = 2 * sizeof(R), EPC = 16 / ES, DK = 128 / ES;
+    // the chunk swizzle of k-contiguous rows: complex128 reads one 16-byte chunk of 16 rows (16 distinct
+    // bank groups), complex64 half a chunk
+    __device__ static inline int swz(int r) { return ES == 16 ? (r & 7) ^ ((r >> 3) & 1) : dl_swz(r); }
+};
+// Byte offset of lane `lane` of wave load `ins` of an operand tile (ROWS rows) from the slice's base.
+template <typename R, int ROWS, bool KC>
+__device__ inline int zl_voff(int ins, int lane, int ld) {
+    typedef ZGeo<R> G;
+    if constexpr (KC) {
+        const int r = ins * 8 + (lane >> 3);
+        return r * ld * G::ES + 16 * ((lane & 7) ^ G::swz(r));
+    } else {
+        constexpr int LPR = ROWS * G::ES / 16;  // lanes per k-row
+        return (ins * (64 / LPR) + lane / LPR) * ld * G::ES + 16 * (lane % LPR);
+    }
+}
+// Place (in elements) of row r, k kk in a staged tile.
+template <typename R, int ROWS, bool KC>
+__device__ inline int zl_at(int r, int kk) {
+    typedef ZGeo<R> G;
+    return KC ? r * G::DK + ((kk / G::EPC) ^ G::swz(r)) * G::EPC + kk % G::EPC : kk * ROWS + r;
+}
+
+template <int B_, int NST_, int U_>
+struct ZlCfg {
+    static constexpr int B = B_, NST = NST_, U = U_, W = B_ / 2, FB = W / 16;
+};
+typedef ZlCfg<64, 2, 1> Zl64;
+typedef ZlCfg<32, 2, 4> Zl32;
+
+template <typename R, class CF, bool TRA, bool CJA, bool TRB, bool CJB, int NPAIR>
+__global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double alpha,
+                                                    const typename ZPrec<R>::cplx *__restrict__ A1,
+                                                    const typename ZPrec<R>::cplx *__restrict__ A2, int64_t lda,
+                                                    const typename ZPrec<R>::cplx *__restrict__ B1,
+                                                    const typename ZPrec<R>::cplx *__restrict__ B2, int64_t ldb,
+                                                    double beta0, const typename ZPrec<R>::cplx *__restrict__ C0,
+                                                    double beta, typename ZPrec<R>::cplx *__restrict__ C, int64_t ldc,
+                                                    int sym, int sps, typename ZPrec<R>::cplx *__restrict__ partial,
+                                                    ZBatch bat) {
+    typedef ZGeo<R> G;
+    typedef typename ZPrec<R>::cplx C2;
+    typedef typename ZPrec<R>::accv AV;
+    constexpr int B = CF::B, NST = CF::NST, U = CF::U, W = CF::W, FB = CF::FB, DK = G::DK;
+    constexpr int LPW = 2 * B * 128 / 1024 / 4;          // wave loads per slice and wave
+    constexpr int SLICE = 2 * B * DK, STAGE = U * SLICE;  // elements: A, then B
+    constexpr bool KCA = TRA, KCB = !TRB;
+    __shared__ __align__(16) C2 smem[NST * STAGE];
+    const int bsys = blockIdx.y;
+    if (bat.active && !bat.active[bsys]) return;  // whole workgroup, before any barrier
+    A1 += bsys * bat.sA;
+    A2 += bsys * bat.sA;
+    B1 += bsys * bat.sB;
+    B2 += bsys * bat.sB;
+    C += bsys * bat.sC;
+    if (C0) C0 += bsys * bat.sC;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    int tm, tn;
+    if (sym)
+        tile_of_lower(blockIdx.x, (m + B - 1) / B, tm, tn);
+    else
+        tile_of(blockIdx.x, (m + B - 1) / B, (n + B - 1) / B, tm, tn);
+    const int i0 = tm * B, j0 = tn * B, wi = i0 + wm * W, wj = j0 + wn * W;
+    const bool live = wi < m && wj < n && !(sym && wj > wi + W - 1);
+    const int nsl = (k + DK - 1) / DK, sb = blockIdx.z * sps, ns = min(NPAIR * nsl, sb + sps) - sb;
+
+    AV are[FB][FB], aim[FB][FB];
+#pragma unroll
+    for (int a = 0; a < FB; ++a)
+#pragma unroll
+        for (int b = 0; b < FB; ++b) {
+            are[a][b] = AV{0, 0, 0, 0};
+            aim[a][b] = AV{0, 0, 0, 0};
+        }
+    // waves 0 and 1 load A, 2 and 3 B; the wave's descriptor advances by one slice each time and starts
+    // over at the second product of a pair
+    const bool on_b = wave >= 2;
+    int voff[LPW];
+#pragma unroll
+    for (int q = 0; q < LPW; ++q) {
+        const int ins = (wave & 1) * LPW + q;
+        voff[q] = on_b ? zl_voff<R, B, KCB>(ins, lane, (int)ldb) : zl_voff<R, B, KCA>(ins, lane, (int)lda);
+    }
+    const bool kc = on_b ? KCB : KCA;
+    const int64_t ld = on_b ? ldb : lda;
+    const int x0 = on_b ? j0 : i0, ext = on_b ? n : m;
+    const int64_t step = G::ES * (kc ? DK : DK * ld), at = G::ES * (kc ? x0 * ld : (int64_t)x0);
+    const int64_t all = G::ES * (kc ? (int64_t)(ext - 1 - x0) * ld + k : (int64_t)(k - 1) * ld + (ext - x0));
+    const char *const first = (const char *)(on_b ? B1 : A1) + at, *const second = (const char *)(on_b ? B2 : A2) + at;
+    const int sb_in = NPAIR == 2 && sb >= nsl ? sb - nsl : sb;
+    const char *pos = (NPAIR == 2 && sb >= nsl ? second : first) + sb_in * step;
+    int64_t left = all - sb_in * step;
+    // slice (of this part) where the second product starts; the last slice of each product if partial
+    const int sw = nsl - sb, t1 = k % DK ? sw - 1 : -1, t2 = NPAIR == 2 && k % DK ? sw + nsl - 1 : -1;
+    auto issue = [&](int s) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int sl = s * U + u;
+            if (U > 1 && sl >= ns) break;
+            C2 *st = smem + (s % NST) * STAGE + u * SLICE + wave * LPW * (1024 / G::ES);
+            if (NPAIR == 2 && sl == sw) {
+                pos = second;
+                left = all;
+            }
+            const __amdgpu_buffer_rsrc_t r = raw_rsrc(pos, (uint32_t)((uint64_t)left >> 31) ? 0x7ffffff8 : (int)left);
+            pos += step;
+            left -= step;
+#pragma unroll
+            for (int q = 0; q < LPW; ++q) {
+                const int vo = voff[q];
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(st + q * (1024 / G::ES)), 16, vo, 0, 0, 0);
+            }
+        }
+    };
+    const int li = lane & 15, lk = lane >> 4;
+    // a = x, b = y of op(A), op(B) before conjugation:
+    //   re += xr yr + s xi yi, im += (sB) xr yi + (sA) xi yr, with sA, sB = -1 where conjugated and s = -sA sB
+    constexpr bool NEG_S = (CJA == CJB), NEG_B = CJB, NEG_A = CJA;
+    auto slice = [&](const C2 *As, const C2 *Bs) {
+        C2 a[2][FB], b[2][FB];
+        auto frag = [&](int ks, C2 (&fa)[FB], C2 (&fb)[FB]) {
+#pragma unroll
+            for (int f = 0; f < FB; ++f) fa[f] = As[zl_at<R, B, KCA>(wm * W + f * 16 + li, ks + lk)];
+#pragma unroll
+            for (int f = 0; f < FB; ++f) fb[f] = Bs[zl_at<R, B, KCB>(wn * W + f * 16 + li, ks + lk)];
+        };
+        frag(0, a[0], b[0]);
+#pragma unroll
+        for (int ks = 0; ks < DK; ks += 4) {
+            const int cur = (ks / 4) & 1;
+            if (ks + 4 < DK) frag(ks + 4, a[cur ^ 1], b[cur ^ 1]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int fm = 0; fm < FB; ++fm) {
+                const C2 x = a[cur][fm];
+                const R xs = NEG_S ? -x.y : x.y, xb = NEG_B ? -x.x : x.x, xa = NEG_A ? -x.y : x.y;
+#pragma unroll
+                for (int fn = 0; fn < FB; ++fn) {  // (y, x): the result's columns run along i
+                    const C2 y = b[cur][fn];
+                    are[fm][fn] = ZPrec<R>::mfma(y.x, x.x, are[fm][fn]);
+                    aim[fm][fn] = ZPrec<R>::mfma(y.y, xb, aim[fm][fn]);
+                    are[fm][fn] = ZPrec<R>::mfma(y.y, xs, are[fm][fn]);
+                    aim[fm][fn] = ZPrec<R>::mfma(y.x, xa, aim[fm][fn]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    const int nst = (ns + U - 1) / U, nfull = ns / U;
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+        if (s < nst) issue(s);
+    auto march = [&](auto work) {  // waves outside the result only load, clear and wait
+        for (int s = 0; s < nst; ++s) {
+            if (NST > 2 && s + NST - 2 < nfull)
+                __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt(LPW * U * (NST - 2)));
+            else
+                __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt(0));
+            wg_barrier();  // stage s has landed for every wave; stage s-1 is no longer read
+            if (s + NST - 1 < nst) issue(s + NST - 1);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int sl = s * U + u;
+                if (U > 1 && sl >= ns) break;
+                C2 *As = smem + (s % NST) * STAGE + u * SLICE, *Bs = As + B * DK;
+                if ((KCA || KCB) && (sl == t1 || (NPAIR == 2 && sl == t2))) {  // k-contiguous rows end at k
+                    for (int e = t; e < B * DK; e += 256)
+                        if (e % DK >= k % DK) {
+                            if (KCA) As[zl_at<R, B, true>(e / DK, e % DK)] = C2{0, 0};
+                            if (KCB) Bs[zl_at<R, B, true>(e / DK, e % DK)] = C2{0, 0};
+                        }
+                    wg_barrier();
+                }
+                if (decltype(work)::value) slice(As, Bs);
+            }
+        }
+    };
+    if (!live) {
+        march(std::false_type{});
+        return;
+    }
+    march(std::true_type{});
+    const int lq = lane >> 4;
+#pragma unroll
+    for (int fm = 0; fm < FB; ++fm)
+#pragma unroll
+        for (int fn = 0; fn < FB; ++fn) {
+            const int i = wi + fm * 16 + li;
+            if (i >= m) continue;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int j = wj + fn * 16 + ZPrec<R>::out_row(lq, v);
+                if (j >= n || (sym && j > i)) continue;
+                const R vr = are[fm][fn][v], vi = aim[fm][fn][v];
+                if (partial) {  // a part of K: the raw sums, reduced in part order later
+                    partial[(int64_t)blockIdx.z * m * n + (int64_t)i + (int64_t)j * m] = C2{vr, vi};
+                    continue;
+                }
+                const int64_t off = (int64_t)i + (int64_t)j * ldc;
+                double rr = alpha * (double)vr, ri = alpha * (double)vi;
+                if (C0) {
+                    rr += beta0 * (double)C0[off].x;
+                    ri += beta0 * (double)C0[off].y;
+                }
+                if (beta != 0.0) {
+                    rr += beta * (double)C[off].x;
+                    ri += beta * (double)C[off].y;
+                }
+                C[off] = C2{(R)rr, (R)ri};
+                if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = C2{(R)rr, (R)-ri};
+            }
+        }
+}
+
+// C := alpha * (sum of the K parts, in part order) + beta0*C0 + beta*C; sym: the lower triangle, and with
+// sym == 2 its conjugate mirror.
+template <typename R>
+__global__ __launch_bounds__(256) void k_zl_reduce(int m, int n, int sym, int splits,
+                                                   const typename ZPrec<R>::cplx *__restrict__ partial, double alpha,
+                                                   double beta0, const typename ZPrec<R>::cplx *__restrict__ C0,
+                                                   double beta, typename ZPrec<R>::cplx *__restrict__ C, int64_t ldc) {
+    typedef typename ZPrec<R>::cplx C2;
+    const int64_t total = (int64_t)m * n;
+    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < total; q += (int64_t)gridDim.x * 256) {
+        const int64_t i = q % m, j = q / m;
+        if (sym && j > i) continue;
+        C2 s = partial[q];
+        for (int z = 1; z < splits; ++z) {
+            const C2 p = partial[(int64_t)z * total + q];
+            s.x += p.x;
+            s.y += p.y;
+        }
+        const int64_t off = i + j * ldc;
+        double rr = alpha * (double)s.x, ri = alpha * (double)s.y;
+        if (C0) {
+            rr += beta0 * (double)C0[off].x;
+            ri += beta0 * (double)C0[off].y;
+        }
+        if (beta != 0.0) {
+            rr += beta * (double)C[off].x;
+            ri += beta * (double)C[off].y;
+        }
+        C[off] = C2{(R)rr, (R)ri};
+        if (sym == 2 && j < i) C[j + i * ldc] = C2{(R)rr, (R)-ri};
+    }
+}
+
+static int64_t zl_tiles(int m, int n, int b, bool sym) {
+    const int64_t tm = (m + b - 1) / b, tn = (n + b - 1) / b;
+    return sym ? tm * (tm + 1) / 2 : tm * tn;
+}
+// Tile and parts of K with the least time: rounds of workgroups over the CUs times the slices of a part,
+// plus the reduction of the parts.  round[r] is a CU's time (us) for one slice of r workgroups resident
+// together (up to four of the 64 tile, two of the 32 one), measured with 250 to 2000 states: a lone
+// workgroup leaves the matrix cores idle while it waits, 1.37 us per slice against 0.92 in a full CU.
+static void zl_shape(omx_ctx ctx, int m, int n, int nsl, bool sym, int nbatch, bool split, int &tile, int &splits) {
+    const int edge[2] = {64, 32}, full[2] = {4, 2};
+    const double round[2][5] = {{0.0, 1.37, 1.96, 2.87, 3.69}, {0.0, 0.29, 0.55, 0.0, 0.0}};
+    double cost = 0.0;
+    tile = 0;
+    for (int q = 0; q < 2; ++q)
+        for (int s : {1, 2, 3, 4, 5, 6, 8, 12}) {
+            if (s > 1 && (!split || nsl < 4 * s)) break;
+            const int64_t units = zl_tiles(m, n, edge[q], sym) * nbatch * s;
+            const int64_t rounds = (units + ctx->num_cus - 1) / ctx->num_cus;
+            const double per = (double)(rounds / full[q]) * round[q][full[q]] + round[q][rounds % full[q]];
+            const double c = 0.55 * rounds + per * ((nsl + s - 1) / s) +
+                             (s > 1 ? 5.3 + 16e-6 * (s + 1) * m * n / 4.9 : 0.0);
+            if (!tile || c < cost) {
+                tile = edge[q];
+                splits = s;
+                cost = c;
+            }
+        }
+}
+
+// Launches the direct-to-LDS product; OMX_ERR_UNSUPPORTED for leading dimensions beyond 2^20.
+template <typename R, bool TRA, bool CJA, bool TRB, bool CJB, int NPAIR>
+static int run_zgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const void *A1, const void *A2, int64_t lda,
+                        const void *B1, const void *B2, int64_t ldb, double beta0, const void *C0, double beta, void *C,
+                        int64_t ldc, int nbatch, const ZBatch &bat, bool allow_split) {
+    typedef typename ZPrec<R>::cplx C2;
+    if (m <= 0 || n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20)) return OMX_ERR_UNSUPPORTED;
+    // A complex64 gradient of an order that is no multiple of 8 stays in three passes: their roundings of
+    // the intermediate results to FP32 are part of a solve's trajectory (one product instead moves an
+    // energy by 3e-6 within 20 CG steps).
+    if (NPAIR == 2 && sizeof(R) == 4 && k % ZBK != 0) return OMX_ERR_UNSUPPORTED;
+    const int sym = (NPAIR == 1 && m == n && !TRA && TRB && CJB) ? ctx->gemm_sym : 0;
+    const int nsl = NPAIR * ((k + ZGeo<R>::DK - 1) / ZGeo<R>::DK);
+    int tile, splits;
+    // batched launches never split K: no workspace, so the launch can be graph-captured
+    zl_shape(ctx, m, n, nsl, sym != 0, nbatch, allow_split && nbatch == 1, tile, splits);
+    const int sps = (nsl + splits - 1) / splits;
+    splits = (nsl + sps - 1) / sps;
+    C2 *partial = nullptr;
+    if (splits > 1) {
+        int rc = ensure_ws(ctx, sizeof(C2) * (size_t)splits * m * n);
+        if (rc) return rc;
+        partial = (C2 *)ctx->ws;
+    }
+    const int64_t tiles = zl_tiles(m, n, tile, sym != 0);
+    OMX_REQUIRE(tiles < (1LL << 31), "complex product: grid too large");
+    const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM;
+    hipEvent_t ev;
+    prof_begin(ctx, cls, &ev);
+    prof_work(ctx, cls, nbatch * 8.0 * (sym ? sym_area(m, tile) : (double)m * n) * NPAIR * k,
+              nbatch * 2.0 * sizeof(R) * ((double)NPAIR * ((double)m * k + (double)k * n) +
+                                          (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
+    const dim3 grid((unsigned)tiles, nbatch, splits);
+#define OMX_ZL_RUN(CF)                                                                                              \
+    hipLaunchKernelGGL((k_zgemm_dl<R, CF, TRA, CJA, TRB, CJB, NPAIR>), grid, dim3(256), 0, ctx->stream, m, n, k, alpha, \
+                       (const C2 *)A1, (const C2 *)A2, lda, (const C2 *)B1, (const C2 *)B2, ldb, beta0,             \
+                       (const C2 *)C0, beta, (C2 *)C, ldc, sym, sps, partial, bat)
+    if (tile == 64)
+        OMX_ZL_RUN(Zl64);
+    else
+        OMX_ZL_RUN(Zl32);
+#undef OMX_ZL_RUN
+    if (partial)
+        hipLaunchKernelGGL((k_zl_reduce<R>), dim3((unsigned)std::min<int64_t>(((int64_t)m * n + 255) / 256, 8192)),
+                           dim3(256), 0, ctx->stream, m, n, sym, splits, partial, alpha, beta0, (const C2 *)C0, beta,
+                           (C2 *)C, ldc);
+    prof_end(ctx, cls, ev);
+    OMX_CHECK_HIP(hipGetLastError());
+    if (sym == 2) ctx->gemm_sym = 3;  // the upper triangle is written too
+    return OMX_OK;
+}
+
 template <typename R, bool TRA, bool CJA, bool TRB, bool CJB, int NPAIR>
 static int run_zgemm(omx_ctx ctx, int m, int n, int k, double alpha, const void *A1, const void *A2, int64_t lda,
                      const void *B1, const void *B2, int64_t ldb, double beta0, const void *C0, double beta, void *C,
                      int64_t ldc, int nbatch = 1, ZBatch bat = ZBatch(), bool allow_split = true) {
     typedef typename ZPrec<R>::cplx C2;
+    {
+        const int rc = run_zgemm_dl<R, TRA, CJA, TRB, CJB, NPAIR>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0,
+                                                                  beta, C, ldc, nbatch, bat, allow_split);
+        if (rc != OMX_ERR_UNSUPPORTED) return rc;
+        if (NPAIR == 2 && k % ZBK != 0) return rc;  // the staged pair's boundary must fall on a slice boundary
+    }
     const int full_tiles = ((m + ZBM - 1) / ZBM) * ((n + ZBN - 1) / ZBN);
     const int ktot = NPAIR * k;
     int splits = 1;
@@ -465,8 +820,9 @@ static int zgemm_herm_r(omx_ctx ctx, int n, int k, double alpha, const void *A, 
     ctx->gemm_sym = 2;
     int rc = run_zgemm<R, false, false, true, true, 1>(ctx, n, n, k, alpha, A, A, lda, B, B, ldb, 0.0, nullptr, 0.0,
                                                        C, ldc, nbatch, bat, allow_split);
+    const bool whole = ctx->gemm_sym == 3;  // the product wrote the upper triangle too
     ctx->gemm_sym = 0;
-    if (rc) return rc;
+    if (rc || whole) return rc;
     const int nt = (n + 31) / 32;
     hipLaunchKernelGGL(k_herm_mirror<R>, dim3(nt * (nt + 1) / 2, nbatch), dim3(256), 0, ctx->stream, n,
                        (typename ZPrec<R>::cplx *)C, ldc, bat);
@@ -500,7 +856,6 @@ int launch_zgemm_pair_batched(omx_ctx ctx, int dt, int m, int n, int k, double a
                               int64_t lda, int64_t sA, const void *B1, const void *B2, int64_t ldb, int64_t sB,
                               double beta0, const void *C0, double beta, void *C, int64_t ldc, int64_t sC, int nbatch,
                               const int *active) {
-    if (k % ZBK != 0) return OMX_ERR_UNSUPPORTED;
     ZBatch bat;
     bat.sA = sA;
     bat.sB = sB;
@@ -516,7 +871,6 @@ int launch_zgemm_pair_batched(omx_ctx ctx, int dt, int m, int n, int k, double a
 int launch_zgemm_pair(omx_ctx ctx, int dt, int m, int n, int k, double alpha, const void *A1, const void *A2,
                       int64_t lda, const void *B1, const void *B2, int64_t ldb, double beta0, const void *C0,
                       double beta, void *C, int64_t ldc) {
-    if (k % ZBK != 0) return OMX_ERR_UNSUPPORTED;  // the pair boundary must fall on a slice boundary
     if (dt == OMX_C128)
         return run_zgemm<double, false, false, false, false, 2>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0,
                                                                 C0, beta, C, ldc);
