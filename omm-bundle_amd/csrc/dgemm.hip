@@ -63,6 +63,12 @@ __device__ inline int64_t dl_left(int extent, int k, int i0, int64_t ld) {
     return 8 * (KC ? (int64_t)(extent - 1 - i0) * ld + k : (int64_t)(k - 1) * ld + (extent - i0));
 }
 
+// Batched products: blockIdx.y selects the product, its operands and result offset by these strides
+// (elements; single products only, no split of K).
+struct DlBatch {
+    int64_t sA = 0, sB = 0, sC = 0;
+};
+
 // EXACT: m, n are multiples of the tile and k of the slice, so nothing needs the descriptors' end, a
 // cleared tail or guarded stores; the 128x128 tile is faster without them (8192 x 8192 x 16384 Gram 29.8
 // against 29.9 ms, gradient 60.4 against 61.6 ms).
@@ -73,10 +79,10 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
                                                                const double *__restrict__ B1,
                                                                const double *__restrict__ B2, int64_t ldb,
                                                                double beta0, const double *__restrict__ C0,
-                                                               double beta, double *__restrict__ C, int64_t ldc,
-                                                               int sym, int tbase, int nsplit, int sps,
+                                                               int64_t ldc0, double beta, double *__restrict__ C,
+                                                               int64_t ldc, int sym, int tbase, int nsplit, int sps,
                                                                double *__restrict__ partial,
-                                                               const int *__restrict__ mask) {
+                                                               const int *__restrict__ mask, DlBatch bat) {
     constexpr int BM = CF::BM, BN = CF::BN, NST = CF::NST, NW = CF::WGM * CF::WGN;
     constexpr int INS = DK * (BM + BN) / 128, LPW = INS / NW, U = CF::U;
     constexpr int SLICE = DK * (BM + BN), STAGE = U * SLICE;
@@ -84,6 +90,9 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
     static_assert(LPW * NW == INS && BM == BN && NW % 2 == 0, "each wave loads one operand");
     __shared__ __align__(16) double smem[NST * STAGE];
     if (mask && !*mask) return;  // system masked off (grouped solver; whole workgroup, before any barrier)
+    A1 += blockIdx.y * bat.sA;
+    B1 += blockIdx.y * bat.sB;
+    C += blockIdx.y * bat.sC;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave / CF::WGN, wn = wave % CF::WGN;
     // tile w of the launch's tile order and the part z of K it takes
@@ -225,7 +234,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
                 const int j = wj + fn * 16 + lq + 4 * v;
                 if ((!EXACT && j >= n) || (sym && j > i)) continue;
                 double r = alpha * acc[fm][fn][v];
-                if (C0) r += beta0 * C0[(int64_t)i + (int64_t)j * ldc];
+                if (C0) r += beta0 * C0[(int64_t)i + (int64_t)j * ldc0];
                 if (beta != 0.0) r += beta * C[(int64_t)i + (int64_t)j * ldc];
                 C[(int64_t)i + (int64_t)j * ldc] = r;
                 if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = r;
@@ -238,8 +247,8 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void k_dl_split_reduce(int m, int n, int sym, int tbase, int nsplit,
                                                          const double *__restrict__ partial, double alpha,
-                                                         double beta0, const double *__restrict__ C0, double beta,
-                                                         double *__restrict__ C, int64_t ldc) {
+                                                         double beta0, const double *__restrict__ C0, int64_t ldc0,
+                                                         double beta, double *__restrict__ C, int64_t ldc) {
     int tm, tn;
     if (sym)
         tile_of_lower(tbase + (int)blockIdx.x, (m + BM - 1) / BM, tm, tn);
@@ -254,7 +263,7 @@ __global__ __launch_bounds__(256) void k_dl_split_reduce(int m, int n, int sym, 
         for (int zz = 0; zz < nsplit; ++zz) sum += pt[(int64_t)zz * (BM * BN) + e];
         const int64_t off = (int64_t)i + (int64_t)j * ldc;
         double r = alpha * sum;
-        if (C0) r += beta0 * C0[off];
+        if (C0) r += beta0 * C0[(int64_t)i + (int64_t)j * ldc0];
         if (beta != 0.0) r += beta * C[off];
         C[off] = r;
         if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = r;
@@ -291,12 +300,13 @@ static int dl_tail_parts(omx_ctx ctx, int m, int tiles, bool sym, int nsl) {
     return parts;
 }
 static const int kDlEdge[3] = {128, 64, 32};
-static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int splits) {
+static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int splits,
+                      int nbatch) {
     const double slice[3] = {1.90, 0.515, 0.172};  // a CU's time for one 16-wide slice of a tile
     const double alone[3] = {2.15, 0.69, 0.172};   // the same with a single workgroup on the CU
-    const int units = tiles_of(m, n, kDlEdge[q], sym) * splits, rounds = (units + ctx->num_cus - 1) / ctx->num_cus;
+    const int units = tiles_of(m, n, kDlEdge[q], sym) * splits * nbatch, rounds = (units + ctx->num_cus - 1) / ctx->num_cus;
     const int sps = (nsl + splits - 1) / splits;
-    const int tail = dl_tail_parts(ctx, q == 0 && splits == 1 ? m : 1, units, sym, nsl);
+    const int tail = dl_tail_parts(ctx, q == 0 && splits == 1 && nbatch == 1 ? m : 1, units, sym, nsl);
     if (tail > 1) {
         const int whole = units / (2 * ctx->num_cus) * 2;  // two workgroups of every round share a CU
         return 9.8 + 0.55 * whole + slice[q] * (whole * sps + 2.0 * sps / tail);
@@ -304,11 +314,11 @@ static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int s
     return 4.5 + 0.55 * rounds + std::max(slice[q] * rounds, alone[q]) * sps +
            (splits > 1 ? 5.3 + 8e-6 * (splits + 1) * m * n / 4.9 : 0.0);
 }
-static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, double *cost = nullptr) {
+static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, double *cost = nullptr) {
     int best = 0;
     double c = 0.0;
     for (int q = 0; q < 3; ++q) {
-        const double t = dl_cost(ctx, q, sym, m, n, nsl, splits);
+        const double t = dl_cost(ctx, q, sym, m, n, nsl, splits, nbatch);
         if (!q || t < c) {
             best = q;
             c = t;
@@ -327,8 +337,8 @@ int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl) {
     for (int s : {1, 2, 3, 4, 5, 6, 8, 12}) {
         if (s > 1 && nsl < 2 * s) break;
         double t, u = 0.0;
-        dl_tile(ctx, false, m, n, nsl, s, &t);
-        if (m == n) dl_tile(ctx, true, m, n, nsl, s, &u);
+        dl_tile(ctx, false, m, n, nsl, s, 1, &t);
+        if (m == n) dl_tile(ctx, true, m, n, nsl, s, 1, &u);
         if (s == 1 || t + u < cost) {
             best = s;
             cost = t + u;
@@ -340,7 +350,8 @@ int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl) {
 template <class CF, bool TRA, bool TRB, int NPAIR>
 static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int k, double alpha, const double *A1,
                     const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
-                    const double *C0, double beta, double *C, int64_t ldc) {
+                    const double *C0, int64_t ldc0, double beta, double *C, int64_t ldc, int nbatch,
+                    const DlBatch &bat) {
     const int tiles = tiles_of(m, n, CF::BM, sym != 0);
     const int nsl = NPAIR * ((k + DK - 1) / DK);
     int whole = tiles, rest = 0, rsplit = 1;
@@ -355,13 +366,13 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
     }
     auto launch = [&](int grid, int tbase, int parts, int per, double *partial, const int *mask) {
         if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
-            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, CF::BM == 128>), dim3(grid), dim3(CF::NT), 0, ctx->stream,
-                               m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, sym, tbase, parts, per,
-                               partial, mask);
+            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, CF::BM == 128>), dim3(grid, nbatch), dim3(CF::NT), 0,
+                               ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
+                               tbase, parts, per, partial, mask, bat);
         else
-            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, false>), dim3(grid), dim3(CF::NT), 0, ctx->stream, m, n,
-                               k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, sym, tbase, parts, per,
-                               partial, mask);
+            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, false>), dim3(grid, nbatch), dim3(CF::NT), 0,
+                               ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
+                               tbase, parts, per, partial, mask, bat);
     };
     if (whole) launch(whole, 0, 1, nsl, nullptr, ctx->launch_mask);
     if (rest) {
@@ -369,8 +380,8 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
         if (rc) return rc;
         launch(rest * rsplit, whole, rsplit, sps, (double *)ctx->ws, nullptr);
         hipLaunchKernelGGL((k_dl_split_reduce<CF::BM, CF::BN>), dim3(rest, CF::BM * CF::BN / 1024), dim3(256), 0,
-                           ctx->stream, m, n, sym, whole, rsplit, (const double *)ctx->ws, alpha, beta0, C0, beta, C,
-                           ldc);
+                           ctx->stream, m, n, sym, whole, rsplit, (const double *)ctx->ws, alpha, beta0, C0,
+                           ldc0, beta, C, ldc);
     }
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
@@ -378,15 +389,15 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
 
 template <bool TRA, bool TRB, int NPAIR>
 static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const double *A1, const double *A2, int64_t lda,
-                   const double *B1, const double *B2, int64_t ldb, double beta0, const double *C0, double beta,
-                   double *C, int64_t ldc) {
+                   const double *B1, const double *B2, int64_t ldb, double beta0, const double *C0, int64_t ldc0,
+                   double beta, double *C, int64_t ldc, int nbatch = 1, const DlBatch &bat = DlBatch()) {
     const int sym = (m == n && NPAIR == 1 && !TRA && TRB) ? ctx->gemm_sym : 0;
     const int nsl = NPAIR * ((k + DK - 1) / DK);
-    int splits = dgemm_k_splits(ctx, m, n, nsl);
+    int splits = nbatch > 1 ? 1 : dgemm_k_splits(ctx, m, n, nsl);
     const int sps = (nsl + splits - 1) / splits;
     splits = (nsl + sps - 1) / sps;
     const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM;
-    const int tile = dl_tile(ctx, sym != 0, m, n, nsl, splits);
+    const int tile = dl_tile(ctx, sym != 0, m, n, nsl, splits, nbatch);
     hipEvent_t ev;
     prof_begin(ctx, cls, &ev);
     prof_work(ctx, cls, 2.0 * (sym ? sym_area(m, kDlEdge[tile]) : (double)m * n) * (double)NPAIR * k,
@@ -394,7 +405,8 @@ static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const double 
                                 (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
     int rc;
 #define OMX_DL_RUN(CF) \
-    run_tile<CF, TRA, TRB, NPAIR>(ctx, sym, splits, sps, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc)
+    run_tile<CF, TRA, TRB, NPAIR>(ctx, sym, splits, sps, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, \
+                                  nbatch, bat)
     if (tile == 0)
         rc = OMX_DL_RUN(Dl128);
     else if (tile == 1)
@@ -409,18 +421,27 @@ static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const double 
 
 int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const double *A1,
                  const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
-                 const double *C0, double beta, double *C, int64_t ldc) {
+                 const double *C0, int64_t ldc0, double beta, double *C, int64_t ldc) {
     if (m <= 0 || n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20))  // 32-bit lane offsets
         return OMX_ERR_UNSUPPORTED;
-    if (npair == 2)
-        return run_ops<false, false, 2>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
-    if (!trA && !trB)
-        return run_ops<false, false, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
-    if (!trA && trB)
-        return run_ops<false, true, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
-    if (trA && !trB)
-        return run_ops<true, false, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
-    return run_ops<true, true, 1>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc);
+#define OMX_DL_OPS(TA, TB, NP) \
+    run_ops<TA, TB, NP>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc)
+    if (npair == 2) return OMX_DL_OPS(false, false, 2);
+    if (!trA && !trB) return OMX_DL_OPS(false, false, 1);
+    if (!trA && trB) return OMX_DL_OPS(false, true, 1);
+    if (trA && !trB) return OMX_DL_OPS(true, false, 1);
+    return OMX_DL_OPS(true, true, 1);
+#undef OMX_DL_OPS
+}
+
+int launch_dgemm_batched(omx_ctx ctx, int m, int n, int k, double alpha, const double *A, int64_t lda, int64_t sA,
+                         const double *B, int64_t ldb, int64_t sB, double *C, int64_t ldc, int64_t sC, int nbatch) {
+    if (m <= 0 || n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20) || nbatch > 65535) return OMX_ERR_UNSUPPORTED;
+    DlBatch bat;
+    bat.sA = sA;
+    bat.sB = sB;
+    bat.sC = sC;
+    return run_ops<false, false, 1>(ctx, m, n, k, alpha, A, A, lda, B, B, ldb, 0.0, nullptr, 0, 0.0, C, ldc, nbatch, bat);
 }
 
 }  // namespace omx

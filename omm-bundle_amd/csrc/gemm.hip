@@ -610,8 +610,8 @@ static int run_cfg_id(int id, omx_ctx ctx, int m, int n, int k, double alpha, co
     typedef CfgSet<TS, PREC, TRA, TRB, NPAIR> CS;
     if constexpr (CS::dl) {
         if (id == 7) {
-            int rc = launch_dgemm(ctx, TRA, TRB, NPAIR, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C,
-                                  ldc);
+            int rc = launch_dgemm(ctx, TRA, TRB, NPAIR, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc, beta,
+                                  C, ldc);
             if (rc != OMX_ERR_UNSUPPORTED) return rc;
             id = 5;  // the staged kernel (5 tiles; 0 with A transposed) for leading dimensions beyond 2^20
         }
@@ -1214,7 +1214,7 @@ int launch_gemm_pair(omx_ctx ctx, int prec, int dt, int m, int n, int k, double 
     if (k % bk != 0) {
         if (dt == OMX_F64 && prec == OMX_PREC_F64 && (ctx->gemm_cfg < 0 || ctx->gemm_cfg == 7))
             return launch_dgemm(ctx, false, false, 2, m, n, k, alpha, (const double *)A1, (const double *)A2, lda,
-                                (const double *)B1, (const double *)B2, ldb, beta0, (const double *)C0, beta,
+                                (const double *)B1, (const double *)B2, ldb, beta0, (const double *)C0, ldc, beta,
                                 (double *)C, ldc);
         return OMX_ERR_UNSUPPORTED;
     }

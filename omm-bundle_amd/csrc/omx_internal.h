@@ -226,7 +226,10 @@ int launch_gemm(omx_ctx ctx, int prec, int dt, bool trA, bool trB, int m, int n,
 // launched) for leading dimensions beyond 2^20.
 int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const double *A1,
                  const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
-                 const double *C0, double beta, double *C, int64_t ldc);
+                 const double *C0, int64_t ldc0, double beta, double *C, int64_t ldc);
+// nbatch products C_b := alpha*A_b*B_b ('n','n') at strides sA, sB, sC elements.
+int launch_dgemm_batched(omx_ctx ctx, int m, int n, int k, double alpha, const double *A, int64_t lda, int64_t sA,
+                         const double *B, int64_t ldb, int64_t sB, double *C, int64_t ldc, int64_t sC, int nbatch);
 // Parts K is split into for an FP64 product of nsl slices of 16; a function of the shape alone, so that
 // every tile configuration and the symmetric form add in the same order.
 int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl);
