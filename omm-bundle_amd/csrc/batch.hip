@@ -361,11 +361,8 @@ static int batch_step(omx_zbatch b) {
     int rc;
     hipLaunchKernelGGL(k_batch_direction<T>, bt_grid(lenC, ns), dim3(BT_NT), 0, ctx->stream, lenC, (const T *)b->G,
                        (T *)b->D, (T *)b->Gp, b->sc, act);
-    if ((rc = launch_spmm_z_batched(ctx, dt, no, nb, b->nbc, b->colptr, b->rowidx, b->hval, sV, b->D, no, lenC, b->HG,
-                                    no, lenC, ns, act)))
-        return rc;
-    if ((rc = launch_spmm_z_batched(ctx, dt, no, nb, b->nbc, b->colptr, b->rowidx, b->sval, sV, b->D, no, lenC, b->SG,
-                                    no, lenC, ns, act)))
+    if ((rc = launch_spmm_z_batched(ctx, dt, no, nb, b->nbc, b->colptr, b->rowidx, b->hval, b->sval, sV, b->D, no, lenC,
+                                    b->HG, b->SG, no, lenC, ns, act)))
         return rc;
     const void *src[4] = {b->HC, b->SC, b->HG, b->SG};
     void *dst[4] = {b->HWd, b->SWd, b->HWdd, b->SWdd};
@@ -523,11 +520,8 @@ int omx_zbatch_solve(omx_zbatch b, double eta, double cg_tol, int max_steps, int
     hipLaunchKernelGGL(k_batch_init_flags, dim3((ns + 63) / 64), dim3(64), 0, st, ns, flag(b, F_ACTIVE),
                        flag(b, F_ICG), flag(b, F_CONV), flag(b, F_NFAIL), b->sc, tol, max_steps);
     int *act = flag(b, F_ACTIVE);
-    if ((rc = launch_spmm_z_batched(ctx, b->dt, no, nb, b->nbc, b->colptr, b->rowidx, b->hval, sV, b->C, no, lenC, b->HC, no,
-                                    lenC, ns, act)))
-        return rc;
-    if ((rc = launch_spmm_z_batched(ctx, b->dt, no, nb, b->nbc, b->colptr, b->rowidx, b->sval, sV, b->C, no, lenC, b->SC, no,
-                                    lenC, ns, act)))
+    if ((rc = launch_spmm_z_batched(ctx, b->dt, no, nb, b->nbc, b->colptr, b->rowidx, b->hval, b->sval, sV, b->C, no, lenC,
+                                    b->HC, b->SC, no, lenC, ns, act)))
         return rc;
     if ((rc = launch_zgemm_herm_batched(ctx, b->dt, no, nb, 1.0, b->HC, no, lenC, b->C, no, lenC, b->HW, no, lenW, ns,
                                         act)))

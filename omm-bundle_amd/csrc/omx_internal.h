@@ -51,7 +51,7 @@ struct ProfEvent {
 // contiguous rows; 1: each XCD walks one row chunk at a time).
 struct omx_spmm_shape_s {
     int batch = 4;
-    int wpg = 4;
+    int wpg = 1;
     int jper = 1;
     int mode = 1;
 };
@@ -267,8 +267,8 @@ int launch_zgemm_pair_batched(omx_ctx ctx, int dt, int m, int n, int k, double a
 
 // Batched pieces of the k-point solver (complex128 or complex64, systems sharing one block pattern).
 int launch_spmm_z_batched(omx_ctx ctx, int dt, int no, int nb, int nbc, const int *colptr, const int *rowidx,
-                          const double *val, int64_t sV, const void *X, int64_t ldx, int64_t sX, void *Y, int64_t ldy,
-                          int64_t sY, int nbatch, const int *active);
+                          const double *val, const double *val2, int64_t sV, const void *X, int64_t ldx, int64_t sX,
+                          void *Y, void *Y2, int64_t ldy, int64_t sY, int nbatch, const int *active);
 // Line-search coefficients (to out[18*s ...]: the 5 coefficients, then the 13 traces) and
 // Polak-Ribiere dots (to out2[2*s ...]) of nbatch systems of element type dt, on the device; a
 // system s with mask && !mask[s] is skipped.

@@ -7,19 +7,32 @@
 //     Y(:,4J+c) = sum over blocks (I,J), r = 0..3 of X(:,4I+r) * A_IJ(r,c),
 // summed in ascending (I, r), the order of the reference's CSC loop.
 //
-// Mapping: a workgroup owns a chunk of RC = 64*VEC*WPG consecutive states (its WPG waves are
-// stacked in rows, each lane loading one 8- or 16-byte vector per basis column) and a run of jper
-// block columns, taken in walk order (the identity, or an order attached to the operator that
-// keeps the basis columns a block column gathers close in time to their other uses, e.g. the
-// lattice in x-y tiles).  Each lane keeps 4*VEC accumulators and issues the loads of a whole
-// batch of NB blocks before using them (memory-level parallelism); the 16 block values are
-// wave-uniform and come through the scalar cache.  Workgroup ids are dealt round-robin over the 8
-// XCDs, and the id -> (row chunk, block-column run) map is XCD-aware:
+// Mapping: a workgroup of four waves owns a chunk of RC = 64*VEC*WPG consecutive states (WPG waves
+// stacked in rows, each lane loading one 8- or 16-byte vector per basis column; the other waves take
+// the neighbouring block columns) and a run of jper block columns per wave, taken in walk order (the
+// identity, or an order attached to the operator that keeps the basis columns a block column gathers
+// close in time to their other uses, e.g. the lattice in x-y tiles).  Each lane keeps 4*VEC
+// accumulators and issues the loads of a whole batch of NB blocks before using them (memory-level
+// parallelism); the 16 block values are wave-uniform and come through the scalar cache.  Workgroup
+// ids are dealt round-robin over the 8 XCDs, and the id -> (row chunk, block-column run) map is
+// XCD-aware:
 //   mode 0: XCD x owns a contiguous eighth of the row chunks and cycles through them for one
 //           block-column run before the next, so the chip reads whole basis columns at once;
 //   mode 1: XCD x owns chunks x, x+8, ... and walks every block column of one chunk before the
 //           next, so an XCD's L2 holds the neighbourhood of the current block columns of a
 //           single chunk.
+// Of the chunks left over (their number mod 8) every XCD walks an eighth of the block columns.
+//
+// What bounds it is how often a basis column crosses from memory into an L2: a column is gathered by
+// seven block columns (a lattice operator), up to two lattice planes apart.  The default is therefore
+// the narrowest chunk (WPG = 1: 1 KB per basis column, so three planes of 256 sites are 3 MB of a 4 MB
+// L2) in mode 1, with large results stored past the L2 (spmm_nt); no load is predicated, and any number
+// of states, leading dimension and alignment takes 16-byte vectors.  Measured, default shapes, us
+// (before: WPG = 4, chunk counts that 8 does not divide spread over all L2s, predicated loads, scalar
+// access unless everything divides and aligns):
+//   FP64  8192 x 16384  797 -> 590    4394 x 8788  332 -> 182    2611 x 5280  128 -> 62   54 x 108  6.5 -> 4.9
+//   FP32  8192 x 16384  427 -> 300    4394 x 8788  179 -> 107    2611 x 5280   72 -> 39   250 x 500 5.1 -> 5.0
+// The copy rate of the card allows 419 and 209 us at the largest size.
 // A zero entry stored inside a block contributes an exact zero, so the per-element sum equals
 // the reference's CSC sum over its stored entries.
 #include <algorithm>
@@ -70,6 +83,35 @@ __device__ inline void vstore(T *p, const T (&in)[VEC]) {
     *reinterpret_cast<V *>(p) = v;
 }
 
+// The same for vectors aligned only to their elements: one 8- or 16-byte access all the same.
+template <typename T, int VEC>
+struct UVec {
+    typedef T type __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+};
+template <typename T>
+struct UVec<T, 1> {
+    typedef T type;
+};
+template <typename T, int VEC>
+__device__ inline void uload(const T *p, T (&out)[VEC]) {
+    const typename UVec<T, VEC>::type u = *reinterpret_cast<const typename UVec<T, VEC>::type *>(p);
+    __builtin_memcpy(out, &u, sizeof out);
+}
+// nt: past the caches (spmm_nt)
+template <typename T, int VEC>
+__device__ inline void ustore(T *p, const T (&in)[VEC], int nt) {
+    typename UVec<T, VEC>::type u;
+    __builtin_memcpy(&u, in, sizeof in);
+    typename UVec<T, VEC>::type *q = reinterpret_cast<typename UVec<T, VEC>::type *>(p);
+    if (nt) {  // the empty statements keep the compiler from merging the two stores into a plain one
+        asm volatile("");
+        __builtin_nontemporal_store(u, q);
+        asm volatile("");
+    } else {
+        *q = u;
+    }
+}
+
 // y := alpha*acc + beta*y_old in FP64 with one explicit rounding sequence (product, then a fused
 // multiply-add), so that every SpMM kernel rounds the epilogue identically whatever the compiler's
 // contraction choices.
@@ -80,37 +122,44 @@ __device__ inline T spmm_out(double alpha, T acc, double beta, T old) {
 }
 
 template <typename T, int VEC, int NB, int WPG>
-__global__ __launch_bounds__(64 * WPG) void k_spmm_bsr4(int no, int nb, int nbc, double alpha,
-                                                      const T *__restrict__ X, int64_t ldx,
-                                                      const int *__restrict__ colptr, const int *__restrict__ rowidx,
-                                                      const double *__restrict__ val, double beta,
-                                                      T *__restrict__ Y, int64_t ldy, int nrc, int njg, int jper,
-                                                      int mode, const int *__restrict__ walk,
-                                                      const int *__restrict__ mask) {
-    constexpr int RC = 64 * VEC * WPG;
+__global__ __launch_bounds__(256) void k_spmm_bsr4(int no, int nb, int nbc, double alpha,
+                                                 const T *__restrict__ X, int64_t ldx,
+                                                 const int *__restrict__ colptr, const int *__restrict__ rowidx,
+                                                 const double *__restrict__ val, double beta,
+                                                 T *__restrict__ Y, int64_t ldy, int nrc, int njg, int jper,
+                                                 int mode, int nt, const int *__restrict__ walk,
+                                                 const int *__restrict__ mask) {
+    constexpr int RC = 64 * VEC * WPG, WJ = 4 / WPG;
     if (mask && !*mask) return;
-    const int w = blockIdx.x;
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;  // dispatch is round-robin over 8 XCDs
+    const int per = nrc >> 3, rest = nrc & 7;
     int rc, jg;
-    if ((nrc & 7) == 0) {
-        const int xcd = w & 7, local = w >> 3;  // dispatch is round-robin over 8 XCDs
+    if (local < per * njg) {
         if (mode == 0) {
-            const int per = nrc >> 3;
             rc = xcd * per + local % per;
             jg = local / per;
         } else {
             rc = (local / njg) * 8 + xcd;
             jg = local % njg;
         }
-    } else {
-        rc = w % nrc;
-        jg = w / nrc;
+    } else {  // the last nrc % 8 chunks: an eighth of the block columns of each on every XCD
+        const int e = local - per * njg, eighth = (njg + 7) >> 3;
+        rc = per * 8 + e / eighth;
+        jg = xcd * eighth + e % eighth;
+        if (rc >= nrc || jg >= njg) return;  // whole workgroup
     }
-    const int i0 = rc * RC + threadIdx.x * VEC;
-    const bool full = (i0 + VEC <= no);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform block columns
+    const int i0 = rc * RC + (threadIdx.x & 63) * VEC + (wave % WPG) * 64 * VEC;
+    // Every lane loads a whole vector (no >= VEC): one that would end past the last state is moved back to
+    // end there, so no load is predicated; of such a vector the first `skip` states belong to the lane
+    // before and are not stored.
+    const int at = min(i0, no - VEC), skip = i0 - at;
     const bool any = (i0 < no);
-    const int jbeg = jg * jper, jend = min(nbc, jbeg + jper);
+    X += at;
+    Y += at;
+    const int jbeg = jg * jper * WJ, jend = min(nbc, jbeg + jper * WJ);
 
-    for (int jj = jbeg; jj < jend; ++jj) {
+    for (int jj = jbeg + wave / WPG; jj < jend; jj += WJ) {
         const int J = walk ? walk[jj] : jj;
         T acc[4][VEC];
 #pragma unroll
@@ -124,27 +173,25 @@ __global__ __launch_bounds__(64 * WPG) void k_spmm_bsr4(int no, int nb, int nbc,
         for (int l0 = lb; l0 < le; l0 += NB) {
             const int nblk = min(NB, le - l0);
             T x[NB][4][VEC];
+            int I[NB];
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 if (b < nblk) {
-                    const int I = rowidx[l0 + b];
+                    I[b] = rowidx[l0 + b];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int kcol = 4 * I + r;
-                        const T *src = X + (int64_t)kcol * ldx + i0;
-                        if (kcol < nb && full) {
-                            vload<T, VEC>(src, x[b][r]);
-                        } else {
-#pragma unroll
-                            for (int q = 0; q < VEC; ++q)
-                                x[b][r][q] = (kcol < nb && any && i0 + q < no) ? src[q] : (T)0;
-                        }
-                    }
+                    for (int r = 0; r < 4; ++r)
+                        uload<T, VEC>(X + (int64_t)min(4 * I[b] + r, nb - 1) * ldx, x[b][r]);
                 }
             }
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 if (b < nblk) {
+                    if (4 * I[b] + 4 > nb) {  // the last block row ends at nb: no basis columns past it
+#pragma unroll
+                        for (int r = 1; r < 4; ++r)
+#pragma unroll
+                            for (int q = 0; q < VEC; ++q) x[b][r][q] = 4 * I[b] + r < nb ? x[b][r][q] : (T)0;
+                    }
                     const double *v = val + 16 * (int64_t)(l0 + b);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
@@ -163,23 +210,23 @@ __global__ __launch_bounds__(64 * WPG) void k_spmm_bsr4(int no, int nb, int nbc,
         for (int c = 0; c < 4; ++c) {
             const int jcol = 4 * J + c;
             if (jcol >= nb) break;
-            T *dst = Y + (int64_t)jcol * ldy + i0;
+            T *dst = Y + (int64_t)jcol * ldy;
             T out[VEC];
-            if (full) {
-                if (beta != 0.0) {
-                    T old[VEC];
-                    vload<T, VEC>(dst, old);
+            if (beta != 0.0) {
+                T old[VEC];
+                uload<T, VEC>(dst, old);
 #pragma unroll
-                    for (int q = 0; q < VEC; ++q) out[q] = spmm_out(alpha, acc[c][q], beta, old[q]);
-                } else {
-#pragma unroll
-                    for (int q = 0; q < VEC; ++q) out[q] = spmm_out(alpha, acc[c][q], 0.0, (T)0);
-                }
-                vstore<T, VEC>(dst, out);
+                for (int q = 0; q < VEC; ++q) out[q] = spmm_out(alpha, acc[c][q], beta, old[q]);
             } else {
 #pragma unroll
-                for (int q = 0; q < VEC; ++q)
-                    if (i0 + q < no) dst[q] = spmm_out(alpha, acc[c][q], beta, beta != 0.0 ? dst[q] : (T)0);
+                for (int q = 0; q < VEC; ++q) out[q] = spmm_out(alpha, acc[c][q], 0.0, (T)0);
+            }
+            if (skip == 0) {
+                ustore<T, VEC>(dst, out, nt);
+            } else {
+#pragma unroll
+                for (int q = 1; q < VEC; ++q)
+                    if (q >= skip) dst[q] = out[q];
             }
         }
     }
@@ -451,16 +498,22 @@ static bool stencil_applies(const omx_ctx ctx, const omx_bsr A, int no, const T 
 
 typedef omx_spmm_shape_s SpmmShape;
 
+// Results go past the caches where they are more than the memory-side cache holds (256 MB), so that the
+// L2s keep the basis columns that later block columns gather (FP64, 8192 x 16384: 566 us against 535,
+// 4394 x 8788: 195 and 171); smaller results stay for the product that reads them next (complex128,
+// 2000 x 4000, SpMM and Gram: 1168 us against 1200).
+static int spmm_nt(double bytes) { return bytes > 256e6; }
+
 template <typename T, int VEC, int NB>
 static void launch_spmm(omx_ctx ctx, const SpmmShape &sh, int no, int nb, double alpha, const T *X, int64_t ldx,
                         omx_bsr A, double beta, T *Y, int64_t ldy) {
     const int nrc = (no + 64 * VEC * sh.wpg - 1) / (64 * VEC * sh.wpg);
-    const int njg = (A->nbc + sh.jper - 1) / sh.jper;
-    const unsigned grid = (unsigned)((int64_t)nrc * njg);
+    const int jg = sh.jper * (4 / sh.wpg), njg = (A->nbc + jg - 1) / jg;
+    const unsigned grid = (unsigned)(8 * ((int64_t)(nrc >> 3) * njg + (nrc & 7) * ((njg + 7) >> 3)));
 #define OMX_SPMM_LAUNCH(W)                                                                                       \
-    hipLaunchKernelGGL((k_spmm_bsr4<T, VEC, NB, W>), dim3(grid), dim3(64 * W), 0, ctx->stream, no, nb, A->nbc, \
+    hipLaunchKernelGGL((k_spmm_bsr4<T, VEC, NB, W>), dim3(grid), dim3(256), 0, ctx->stream, no, nb, A->nbc, \
                        alpha, X, ldx, A->d_colptr, A->d_rowidx, A->d_val, beta, Y, ldy, nrc, njg, sh.jper,   \
-                       sh.mode, A->d_walk, ctx->launch_mask)
+                       sh.mode, spmm_nt(sizeof(T) * (double)no * nb), A->d_walk, ctx->launch_mask)
     if (sh.wpg == 1)
         OMX_SPMM_LAUNCH(1);
     else if (sh.wpg == 2)
@@ -483,7 +536,7 @@ static void launch_spmm_shape(omx_ctx ctx, const SpmmShape &sh, int no, int nb, 
 
 static int64_t spmm_grid(const SpmmShape &sh, int rows_per_wave, int no, int nbc) {
     const int64_t nrc = (no + (int64_t)rows_per_wave * sh.wpg - 1) / ((int64_t)rows_per_wave * sh.wpg);
-    return nrc * ((nbc + sh.jper - 1) / sh.jper);
+    return (nrc + 8) * ((nbc + sh.jper - 1) / sh.jper + 8);
 }
 
 // Autotuner for the SpMM launch shape: the first time an operator shape is seen with tuning on,
@@ -732,109 +785,139 @@ static int run_spmm(omx_ctx ctx, int no, int nb, double alpha, const T *X, int64
     return OMX_OK;
 }
 
-// Complex operator and complex X, Y (interleaved (re, im), element type R per part): the same
-// band-major mapping; each lane holds VEC complex states.
-template <typename R, int VEC, int WPG>
+// Complex operator and complex X, Y (interleaved (re, im), element type R per part): each lane holds
+// VEC complex states, the workgroup's waves take neighbouring block columns of one 64*VEC-state band;
+// DUAL: the products with two operators of one block pattern, X read once.  Measured, complex128:
+// 2000 x 4000 165 -> 75 us (copy rate: 50), 701 x 1512 32 -> 13; complex64 2000 x 4000 83 -> 47 (before:
+// the block values loaded by every lane, since the block column came from the thread id, and loads
+// predicated).
+template <typename R, int VEC, int WPG, bool DUAL>
 __global__ __launch_bounds__(64 * WPG) void k_spmm_bsr4_z(int no, int nb, int nbc, double alpha,
                                                         const R *__restrict__ X, int64_t ldx,
                                                         const int *__restrict__ colptr, const int *__restrict__ rowidx,
                                                         const double *__restrict__ val, double beta,
-                                                        R *__restrict__ Y, int64_t ldy, int nbands, int jgroups,
-                                                        int64_t sX, int64_t sY, int64_t sV,
-                                                        const int *__restrict__ active) {
+                                                        R *__restrict__ Y, int64_t ldy, int nbands, int jgroups, int nt,
+                                                        int64_t sX, int64_t sY, int64_t sV, int nbatch,
+                                                        const int *__restrict__ active,
+                                                        const double *__restrict__ val2, R *__restrict__ Y2) {
     constexpr int ROWS = 64 * VEC;
-    constexpr int NB = 4;
-    // batched use: blockIdx.y selects the system (operator values, X and Y offset by its strides)
-    const int bsys = blockIdx.y;
-    if (active && !active[bsys]) return;
-    X += bsys * sX;
-    Y += bsys * sY;
-    val += bsys * sV;
-    const int w = blockIdx.x;
-    int band, jg;
-    if ((nbands & 7) == 0) {
-        const int xcd = w & 7, local = w >> 3;
-        band = (local / jgroups) * 8 + xcd;
-        jg = local % jgroups;
-    } else {
+    constexpr int NB = 4, NO = DUAL ? 2 : 1;
+    // ids are dealt round-robin over the 8 XCDs: a system of a batch (operator values, X and Y offset by
+    // its strides), else a row band, stays on one XCD
+    int w = blockIdx.x, band, jg, sys = 0;
+    if (nbatch > 1) {
+        const int per = nbands * jgroups;
+        if ((nbatch & 7) == 0) {
+            sys = (w >> 3) / per * 8 + (w & 7);
+            w = (w >> 3) % per;
+        } else {
+            sys = w / per;
+            w = w % per;
+        }
         band = w / jgroups;
         jg = w % jgroups;
+    } else {  // as in k_spmm_bsr4, mode 1
+        const int xcd = w & 7, local = w >> 3, whole = (nbands >> 3) * jgroups, eighth = (jgroups + 7) >> 3;
+        if (local < whole) {
+            band = (local / jgroups) * 8 + xcd;
+            jg = local % jgroups;
+        } else {
+            band = (nbands & ~7) + (local - whole) / eighth;
+            jg = xcd * eighth + (local - whole) % eighth;
+            if (band >= nbands || jg >= jgroups) return;
+        }
     }
-    const int J = jg * WPG + (threadIdx.x >> 6);
+    if (active && !active[sys]) return;
+    // wave-uniform, so that the block values come through the scalar cache
+    const int J = jg * WPG + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (J >= nbc) return;  // whole wave; the kernel has no barriers
-    const int i0 = band * ROWS + (threadIdx.x & 63) * VEC;
-    const bool full = (i0 + VEC <= no);
-    const bool any = (i0 < no);
-    R ar[4][VEC], ai[4][VEC];
+    // as in k_spmm_bsr4: a vector that would end past the last state is moved back
+    const int i0 = band * ROWS + (threadIdx.x & 63) * VEC, at = min(i0, no - VEC), skip = i0 - at;
+    X += sys * sX + 2 * at;
+    const double *const vals[2] = {val + sys * sV, DUAL ? val2 + sys * sV : nullptr};
+    R *const out[2] = {Y + sys * sY + 2 * at, DUAL ? Y2 + sys * sY + 2 * at : nullptr};
+    R ar[NO][4][VEC], ai[NO][4][VEC];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int o = 0; o < NO; ++o)
 #pragma unroll
-        for (int q = 0; q < VEC; ++q) ar[c][q] = ai[c][q] = (R)0;
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int q = 0; q < VEC; ++q) ar[o][c][q] = ai[o][c][q] = (R)0;
     const int lb = colptr[J], le = colptr[J + 1];
     for (int l0 = lb; l0 < le; l0 += NB) {
         const int nblk = min(NB, le - l0);
-        R xr[NB][4][VEC], xi[NB][4][VEC];
+        R x[NB][4][2 * VEC];
+        int I[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             if (b < nblk) {
-                const int I = rowidx[l0 + b];
+                I[b] = rowidx[l0 + b];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int kcol = 4 * I + r;
-                    const R *src = X + 2 * ((int64_t)kcol * ldx + i0);
-                    R tmp[2 * VEC];
-                    if (kcol < nb && full) {
-                        vload<R, 2 * VEC>(src, tmp);
-                    } else {
+                for (int r = 0; r < 4; ++r)
+                    uload<R, 2 * VEC>(X + 2 * (int64_t)min(4 * I[b] + r, nb - 1) * ldx, x[b][r]);
+            }
+        }
 #pragma unroll
-                        for (int q = 0; q < 2 * VEC; ++q) tmp[q] = (kcol < nb && any && i0 + q / 2 < no) ? src[q] : (R)0;
-                    }
+        for (int b = 0; b < NB; ++b) {
+            if (b < nblk) {
+                if (4 * I[b] + 4 > nb) {  // the last block row ends at nb: no basis columns past it
 #pragma unroll
-                    for (int q = 0; q < VEC; ++q) {
-                        xr[b][r][q] = tmp[2 * q];
-                        xi[b][r][q] = tmp[2 * q + 1];
-                    }
+                    for (int r = 1; r < 4; ++r)
+#pragma unroll
+                        for (int q = 0; q < 2 * VEC; ++q) x[b][r][q] = 4 * I[b] + r < nb ? x[b][r][q] : (R)0;
+                }
+#pragma unroll
+                for (int o = 0; o < NO; ++o) {
+                    const double *v = vals[o] + 32 * (int64_t)(l0 + b);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            const R vr = (R)v[2 * (r + 4 * c)], vi = (R)v[2 * (r + 4 * c) + 1];
+#pragma unroll
+                            for (int q = 0; q < VEC; ++q) {
+                                const R xr = x[b][r][2 * q], xi = x[b][r][2 * q + 1];
+                                ar[o][c][q] = fma(xr, vr, ar[o][c][q]);
+                                ar[o][c][q] = fma(-xi, vi, ar[o][c][q]);
+                                ai[o][c][q] = fma(xr, vi, ai[o][c][q]);
+                                ai[o][c][q] = fma(xi, vr, ai[o][c][q]);
+                            }
+                        }
                 }
             }
         }
+    }
+    if (i0 >= no) return;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            if (b < nblk) {
-                const double *v = val + 32 * (int64_t)(l0 + b);
+    for (int o = 0; o < NO; ++o)
 #pragma unroll
-                for (int r = 0; r < 4; ++r)
+        for (int c = 0; c < 4; ++c) {
+            const int jcol = 4 * J + c;
+            if (jcol >= nb) break;
+            R *dst = out[o] + 2 * (int64_t)jcol * ldy;
+            R res[2 * VEC], old[2 * VEC];
+            if (beta != 0.0) uload<R, 2 * VEC>(dst, old);
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        const R vr = (R)v[2 * (r + 4 * c)], vi = (R)v[2 * (r + 4 * c) + 1];
+            for (int q = 0; q < VEC; ++q) {
+                double orr = alpha * (double)ar[o][c][q], oii = alpha * (double)ai[o][c][q];
+                if (beta != 0.0) {
+                    orr += beta * (double)old[2 * q];
+                    oii += beta * (double)old[2 * q + 1];
+                }
+                res[2 * q] = (R)orr;
+                res[2 * q + 1] = (R)oii;
+            }
+            if (skip == 0) {
+                ustore<R, 2 * VEC>(dst, res, nt);
+            } else {
 #pragma unroll
-                        for (int q = 0; q < VEC; ++q) {
-                            ar[c][q] = fma(xr[b][r][q], vr, ar[c][q]);
-                            ar[c][q] = fma(-xi[b][r][q], vi, ar[c][q]);
-                            ai[c][q] = fma(xr[b][r][q], vi, ai[c][q]);
-                            ai[c][q] = fma(xi[b][r][q], vr, ai[c][q]);
-                        }
+                for (int q = 1; q < VEC; ++q)
+                    if (q >= skip) {
+                        dst[2 * q] = res[2 * q];
+                        dst[2 * q + 1] = res[2 * q + 1];
                     }
             }
         }
-    }
-    if (!any) return;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        const int jcol = 4 * J + c;
-        if (jcol >= nb) break;
-        R *dst = Y + 2 * ((int64_t)jcol * ldy + i0);
-#pragma unroll
-        for (int q = 0; q < VEC; ++q) {
-            if (!full && i0 + q >= no) continue;
-            double orr = alpha * (double)ar[c][q], oii = alpha * (double)ai[c][q];
-            if (beta != 0.0) {
-                orr += beta * (double)dst[2 * q];
-                oii += beta * (double)dst[2 * q + 1];
-            }
-            dst[2 * q] = (R)orr;
-            dst[2 * q + 1] = (R)oii;
-        }
-    }
 }
 
 template <typename R, int VEC>
@@ -843,44 +926,49 @@ static int run_spmm_z(omx_ctx ctx, int no, int nb, double alpha, const R *X, int
     constexpr int ROWS = 64 * VEC, WPG = 4;
     const int nbands = (no + ROWS - 1) / ROWS;
     const int jgroups = (A->nbc + WPG - 1) / WPG;
-    const int64_t total = (int64_t)nbands * jgroups;
+    const int64_t total = 8 * ((int64_t)(nbands >> 3) * jgroups + (nbands & 7) * ((jgroups + 7) >> 3));
     OMX_REQUIRE(total < (1LL << 31), "omx_spmm: grid too large");
     hipEvent_t ev;
     prof_begin(ctx, OMX_K_SPMM, &ev);
     prof_work(ctx, OMX_K_SPMM, 8.0 * 16.0 * A->nnzb * no,
               2.0 * sizeof(R) * 2.0 * (double)no * nb * (beta != 0.0 ? 1.5 : 1.0) + A->nnzb * (32.0 * 8 + 4) +
                   4.0 * (A->nbc + 1));
-    hipLaunchKernelGGL((k_spmm_bsr4_z<R, VEC, WPG>), dim3((unsigned)total), dim3(64 * WPG), 0, ctx->stream, no, nb,
-                       A->nbc, alpha, X, ldx, A->d_colptr, A->d_rowidx, A->d_val, beta, Y, ldy, nbands, jgroups,
-                       (int64_t)0, (int64_t)0, (int64_t)0, (const int *)nullptr);
+    hipLaunchKernelGGL((k_spmm_bsr4_z<R, VEC, WPG, false>), dim3((unsigned)total), dim3(64 * WPG), 0, ctx->stream, no,
+                       nb, A->nbc, alpha, X, ldx, A->d_colptr, A->d_rowidx, A->d_val, beta, Y, ldy, nbands, jgroups,
+                       spmm_nt(2.0 * sizeof(R) * no * nb), (int64_t)0, (int64_t)0, (int64_t)0, 1, (const int *)nullptr, (const double *)nullptr,
+                       (R *)nullptr);
     prof_end(ctx, OMX_K_SPMM, ev);
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
 }
 
-static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
-
-// Batched complex SpMM (complex128, or complex64 with the FP64 operator values rounded to FP32)
-// over nbatch systems sharing one block pattern: Y_s := X_s * A_s (beta 0), A_s values at
-// val + s*sV (doubles), X_s, Y_s at s*sX, s*sY (complex elements).
-int launch_spmm_z_batched(omx_ctx ctx, int dt, int no, int nb, int nbc, const int *colptr, const int *rowidx,
-                          const double *val, int64_t sV, const void *X, int64_t ldx, int64_t sX, void *Y, int64_t ldy,
-                          int64_t sY, int nbatch, const int *active) {
-    constexpr int VEC = 1, ROWS = 64 * VEC, WPG = 4;
-    const int nbands = (no + ROWS - 1) / ROWS;
-    const int jgroups = (nbc + WPG - 1) / WPG;
-    const int64_t total = (int64_t)nbands * jgroups;
-    OMX_REQUIRE(total < (1LL << 31) && nbatch < 65536, "batched spmm: grid too large");
-    if (dt == OMX_C64)
-        hipLaunchKernelGGL((k_spmm_bsr4_z<float, VEC, WPG>), dim3((unsigned)total, nbatch), dim3(64 * WPG), 0,
-                           ctx->stream, no, nb, nbc, 1.0, (const float *)X, ldx, colptr, rowidx, val, 0.0, (float *)Y,
-                           ldy, nbands, jgroups, 2 * sX, 2 * sY, sV, active);
-    else
-        hipLaunchKernelGGL((k_spmm_bsr4_z<double, VEC, WPG>), dim3((unsigned)total, nbatch), dim3(64 * WPG), 0,
-                           ctx->stream, no, nb, nbc, 1.0, (const double *)X, ldx, colptr, rowidx, val, 0.0,
-                           (double *)Y, ldy, nbands, jgroups, 2 * sX, 2 * sY, sV, active);
+template <typename R, int VEC>
+static int run_spmm_z_batched(omx_ctx ctx, int no, int nb, int nbc, const int *colptr, const int *rowidx, const double *val,
+                              const double *val2, int64_t sV, const void *X, int64_t ldx, int64_t sX, void *Y, void *Y2,
+                              int64_t ldy, int64_t sY, int nbatch, const int *active) {
+    constexpr int ROWS = 64 * VEC, WPG = 4;
+    const int nbands = (no + ROWS - 1) / ROWS, jgroups = (nbc + WPG - 1) / WPG;
+    const int64_t total = (int64_t)nbands * jgroups * nbatch;
+    OMX_REQUIRE(total < (1LL << 31), "batched spmm: grid too large");
+    hipLaunchKernelGGL((k_spmm_bsr4_z<R, VEC, WPG, true>), dim3((unsigned)total), dim3(64 * WPG), 0, ctx->stream, no, nb, nbc,
+                       1.0, (const R *)X, ldx, colptr, rowidx, val, 0.0, (R *)Y, ldy, nbands, jgroups, 0, 2 * sX, 2 * sY, sV,
+                       nbatch, active, val2, (R *)Y2);
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
+}
+
+// Batched complex SpMM (complex128, or complex64 with the FP64 operator values rounded to FP32) of two
+// operators over nbatch systems sharing one block pattern: Y_s := X_s * A_s, Y2_s := X_s * B_s, the
+// values of A_s and B_s at val + s*sV, val2 + s*sV (doubles), X_s, Y_s and Y2_s at s*sX, s*sY (complex
+// elements).
+int launch_spmm_z_batched(omx_ctx ctx, int dt, int no, int nb, int nbc, const int *colptr, const int *rowidx,
+                          const double *val, const double *val2, int64_t sV, const void *X, int64_t ldx, int64_t sX,
+                          void *Y, void *Y2, int64_t ldy, int64_t sY, int nbatch, const int *active) {
+    if (dt == OMX_C128)
+        return run_spmm_z_batched<double, 1>(ctx, no, nb, nbc, colptr, rowidx, val, val2, sV, X, ldx, sX, Y, Y2, ldy, sY,
+                                             nbatch, active);
+    return run_spmm_z_batched<float, 1>(ctx, no, nb, nbc, colptr, rowidx, val, val2, sV, X, ldx, sX, Y, Y2, ldy, sY, nbatch,
+                                        active);
 }
 
 }  // namespace omx
@@ -941,6 +1029,13 @@ extern "C" int omx_bsr_set_walk(omx_bsr A, const int *order) {
     return OMX_OK;
 }
 
+// 16-byte vectors once they make more than two waves per CU; below that a lane with one state has the
+// shorter chain (FP32, 250 x 500: 5.0 us against 5.9; 432 x 864: 5.2 and 5.9; 686 x 1372, four waves per
+// CU: 7.4 and 6.8.  FP64: 250 x 500 4.8 and 5.1, 432 x 864 5.6 and 5.4).
+static bool spmm_wide(omx_ctx ctx, int no, int vec, omx_bsr A) {
+    return no >= vec && (int64_t)((no + 64 * vec - 1) / (64 * vec)) * A->nbc > 2 * ctx->num_cus;
+}
+
 extern "C" int omx_spmm(omx_ctx ctx, int dt, int no, int nb, double alpha, const void *X, int64_t ldx, omx_bsr A,
                         double beta, void *Y, int64_t ldy) {
     OMX_REQUIRE(ctx && A, "omx_spmm: null argument");
@@ -954,18 +1049,15 @@ extern "C" int omx_spmm(omx_ctx ctx, int dt, int no, int nb, double alpha, const
     if (zdt) {
         OMX_REQUIRE(A->is_complex, "omx_spmm: complex X needs a complex operator");
         if (dt == OMX_C128) return run_spmm_z<double, 1>(ctx, no, nb, alpha, (const double *)X, ldx, A, beta, (double *)Y, ldy);
-        const bool vec = (no % 2 == 0) && (ldx % 2 == 0) && (ldy % 2 == 0) && aligned16(X) && aligned16(Y);
-        if (vec) return run_spmm_z<float, 2>(ctx, no, nb, alpha, (const float *)X, ldx, A, beta, (float *)Y, ldy);
+        if (no >= 2) return run_spmm_z<float, 2>(ctx, no, nb, alpha, (const float *)X, ldx, A, beta, (float *)Y, ldy);
         return run_spmm_z<float, 1>(ctx, no, nb, alpha, (const float *)X, ldx, A, beta, (float *)Y, ldy);
     }
     if (dt == OMX_F64) {
-        bool vec = (no % 2 == 0) && (ldx % 2 == 0) && (ldy % 2 == 0) && aligned16(X) && aligned16(Y);
-        if (vec) return run_spmm<double, 2>(ctx, no, nb, alpha, (const double *)X, ldx, A, beta, (double *)Y, ldy);
+        if (spmm_wide(ctx, no, 2, A)) return run_spmm<double, 2>(ctx, no, nb, alpha, (const double *)X, ldx, A, beta, (double *)Y, ldy);
         return run_spmm<double, 1>(ctx, no, nb, alpha, (const double *)X, ldx, A, beta, (double *)Y, ldy);
     }
     if (dt == OMX_F32) {
-        bool vec = (no % 4 == 0) && (ldx % 4 == 0) && (ldy % 4 == 0) && aligned16(X) && aligned16(Y);
-        if (vec) return run_spmm<float, 4>(ctx, no, nb, alpha, (const float *)X, ldx, A, beta, (float *)Y, ldy);
+        if (spmm_wide(ctx, no, 4, A)) return run_spmm<float, 4>(ctx, no, nb, alpha, (const float *)X, ldx, A, beta, (float *)Y, ldy);
         return run_spmm<float, 1>(ctx, no, nb, alpha, (const float *)X, ldx, A, beta, (float *)Y, ldy);
     }
     set_error("omx_spmm: unsupported element type %d", dt);
