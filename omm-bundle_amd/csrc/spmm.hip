@@ -39,6 +39,7 @@
 #include <utility>
 
 #include "omx_internal.h"
+#include "omx_mfma.h"
 
 namespace omx {
 
@@ -1072,90 +1073,128 @@ extern "C" int omx_spmm(omx_ctx ctx, int dt, int no, int nb, double alpha, const
 // op = 'c','n'), used for the density matrix D = C^T (QW C) on the pattern of H
 // (libOMM/src/omm_ops.F90:104-124 with a sparse D_min) and for dE/dH.
 //
-// Mapping: a workgroup owns a chunk of SD_NT*VEC*SD_STR states and one block column J; it holds
-// B's four columns 4J..4J+3 of the chunk in registers and, per stored block, reads A's four
-// columns, accumulates the 16 products per thread over its SD_STR strides and reduces them over
-// each wave (a reduce-scatter, no barrier).  Per-wave partial blocks go to the workspace and a
-// second kernel adds them in (chunk, wave) order (deterministic).
+// Mapping: a wave owns one block column J and a chunk of states.  The 4 x 4 result of a stored block is a
+// sum over states, so it runs on v_mfma_f64_4x4x4 (four independent 4x4x4 products): lane l holds column
+// l & 3 of the block at the VEC consecutive states that l >> 2 numbers, and the sum over states needs no
+// shuffles until the chunk's end, where two add the four products.  A step is 16*VEC states: one load of
+// 1 KB straight into LDS for B's columns and one for every stored block's, four runs of 256 bytes each
+// (loaded in the matrix core's own layout, neighbouring lanes fall into different lines, and the L1 takes
+// 64 cycles per load: 0.92 ms instead of 0.66 at 8192 x 16384).  The tiles' 16-byte vectors are swizzled
+// by column (no bank conflicts), and a wave has only one set of them: with 8 KB per wave 20 waves fit on a
+// CU and hide each other's waits (two sets, 8 waves: 0.70 ms; three: 1.02).
+// The block's partial result goes to the workspace, and a second kernel adds the chunks in order
+// (deterministic).  The id -> (chunk, block columns) map is that of k_spmm_bsr4, mode 1.
+//
+// Bound by gathers through the L2s, like the SpMM: 2.14 GB come from memory, all there is.  Measured, us,
+// before (a thread per state, 17 shuffles per block, wave and chunk) and after:
+//   FP64  8192 x 16384   976 -> 660   4394 x 8788  337 -> 244   1458 x 2916  34 -> 30   54 x 108  15 -> 8
+//   FP32  8192 x 16384  1610 -> 357   4394 x 8788  548 -> 121    250 x 500  20 ->  8
 // =============================================================================================
 namespace omx {
 
-constexpr int SD_NT = 256;
-// strides of SD_NT*VEC states per thread: one workgroup reduction per stored block per SD_STR strides
-constexpr int SD_STR = 4;
+constexpr int SD_NBK = 7;           // stored blocks taken together (a lattice column's)
+constexpr int64_t SD_LD = 1 << 26;  // leading dimensions whose block columns 32-bit offsets reach
 
-template <typename T, int VEC>
-__global__ __launch_bounds__(SD_NT) void k_sddmm_bsr4_partial(int no, int nb, const T *__restrict__ A, int64_t lda,
-                                                              const T *__restrict__ B, int64_t ldb,
-                                                              const int *__restrict__ colptr,
-                                                              const int *__restrict__ rowidx, int rchunks,
-                                                              int64_t nnzb, double *__restrict__ partial) {
-    constexpr int ROWS = SD_NT * VEC * SD_STR;
-    const int rc = blockIdx.x % rchunks, J = blockIdx.x / rchunks;
-    double bcol[SD_STR][4][VEC];
-#pragma unroll
-    for (int st = 0; st < SD_STR; ++st) {
-        const int i0 = rc * ROWS + st * SD_NT * VEC + threadIdx.x * VEC;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int j = 4 * J + c;
-#pragma unroll
-            for (int q = 0; q < VEC; ++q)
-                bcol[st][c][q] = (j < nb && i0 + q < no) ? (double)B[(int64_t)j * ldb + i0 + q] : 0.0;
-        }
+template <typename T>
+__global__ __launch_bounds__(256) void k_sddmm_bsr4_partial(int no, int nb, int nbc, const T *__restrict__ A, int64_t lda,
+                                                          const T *__restrict__ B, int64_t ldb,
+                                                          const int *__restrict__ colptr, const int *__restrict__ rowidx,
+                                                          int chunk, int nrc, int njg, int64_t nnzb,
+                                                          double *__restrict__ partial) {
+    constexpr int VEC = 16 / sizeof(T), SV = 16 * VEC, TILE = 4 * SV;  // states of a step, elements of its tile
+    __shared__ __align__(16) T smem[4 * (SD_NBK + 1) * TILE];
+    const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3, whole = (nrc >> 3) * njg, eighth = (njg + 7) >> 3;
+    int rc, jg;
+    if (local < whole) {
+        rc = (local / njg) * 8 + xcd;
+        jg = local % njg;
+    } else {
+        rc = (nrc & ~7) + (local - whole) / eighth;
+        jg = xcd * eighth + (local - whole) % eighth;
+        if (rc >= nrc || jg >= njg) return;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int l = colptr[J]; l < colptr[J + 1]; ++l) {
-        const int I = rowidx[l];
-        double s[16];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int J = jg * 4 + wave;
+    if (J >= nbc) return;  // whole wave; the kernel has no barriers, each wave has its own tiles
+    T *const tb = smem + wave * (SD_NBK + 1) * TILE, *const ta = tb + TILE;
+    const int lane = threadIdx.x & 63;
+    // loads: lane l brings vector (l & 15) ^ 4 c of column c = l >> 4; reads: lane l takes vector l >> 2 of column l & 3
+    const int lc = lane >> 4, lv = ((lane & 15) ^ (4 * lc)) * VEC;
+    const int col = lane & 3, rv = lane >> 2, at = (col * 16 + (rv ^ (4 * col))) * VEC;
+    const int beg = rc * chunk, len = min(no - beg, chunk);
+    const int nfull = max(lda, ldb) < SD_LD ? len / SV : 0;  // steps through LDS (32-bit offsets in a block)
+    const T *const pb = B + (int64_t)4 * J * ldb + beg;
+    const int ob = (min(lc, nb - 1 - 4 * J) * (int)ldb + lv) * (int)sizeof(T);
+    const bool jin = 4 * J + col < nb;
+    const int le = colptr[J + 1];
+    for (int l0 = colptr[J]; l0 < le; l0 += SD_NBK) {
+        const int nblk = min(SD_NBK, le - l0);
+        int I[SD_NBK];
+        int oa[SD_NBK];
+        double acc[SD_NBK];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = 0.0;
+        for (int b = 0; b < SD_NBK; ++b) {
+            I[b] = rowidx[l0 + min(b, nblk - 1)];
+            oa[b] = (min(lc, nb - 1 - 4 * I[b]) * (int)lda + lv) * (int)sizeof(T);
+            acc[b] = 0.0;
+        }
+        // products of one step: xb and the xa(b) are this lane's vectors of B and of A's block b
+        auto products = [&](T (&xb)[VEC], auto xa) {
+            if (4 * J + 4 > nb) {  // no basis columns past nb: their results are zero
 #pragma unroll
-        for (int st = 0; st < SD_STR; ++st) {
-            const int i0 = rc * ROWS + st * SD_NT * VEC + threadIdx.x * VEC;
-            const bool full = (i0 + VEC <= no);
-            double acol[4][VEC];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int k = 4 * I + r;
-                const T *src = A + (int64_t)k * lda + i0;
-#pragma unroll
-                for (int q = 0; q < VEC; ++q) acol[r][q] = (k < nb && (full || i0 + q < no)) ? (double)src[q] : 0.0;
+                for (int q = 0; q < VEC; ++q) xb[q] = jin ? xb[q] : (T)0;
             }
+            T x[SD_NBK][VEC];
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+            for (int b = 0; b < SD_NBK; ++b)
+                if (b < nblk) xa(b, x[b]);
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
+            for (int b = 0; b < SD_NBK; ++b)
+                if (b < nblk) {
+                    if (4 * I[b] + 4 > nb) {
 #pragma unroll
-                    for (int q = 0; q < VEC; ++q) s[r + 4 * c] = fma(acol[r][q], bcol[st][c][q], s[r + 4 * c]);
+                        for (int q = 0; q < VEC; ++q) x[b][q] = 4 * I[b] + col < nb ? x[b][q] : (T)0;
+                    }
+#pragma unroll
+                    for (int q = 0; q < VEC; ++q)
+                        acc[b] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x[b][q], (double)xb[q], acc[b], 0, 0, 0);
+                }
+        };
+        auto load = [&](const T *p, T *to, int o) {
+            const __amdgpu_buffer_rsrc_t r = raw_rsrc(p);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)to, 16, o, 0, 0, 0);
+        };
+        for (int st = 0; st < nfull; ++st) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt 0: the tiles of the step before are read
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            load(pb + st * SV, tb, ob);
+#pragma unroll
+            for (int b = 0; b < SD_NBK; ++b)
+                if (b < nblk) load(A + (int64_t)4 * I[b] * lda + beg + st * SV, ta + b * TILE, oa[b]);
+            __builtin_amdgcn_s_waitcnt(waitcnt_vmcnt(0));
+            __atomic_signal_fence(__ATOMIC_SEQ_CST);
+            T xb[VEC];
+            uload<T, VEC>(tb + at, xb);
+            products(xb, [&](int b, T (&x)[VEC]) { uload<T, VEC>(ta + b * TILE + at, x); });
         }
-        // Reduce-scatter of the 16 sums over the wave by recursive halving: at offset 32 a lane keeps
-        // half of its values and adds its partner's copy of that half (8 shuffles), then 4, 2 and 1;
-        // lane l ends with output (l >> 2) & 15, and two more steps add the four lanes that share
-        // it.  17 shuffles instead of 16 x 6; the order is fixed, and each wave writes its own
-        // partial block, so no barrier is needed.
-        double h8[8], h4[4], h2[2];
-        const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8, b2 = lane & 4;
+        for (int st = nfull; st * SV < len; ++st) {  // the last states
+            const int s = st * SV + rv * VEC;
+            auto tail = [&](const T *p, T (&x)[VEC]) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const double keep = b5 ? s[e + 8] : s[e], send = b5 ? s[e] : s[e + 8];
-            h8[e] = keep + __shfl_xor(send, 32, 64);
+                for (int q = 0; q < VEC; ++q) x[q] = s + q < len ? p[beg + s + q] : (T)0;
+            };
+            T xb[VEC];
+            tail(B + (int64_t)min(4 * J + col, nb - 1) * ldb, xb);
+            products(xb, [&](int b, T (&x)[VEC]) { tail(A + (int64_t)min(4 * I[b] + col, nb - 1) * lda, x); });
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const double keep = b4 ? h8[e + 4] : h8[e], send = b4 ? h8[e] : h8[e + 4];
-            h4[e] = keep + __shfl_xor(send, 16, 64);
-        }
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const double keep = b3 ? h4[e + 2] : h4[e], send = b3 ? h4[e] : h4[e + 2];
-            h2[e] = keep + __shfl_xor(send, 8, 64);
-        }
-        double t = (b2 ? h2[1] : h2[0]) + __shfl_xor(b2 ? h2[0] : h2[1], 4, 64);
-        t += __shfl_xor(t, 1, 64);
-        t += __shfl_xor(t, 2, 64);
-        if ((lane & 3) == 0)
-            partial[(((int64_t)rc * (SD_NT / 64) + wave) * nnzb + l) * 16 + ((lane >> 2) & 15)] = t;
+        for (int b = 0; b < SD_NBK; ++b)
+            if (b < nblk) {  // lane j + 4 g + 16 i holds entry (i, j) of product g
+                double t = acc[b];
+                t += __shfl_xor(t, 4, 64);
+                t += __shfl_xor(t, 8, 64);
+                if ((lane & 12) == 0) partial[((int64_t)rc * nnzb + l0 + b) * 16 + (lane >> 4) + 4 * col] = t;
+            }
     }
 }
 
@@ -1169,14 +1208,16 @@ __global__ void k_sddmm_bsr4_final(int64_t nnzb, int nparts, const double *__res
     }
 }
 
-template <typename T, int VEC>
+template <typename T>
 static int run_sddmm(omx_ctx ctx, int no, int nb, double alpha, const T *A, int64_t lda, const T *B, int64_t ldb,
                      double beta, omx_bsr C) {
-    constexpr int ROWS = SD_NT * VEC * SD_STR;
-    const int rchunks = (no + ROWS - 1) / ROWS;
-    const int64_t grid = (int64_t)rchunks * C->nbc;
+    // chunks of 512 states (more of them cost partial results), shorter ones while that leaves less than
+    // eight waves per CU (432 x 864: 128 states 10 us, 256 12, 512 18; 1458 x 2916: 31, 32, 30)
+    int chunk = 512;
+    while (chunk > 128 && (int64_t)((no + chunk - 1) / chunk) * C->nbc < 8 * ctx->num_cus) chunk /= 2;
+    const int nparts = (no + chunk - 1) / chunk, njg = (C->nbc + 3) / 4;
+    const int64_t grid = 8 * ((int64_t)(nparts >> 3) * njg + (nparts & 7) * ((njg + 7) >> 3));
     OMX_REQUIRE(grid < (1LL << 31), "omx_sddmm_bsr: grid too large");
-    const int nparts = rchunks * (SD_NT / 64);  // one partial block per wave of every chunk
     const size_t bytes = sizeof(double) * 16 * (size_t)C->nnzb * nparts;
     int rc = ensure_ws(ctx, bytes);
     if (rc) return rc;
@@ -1184,8 +1225,8 @@ static int run_sddmm(omx_ctx ctx, int no, int nb, double alpha, const T *A, int6
     hipEvent_t ev;
     prof_begin(ctx, OMX_K_SPMM, &ev);
     prof_work(ctx, OMX_K_SPMM, 2.0 * 16.0 * C->nnzb * no, sizeof(T) * 2.0 * (double)no * nb + C->nnzb * (16.0 * 8 + 4));
-    hipLaunchKernelGGL((k_sddmm_bsr4_partial<T, VEC>), dim3((unsigned)grid), dim3(SD_NT), 0, ctx->stream, no, nb, A,
-                       lda, B, ldb, C->d_colptr, C->d_rowidx, rchunks, C->nnzb, partial);
+    hipLaunchKernelGGL(k_sddmm_bsr4_partial<T>, dim3((unsigned)grid), dim3(256), 0, ctx->stream, no, nb, C->nbc, A, lda, B,
+                       ldb, C->d_colptr, C->d_rowidx, chunk, nparts, njg, C->nnzb, partial);
     const int64_t total = C->nnzb * 16;
     const int g2 = (int)std::max<int64_t>(1, std::min<int64_t>((total + 255) / 256, 8192));
     hipLaunchKernelGGL(k_sddmm_bsr4_final, dim3(g2), dim3(256), 0, ctx->stream, C->nnzb, nparts, partial, alpha, beta,
@@ -1211,8 +1252,8 @@ extern "C" int omx_sddmm_bsr(omx_ctx ctx, int dt, int no, int nb, double alpha, 
         return OMX_OK;
     }
     OMX_REQUIRE(A && B, "omx_sddmm_bsr: null operand");
-    if (dt == OMX_F64) return run_sddmm<double, 2>(ctx, no, nb, alpha, (const double *)A, lda, (const double *)B, ldb, beta, C);
-    if (dt == OMX_F32) return run_sddmm<float, 2>(ctx, no, nb, alpha, (const float *)A, lda, (const float *)B, ldb, beta, C);
+    if (dt == OMX_F64) return run_sddmm<double>(ctx, no, nb, alpha, (const double *)A, lda, (const double *)B, ldb, beta, C);
+    if (dt == OMX_F32) return run_sddmm<float>(ctx, no, nb, alpha, (const float *)A, lda, (const float *)B, ldb, beta, C);
     set_error("omx_sddmm_bsr: unsupported element type %d", dt);
     return OMX_ERR_UNSUPPORTED;
 }
