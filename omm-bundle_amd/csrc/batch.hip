@@ -6,14 +6,17 @@
 //
 // Per step (all systems; libOMM/src/omm.F90:436-552 for one system):
 //   D = G + lambda*D, G_p = G                         batched element-wise (lambda per system)
-//   HG = D*H_s, SG = D*S_s                            batched complex BSR SpMM
-//   HWd = HC*D^H, SWd = SC*D^H, HWdd = HG*D^H,       batched complex MFMA GEMMs
+//   HG = D*H_s, SG = D*S_s                            one batched complex BSR SpMM
+//   HWd = HC*D^H, SWd = SC*D^H, HWdd = HG*D^H,       one launch of batched complex MFMA GEMMs
 //   SWdd = SG*D^H
-//   coefficients                                      batched fused reduction, on the device
-//   quartic, energy, e_diff, convergence, ls_fail     one thread per system (k_batch_quartic)
-//   C, SW updates; then (not converged) HW, HC, SC    per-system element-wise with x_min
+//   coefficients, quartic, energy, e_diff,            batched fused reduction; one workgroup per system adds
+//   convergence, ls_fail                              its parts and decides (k_batch_quartic)
+//   C, SW updates; then (not converged) HW, HC, SC    two launches, per-system element-wise with x_min
 //   G = 4HC - 2SW*HC - 2HW*SC                         batched pair GEMM (systems still running)
-//   Polak-Ribiere lambda                              batched dots, divided on the device
+//   Polak-Ribiere lambda                              batched dots, added and divided on the device
+// A small batch is bound by its launches (a dependent kernel of a graph takes 4.5 us even when it does
+// nothing): ten per step instead of eighteen, and TrQS of all systems in one reduction at the end instead
+// of two reductions and readbacks per system: 16 systems of 128 x 256, 20 steps, 5.4 -> 3.9 ms.
 // The first step of a CG run recomputes the line-search products from D = G, which is what the
 // reference's initial pass computes (omm.F90:350-413).  A converged system is frozen: its
 // `active` flag masks every later launch, and its final state is the reference's (the HW, HC and
@@ -32,6 +35,7 @@
 #include <vector>
 
 #include "omx_internal.h"
+#include "omx_reduce.h"
 
 struct omx_zbatch_s {
     omx_ctx ctx = nullptr;
@@ -40,15 +44,17 @@ struct omx_zbatch_s {
     int *colptr = nullptr, *rowidx = nullptr;
     double *hval = nullptr, *sval = nullptr;  // nsys * nnzb * 32
     int dt = OMX_C128;  // element type of the state: OMX_C128 or OMX_C64
-    // state, system s at s * (no*nb) or s * (no*no) complex elements, ld = no
+    // state, system s at s * (no*nb) or s * (no*no) complex elements, ld = no; HC, SC, HG, SG and HWd, SWd,
+    // HWdd, SWdd each in one allocation, in this order (one launch makes the four line-search products)
     void *C = nullptr, *HC = nullptr, *SC = nullptr, *G = nullptr, *Gp = nullptr, *D = nullptr, *HG = nullptr,
          *SG = nullptr;
     void *HW = nullptr, *SW = nullptr, *HWd = nullptr, *SWd = nullptr, *HWdd = nullptr, *SWdd = nullptr;
     // per-system scalars
     double *coeff = nullptr;  // 18 per system
-    double *dots = nullptr;   // 2 per system
-    double *sc = nullptr;     // [x, lambda, e_min, e_diff] per system, then the solve's [cg_tol, max_steps]
-    int *active = nullptr;    // per-system flags, F_COUNT arrays of nsys (see flag())
+    // one allocation, read back at the end of a solve: sc, dots, active
+    double *sc = nullptr;    // [x, lambda, e_min, e_diff] per system, then the solve's [cg_tol, max_steps]
+    double *dots = nullptr;  // [Re tr SW, <SW, SW>] per system
+    int *active = nullptr;   // per-system flags, F_COUNT arrays of nsys (see flag())
     double *partial = nullptr, *partial2 = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -57,7 +63,7 @@ struct omx_zbatch_s {
 
 namespace omx {
 
-constexpr int BT_NT = 256;
+constexpr int BT_NT = EW_NT;
 
 // The quartic line search of omm_solve_quartic (libOMM/src/omm_quartic.F90:60-153), the energy at
 // the minimum and the convergence test, for one system.
@@ -119,18 +125,24 @@ __device__ inline void quartic_min(const double *c, double &x_min, bool &fail) {
 // current solve, in device memory so a captured step reads the values of the solve that replays it.
 // A system that reaches max_steps stops like a converged one (before the updates) but keeps
 // conv = 0; the steps that follow in the same graph are no-ops for it.
-__global__ void k_batch_quartic(int nsys, const double *__restrict__ coeff, double *__restrict__ sc,
-                                const int *__restrict__ active, int *__restrict__ failf, int *__restrict__ cont,
-                                int *__restrict__ grad, int *__restrict__ icg, int *__restrict__ conv,
-                                int *__restrict__ nfail, const double *__restrict__ params) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsys) return;
-    if (!active[s]) {
-        failf[s] = 0;
-        cont[s] = 0;
-        grad[s] = 0;
+// One workgroup per system: adds the coefficients' partial sums (nblocks groups per system) first.
+__global__ __launch_bounds__(BT_NT) void k_batch_quartic(int nblocks, const double *__restrict__ partial,
+                                                       double *__restrict__ coeff, double *__restrict__ sc,
+                                                       const int *__restrict__ active, int *__restrict__ failf,
+                                                       int *__restrict__ cont, int *__restrict__ grad,
+                                                       int *__restrict__ icg, int *__restrict__ conv,
+                                                       int *__restrict__ nfail, const double *__restrict__ params) {
+    const int s = blockIdx.x;
+    if (!active[s]) {  // whole workgroup
+        if (threadIdx.x == 0) {
+            failf[s] = 0;
+            cont[s] = 0;
+            grad[s] = 0;
+        }
         return;
     }
+    coeff_final(nblocks, partial + 13 * (int64_t)s * nblocks, coeff + 18 * s);
+    if (threadIdx.x) return;  // the coefficients are thread 0's own
     const double *c = coeff + 18 * s;
     double *v = sc + 4 * s;
     const double e_old = (icg[s] == 0) ? c[0] : v[2];
@@ -185,39 +197,61 @@ __global__ __launch_bounds__(BT_NT) void k_batch_direction(int64_t len, const T 
     }
 }
 
-// For systems with mask[s]: Y := Y + x*X, or Y := fail_scale*Y after a failed line search.
+// After the line search, one pass: C := C + x*D for the systems that stepped (act); HC := HC + x*HG and
+// SC := SC + x*SG for those still running (cont).  After a failed line search all are halved instead, and
+// where the system runs on, G_p := G and G := 1.5*HC + G with the halved HC (omm.F90:470-523).
 template <typename T>
-__global__ __launch_bounds__(BT_NT) void k_batch_axpy(int64_t len, const T *__restrict__ X, T *__restrict__ Y,
-                                                      const double *__restrict__ sc, const int *__restrict__ mask,
-                                                      const int *__restrict__ failf, double fail_scale) {
+__global__ __launch_bounds__(BT_NT) void k_batch_update_c(int64_t len, const T *__restrict__ D, const T *__restrict__ HG,
+                                                        const T *__restrict__ SG, T *__restrict__ C,
+                                                        T *__restrict__ HC, T *__restrict__ SC, T *__restrict__ G,
+                                                        T *__restrict__ Gp, const double *__restrict__ sc,
+                                                        const int *__restrict__ act, const int *__restrict__ cont,
+                                                        const int *__restrict__ failf) {
     typedef El<T> E;
     const int s = blockIdx.y;
-    if (!mask[s]) return;
-    const bool failed = failf[s] != 0;
+    if (!act[s]) return;
+    const bool failed = failf[s] != 0, on = cont[s] != 0;
     const double x = sc[4 * s];
     const int64_t o = (int64_t)s * len;
-    for (int64_t q = (int64_t)blockIdx.x * BT_NT + threadIdx.x; q < len; q += (int64_t)gridDim.x * BT_NT) {
-        const T y = Y[o + q];
+    auto moved = [&](const T y, const T *X, int64_t q) {
+        if (failed) return E::make(E::re(y) * 0.5, E::im(y) * 0.5);
+        const T xx = X[q];
+        return E::make(E::re(y) + x * E::re(xx), E::cplx ? E::im(y) + x * E::im(xx) : 0.0);
+    };
+    for (int64_t q = o + (int64_t)blockIdx.x * BT_NT + threadIdx.x; q < o + len; q += (int64_t)gridDim.x * BT_NT) {
+        C[q] = moved(C[q], D, q);
+        if (!on) continue;
+        const T h = moved(HC[q], HG, q);
+        HC[q] = h;
+        SC[q] = moved(SC[q], SG, q);
         if (failed) {
-            Y[o + q] = E::make(E::re(y) * fail_scale, E::im(y) * fail_scale);
-        } else {
-            const T xx = X[o + q];
-            Y[o + q] = E::make(E::re(y) + x * E::re(xx), E::cplx ? E::im(y) + x * E::im(xx) : 0.0);
+            const T g = G[q];
+            Gp[q] = g;
+            G[q] = E::make(1.5 * E::re(h) + E::re(g), E::cplx ? 1.5 * E::im(h) + E::im(g) : 0.0);
         }
     }
 }
 
-// For systems with mask[s]: W := W + x*Wd^H + x*Wd + x^2*Wdd (the reference's order), or
-// W := 0.25*W after a failed line search.
+// W := W + x*Wd^H + x*Wd + x^2*Wdd (the reference's order), or W := 0.25*W after a failed line search:
+// SW of the systems that stepped (act) for z < nsys, HW of those still running (cont) from there to 2*nsys
+// (z = blockIdx.z + z0).
 template <typename T>
-__global__ __launch_bounds__(BT_NT) void k_batch_update_w(int n, const T *__restrict__ Wd, const T *__restrict__ Wdd,
-                                                          T *__restrict__ W, const double *__restrict__ sc,
-                                                          const int *__restrict__ mask, const int *__restrict__ failf) {
+__global__ __launch_bounds__(BT_NT) void k_batch_update_w(int n, const T *__restrict__ SWd, const T *__restrict__ SWdd,
+                                                          T *__restrict__ SW, const T *__restrict__ HWd,
+                                                          const T *__restrict__ HWdd, T *__restrict__ HW,
+                                                          const double *__restrict__ sc, const int *__restrict__ act,
+                                                          const int *__restrict__ cont, const int *__restrict__ failf,
+                                                          int nsys, int z0) {
     typedef El<T> E;
+    const int z = blockIdx.z + z0;
+    const bool second = z >= nsys;
+    const int *const mask = second ? cont : act;
+    const T *const Wd = second ? HWd : SWd, *const Wdd = second ? HWdd : SWdd;
+    T *const W = second ? HW : SW;
     constexpr int TS = 32;
     __shared__ double tr[TS][TS + 1];
     __shared__ double ti[E::cplx ? TS : 1][TS + 1];
-    const int s = blockIdx.z;
+    const int s = second ? z - nsys : z;
     if (!mask[s]) return;  // whole workgroup, before the barrier
     const int64_t o = (int64_t)s * n * n;
     const bool failed = failf[s] != 0;
@@ -256,34 +290,23 @@ __global__ __launch_bounds__(BT_NT) void k_batch_update_w(int n, const T *__rest
     }
 }
 
-// After a rescaling (omm.F90:519-523): G_p := G; G := 1.5*HC + G (HC already halved).
-template <typename T>
-__global__ __launch_bounds__(BT_NT) void k_batch_fail_grad(int64_t len, const T *__restrict__ HC, T *__restrict__ G,
-                                                           T *__restrict__ Gp, const int *__restrict__ cont,
-                                                           const int *__restrict__ failf) {
-    typedef El<T> E;
-    const int s = blockIdx.y;
-    if (!cont[s] || !failf[s]) return;
-    const int64_t o = (int64_t)s * len;
-    for (int64_t q = (int64_t)blockIdx.x * BT_NT + threadIdx.x; q < len; q += (int64_t)gridDim.x * BT_NT) {
-        const T g = G[o + q], h = HC[o + q];
-        Gp[o + q] = g;
-        G[o + q] = E::make(1.5 * E::re(h) + E::re(g), E::cplx ? 1.5 * E::im(h) + E::im(g) : 0.0);
-    }
-}
-
 // lambda := <G, G - G_p> / <G_p, G_p> where the gradient was recomputed, 0 after a rescaling
 // (the restart of the inner loop); the next step's active set is the running set.
-__global__ void k_batch_lambda(int nsys, const double *__restrict__ dots, double *__restrict__ sc,
-                               const int *__restrict__ grad, const int *__restrict__ failf,
-                               const int *__restrict__ cont, int *__restrict__ active) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsys) return;
-    if (grad[s])
-        sc[4 * s + 1] = dots[2 * s] / dots[2 * s + 1];
-    else if (failf[s])
+// One workgroup per system: adds the dots' partial sums first.
+__global__ __launch_bounds__(BT_NT) void k_batch_lambda(int nblocks, const double *__restrict__ partial,
+                                                      double *__restrict__ sc, const int *__restrict__ grad,
+                                                      const int *__restrict__ failf, const int *__restrict__ cont,
+                                                      int *__restrict__ active) {
+    const int s = blockIdx.x;
+    if (grad[s]) {  // whole workgroup
+        __shared__ double dots[2];
+        reduce_partials<2>(nblocks, partial + 2 * (int64_t)s * nblocks, dots);
+        __syncthreads();
+        if (threadIdx.x == 0) sc[4 * s + 1] = dots[0] / dots[1];
+    } else if (threadIdx.x == 0 && failf[s]) {
         sc[4 * s + 1] = 0.0;
-    active[s] = cont[s];
+    }
+    if (threadIdx.x == 0) active[s] = cont[s];
 }
 
 // Start of a solve: every system active, counters cleared, and the solve's parameters
@@ -318,6 +341,17 @@ __global__ __launch_bounds__(BT_NT) void k_batch_scale_copy(int64_t len, const T
         const T x = X[o + q];
         Y[o + q] = E::make(a * E::re(x), a * E::im(x));
     }
+}
+
+// k_batch_update_w over both W of nsys systems, in one launch where the grid allows it.
+template <typename T>
+static void launch_update_w(omx_ctx ctx, int n, const void *SWd, const void *SWdd, void *SW, const void *HWd, const void *HWdd,
+                            void *HW, const double *sc, const int *act, const int *cont, const int *failf, int nsys) {
+    const int per = 2LL * nsys < 65536 ? 2 * nsys : nsys;
+    for (int z0 = 0; z0 < 2 * nsys; z0 += per)
+        hipLaunchKernelGGL(k_batch_update_w<T>, dim3((n + 31) / 32, (n + 31) / 32, per), dim3(BT_NT), 0, ctx->stream, n,
+                           (const T *)SWd, (const T *)SWdd, (T *)SW, (const T *)HWd, (const T *)HWdd, (T *)HW, sc, act, cont,
+                           failf, nsys, z0);
 }
 
 static inline dim3 bt_grid(int64_t len, int nsys) {
@@ -364,41 +398,24 @@ static int batch_step(omx_zbatch b) {
     if ((rc = launch_spmm_z_batched(ctx, dt, no, nb, b->nbc, b->colptr, b->rowidx, b->hval, b->sval, sV, b->D, no, lenC,
                                     b->HG, b->SG, no, lenC, ns, act)))
         return rc;
-    const void *src[4] = {b->HC, b->SC, b->HG, b->SG};
-    void *dst[4] = {b->HWd, b->SWd, b->HWdd, b->SWdd};
-    // HG D^H = D H D^H and SG D^H are Hermitian: lower-triangle tiles and a mirror
-    for (int q = 0; q < 4; ++q)
-        if ((rc = q < 2 ? launch_zgemm_batched(ctx, dt, 'n', 'c', no, no, nb, 1.0, src[q], no, lenC, b->D, no, lenC,
-                                               0.0, dst[q], no, lenW, ns, act)
-                        : launch_zgemm_herm_batched(ctx, dt, no, nb, 1.0, src[q], no, lenC, b->D, no, lenC, dst[q],
-                                                    no, lenW, ns, act)))
-            return rc;
-    if ((rc = launch_coeff_batched(ctx, dt, no, no, lenW, b->HW, b->SW, b->HWd, b->SWd, b->HWdd, b->SWdd, ns,
-                                   b->partial, b->coeff, nullptr)))
+    // HC D^H, SC D^H, and the Hermitian HG D^H = D H D^H and SG D^H
+    if ((rc = launch_zgemm_search_batched(ctx, dt, no, nb, b->HC, no, lenC, b->D, no, lenC, b->HWd, no, lenW, ns, act)))
         return rc;
-    hipLaunchKernelGGL(k_batch_quartic, dim3((ns + 63) / 64), dim3(64), 0, ctx->stream, ns, b->coeff, b->sc, act,
-                       failf, cont, grad, flag(b, F_ICG), flag(b, F_CONV), flag(b, F_NFAIL), b->sc + 4 * ns);
-    // C and SW for every system that stepped (omm.F90:470-502)
-    hipLaunchKernelGGL(k_batch_axpy<T>, bt_grid(lenC, ns), dim3(BT_NT), 0, ctx->stream, lenC, (const T *)b->D,
-                       (T *)b->C, b->sc, act, failf, 0.5);
-    const dim3 wgrid((no + 31) / 32, (no + 31) / 32, ns);
-    hipLaunchKernelGGL(k_batch_update_w<T>, wgrid, dim3(BT_NT), 0, ctx->stream, no, (const T *)b->SWd,
-                       (const T *)b->SWdd, (T *)b->SW, b->sc, act, failf);
-    // HW, HC, SC for the systems still running (omm.F90:511-527)
-    hipLaunchKernelGGL(k_batch_update_w<T>, wgrid, dim3(BT_NT), 0, ctx->stream, no, (const T *)b->HWd,
-                       (const T *)b->HWdd, (T *)b->HW, b->sc, cont, failf);
-    hipLaunchKernelGGL(k_batch_axpy<T>, bt_grid(lenC, ns), dim3(BT_NT), 0, ctx->stream, lenC, (const T *)b->HG,
-                       (T *)b->HC, b->sc, cont, failf, 0.5);
-    hipLaunchKernelGGL(k_batch_axpy<T>, bt_grid(lenC, ns), dim3(BT_NT), 0, ctx->stream, lenC, (const T *)b->SG,
-                       (T *)b->SC, b->sc, cont, failf, 0.5);
-    hipLaunchKernelGGL(k_batch_fail_grad<T>, bt_grid(lenC, ns), dim3(BT_NT), 0, ctx->stream, lenC, (const T *)b->HC,
-                       (T *)b->G, (T *)b->Gp, cont, failf);
+    if ((rc = launch_coeff_batched(ctx, dt, no, no, lenW, b->HW, b->SW, b->HWd, b->SWd, b->HWdd, b->SWdd, ns,
+                                   b->partial, act)))
+        return rc;
+    hipLaunchKernelGGL(k_batch_quartic, dim3(ns), dim3(BT_NT), 0, ctx->stream, coeff_blocks(no), b->partial, b->coeff, b->sc,
+                       act, failf, cont, grad, flag(b, F_ICG), flag(b, F_CONV), flag(b, F_NFAIL), b->sc + 4 * ns);
+    // C and SW for every system that stepped, HC, SC and HW for those still running (omm.F90:470-527)
+    hipLaunchKernelGGL(k_batch_update_c<T>, bt_grid(lenC, ns), dim3(BT_NT), 0, ctx->stream, lenC, (const T *)b->D,
+                       (const T *)b->HG, (const T *)b->SG, (T *)b->C, (T *)b->HC, (T *)b->SC, (T *)b->G, (T *)b->Gp, b->sc,
+                       act, cont, failf);
+    launch_update_w<T>(ctx, no, b->SWd, b->SWdd, b->SW, b->HWd, b->HWdd, b->HW, b->sc, act, cont, failf, ns);
     // G = 4HC - 2SW*HC - 2HW*SC where the line search succeeded, then Polak-Ribiere
     if ((rc = batch_calc_G<T>(b, grad))) return rc;
-    if ((rc = launch_pr_batched(ctx, dt, no, nb, no, lenC, b->G, b->Gp, ns, b->partial2, b->dots, nullptr)))
-        return rc;
-    hipLaunchKernelGGL(k_batch_lambda, dim3((ns + 63) / 64), dim3(64), 0, ctx->stream, ns, b->dots, b->sc, grad, failf,
-                       cont, act);
+    if ((rc = launch_pr_batched(ctx, dt, no, nb, no, lenC, b->G, b->Gp, ns, b->partial2, grad))) return rc;
+    hipLaunchKernelGGL(k_batch_lambda, dim3(ns), dim3(BT_NT), 0, ctx->stream, pr_blocks(no, nb), b->partial2, b->sc, grad,
+                       failf, cont, act);
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
 }
@@ -411,14 +428,16 @@ static int batch_calc_G_any(omx_zbatch b, const int *mask) {
 }
 static size_t batch_esize(omx_zbatch b) { return b->dt == OMX_C64 ? 8 : 16; }
 
+// sc, dots and active of a batch, one allocation
+static size_t batch_result_bytes(int nsys) { return sizeof(double) * (6 * (size_t)nsys + 2) + sizeof(int) * F_COUNT * nsys; }
+
 static void batch_free(omx_zbatch b) {
     if (!b) return;
     if (b->ctx) (void)hipStreamSynchronize(b->ctx->stream);
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
-    void *ptrs[] = {b->colptr, b->rowidx, b->hval, b->sval, b->C, b->HC, b->SC, b->G, b->Gp, b->D, b->HG, b->SG,
-                    b->HW, b->SW, b->HWd, b->SWd, b->HWdd, b->SWdd, b->coeff, b->dots, b->sc, b->active,
-                    b->partial, b->partial2};
+    void *ptrs[] = {b->colptr, b->rowidx, b->hval, b->sval, b->C, b->HC, b->G, b->Gp, b->D, b->HW, b->SW, b->HWd, b->coeff,
+                    b->sc, b->partial, b->partial2};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     delete b;
@@ -454,21 +473,27 @@ int omx_zbatch_create_dt(omx_ctx ctx, int dt, int nsys, int no, int nb, const in
               hipMalloc(&b->hval, sizeof(double) * 32 * std::max<int64_t>(b->nnzb, 1) * nsys) == hipSuccess &&
               hipMalloc(&b->sval, sizeof(double) * 32 * std::max<int64_t>(b->nnzb, 1) * nsys) == hipSuccess;
     const size_t es = batch_esize(b);
-    void **nm[] = {&b->C, &b->HC, &b->SC, &b->G, &b->Gp, &b->D, &b->HG, &b->SG};
+    void **nm[] = {&b->C, &b->G, &b->Gp, &b->D};
     for (auto p : nm) ok = ok && hipMalloc(p, es * lenC) == hipSuccess;
-    void **nn[] = {&b->HW, &b->SW, &b->HWd, &b->SWd, &b->HWdd, &b->SWdd};
+    void **nn[] = {&b->HW, &b->SW};
     for (auto p : nn) ok = ok && hipMalloc(p, es * lenW) == hipSuccess;
-    ok = ok && hipMalloc(&b->coeff, sizeof(double) * 18 * nsys) == hipSuccess &&
-         hipMalloc(&b->dots, sizeof(double) * 2 * nsys) == hipSuccess &&
-         hipMalloc(&b->sc, sizeof(double) * (4 * nsys + 2)) == hipSuccess &&
-         hipMalloc(&b->active, sizeof(int) * F_COUNT * nsys) == hipSuccess &&
-         hipMalloc(&b->partial, sizeof(double) * coeff_partial_doubles(no, nsys)) == hipSuccess &&
-         hipMalloc(&b->partial2, sizeof(double) * pr_partial_doubles(no, nb, nsys)) == hipSuccess;
+    ok = ok && hipMalloc(&b->HC, es * 4 * lenC) == hipSuccess && hipMalloc(&b->HWd, es * 4 * lenW) == hipSuccess &&
+         hipMalloc(&b->coeff, sizeof(double) * 18 * nsys) == hipSuccess &&
+         hipMalloc(&b->sc, batch_result_bytes(nsys)) == hipSuccess &&
+         hipMalloc(&b->partial, sizeof(double) * 13 * coeff_blocks(no) * nsys) == hipSuccess &&
+         hipMalloc(&b->partial2, sizeof(double) * 2 * pr_blocks(no, nb) * nsys) == hipSuccess;
     if (!ok) {
         batch_free(b);
         set_error("omx_zbatch_create: device allocation failed");
         return OMX_ERR_NOMEM;
     }
+    void **const x[] = {&b->SC, &b->HG, &b->SG}, **const w[] = {&b->SWd, &b->HWdd, &b->SWdd};
+    for (size_t q = 0; q < 3; ++q) {
+        *x[q] = (char *)b->HC + (q + 1) * es * lenC;
+        *w[q] = (char *)b->HWd + (q + 1) * es * lenW;
+    }
+    b->dots = b->sc + 4 * nsys + 2;
+    b->active = (int *)(b->dots + 2 * nsys);
     hipStream_t st = ctx->stream;
     (void)hipMemcpyAsync(b->colptr, bcolptr, sizeof(int) * (nbc + 1), hipMemcpyHostToDevice, st);
     if (b->nnzb) {
@@ -573,21 +598,17 @@ int omx_zbatch_solve(omx_zbatch b, double eta, double cg_tol, int max_steps, int
     }
     if (steps_run) *steps_run = done_steps;  // step sequences issued (masked ones included)
     // results: e_min + eta*TrQS with TrQS = Re tr[(2I - SW) SW] = 2 Re tr(SW) - <SW, SW>
-    std::vector<double> sc(4 * ns);
-    std::vector<int> h_icg(ns), h_conv(ns);
-    OMX_CHECK_HIP(hipMemcpyAsync(sc.data(), b->sc, sizeof(double) * 4 * ns, hipMemcpyDeviceToHost, st));
-    OMX_CHECK_HIP(hipMemcpyAsync(h_icg.data(), flag(b, F_ICG), sizeof(int) * ns, hipMemcpyDeviceToHost, st));
-    OMX_CHECK_HIP(hipMemcpyAsync(h_conv.data(), flag(b, F_CONV), sizeof(int) * ns, hipMemcpyDeviceToHost, st));
+    if ((rc = launch_trqs_batched(ctx, b->dt, no, lenW, b->SW, ns, pr_blocks(no, nb), b->partial2, b->dots))) return rc;
+    std::vector<double> res((batch_result_bytes(ns) + sizeof(double) - 1) / sizeof(double));
+    OMX_CHECK_HIP(hipMemcpyAsync(res.data(), b->sc, batch_result_bytes(ns), hipMemcpyDeviceToHost, st));
     OMX_CHECK_HIP(hipStreamSynchronize(st));
+    const double *dots = res.data() + 4 * ns + 2;
+    const int *flags = (const int *)(dots + 2 * ns);
     for (int s = 0; s < ns; ++s) {
-        double tr[2], dd[2];
-        const void *W = (const char *)b->SW + batch_esize(b) * (size_t)s * lenW;
-        if ((rc = omx_trace(ctx, b->dt, no, W, no, tr))) return rc;
-        if ((rc = omx_mm_trace(ctx, b->dt, no, no, W, no, W, no, dd))) return rc;
-        const double TrQS = 2.0 * tr[0] - dd[0];
-        e_min[s] = sc[4 * s + 2] + eta * TrQS;
-        icg[s] = h_icg[s];
-        converged[s] = h_conv[s];
+        const double TrQS = 2.0 * dots[2 * s] - dots[2 * s + 1];
+        e_min[s] = res[4 * s + 2] + eta * TrQS;
+        icg[s] = flags[F_ICG * ns + s];
+        converged[s] = flags[F_CONV * ns + s];
     }
     return OMX_OK;
 }
@@ -671,32 +692,20 @@ static int group_sys_step(omx_group g, int s) {
     if (!rc) rc = group_gram(g, s, M[M_SG], M[M_D], M[M_SWDD], true);
     if (!rc)
         rc = launch_coeff_batched(ctx, OMX_F64, no, no, 0, M[M_HW], M[M_SW], M[M_HWD], M[M_SWD], M[M_HWDD],
-                                  M[M_SWDD], 1, g->partial[s], g->coeff + 18 * s, act);
+                                  M[M_SWDD], 1, g->partial[s], act);
     ctx->launch_mask = nullptr;
     if (rc) return rc;
-    hipLaunchKernelGGL(k_batch_quartic, dim3(1), dim3(64), 0, ctx->stream, 1, g->coeff + 18 * s, scs, act, failf,
-                       cont, grad, gflag(g, F_ICG, s), gflag(g, F_CONV, s), gflag(g, F_NFAIL, s),
-                       g->sc + 4 * g->nsys);
+    hipLaunchKernelGGL(k_batch_quartic, dim3(1), dim3(BT_NT), 0, ctx->stream, coeff_blocks(no), g->partial[s],
+                       g->coeff + 18 * s, scs, act, failf, cont, grad, gflag(g, F_ICG, s), gflag(g, F_CONV, s),
+                       gflag(g, F_NFAIL, s), g->sc + 4 * g->nsys);
     // C and SW when the system stepped; HW, HC, SC when it is still running (omm.F90:470-527)
-    hipLaunchKernelGGL(k_batch_axpy<double>, bt_grid(lenC, 1), dim3(BT_NT), 0, ctx->stream, lenC, M[M_D], M[M_C],
-                       scs, act, failf, 0.5);
-    const dim3 wgrid((no + 31) / 32, (no + 31) / 32, 1);
-    hipLaunchKernelGGL(k_batch_update_w<double>, wgrid, dim3(BT_NT), 0, ctx->stream, no, M[M_SWD], M[M_SWDD], M[M_SW],
-                       scs, act, failf);
-    hipLaunchKernelGGL(k_batch_update_w<double>, wgrid, dim3(BT_NT), 0, ctx->stream, no, M[M_HWD], M[M_HWDD], M[M_HW],
-                       scs, cont, failf);
-    hipLaunchKernelGGL(k_batch_axpy<double>, bt_grid(lenC, 1), dim3(BT_NT), 0, ctx->stream, lenC, M[M_HG], M[M_HC],
-                       scs, cont, failf, 0.5);
-    hipLaunchKernelGGL(k_batch_axpy<double>, bt_grid(lenC, 1), dim3(BT_NT), 0, ctx->stream, lenC, M[M_SG], M[M_SC],
-                       scs, cont, failf, 0.5);
-    hipLaunchKernelGGL(k_batch_fail_grad<double>, bt_grid(lenC, 1), dim3(BT_NT), 0, ctx->stream, lenC, M[M_HC],
-                       M[M_G], M[M_GP], cont, failf);
+    hipLaunchKernelGGL(k_batch_update_c<double>, bt_grid(lenC, 1), dim3(BT_NT), 0, ctx->stream, lenC, M[M_D], M[M_HG],
+                       M[M_SG], M[M_C], M[M_HC], M[M_SC], M[M_G], M[M_GP], scs, act, cont, failf);
+    launch_update_w<double>(ctx, no, M[M_SWD], M[M_SWDD], M[M_SW], M[M_HWD], M[M_HWDD], M[M_HW], scs, act, cont, failf, 1);
     if ((rc = group_calc_G(g, s, grad))) return rc;
-    if ((rc = launch_pr_batched(ctx, OMX_F64, no, nb, no, 0, M[M_G], M[M_GP], 1, g->partial2[s], g->dots + 2 * s,
-                                grad)))
-        return rc;
-    hipLaunchKernelGGL(k_batch_lambda, dim3(1), dim3(64), 0, ctx->stream, 1, g->dots + 2 * s, scs, grad, failf, cont,
-                       act);
+    if ((rc = launch_pr_batched(ctx, OMX_F64, no, nb, no, 0, M[M_G], M[M_GP], 1, g->partial2[s], grad))) return rc;
+    hipLaunchKernelGGL(k_batch_lambda, dim3(1), dim3(BT_NT), 0, ctx->stream, pr_blocks(no, nb), g->partial2[s], scs, grad,
+                       failf, cont, act);
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
 }
@@ -795,8 +804,8 @@ int omx_group_create(omx_ctx ctx, int nsys, const int *no, const omx_bsr *H, con
             ok = hipMalloc(&g->m[s][q], sizeof(double) * elems) == hipSuccess;
             if (ok) ok = hipMemsetAsync(g->m[s][q], 0, sizeof(double) * elems, ctx->stream) == hipSuccess;
         }
-        ok = ok && hipMalloc(&g->partial[s], sizeof(double) * coeff_partial_doubles(o, 1)) == hipSuccess &&
-             hipMalloc(&g->partial2[s], sizeof(double) * pr_partial_doubles(o, n, 1)) == hipSuccess &&
+        ok = ok && hipMalloc(&g->partial[s], sizeof(double) * 13 * coeff_blocks(o)) == hipSuccess &&
+             hipMalloc(&g->partial2[s], sizeof(double) * 2 * pr_blocks(o, n)) == hipSuccess &&
              hipStreamCreateWithFlags(&g->streams[s], hipStreamNonBlocking) == hipSuccess &&
              hipEventCreateWithFlags(&g->joins[s], hipEventDisableTiming) == hipSuccess;
     }
@@ -906,18 +915,19 @@ int omx_group_solve(omx_group g, const double *eta, double cg_tol, int max_steps
     }
     if (steps_run) *steps_run = done_steps;  // step sequences issued (masked ones included)
     // e_min + eta*TrQS, TrQS = tr[(2I - SW) SW] = 2 tr(SW) - <SW, SW> (omm.F90:576-593)
-    std::vector<double> sc(4 * ns);
+    for (int s = 0; s < ns; ++s)
+        if ((rc = launch_trqs_batched(ctx, OMX_F64, g->no[s], 0, g->m[s][M_SW], 1, pr_blocks(g->no[s], g->nb[s]),
+                                      g->partial2[s], g->dots + 2 * s)))
+            return rc;
+    std::vector<double> sc(4 * ns), dots(2 * ns);
     std::vector<int> h_icg(ns), h_conv(ns);
     OMX_CHECK_HIP(hipMemcpyAsync(sc.data(), g->sc, sizeof(double) * 4 * ns, hipMemcpyDeviceToHost, st));
+    OMX_CHECK_HIP(hipMemcpyAsync(dots.data(), g->dots, sizeof(double) * 2 * ns, hipMemcpyDeviceToHost, st));
     OMX_CHECK_HIP(hipMemcpyAsync(h_icg.data(), g->flags + F_ICG * ns, sizeof(int) * ns, hipMemcpyDeviceToHost, st));
     OMX_CHECK_HIP(hipMemcpyAsync(h_conv.data(), g->flags + F_CONV * ns, sizeof(int) * ns, hipMemcpyDeviceToHost, st));
     OMX_CHECK_HIP(hipStreamSynchronize(st));
     for (int s = 0; s < ns; ++s) {
-        double tr[2], dd[2];
-        const double *W = g->m[s][M_SW];
-        if ((rc = omx_trace(ctx, OMX_F64, g->no[s], W, g->no[s], tr))) return rc;
-        if ((rc = omx_mm_trace(ctx, OMX_F64, g->no[s], g->no[s], W, g->no[s], W, g->no[s], dd))) return rc;
-        e_min[s] = sc[4 * s + 2] + eta[s] * (2.0 * tr[0] - dd[0]);
+        e_min[s] = sc[4 * s + 2] + eta[s] * (2.0 * dots[2 * s] - dots[2 * s + 1]);
         icg[s] = h_icg[s];
         converged[s] = h_conv[s];
     }

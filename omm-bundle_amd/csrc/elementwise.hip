@@ -8,52 +8,20 @@
 #include <mutex>
 
 #include "omx_internal.h"
+#include "omx_reduce.h"
 
 namespace omx {
 
-constexpr int EW_NT = 256;
 constexpr int TT = 32;  // transpose / trace tile edge
 
 template <typename T>
 __device__ inline double ld(const T *p) { return (double)*p; }
 
-// ---- block reduction helpers ----------------------------------------------------------------
-
-template <int NV>
-__device__ inline void block_reduce_store(double (&v)[NV], double *__restrict__ out) {
-    __shared__ double red[NV][EW_NT / 64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double s = v[q];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-        if (lane == 0) red[q][wave] = s;
-    }
-    __syncthreads();
-    if (threadIdx.x < NV) {
-        double s = 0.0;
-#pragma unroll
-        for (int w = 0; w < EW_NT / 64; ++w) s += red[threadIdx.x][w];
-        out[threadIdx.x] = s;
-    }
-}
-
-// Final stage: out[q] = sum over blocks b (ascending) of partial[b*NV + q].
+// Final stage: out[q] = sum over blocks b (ascending) of partial[b*NV + q]; one workgroup per system.
 template <int NV>
 __global__ __launch_bounds__(EW_NT) void k_reduce_partials(int nblocks, const double *__restrict__ partial,
-                                                           double *__restrict__ out,
-                                                           const int *__restrict__ mask = nullptr) {
-    if (mask && !mask[blockIdx.x]) return;          // system masked off (whole workgroup)
-    partial += (int64_t)blockIdx.x * nblocks * NV;  // one workgroup per system in batched use
-    out += blockIdx.x * NV;
-    double v[NV];
-#pragma unroll
-    for (int q = 0; q < NV; ++q) v[q] = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += EW_NT)
-#pragma unroll
-        for (int q = 0; q < NV; ++q) v[q] += partial[(int64_t)b * NV + q];
-    block_reduce_store<NV>(v, out);
+                                                           double *__restrict__ out) {
+    reduce_partials<NV>(nblocks, partial + (int64_t)blockIdx.x * nblocks * NV, out + blockIdx.x * NV);
 }
 
 // ---- m_add / m_scale / m_set -----------------------------------------------------------------
@@ -167,6 +135,23 @@ __global__ __launch_bounds__(EW_NT) void k_trace_partial(int n, const T *__restr
         if constexpr (El<T>::cplx) v[1] += El<T>::im(a);
     }
     block_reduce_store<2>(v, partial + 2 * (int64_t)blockIdx.x);
+}
+
+// Re tr(W) and <W, W> of the n x n matrices of a batch (blockIdx.y, sW elements apart, ld = n)
+template <typename T>
+__global__ __launch_bounds__(EW_NT) void k_trqs_partial(int n, const T *__restrict__ W, int64_t sW,
+                                                        double *__restrict__ partial) {
+    typedef El<T> E;
+    W += blockIdx.y * sW;
+    double v[2] = {0.0, 0.0};
+    const int first = blockIdx.x * EW_NT + threadIdx.x, stride = gridDim.x * EW_NT;
+    for (int i = first; i < n; i += stride) v[0] += E::re(W[(int64_t)i * (n + 1)]);
+    for (int64_t q = first; q < (int64_t)n * n; q += stride) {
+        const T w = W[q];
+        v[1] += E::re(w) * E::re(w);
+        if constexpr (E::cplx) v[1] += E::im(w) * E::im(w);
+    }
+    block_reduce_store<2>(v, partial + 2 * ((int64_t)blockIdx.y * gridDim.x + blockIdx.x));
 }
 
 // (re, im) of sum_ij conj(A_ij)*B_ij
@@ -300,33 +285,9 @@ __global__ __launch_bounds__(EW_NT) void k_coeff_partial(int n, int64_t ldm, con
     block_reduce_store<13>(v, partial + 13 * (int64_t)blockIdx.x);
 }
 
-__global__ void k_coeff_final(int nblocks, const double *__restrict__ partial, double *__restrict__ out,
-                              const int *__restrict__ mask = nullptr) {
-    // One workgroup (per system in batched use): deterministic per-term sums, then the closed-form
-    // coefficients.
-    if (mask && !mask[blockIdx.x]) return;
-    partial += 13 * (int64_t)blockIdx.x * nblocks;
-    out += 18 * blockIdx.x;
-    double v[13];
-#pragma unroll
-    for (int q = 0; q < 13; ++q) v[q] = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += EW_NT)
-#pragma unroll
-        for (int q = 0; q < 13; ++q) v[q] += partial[(int64_t)b * 13 + q];
-    __shared__ double tr[13];
-    block_reduce_store<13>(v, tr);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const double TrH = tr[0], TrHS = tr[1], TrHd = tr[2], TrHdS = tr[3], TrHSd = tr[4], TrHdd = tr[5],
-                     TrHddS = tr[6], TrHSdd = tr[7], TrHdSd = tr[8], TrHdSdH = tr[9], TrHddSd = tr[10],
-                     TrHdSdd = tr[11], TrHddSdd = tr[12];
-        out[0] = 2.0 * TrH - TrHS;
-        out[1] = 2.0 * (2.0 * TrHd - TrHdS - TrHSd);
-        out[2] = 2.0 * (TrHdd - TrHdSd - TrHdSdH) - TrHddS - TrHSdd;
-        out[3] = -2.0 * (TrHddSd + TrHdSdd);
-        out[4] = -TrHddSdd;
-        for (int q = 0; q < 13; ++q) out[5 + q] = tr[q];
-    }
+__global__ __launch_bounds__(EW_NT) void k_coeff_final(int nblocks, const double *__restrict__ partial,
+                                                       double *__restrict__ out) {
+    coeff_final(nblocks, partial, out);
 }
 
 // ---- fused CG updates ------------------------------------------------------------------------
@@ -405,17 +366,6 @@ inline bool with_type(int dt, F &&f) {
         default: return false;
     }
 }
-
-// Batched complex128 reductions over nbatch systems (used by the batched solver): coefficients to
-// out[18*s ...] (5 coefficients then the 13 traces) and Polak-Ribiere dots to out2[2*s ...], on
-// the device, no readback.
-int launch_coeff_batched(omx_ctx ctx, int dt, int n, int64_t ldm, int64_t sW, const void *HW, const void *SW,
-                         const void *HWd, const void *SWd, const void *HWdd, const void *SWdd, int nbatch,
-                         double *partial, double *out, const int *mask);
-int launch_pr_batched(omx_ctx ctx, int dt, int n, int m, int64_t ld, int64_t sG, const void *G, const void *Gp,
-                      int nbatch, double *partial, double *out2, const int *mask);
-size_t coeff_partial_doubles(int n, int nbatch);
-size_t pr_partial_doubles(int n, int m, int nbatch);
 
 inline int grid_for(int64_t total) { return (int)std::max<int64_t>(1, std::min<int64_t>((total + EW_NT - 1) / EW_NT, 65536)); }
 
@@ -728,42 +678,45 @@ int omx_omm_update_w(omx_ctx ctx, int dt, int n, int64_t ld, double x, const voi
 
 namespace omx {
 
-size_t coeff_partial_doubles(int n, int nbatch) {
-    const int64_t tiles = (n + TT - 1) / TT;
-    return (size_t)13 * tiles * tiles * nbatch;
-}
-size_t pr_partial_doubles(int n, int m, int nbatch) {
-    return (size_t)2 * std::min(2048, grid_for((int64_t)n * m)) * nbatch;
-}
+int coeff_blocks(int n) { return ((n + TT - 1) / TT) * ((n + TT - 1) / TT); }
+int pr_blocks(int n, int m) { return std::min(2048, grid_for((int64_t)n * m)); }
 
 int launch_coeff_batched(omx_ctx ctx, int dt, int n, int64_t ldm, int64_t sW, const void *HW, const void *SW,
                          const void *HWd, const void *SWd, const void *HWdd, const void *SWdd, int nbatch,
-                         double *partial, double *out, const int *mask) {
-    const int tiles = (n + TT - 1) / TT;
-    const int blocks = tiles * tiles;
+                         double *partial, const int *mask) {
     const bool ok = with_type(dt, [&](auto tag) {
         typedef decltype(tag) T;
-        hipLaunchKernelGGL(k_coeff_partial<T>, dim3((unsigned)blocks, nbatch), dim3(EW_NT), 0, ctx->stream, n, ldm,
+        hipLaunchKernelGGL(k_coeff_partial<T>, dim3(coeff_blocks(n), nbatch), dim3(EW_NT), 0, ctx->stream, n, ldm,
                            (const T *)HW, (const T *)SW, (const T *)HWd, (const T *)SWd, (const T *)HWdd,
                            (const T *)SWdd, partial, sW, mask);
     });
     OMX_REQUIRE(ok, "batched coefficients: unsupported element type %d", dt);
-    hipLaunchKernelGGL(k_coeff_final, dim3(nbatch), dim3(EW_NT), 0, ctx->stream, blocks, partial, out, mask);
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
 }
 
 int launch_pr_batched(omx_ctx ctx, int dt, int n, int m, int64_t ld, int64_t sG, const void *G, const void *Gp,
-                      int nbatch, double *partial, double *out2, const int *mask) {
-    const int64_t total = (int64_t)n * m;
-    const int blocks = std::min(2048, grid_for(total));
+                      int nbatch, double *partial, const int *mask) {
     const bool ok = with_type(dt, [&](auto tag) {
         typedef decltype(tag) T;
-        hipLaunchKernelGGL(k_pr_partial<T>, dim3(blocks, nbatch), dim3(EW_NT), 0, ctx->stream, total, n,
-                           (const T *)G, (const T *)Gp, ld, partial, sG, mask);
+        hipLaunchKernelGGL(k_pr_partial<T>, dim3(pr_blocks(n, m), nbatch), dim3(EW_NT), 0, ctx->stream,
+                           (int64_t)n * m, n, (const T *)G, (const T *)Gp, ld, partial, sG, mask);
     });
     OMX_REQUIRE(ok, "batched dots: unsupported element type %d", dt);
-    hipLaunchKernelGGL((k_reduce_partials<2>), dim3(nbatch), dim3(EW_NT), 0, ctx->stream, blocks, partial, out2, mask);
+    OMX_CHECK_HIP(hipGetLastError());
+    return OMX_OK;
+}
+
+int launch_trqs_batched(omx_ctx ctx, int dt, int n, int64_t sW, const void *W, int nbatch, int maxblocks,
+                        double *partial, double *out2) {
+    const int blocks = std::min(std::min(64, maxblocks), grid_for((int64_t)n * n));
+    const bool ok = with_type(dt, [&](auto tag) {
+        typedef decltype(tag) T;
+        hipLaunchKernelGGL(k_trqs_partial<T>, dim3(blocks, nbatch), dim3(EW_NT), 0, ctx->stream, n, (const T *)W, sW,
+                           partial);
+    });
+    OMX_REQUIRE(ok, "batched traces: unsupported element type %d", dt);
+    hipLaunchKernelGGL((k_reduce_partials<2>), dim3(nbatch), dim3(EW_NT), 0, ctx->stream, blocks, partial, out2);
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
 }

@@ -260,6 +260,12 @@ int launch_zgemm_herm(omx_ctx ctx, int dt, int n, int k, double alpha, const voi
 int launch_zgemm_herm_batched(omx_ctx ctx, int dt, int n, int k, double alpha, const void *A, int64_t lda,
                               int64_t sA, const void *B, int64_t ldb, int64_t sB, void *C, int64_t ldc, int64_t sC,
                               int nbatch, const int *active);
+// The four line-search products of nbatch systems, X_q D^H with X_q at X + q*nbatch*sX (q = 0..3, system s at
+// + s*sX) and the results likewise at C, sC apart; products 2 and 3 are Hermitian.  One launch where the
+// kernel allows it.
+int launch_zgemm_search_batched(omx_ctx ctx, int dt, int n, int k, const void *X, int64_t ldx, int64_t sX,
+                                const void *D, int64_t ldd, int64_t sD, void *C, int64_t ldc, int64_t sC, int nbatch,
+                                const int *active);
 int launch_zgemm_pair_batched(omx_ctx ctx, int dt, int m, int n, int k, double alpha, const void *A1, const void *A2,
                               int64_t lda, int64_t sA, const void *B1, const void *B2, int64_t ldb, int64_t sB,
                               double beta0, const void *C0, double beta, void *C, int64_t ldc, int64_t sC, int nbatch,
@@ -269,15 +275,19 @@ int launch_zgemm_pair_batched(omx_ctx ctx, int dt, int m, int n, int k, double a
 int launch_spmm_z_batched(omx_ctx ctx, int dt, int no, int nb, int nbc, const int *colptr, const int *rowidx,
                           const double *val, const double *val2, int64_t sV, const void *X, int64_t ldx, int64_t sX,
                           void *Y, void *Y2, int64_t ldy, int64_t sY, int nbatch, const int *active);
-// Line-search coefficients (to out[18*s ...]: the 5 coefficients, then the 13 traces) and
-// Polak-Ribiere dots (to out2[2*s ...]) of nbatch systems of element type dt, on the device; a
-// system s with mask && !mask[s] is skipped.
+// Partial sums of the line-search coefficients (13 values per workgroup, coeff_blocks(n) workgroups per
+// system) and of the Polak-Ribiere dots (2 values, pr_blocks(n, m)) of nbatch systems of element type dt; a
+// system s with mask && !mask[s] is skipped.  The solver's own kernels add them (omx_reduce.h).
+int coeff_blocks(int n);
+int pr_blocks(int n, int m);
 int launch_coeff_batched(omx_ctx ctx, int dt, int n, int64_t ldm, int64_t sW, const void *HW, const void *SW,
                          const void *HWd, const void *SWd, const void *HWdd, const void *SWdd, int nbatch,
-                         double *partial, double *out, const int *mask);
+                         double *partial, const int *mask);
 int launch_pr_batched(omx_ctx ctx, int dt, int n, int m, int64_t ld, int64_t sG, const void *G, const void *Gp,
-                      int nbatch, double *partial, double *out2, const int *mask);
-size_t coeff_partial_doubles(int n, int nbatch);
-size_t pr_partial_doubles(int n, int m, int nbatch);
+                      int nbatch, double *partial, const int *mask);
+// Re tr(W_s) and <W_s, W_s> to out2[2*s ...] (W_s n x n, ld = n, sW elements apart); partial holds
+// 2*maxblocks values per system.
+int launch_trqs_batched(omx_ctx ctx, int dt, int n, int64_t sW, const void *W, int nbatch, int maxblocks,
+                        double *partial, double *out2);
 
 }  // namespace omx

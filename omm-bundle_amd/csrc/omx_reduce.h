@@ -1,0 +1,63 @@
+// Workgroup reductions shared by the element-wise kernels and the batched solver (EW_NT threads).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace omx {
+
+constexpr int EW_NT = 256;
+
+template <int NV>
+__device__ inline void block_reduce_store(double (&v)[NV], double *__restrict__ out) {
+    __shared__ double red[NV][EW_NT / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        double s = v[q];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+        if (lane == 0) red[q][wave] = s;
+    }
+    __syncthreads();
+    if (threadIdx.x < NV) {
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < EW_NT / 64; ++w) s += red[threadIdx.x][w];
+        out[threadIdx.x] = s;
+    }
+}
+
+// Sums of nblocks groups of NV partial values each, ascending, into out.
+template <int NV>
+__device__ inline void reduce_partials(int nblocks, const double *__restrict__ partial, double *__restrict__ out) {
+    double v[NV];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) v[q] = 0.0;
+    for (int b = threadIdx.x; b < nblocks; b += EW_NT)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) v[q] += partial[(int64_t)b * NV + q];
+    block_reduce_store<NV>(v, out);
+}
+
+// The line-search coefficients and then their thirteen sums (k_coeff_partial's order) into out[0..17]:
+// deterministic per-term sums, then the closed forms, written by thread 0.
+__device__ inline void coeff_final(int nblocks, const double *__restrict__ partial, double *__restrict__ out) {
+    __shared__ double tr[13];
+    reduce_partials<13>(nblocks, partial, tr);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double TrH = tr[0], TrHS = tr[1], TrHd = tr[2], TrHdS = tr[3], TrHSd = tr[4], TrHdd = tr[5],
+                     TrHddS = tr[6], TrHSdd = tr[7], TrHdSd = tr[8], TrHdSdH = tr[9], TrHddSd = tr[10],
+                     TrHdSdd = tr[11], TrHddSdd = tr[12];
+        out[0] = 2.0 * TrH - TrHS;
+        out[1] = 2.0 * (2.0 * TrHd - TrHdS - TrHSd);
+        out[2] = 2.0 * (TrHdd - TrHdSd - TrHdSdH) - TrHddS - TrHSdd;
+        out[3] = -2.0 * (TrHddSd + TrHdSdd);
+        out[4] = -TrHddSdd;
+        for (int q = 0; q < 13; ++q) out[5 + q] = tr[q];
+    }
+}
+
+}  // namespace omx

@@ -52,6 +52,9 @@ constexpr int ZBM = 64, ZBN = 128, ZBK = 8, ZNT = 256, ZPAD = 4;
 struct ZBatch {
     int64_t sA = 0, sB = 0, sC = 0;
     const int *active = nullptr;
+    // several products per system (direct-to-LDS kernel only): entry y of the batch is product y / nsys of
+    // system y % nsys, B is the system's, and with sym the products from entry `herm` on are Hermitian
+    int nsys = 0, herm = 0;
 };
 constexpr int ZWM = ZBM / 2, ZWN = ZBN / 2, ZFBM = ZWM / 16, ZFBN = ZWN / 16;
 static_assert(ZBN == 2 * ZBM, "the lower-triangle tile count assumes tiles twice as wide as tall");
@@ -370,12 +373,19 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double
     constexpr int SLICE = 2 * B * DK, STAGE = U * SLICE;  // elements: A, then B
     constexpr bool KCA = TRA, KCB = !TRB;
     __shared__ __align__(16) C2 smem[NST * STAGE];
-    const int bsys = blockIdx.y;
-    if (bat.active && !bat.active[bsys]) return;  // whole workgroup, before any barrier
+    const int bsys = blockIdx.y, sys = bat.nsys ? bsys % bat.nsys : bsys;
+    if (bat.active && !bat.active[sys]) return;  // whole workgroup, before any barrier
+    if (bat.nsys) {
+        const int T = (m + B - 1) / B;
+        if (bsys < bat.herm)
+            sym = 0;
+        else if (sym && (int)blockIdx.x >= T * (T + 1) / 2)
+            return;  // the tiles above the diagonal
+    }
     A1 += bsys * bat.sA;
     A2 += bsys * bat.sA;
-    B1 += bsys * bat.sB;
-    B2 += bsys * bat.sB;
+    B1 += sys * bat.sB;
+    B2 += sys * bat.sB;
     C += bsys * bat.sC;
     if (C0) C0 += bsys * bat.sC;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -614,7 +624,8 @@ static int run_zgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const vo
     const int nsl = NPAIR * ((k + ZGeo<R>::DK - 1) / ZGeo<R>::DK);
     int tile, splits;
     // batched launches never split K: no workspace, so the launch can be graph-captured
-    zl_shape(ctx, m, n, nsl, sym != 0, nbatch, allow_split && nbatch == 1, tile, splits);
+    const bool lower = sym && !bat.nsys;  // a grid of lower-triangle tiles
+    zl_shape(ctx, m, n, nsl, lower, bat.nsys ? (nbatch + bat.herm) / 2 : nbatch, allow_split && nbatch == 1, tile, splits);
     const int sps = (nsl + splits - 1) / splits;
     splits = (nsl + sps - 1) / sps;
     C2 *partial = nullptr;
@@ -623,12 +634,12 @@ static int run_zgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const vo
         if (rc) return rc;
         partial = (C2 *)ctx->ws;
     }
-    const int64_t tiles = zl_tiles(m, n, tile, sym != 0);
+    const int64_t tiles = zl_tiles(m, n, tile, lower);
     OMX_REQUIRE(tiles < (1LL << 31), "complex product: grid too large");
-    const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM;
+    const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM, nherm = sym ? nbatch - bat.herm : 0;
     hipEvent_t ev;
     prof_begin(ctx, cls, &ev);
-    prof_work(ctx, cls, nbatch * 8.0 * (sym ? sym_area(m, tile) : (double)m * n) * NPAIR * k,
+    prof_work(ctx, cls, 8.0 * (nherm * (nherm ? sym_area(m, tile) : 0.0) + (nbatch - nherm) * (double)m * n) * NPAIR * k,
               nbatch * 2.0 * sizeof(R) * ((double)NPAIR * ((double)m * k + (double)k * n) +
                                           (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
     const dim3 grid((unsigned)tiles, nbatch, splits);
@@ -838,6 +849,38 @@ int launch_zgemm_herm(omx_ctx ctx, int dt, int n, int k, double alpha, const voi
     return OMX_ERR_UNSUPPORTED;
 }
 
+int launch_zgemm_search_batched(omx_ctx ctx, int dt, int n, int k, const void *X, int64_t ldx, int64_t sX,
+                                const void *D, int64_t ldd, int64_t sD, void *C, int64_t ldc, int64_t sC, int nbatch,
+                                const int *active) {
+    OMX_REQUIRE(dt == OMX_C128 || dt == OMX_C64, "batched complex products: unsupported element type %d", dt);
+    int rc = OMX_ERR_UNSUPPORTED;
+    if (4LL * nbatch < 65536) {
+        ZBatch bat;
+        bat.sA = sX;
+        bat.sB = sD;
+        bat.sC = sC;
+        bat.active = active;
+        bat.nsys = nbatch;
+        bat.herm = 2 * nbatch;
+        ctx->gemm_sym = 2;
+        rc = dt == OMX_C128 ? run_zgemm_dl<double, false, false, true, true, 1>(ctx, n, n, k, 1.0, X, X, ldx, D, D, ldd, 0.0,
+                                                                                nullptr, 0.0, C, ldc, 4 * nbatch, bat, false)
+                            : run_zgemm_dl<float, false, false, true, true, 1>(ctx, n, n, k, 1.0, X, X, ldx, D, D, ldd, 0.0,
+                                                                               nullptr, 0.0, C, ldc, 4 * nbatch, bat, false);
+        ctx->gemm_sym = 0;
+    }
+    if (rc != OMX_ERR_UNSUPPORTED) return rc;
+    const size_t es = dt == OMX_C128 ? 16 : 8;
+    for (int q = 0; q < 4; ++q) {
+        const void *x = (const char *)X + es * q * nbatch * sX;
+        void *c = (char *)C + es * q * nbatch * sC;
+        rc = q < 2 ? launch_zgemm_batched(ctx, dt, 'n', 'c', n, n, k, 1.0, x, ldx, sX, D, ldd, sD, 0.0, c, ldc, sC, nbatch,
+                                          active)
+                   : launch_zgemm_herm_batched(ctx, dt, n, k, 1.0, x, ldx, sX, D, ldd, sD, c, ldc, sC, nbatch, active);
+        if (rc) return rc;
+    }
+    return OMX_OK;
+}
 int launch_zgemm_herm_batched(omx_ctx ctx, int dt, int n, int k, double alpha, const void *A, int64_t lda,
                               int64_t sA, const void *B, int64_t ldb, int64_t sB, void *C, int64_t ldc, int64_t sC,
                               int nbatch, const int *active) {
