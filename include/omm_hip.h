@@ -89,7 +89,9 @@ const char *omx_last_error(void);
 /* hipStream_t of the context, as void*, for callers that enqueue their own work. */
 void *omx_stream(omx_ctx ctx);
 
-/* Device allocation, zero-filled, as m_allocate (MatrixSwitch/src/MatrixSwitch.F90:394-415). */
+/* Device allocation, zero-filled, as m_allocate (MatrixSwitch/src/MatrixSwitch.F90:394-415).  omx_free waits
+ * for the device; up to 64 freed blocks and 1/64 of the device's memory stay with the library for later
+ * omx_malloc calls, and go back when an allocation fails or a context is finalized. */
 int omx_malloc(omx_ctx ctx, size_t bytes, void **dptr);
 int omx_free(omx_ctx ctx, void *dptr);
 /* Zero `bytes` of device memory with a fill kernel (safe under stream capture). */

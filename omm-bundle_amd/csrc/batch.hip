@@ -468,20 +468,20 @@ int omx_zbatch_create_dt(omx_ctx ctx, int dt, int nsys, int no, int nb, const in
     b->nbc = nbc;
     b->nnzb = bcolptr[nbc];
     const size_t lenC = (size_t)no * nb * nsys, lenW = (size_t)no * no * nsys;
-    bool ok = hipMalloc(&b->colptr, sizeof(int) * (nbc + 1)) == hipSuccess &&
-              hipMalloc(&b->rowidx, sizeof(int) * std::max<int64_t>(b->nnzb, 1)) == hipSuccess &&
-              hipMalloc(&b->hval, sizeof(double) * 32 * std::max<int64_t>(b->nnzb, 1) * nsys) == hipSuccess &&
-              hipMalloc(&b->sval, sizeof(double) * 32 * std::max<int64_t>(b->nnzb, 1) * nsys) == hipSuccess;
+    bool ok = dev_malloc((void **)&b->colptr, sizeof(int) * (nbc + 1)) == hipSuccess &&
+              dev_malloc((void **)&b->rowidx, sizeof(int) * std::max<int64_t>(b->nnzb, 1)) == hipSuccess &&
+              dev_malloc((void **)&b->hval, sizeof(double) * 32 * std::max<int64_t>(b->nnzb, 1) * nsys) == hipSuccess &&
+              dev_malloc((void **)&b->sval, sizeof(double) * 32 * std::max<int64_t>(b->nnzb, 1) * nsys) == hipSuccess;
     const size_t es = batch_esize(b);
     void **nm[] = {&b->C, &b->G, &b->Gp, &b->D};
-    for (auto p : nm) ok = ok && hipMalloc(p, es * lenC) == hipSuccess;
+    for (auto p : nm) ok = ok && dev_malloc(p, es * lenC) == hipSuccess;
     void **nn[] = {&b->HW, &b->SW};
-    for (auto p : nn) ok = ok && hipMalloc(p, es * lenW) == hipSuccess;
-    ok = ok && hipMalloc(&b->HC, es * 4 * lenC) == hipSuccess && hipMalloc(&b->HWd, es * 4 * lenW) == hipSuccess &&
-         hipMalloc(&b->coeff, sizeof(double) * 18 * nsys) == hipSuccess &&
-         hipMalloc(&b->sc, batch_result_bytes(nsys)) == hipSuccess &&
-         hipMalloc(&b->partial, sizeof(double) * 13 * coeff_blocks(no) * nsys) == hipSuccess &&
-         hipMalloc(&b->partial2, sizeof(double) * 2 * pr_blocks(no, nb) * nsys) == hipSuccess;
+    for (auto p : nn) ok = ok && dev_malloc(p, es * lenW) == hipSuccess;
+    ok = ok && dev_malloc((void **)&b->HC, es * 4 * lenC) == hipSuccess && dev_malloc((void **)&b->HWd, es * 4 * lenW) == hipSuccess &&
+         dev_malloc((void **)&b->coeff, sizeof(double) * 18 * nsys) == hipSuccess &&
+         dev_malloc((void **)&b->sc, batch_result_bytes(nsys)) == hipSuccess &&
+         dev_malloc((void **)&b->partial, sizeof(double) * 13 * coeff_blocks(no) * nsys) == hipSuccess &&
+         dev_malloc((void **)&b->partial2, sizeof(double) * 2 * pr_blocks(no, nb) * nsys) == hipSuccess;
     if (!ok) {
         batch_free(b);
         set_error("omx_zbatch_create: device allocation failed");
@@ -801,18 +801,18 @@ int omx_group_create(omx_ctx ctx, int nsys, const int *no, const omx_bsr *H, con
         g->m[s].fill(nullptr);
         for (int q = 0; q < 14 && ok; ++q) {
             const size_t elems = (size_t)o * (q < M_HW ? n : o);
-            ok = hipMalloc(&g->m[s][q], sizeof(double) * elems) == hipSuccess;
+            ok = dev_malloc((void **)&g->m[s][q], sizeof(double) * elems) == hipSuccess;
             if (ok) ok = hipMemsetAsync(g->m[s][q], 0, sizeof(double) * elems, ctx->stream) == hipSuccess;
         }
-        ok = ok && hipMalloc(&g->partial[s], sizeof(double) * 13 * coeff_blocks(o)) == hipSuccess &&
-             hipMalloc(&g->partial2[s], sizeof(double) * 2 * pr_blocks(o, n)) == hipSuccess &&
+        ok = ok && dev_malloc((void **)&g->partial[s], sizeof(double) * 13 * coeff_blocks(o)) == hipSuccess &&
+             dev_malloc((void **)&g->partial2[s], sizeof(double) * 2 * pr_blocks(o, n)) == hipSuccess &&
              hipStreamCreateWithFlags(&g->streams[s], hipStreamNonBlocking) == hipSuccess &&
              hipEventCreateWithFlags(&g->joins[s], hipEventDisableTiming) == hipSuccess;
     }
-    ok = ok && hipMalloc(&g->coeff, sizeof(double) * 18 * nsys) == hipSuccess &&
-         hipMalloc(&g->dots, sizeof(double) * 2 * nsys) == hipSuccess &&
-         hipMalloc(&g->sc, sizeof(double) * (4 * nsys + 2)) == hipSuccess &&
-         hipMalloc(&g->flags, sizeof(int) * F_COUNT * nsys) == hipSuccess &&
+    ok = ok && dev_malloc((void **)&g->coeff, sizeof(double) * 18 * nsys) == hipSuccess &&
+         dev_malloc((void **)&g->dots, sizeof(double) * 2 * nsys) == hipSuccess &&
+         dev_malloc((void **)&g->sc, sizeof(double) * (4 * nsys + 2)) == hipSuccess &&
+         dev_malloc((void **)&g->flags, sizeof(int) * F_COUNT * nsys) == hipSuccess &&
          hipEventCreateWithFlags(&g->fork, hipEventDisableTiming) == hipSuccess;
     if (!ok) {
         group_free(g);

@@ -400,7 +400,10 @@ struct DevBuf {
     double *p = nullptr;
     DevBuf(omx_ctx c) : ctx(c) {}
     int alloc(size_t count) {
-        if (hipMallocAsync((void **)&p, sizeof(double) * std::max<size_t>(count, 1), ctx->stream) != hipSuccess) {
+        const size_t bytes = sizeof(double) * std::max<size_t>(count, 1);
+        hipError_t e = hipMallocAsync((void **)&p, bytes, ctx->stream);
+        if (e != hipSuccess && dev_release()) e = hipMallocAsync((void **)&p, bytes, ctx->stream);
+        if (e != hipSuccess) {
             p = nullptr;
             set_error("dense factorisation: device allocation of %zu doubles failed", count);
             return OMX_ERR_NOMEM;

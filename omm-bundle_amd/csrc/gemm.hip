@@ -677,7 +677,7 @@ static int tuned_cfg(omx_ctx ctx, int m, int n, int k, const TS *A1, const TS *A
         return OMX_OK;
     }
     TS *tmp = nullptr;
-    OMX_CHECK_HIP(hipMalloc((void **)&tmp, sizeof(TS) * (size_t)std::max(m, 1) * std::max(n, 1)));
+    OMX_CHECK_HIP(dev_malloc((void **)&tmp, sizeof(TS) * (size_t)std::max(m, 1) * std::max(n, 1)));
     hipEvent_t e0, e1;
     OMX_CHECK_HIP(hipEventCreate(&e0));
     OMX_CHECK_HIP(hipEventCreate(&e1));

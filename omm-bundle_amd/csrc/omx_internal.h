@@ -147,6 +147,10 @@ struct El<double2> {
 };
 
 // Ensure ctx->ws holds at least `bytes`.  Returns OMX_OK or an error.
+// hipMalloc that gives back omx_malloc's idle blocks before it fails
+hipError_t dev_malloc(void **p, size_t bytes);
+// Gives them back; false if there are none.
+bool dev_release();
 int ensure_ws(omx_ctx ctx, size_t bytes);
 
 // Look up this device's copy of the static scratch of omx_omm_pr_dots_noalloc (once per device,

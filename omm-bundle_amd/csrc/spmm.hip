@@ -567,7 +567,7 @@ static int tuned_spmm_shape(omx_ctx ctx, int no, int nb, const T *X, int64_t ldx
                 }
     OMX_REQUIRE(!cands.empty(), "omx_spmm: grid too large");
     T *tmp = nullptr;
-    OMX_CHECK_HIP(hipMalloc((void **)&tmp, sizeof(T) * (size_t)no * nb));
+    OMX_CHECK_HIP(dev_malloc((void **)&tmp, sizeof(T) * (size_t)no * nb));
     hipEvent_t e0, e1;
     OMX_CHECK_HIP(hipEventCreate(&e0));
     OMX_CHECK_HIP(hipEventCreate(&e1));
@@ -1024,7 +1024,7 @@ extern "C" int omx_bsr_set_walk(omx_bsr A, const int *order) {
                     "omx_bsr_set_walk: order is not a permutation of the %d block columns (entry %d)", A->nbc, j);
         seen[order[j]] = 1;
     }
-    if (!A->d_walk) OMX_CHECK_HIP(hipMalloc((void **)&A->d_walk, sizeof(int) * std::max(A->nbc, 1)));
+    if (!A->d_walk) OMX_CHECK_HIP(dev_malloc((void **)&A->d_walk, sizeof(int) * std::max(A->nbc, 1)));
     OMX_CHECK_HIP(hipMemcpyAsync(A->d_walk, order, sizeof(int) * A->nbc, hipMemcpyHostToDevice, ctx->stream));
     OMX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     return OMX_OK;
@@ -1295,9 +1295,9 @@ extern "C" int omx_bsr_set_walk_groups(omx_bsr A, const int *order, int group) {
         uidx.insert(uidx.end(), u.begin(), u.end());
         gptr[g + 1] = (int)uidx.size();
     }
-    bool ok = hipMalloc((void **)&A->d_gptr, sizeof(int) * (ngroups + 1)) == hipSuccess &&
-              hipMalloc((void **)&A->d_uidx, sizeof(int) * std::max<size_t>(uidx.size(), 1)) == hipSuccess &&
-              hipMalloc((void **)&A->d_slot, slot.size()) == hipSuccess;
+    bool ok = dev_malloc((void **)&A->d_gptr, sizeof(int) * (ngroups + 1)) == hipSuccess &&
+              dev_malloc((void **)&A->d_uidx, sizeof(int) * std::max<size_t>(uidx.size(), 1)) == hipSuccess &&
+              dev_malloc((void **)&A->d_slot, slot.size()) == hipSuccess;
     if (!ok) {
         clear_patch_plan(A);
         set_error("omx_bsr_set_walk_groups: device allocation failed");
