@@ -288,7 +288,9 @@ static int tiles_of(int m, int n, int b, bool sym) {
 // the CUs (workgroups that share a CU share its matrix cores) times the slices of a part, plus what a launch,
 // a round and the reduction of the parts cost.  The constants are a least-squares fit to 60 shapes (54 x 54
 // x 108 to 4394 x 4394 x 8788, Grams, symmetric Grams and pairs; every tile and 1 to 12 parts): 11 % rms, and
-// the choices they lead to are within 1.6 % of the fastest of all on average.
+// the choices they lead to are within 1.6 % of the fastest of all on average.  How the last rounds fill the
+// CUs is modelled apart (1458 x 1458 x 2916: 64 tiles, 4 parts 240 us instead of 128, 5 parts 267; the pair
+// 1700 x 3456 x 1700: 64 tiles 644 us instead of 128, 2 parts 740).
 // A symmetric product in 128x128 tiles whose last round of resident workgroups (two per CU) is not full:
 // the parts along K that each tile of that round is split into (1: it is not split).  Only for orders
 // that are multiples of 128; elsewhere the symmetric form adds exactly as the full product does.
@@ -311,8 +313,13 @@ static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int s
         const int whole = units / (2 * ctx->num_cus) * 2;  // two workgroups of every round share a CU
         return 9.8 + 0.55 * whole + slice[q] * (whole * sps + 2.0 * sps / tail);
     }
-    return 4.5 + 0.55 * rounds + std::max(slice[q] * rounds, alone[q]) * sps +
-           (splits > 1 ? 5.3 + 8e-6 * (splits + 1) * m * n / 4.9 : 0.0);
+    // 64: three workgroups share a CU, so a last one alone costs more; with many rounds the CUs drift apart
+    // and the last is half empty on average.  128: two share a CU, and the parts of most of a third round land in pairs.
+    double per = std::max(slice[q] * rounds, alone[q]);
+    if (q == 1 && rounds % 3 == 1 && rounds < 6) per = slice[q] * (rounds - 1) + alone[q];
+    if (q == 1 && rounds >= 6) per = slice[q] * 0.5 * (rounds + (double)units / ctx->num_cus);
+    if (q == 0 && splits > 1 && rounds == 3 && 2 * units > 5 * ctx->num_cus && units < 3 * ctx->num_cus) per *= 1.1;
+    return 4.5 + 0.55 * rounds + per * sps + (splits > 1 ? 5.3 + 8e-6 * (splits + 1) * m * n / 4.9 : 0.0);
 }
 static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, double *cost = nullptr) {
     int best = 0;
