@@ -226,11 +226,10 @@ int omx_bsr_set_walk_groups(omx_bsr A, const int *order, int group);
 /* Force the GEMM tile configuration of later products on this context (-1 restores the default)
  * for the Gram and gradient products: 0 = 128x128 tiles, 4 waves, two workgroups per CU;
  * 1 = 128x128, one per CU; 2 = 256x128; 3 = 128x256; 5 = 128x128 with 8 waves of 32x64 and 6 =
- * 128x128 with 8 waves of 64x32 (FP64 products); 4 = 256x256 with 8 waves (FP32 and BF16 products
- * on FP32 storage); 7 = the operands loaded straight into LDS (every FP64 product on FP64 storage
- * with leading dimensions up to 2^20, in 128x128, 64x64 or 32x32 tiles by shape, the default
- * there; and FP32 'n','t' Grams on FP32 storage with m, n % 128 == 0 and k % 32 == 0 whose tiles
- * fill the chip, the default there; other shapes take 0).  A configuration that does not apply to
+ * 128x128 with 8 waves of 64x32 (FP64 products); 4 = 256x256 with 8 waves (BF16 products on
+ * FP32 storage); 7 = the operands loaded straight into LDS (every FP64 product on FP64 storage
+ * and every FP32 product on FP32 storage with leading dimensions up to 2^20, in 128x128, 64x64 or
+ * 32x32 tiles by shape, the default there).  A configuration that does not apply to
  * a product falls back to 0.  Used by the tile autotuner; results do not depend on it. */
 int omx_gemm_set_tile(omx_ctx ctx, int cfg);
 /* Autotuner (project-written; no counterpart in the reference): with enable != 0, the first

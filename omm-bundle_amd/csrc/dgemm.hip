@@ -1,11 +1,11 @@
-// FP64 products C := alpha * sum_p op(A_p) op(B_p) + beta0*C0 + beta*C on the FP64 matrix cores, with the
-// operands loaded straight into LDS, for every m, n, k and every leading dimension up to 2^20 (NPAIR = 2:
-// calc_G's two products back to back along K).
+// FP64 products C := alpha * sum_p op(A_p) op(B_p) + beta0*C0 + beta*C on the FP64 matrix cores, and FP32
+// ones of FP32 operands on the FP32 ones, with the operands loaded straight into LDS, for every m, n, k and
+// every leading dimension up to 2^20 (NPAIR = 2: calc_G's two products back to back along K).
 //
-// Staging.  K is taken in slices of 16.  An operand whose row index is contiguous (A 'n', B 't') lands
-// k-major: ROWS doubles per k-row, 128 / ROWS k-rows per wave load.  One whose k is contiguous (A 't',
-// B 'n') lands row-major: 16 k values (128 bytes) per row, 8 rows per wave load, logical 16-byte chunk c
-// of row r at physical chunk c ^ ((r >> 1) & 7).  A wave load is one buffer_load_dwordx4 ... lds, 16 bytes
+// Staging.  K is taken in slices of 16 (FP32: 32), 128 bytes.  An operand whose row index is contiguous (A
+// 'n', B 't') lands k-major: ROWS elements per k-row, several k-rows per wave load (FP32: with the 16-byte
+// chunks rotated by k-row, dl_rot).  One whose k is contiguous (A 't', B 'n') lands row-major: 128 bytes
+// per row, 8 rows per wave load, logical 16-byte chunk c of row r at physical chunk c ^ ((r >> 1) & 7).  A wave load is one buffer_load_dwordx4 ... lds, 16 bytes
 // per lane, lane l landing at byte 16*l.  The descriptors are rebased at every slice, so a lane's byte
 // offset is the same for every slice, and they end exactly where the matrix ends: the hardware's range
 // check is per dword, so anything past the last element arrives as zero and an odd size, an odd leading
@@ -18,6 +18,12 @@
 // the launch.  Before, only m, n % 128 == 0 with k % 16 == 0 took this path and everything else was staged
 // through registers in 128x128 tiles: 54 x 54 x 108 22 us (now 5.5), 432 x 432 x 864 about 35 us (16),
 // 1458 x 1458 x 2916 340 us (236), 4394 x 4394 x 8788 5.84 ms (5.17), gradient of 2662 x 5324 2.96 ms (2.32).
+// FP32: an FP32 step takes half the time of an FP64 one, so a slice of 32 takes as long as an FP64 slice of
+// 16 and the same tiles and model serve.  Before, only Grams of whole 128 tiles that fill the chip were
+// loaded this way: 54 x 54 x 108 21 us (now 5.8), 250 x 250 x 500 30 (6.2), 1458 x 1458 x 2916 242 (124;
+// symmetric 252, now 75; pair 512, now 237), 4394 x 4394 x 8788 4.14 ms (2.70; symmetric 2.61, now 1.37), pair
+// of 4394 x 8788 8.64 ms (5.17), 4096 x 4096 x 8192 1.90 (1.91).  Errors against FP64 (relative, Gram): 250 x
+// 500 2.4e-7 (2.1e-7), 1458 x 2916 4.9e-7 (2.1e-7), 4096 x 8192 1.6e-6 (2.5e-7); the carry costs 2 %.
 //
 // Tiles.  Three tile sizes with the same K chain per element (K in order, so the results do not depend
 // on the tile): 128x128 (8 waves of 32x64, two stages), 64x64 (4 waves of 32x32, three stages) and 32x32
@@ -32,35 +38,67 @@
 
 namespace omx {
 
-constexpr int DK = 16;  // K slice
+// Per element type: a slice of K is 128 bytes of a k-contiguous row, one matrix-core step is 16x16x4.
+template <typename R>
+struct DlT;
+template <>
+struct DlT<double> {
+    typedef d4v acc;
+    static constexpr int DK = 16, CH = 2;  // K slice; elements of a 16-byte chunk
+    __device__ static inline acc mfma(double a, double b, acc c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    __device__ static inline int row(int lq, int v) { return lq + 4 * v; }  // of a result register
+};
+template <>
+struct DlT<float> {
+    typedef f4v acc;
+    static constexpr int DK = 32, CH = 4;
+    __device__ static inline acc mfma(float a, float b, acc c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    __device__ static inline int row(int lq, int v) { return 4 * lq + v; }
+};
 
+// XOR of the 16-byte chunks of FP32 k-row kk of a k-major tile: a step reads 16 consecutive floats from each
+// of four consecutive k-rows, which would share their banks.
+template <typename R, int ROWS>
+__device__ inline int dl_rot(int kk) {
+    return sizeof(R) == 8 ? 0 : ROWS == 32 ? (kk & 2) << 1 : (kk & 3) << 2;
+}
 // Byte offset of lane `lane` of wave load `ins` of an operand tile (ROWS rows x DK) from the slice's
 // descriptor base.  KC: k contiguous.
-template <int ROWS, bool KC>
+template <typename R, int ROWS, bool KC>
 __device__ inline int dl_voff(int ins, int lane, int ld) {
+    constexpr int ES = sizeof(R);
     if constexpr (KC) {
         const int r = ins * 8 + (lane >> 3);
-        return 8 * (r * ld + 2 * ((lane & 7) ^ dl_swz(r)));
+        return ES * r * ld + 16 * ((lane & 7) ^ dl_swz(r));
     } else {
-        constexpr int LPR = ROWS / 2;  // lanes per k-row
-        return 8 * ((ins * (64 / LPR) + lane / LPR) * ld + 2 * (lane % LPR));
+        constexpr int LPR = ROWS * ES / 16;  // lanes per k-row
+        const int kk = ins * (64 / LPR) + lane / LPR;
+        return ES * kk * ld + 16 * ((lane % LPR) ^ dl_rot<R, ROWS>(kk));
     }
 }
 // The element (row r, k kk) of a staged tile; dl_at: its place in a k-contiguous one.
-__device__ inline int dl_at(int r, int kk) { return r * DK + (((kk >> 1) ^ dl_swz(r)) << 1) + (kk & 1); }
-template <int ROWS, bool KC>
-__device__ inline double dl_elem(const double *t, int r, int kk) {
-    return t[KC ? dl_at(r, kk) : kk * ROWS + r];
+template <typename R>
+__device__ inline int dl_at(int r, int kk) {
+    constexpr int CH = DlT<R>::CH;
+    return r * DlT<R>::DK + ((kk / CH) ^ dl_swz(r)) * CH + kk % CH;
+}
+template <typename R, int ROWS, bool KC>
+__device__ inline R dl_elem(const R *t, int r, int kk) {
+    return t[KC ? dl_at<R>(r, kk) : kk * ROWS + (r ^ dl_rot<R, ROWS>(kk) * DlT<R>::CH)];
 }
 // Start of an operand tile (row i0, k 0), and the bytes from there to the end of the operand (extent rows
 // x k, leading dimension ld).
-template <bool KC>
-__device__ inline const char *dl_base(const double *P, int i0, int64_t ld) {
+template <typename R, bool KC>
+__device__ inline const char *dl_base(const R *P, int i0, int64_t ld) {
     return (const char *)(P + (KC ? (int64_t)i0 * ld : i0));
 }
-template <bool KC>
+template <typename R, bool KC>
 __device__ inline int64_t dl_left(int extent, int k, int i0, int64_t ld) {
-    return 8 * (KC ? (int64_t)(extent - 1 - i0) * ld + k : (int64_t)(k - 1) * ld + (extent - i0));
+    return (int64_t)sizeof(R) * (KC ? (int64_t)(extent - 1 - i0) * ld + k : (int64_t)(k - 1) * ld + (extent - i0));
 }
 
 // Batched products: blockIdx.y selects the product, its operands and result offset by these strides
@@ -72,23 +110,24 @@ struct DlBatch {
 // EXACT: m, n are multiples of the tile and k of the slice, so nothing needs the descriptors' end, a
 // cleared tail or guarded stores; the 128x128 tile is faster without them (8192 x 8192 x 16384 Gram 29.8
 // against 29.9 ms, gradient 60.4 against 61.6 ms).
-template <class CF, bool TRA, bool TRB, int NPAIR, bool EXACT>
+template <typename R, class CF, bool TRA, bool TRB, int NPAIR, bool EXACT>
 __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int k, double alpha,
-                                                               const double *__restrict__ A1,
-                                                               const double *__restrict__ A2, int64_t lda,
-                                                               const double *__restrict__ B1,
-                                                               const double *__restrict__ B2, int64_t ldb,
-                                                               double beta0, const double *__restrict__ C0,
-                                                               int64_t ldc0, double beta, double *__restrict__ C,
+                                                               const R *__restrict__ A1,
+                                                               const R *__restrict__ A2, int64_t lda,
+                                                               const R *__restrict__ B1,
+                                                               const R *__restrict__ B2, int64_t ldb,
+                                                               double beta0, const R *__restrict__ C0,
+                                                               int64_t ldc0, double beta, R *__restrict__ C,
                                                                int64_t ldc, int sym, int tbase, int nsplit, int sps,
-                                                               double *__restrict__ partial,
+                                                               R *__restrict__ partial,
                                                                const int *__restrict__ mask, DlBatch bat) {
     constexpr int BM = CF::BM, BN = CF::BN, NST = CF::NST, NW = CF::WGM * CF::WGN;
-    constexpr int INS = DK * (BM + BN) / 128, LPW = INS / NW, U = CF::U;
+    constexpr int DK = DlT<R>::DK, LD = 1024 / sizeof(R);  // K slice, elements of a wave load
+    constexpr int INS = DK * (BM + BN) / LD, LPW = INS / NW, U = CF::U;
     constexpr int SLICE = DK * (BM + BN), STAGE = U * SLICE;
     constexpr bool KCA = TRA, KCB = !TRB;
     static_assert(LPW * NW == INS && BM == BN && NW % 2 == 0, "each wave loads one operand");
-    __shared__ __align__(16) double smem[NST * STAGE];
+    __shared__ __align__(16) R smem[NST * STAGE];
     if (mask && !*mask) return;  // system masked off (grouped solver; whole workgroup, before any barrier)
     A1 += blockIdx.y * bat.sA;
     B1 += blockIdx.y * bat.sB;
@@ -108,11 +147,19 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
     const int nsl = (k + DK - 1) / DK;  // slices of one product
     const int sb = z * sps, ns = min(NPAIR * nsl, sb + sps) - sb;
 
-    d4v acc[CF::FBM][CF::FBN];
+    typename DlT<R>::acc acc[CF::FBM][CF::FBN];
 #pragma unroll
     for (int a = 0; a < CF::FBM; ++a)
 #pragma unroll
-        for (int b = 0; b < CF::FBN; ++b) acc[a][b] = d4v{0, 0, 0, 0};
+        for (int b = 0; b < CF::FBN; ++b) acc[a][b] = typename DlT<R>::acc{0, 0, 0, 0};
+    constexpr bool CARRY = sizeof(R) == 4;
+    typename DlT<R>::acc tot[CARRY ? CF::FBM : 1][CARRY ? CF::FBN : 1];  // FP32 (see f32_carry)
+    if constexpr (CARRY) {
+#pragma unroll
+        for (int a = 0; a < CF::FBM; ++a)
+#pragma unroll
+            for (int b = 0; b < CF::FBN; ++b) tot[a][b] = typename DlT<R>::acc{0, 0, 0, 0};
+    }
     // The first half of the waves loads A, the second half B.  Slices are issued in order: the wave's
     // descriptor advances by one slice each time, and starts over at the second product of a pair.
     const bool on_b = wave >= NW / 2;
@@ -120,11 +167,11 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
     int voff[LPW];
 #pragma unroll
     for (int q = 0; q < LPW; ++q)
-        voff[q] = on_b ? dl_voff<BN, KCB>(ins0 + q, lane, (int)ldb) : dl_voff<BM, KCA>(ins0 + q, lane, (int)lda);
-    const int64_t step = 8 * (on_b ? (KCB ? DK : DK * ldb) : (KCA ? DK : DK * lda));
-    const int64_t all = on_b ? dl_left<KCB>(n, k, j0, ldb) : dl_left<KCA>(m, k, i0, lda);
-    const char *const first = on_b ? dl_base<KCB>(B1, j0, ldb) : dl_base<KCA>(A1, i0, lda);
-    const char *const second = on_b ? dl_base<KCB>(B2, j0, ldb) : dl_base<KCA>(A2, i0, lda);
+        voff[q] = on_b ? dl_voff<R, BN, KCB>(ins0 + q, lane, (int)ldb) : dl_voff<R, BM, KCA>(ins0 + q, lane, (int)lda);
+    const int64_t step = (int64_t)sizeof(R) * (on_b ? (KCB ? DK : DK * ldb) : (KCA ? DK : DK * lda));
+    const int64_t all = on_b ? dl_left<R, KCB>(n, k, j0, ldb) : dl_left<R, KCA>(m, k, i0, lda);
+    const char *const first = on_b ? dl_base<R, KCB>(B1, j0, ldb) : dl_base<R, KCA>(A1, i0, lda);
+    const char *const second = on_b ? dl_base<R, KCB>(B2, j0, ldb) : dl_base<R, KCA>(A2, i0, lda);
     const int sb_in = NPAIR == 2 && sb >= nsl ? sb - nsl : sb;
     const char *pos = (NPAIR == 2 && sb >= nsl ? second : first) + sb_in * step;
     int64_t left = all - sb_in * step;
@@ -135,7 +182,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
         for (int u = 0; u < U; ++u) {
             const int sl = s * U + u;
             if (U > 1 && sl >= ns) break;
-            double *st = smem + (s % NST) * STAGE + u * SLICE + wave * LPW * 128;
+            R *st = smem + (s % NST) * STAGE + u * SLICE + wave * LPW * LD;
             if (NPAIR == 2 && sl == sw) {
                 pos = second;
                 left = all;
@@ -146,20 +193,20 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
 #pragma unroll
             for (int q = 0; q < LPW; ++q) {
                 const int vo = voff[q];  // (a local: see k_bgemm_tn)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(st + q * 128), 16, vo, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)(st + q * LD), 16, vo, 0, 0, 0);
             }
         }
     };
     const int li = lane & 15, lk = lane >> 4;
     // one slice: the fragments of k step ks + 4 are read before the MFMAs of step ks
-    auto slice = [&](const double *As, const double *Bs) {
-        double a[2][CF::FBM], b[2][CF::FBN];
-        auto frag = [&](int ks, double (&fa)[CF::FBM], double (&fb)[CF::FBN]) {
+    auto slice = [&](const R *As, const R *Bs) {
+        R a[2][CF::FBM], b[2][CF::FBN];
+        auto frag = [&](int ks, R (&fa)[CF::FBM], R (&fb)[CF::FBN]) {
             const int kk = ks + lk;
 #pragma unroll
-            for (int f = 0; f < CF::FBM; ++f) fa[f] = dl_elem<BM, KCA>(As, wm * CF::WM + f * 16 + li, kk);
+            for (int f = 0; f < CF::FBM; ++f) fa[f] = dl_elem<R, BM, KCA>(As, wm * CF::WM + f * 16 + li, kk);
 #pragma unroll
-            for (int f = 0; f < CF::FBN; ++f) fb[f] = dl_elem<BN, KCB>(Bs, wn * CF::WN + f * 16 + li, kk);
+            for (int f = 0; f < CF::FBN; ++f) fb[f] = dl_elem<R, BN, KCB>(Bs, wn * CF::WN + f * 16 + li, kk);
         };
         frag(0, a[0], b[0]);
 #pragma unroll
@@ -171,7 +218,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
             for (int fm = 0; fm < CF::FBM; ++fm)
 #pragma unroll
                 for (int fn = 0; fn < CF::FBN; ++fn)  // (b, a): the result's columns run along i
-                    acc[fm][fn] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[cur][fn], a[cur][fm], acc[fm][fn], 0, 0, 0);
+                    acc[fm][fn] = DlT<R>::mfma(b[cur][fn], a[cur][fm], acc[fm][fn]);
             __builtin_amdgcn_sched_barrier(0);
         }
     };
@@ -192,17 +239,22 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
             for (int u = 0; u < U; ++u) {
                 const int sl = s * U + u;
                 if (U > 1 && sl >= ns) break;
-                double *As = smem + (s % NST) * STAGE + u * SLICE, *Bs = As + DK * BM;
+                R *As = smem + (s % NST) * STAGE + u * SLICE, *Bs = As + DK * BM;
                 if (!EXACT && (KCA || KCB) && (sl == t1 || (NPAIR == 2 && sl == t2))) {  // k-contiguous rows end at k
                     if (KCA)
                         for (int e = t; e < BM * DK; e += CF::NT)
-                            if (e % DK >= k % DK) As[dl_at(e / DK, e % DK)] = 0.0;
+                            if (e % DK >= k % DK) As[dl_at<R>(e / DK, e % DK)] = (R)0;
                     if (KCB)
                         for (int e = t; e < BN * DK; e += CF::NT)
-                            if (e % DK >= k % DK) Bs[dl_at(e / DK, e % DK)] = 0.0;
+                            if (e % DK >= k % DK) Bs[dl_at<R>(e / DK, e % DK)] = (R)0;
                     wg_barrier();
                 }
-                if (decltype(work)::value) slice(As, Bs);
+                if (decltype(work)::value) {
+                    slice(As, Bs);
+                    if constexpr (CARRY) {
+                        if (sl % 4 == 3 || (NPAIR == 2 && sl + 1 == sw)) f32_carry(acc, tot);
+                    }
+                }
             }
         }
     };
@@ -211,16 +263,22 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
         return;
     }
     march(std::true_type{});
+    if constexpr (CARRY) {
+#pragma unroll
+        for (int a = 0; a < CF::FBM; ++a)
+#pragma unroll
+            for (int b = 0; b < CF::FBN; ++b) acc[a][b] = tot[a][b] + acc[a][b];
+    }
     const int lq = lane >> 4;
     if (partial) {  // a K part of a split tile: the raw sums, reduced in part order later
-        double *pt = partial + (int64_t)blockIdx.x * (BM * BN);
+        R *pt = partial + (int64_t)blockIdx.x * (BM * BN);
 #pragma unroll
         for (int fm = 0; fm < CF::FBM; ++fm)
 #pragma unroll
             for (int fn = 0; fn < CF::FBN; ++fn)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    pt[(wm * CF::WM + fm * 16 + li) + (wn * CF::WN + fn * 16 + lq + 4 * v) * BM] = acc[fm][fn][v];
+                    pt[(wm * CF::WM + fm * 16 + li) + (wn * CF::WN + fn * 16 + DlT<R>::row(lq, v)) * BM] = acc[fm][fn][v];
         return;
     }
 #pragma unroll
@@ -231,42 +289,42 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
             if (!EXACT && i >= m) continue;
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int j = wj + fn * 16 + lq + 4 * v;
+                const int j = wj + fn * 16 + DlT<R>::row(lq, v);
                 if ((!EXACT && j >= n) || (sym && j > i)) continue;
-                double r = alpha * acc[fm][fn][v];
-                if (C0) r += beta0 * C0[(int64_t)i + (int64_t)j * ldc0];
-                if (beta != 0.0) r += beta * C[(int64_t)i + (int64_t)j * ldc];
-                C[(int64_t)i + (int64_t)j * ldc] = r;
-                if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = r;
+                double r = alpha * (double)acc[fm][fn][v];
+                if (C0) r += beta0 * (double)C0[(int64_t)i + (int64_t)j * ldc0];
+                if (beta != 0.0) r += beta * (double)C[(int64_t)i + (int64_t)j * ldc];
+                C[(int64_t)i + (int64_t)j * ldc] = (R)r;
+                if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = (R)r;
             }
         }
 }
 
 // C tile := alpha * (sum of its nsplit K parts, in part order) + beta0*C0 + beta*C for the tiles tbase..
 // of the launch's tile order (blockIdx.x: tile, blockIdx.y: a 1024-element slice of it).
-template <int BM, int BN>
+template <typename R, int BM, int BN>
 __global__ __launch_bounds__(256) void k_dl_split_reduce(int m, int n, int sym, int tbase, int nsplit,
-                                                         const double *__restrict__ partial, double alpha,
-                                                         double beta0, const double *__restrict__ C0, int64_t ldc0,
-                                                         double beta, double *__restrict__ C, int64_t ldc) {
+                                                         const R *__restrict__ partial, double alpha,
+                                                         double beta0, const R *__restrict__ C0, int64_t ldc0,
+                                                         double beta, R *__restrict__ C, int64_t ldc) {
     int tm, tn;
     if (sym)
         tile_of_lower(tbase + (int)blockIdx.x, (m + BM - 1) / BM, tm, tn);
     else
         tile_of(tbase + (int)blockIdx.x, (m + BM - 1) / BM, (n + BN - 1) / BN, tm, tn);
-    const double *pt = partial + (int64_t)blockIdx.x * nsplit * (BM * BN);
+    const R *pt = partial + (int64_t)blockIdx.x * nsplit * (BM * BN);
     const int e0 = blockIdx.y * 1024;
     for (int e = e0 + threadIdx.x; e < e0 + 1024; e += 256) {
         const int i = tm * BM + e % BM, j = tn * BN + e / BM;
         if (i >= m || j >= n || (sym && j > i)) continue;  // (parts above the diagonal are not written)
-        double sum = 0.0;
+        R sum = (R)0;
         for (int zz = 0; zz < nsplit; ++zz) sum += pt[(int64_t)zz * (BM * BN) + e];
         const int64_t off = (int64_t)i + (int64_t)j * ldc;
-        double r = alpha * sum;
-        if (C0) r += beta0 * C0[(int64_t)i + (int64_t)j * ldc0];
-        if (beta != 0.0) r += beta * C[off];
-        C[off] = r;
-        if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = r;
+        double r = alpha * (double)sum;
+        if (C0) r += beta0 * (double)C0[(int64_t)i + (int64_t)j * ldc0];
+        if (beta != 0.0) r += beta * (double)C[off];
+        C[off] = (R)r;
+        if (sym == 2 && j < i) C[(int64_t)j + (int64_t)i * ldc] = (R)r;
     }
 }
 
@@ -302,13 +360,12 @@ static int dl_tail_parts(omx_ctx ctx, int m, int tiles, bool sym, int nsl) {
     return parts;
 }
 static const int kDlEdge[3] = {128, 64, 32};
-static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int splits,
-                      int nbatch) {
+static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int splits, int nbatch, int es) {
     const double slice[3] = {1.90, 0.515, 0.172};  // a CU's time for one 16-wide slice of a tile
     const double alone[3] = {2.15, 0.69, 0.172};   // the same with a single workgroup on the CU
     const int units = tiles_of(m, n, kDlEdge[q], sym) * splits * nbatch, rounds = (units + ctx->num_cus - 1) / ctx->num_cus;
     const int sps = (nsl + splits - 1) / splits;
-    const int tail = dl_tail_parts(ctx, q == 0 && splits == 1 && nbatch == 1 ? m : 1, units, sym, nsl);
+    const int tail = dl_tail_parts(ctx, q == 0 && splits == 1 && nbatch == 1 && es == 8 ? m : 1, units, sym, nsl);
     if (tail > 1) {
         const int whole = units / (2 * ctx->num_cus) * 2;  // two workgroups of every round share a CU
         return 9.8 + 0.55 * whole + slice[q] * (whole * sps + 2.0 * sps / tail);
@@ -319,13 +376,13 @@ static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int s
     if (q == 1 && rounds % 3 == 1 && rounds < 6) per = slice[q] * (rounds - 1) + alone[q];
     if (q == 1 && rounds >= 6) per = slice[q] * 0.5 * (rounds + (double)units / ctx->num_cus);
     if (q == 0 && splits > 1 && rounds == 3 && 2 * units > 5 * ctx->num_cus && units < 3 * ctx->num_cus) per *= 1.1;
-    return 4.5 + 0.55 * rounds + per * sps + (splits > 1 ? 5.3 + 8e-6 * (splits + 1) * m * n / 4.9 : 0.0);
+    return 4.5 + 0.55 * rounds + per * sps + (splits > 1 ? 5.3 + 1e-6 * es * (splits + 1) * m * n / 4.9 : 0.0);
 }
-static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, double *cost = nullptr) {
+static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, int es, double *cost = nullptr) {
     int best = 0;
     double c = 0.0;
     for (int q = 0; q < 3; ++q) {
-        const double t = dl_cost(ctx, q, sym, m, n, nsl, splits, nbatch);
+        const double t = dl_cost(ctx, q, sym, m, n, nsl, splits, nbatch, es);
         if (!q || t < c) {
             best = q;
             c = t;
@@ -337,15 +394,15 @@ static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int
 
 // The number of parts with the least time; for a square result that of the full and the symmetric form
 // together, so that both add the same parts.
-int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl) {
+int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es) {
     if (ctx->launch_mask) return 1;
     int best = 1;
     double cost = 0.0;
     for (int s : {1, 2, 3, 4, 5, 6, 8, 12}) {
         if (s > 1 && nsl < 2 * s) break;
         double t, u = 0.0;
-        dl_tile(ctx, false, m, n, nsl, s, 1, &t);
-        if (m == n) dl_tile(ctx, true, m, n, nsl, s, 1, &u);
+        dl_tile(ctx, false, m, n, nsl, s, 1, es, &t);
+        if (m == n) dl_tile(ctx, true, m, n, nsl, s, 1, es, &u);
         if (s == 1 || t + u < cost) {
             best = s;
             cost = t + u;
@@ -354,11 +411,12 @@ int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl) {
     return best;
 }
 
-template <class CF, bool TRA, bool TRB, int NPAIR>
-static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int k, double alpha, const double *A1,
-                    const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
-                    const double *C0, int64_t ldc0, double beta, double *C, int64_t ldc, int nbatch,
+template <typename R, class CF, bool TRA, bool TRB, int NPAIR>
+static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int k, double alpha, const R *A1,
+                    const R *A2, int64_t lda, const R *B1, const R *B2, int64_t ldb, double beta0,
+                    const R *C0, int64_t ldc0, double beta, R *C, int64_t ldc, int nbatch,
                     const DlBatch &bat) {
+    constexpr int DK = DlT<R>::DK;
     const int tiles = tiles_of(m, n, CF::BM, sym != 0);
     const int nsl = NPAIR * ((k + DK - 1) / DK);
     int whole = tiles, rest = 0, rsplit = 1;
@@ -366,53 +424,53 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
         whole = 0;
         rest = tiles;
         rsplit = splits;
-    } else if (CF::BM == 128 && (rsplit = dl_tail_parts(ctx, m, tiles, sym != 0, nsl)) > 1) {
+    } else if (CF::BM == 128 && sizeof(R) == 8 && (rsplit = dl_tail_parts(ctx, m, tiles, sym != 0, nsl)) > 1) {
         rest = tiles % (2 * ctx->num_cus);
         whole = tiles - rest;
         sps = nsl / rsplit;
     }
-    auto launch = [&](int grid, int tbase, int parts, int per, double *partial, const int *mask) {
+    auto launch = [&](int grid, int tbase, int parts, int per, R *partial, const int *mask) {
         if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
-            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, CF::BM == 128>), dim3(grid, nbatch), dim3(CF::NT), 0,
+            hipLaunchKernelGGL((k_dgemm_dl<R, CF, TRA, TRB, NPAIR, CF::BM == 128>), dim3(grid, nbatch), dim3(CF::NT), 0,
                                ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
                                tbase, parts, per, partial, mask, bat);
         else
-            hipLaunchKernelGGL((k_dgemm_dl<CF, TRA, TRB, NPAIR, false>), dim3(grid, nbatch), dim3(CF::NT), 0,
+            hipLaunchKernelGGL((k_dgemm_dl<R, CF, TRA, TRB, NPAIR, false>), dim3(grid, nbatch), dim3(CF::NT), 0,
                                ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
                                tbase, parts, per, partial, mask, bat);
     };
     if (whole) launch(whole, 0, 1, nsl, nullptr, ctx->launch_mask);
     if (rest) {
-        int rc = ensure_ws(ctx, sizeof(double) * (size_t)rest * rsplit * CF::BM * CF::BN);
+        int rc = ensure_ws(ctx, sizeof(R) * (size_t)rest * rsplit * CF::BM * CF::BN);
         if (rc) return rc;
-        launch(rest * rsplit, whole, rsplit, sps, (double *)ctx->ws, nullptr);
-        hipLaunchKernelGGL((k_dl_split_reduce<CF::BM, CF::BN>), dim3(rest, CF::BM * CF::BN / 1024), dim3(256), 0,
-                           ctx->stream, m, n, sym, whole, rsplit, (const double *)ctx->ws, alpha, beta0, C0,
+        launch(rest * rsplit, whole, rsplit, sps, (R *)ctx->ws, nullptr);
+        hipLaunchKernelGGL((k_dl_split_reduce<R, CF::BM, CF::BN>), dim3(rest, CF::BM * CF::BN / 1024), dim3(256), 0,
+                           ctx->stream, m, n, sym, whole, rsplit, (const R *)ctx->ws, alpha, beta0, C0,
                            ldc0, beta, C, ldc);
     }
     OMX_CHECK_HIP(hipGetLastError());
     return OMX_OK;
 }
 
-template <bool TRA, bool TRB, int NPAIR>
-static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const double *A1, const double *A2, int64_t lda,
-                   const double *B1, const double *B2, int64_t ldb, double beta0, const double *C0, int64_t ldc0,
-                   double beta, double *C, int64_t ldc, int nbatch = 1, const DlBatch &bat = DlBatch()) {
+template <typename R, bool TRA, bool TRB, int NPAIR>
+static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const R *A1, const R *A2, int64_t lda,
+                   const R *B1, const R *B2, int64_t ldb, double beta0, const R *C0, int64_t ldc0,
+                   double beta, R *C, int64_t ldc, int nbatch = 1, const DlBatch &bat = DlBatch()) {
     const int sym = (m == n && NPAIR == 1 && !TRA && TRB) ? ctx->gemm_sym : 0;
-    const int nsl = NPAIR * ((k + DK - 1) / DK);
-    int splits = nbatch > 1 ? 1 : dgemm_k_splits(ctx, m, n, nsl);
+    const int nsl = NPAIR * ((k + DlT<R>::DK - 1) / DlT<R>::DK);
+    int splits = nbatch > 1 ? 1 : dgemm_k_splits(ctx, m, n, nsl, sizeof(R));
     const int sps = (nsl + splits - 1) / splits;
     splits = (nsl + sps - 1) / sps;
     const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM;
-    const int tile = dl_tile(ctx, sym != 0, m, n, nsl, splits, nbatch);
+    const int tile = dl_tile(ctx, sym != 0, m, n, nsl, splits, nbatch, sizeof(R));
     hipEvent_t ev;
     prof_begin(ctx, cls, &ev);
     prof_work(ctx, cls, 2.0 * (sym ? sym_area(m, kDlEdge[tile]) : (double)m * n) * (double)NPAIR * k,
-              sizeof(double) * ((double)NPAIR * ((double)m * k + (double)k * n) +
+              sizeof(R) * ((double)NPAIR * ((double)m * k + (double)k * n) +
                                 (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
     int rc;
 #define OMX_DL_RUN(CF) \
-    run_tile<CF, TRA, TRB, NPAIR>(ctx, sym, splits, sps, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, \
+    run_tile<R, CF, TRA, TRB, NPAIR>(ctx, sym, splits, sps, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, \
                                   nbatch, bat)
     if (tile == 0)
         rc = OMX_DL_RUN(Dl128);
@@ -426,19 +484,32 @@ static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const double 
     return rc;
 }
 
-int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const double *A1,
-                 const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
-                 const double *C0, int64_t ldc0, double beta, double *C, int64_t ldc) {
+template <typename R>
+static int launch_dl(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const R *A1, const R *A2,
+                     int64_t lda, const R *B1, const R *B2, int64_t ldb, double beta0, const R *C0, int64_t ldc0, double beta,
+                     R *C, int64_t ldc) {
     if (m <= 0 || n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20))  // 32-bit lane offsets
         return OMX_ERR_UNSUPPORTED;
 #define OMX_DL_OPS(TA, TB, NP) \
-    run_ops<TA, TB, NP>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc)
+    run_ops<R, TA, TB, NP>(ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc)
     if (npair == 2) return OMX_DL_OPS(false, false, 2);
     if (!trA && !trB) return OMX_DL_OPS(false, false, 1);
     if (!trA && trB) return OMX_DL_OPS(false, true, 1);
     if (trA && !trB) return OMX_DL_OPS(true, false, 1);
     return OMX_DL_OPS(true, true, 1);
 #undef OMX_DL_OPS
+}
+
+int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const double *A1,
+                 const double *A2, int64_t lda, const double *B1, const double *B2, int64_t ldb, double beta0,
+                 const double *C0, int64_t ldc0, double beta, double *C, int64_t ldc) {
+    return launch_dl(ctx, trA, trB, npair, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc);
+}
+
+int launch_sgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const float *A1,
+                 const float *A2, int64_t lda, const float *B1, const float *B2, int64_t ldb, double beta0, const float *C0,
+                 double beta, float *C, int64_t ldc) {
+    return launch_dl(ctx, trA, trB, npair, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc, beta, C, ldc);
 }
 
 int launch_dgemm_batched(omx_ctx ctx, int m, int n, int k, double alpha, const double *A, int64_t lda, int64_t sA,
@@ -448,7 +519,7 @@ int launch_dgemm_batched(omx_ctx ctx, int m, int n, int k, double alpha, const d
     bat.sA = sA;
     bat.sB = sB;
     bat.sC = sC;
-    return run_ops<false, false, 1>(ctx, m, n, k, alpha, A, A, lda, B, B, ldb, 0.0, nullptr, 0, 0.0, C, ldc, nbatch, bat);
+    return run_ops<double, false, false, 1>(ctx, m, n, k, alpha, A, A, lda, B, B, ldb, 0.0, nullptr, 0, 0.0, C, ldc, nbatch, bat);
 }
 
 }  // namespace omx

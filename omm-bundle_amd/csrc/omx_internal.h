@@ -234,9 +234,13 @@ int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k
 // nbatch products C_b := alpha*A_b*B_b ('n','n') at strides sA, sB, sC elements.
 int launch_dgemm_batched(omx_ctx ctx, int m, int n, int k, double alpha, const double *A, int64_t lda, int64_t sA,
                          const double *B, int64_t ldb, int64_t sB, double *C, int64_t ldc, int64_t sC, int nbatch);
-// Parts K is split into for an FP64 product of nsl slices of 16; a function of the shape alone, so that
-// every tile configuration and the symmetric form add in the same order.
-int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl);
+// The same for FP32 products on FP32 storage (C0 has C's leading dimension).
+int launch_sgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const float *A1,
+                 const float *A2, int64_t lda, const float *B1, const float *B2, int64_t ldb, double beta0, const float *C0,
+                 double beta, float *C, int64_t ldc);
+// Parts K is split into for such a product of nsl slices of 128 bytes (es: element size); a function of the
+// shape alone, so that every tile configuration and the symmetric form add in the same order.
+int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es);
 // C := alpha*A*B^T known to be symmetric (n x n, 'n','t' operands of k columns): the lower-triangle
 // tiles where the kernels allow it, then a mirror of the lower triangle onto the upper (both honour
 // ctx->launch_mask).
