@@ -355,7 +355,11 @@ struct ZlCfg {
 typedef ZlCfg<64, 2, 1> Zl64;
 typedef ZlCfg<32, 2, 4> Zl32;
 
-template <typename R, class CF, bool TRA, bool CJA, bool TRB, bool CJB, int NPAIR>
+// CARRY (complex64, single products): sums of 32 values of K are added up apart (see f32_carry), which keeps
+// the error at or below that of the many parts K used to be split into (Gram 54 x 108: 1.6e-7 -> 1.4e-7, 2000 x
+// 4000: 1.6e-6 -> 2.5e-7; with one chain 900 x 2916 1.3e-6) for 3 %.  Batched products keep one chain: their
+// roundings are part of a k-point solve's trajectory.
+template <typename R, class CF, bool TRA, bool CJA, bool TRB, bool CJB, int NPAIR, bool CARRY>
 __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double alpha,
                                                     const typename ZPrec<R>::cplx *__restrict__ A1,
                                                     const typename ZPrec<R>::cplx *__restrict__ A2, int64_t lda,
@@ -407,6 +411,16 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double
             are[a][b] = AV{0, 0, 0, 0};
             aim[a][b] = AV{0, 0, 0, 0};
         }
+    AV tre[CARRY ? FB : 1][CARRY ? FB : 1], tim[CARRY ? FB : 1][CARRY ? FB : 1];
+    if constexpr (CARRY) {
+#pragma unroll
+        for (int a = 0; a < FB; ++a)
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                tre[a][b] = AV{0, 0, 0, 0};
+                tim[a][b] = AV{0, 0, 0, 0};
+            }
+    }
     // waves 0 and 1 load A, 2 and 3 B; the wave's descriptor advances by one slice each time and starts
     // over at the second product of a pair
     const bool on_b = wave >= 2;
@@ -506,7 +520,15 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double
                         }
                     wg_barrier();
                 }
-                if (decltype(work)::value) slice(As, Bs);
+                if (decltype(work)::value) {
+                    slice(As, Bs);
+                    if constexpr (CARRY) {
+                        if (sl % 2 == 1 || (NPAIR == 2 && sl + 1 == sw)) {
+                            f32_carry(are, tre);
+                            f32_carry(aim, tim);
+                        }
+                    }
+                }
             }
         }
     };
@@ -515,6 +537,15 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double
         return;
     }
     march(std::true_type{});
+    if constexpr (CARRY) {
+#pragma unroll
+        for (int a = 0; a < FB; ++a)
+#pragma unroll
+            for (int b = 0; b < FB; ++b) {
+                are[a][b] = tre[a][b] + are[a][b];
+                aim[a][b] = tim[a][b] + aim[a][b];
+            }
+    }
     const int lq = lane >> 4;
 #pragma unroll
     for (int fm = 0; fm < FB; ++fm)
@@ -643,14 +674,22 @@ static int run_zgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const vo
               nbatch * 2.0 * sizeof(R) * ((double)NPAIR * ((double)m * k + (double)k * n) +
                                           (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
     const dim3 grid((unsigned)tiles, nbatch, splits);
-#define OMX_ZL_RUN(CF)                                                                                              \
-    hipLaunchKernelGGL((k_zgemm_dl<R, CF, TRA, CJA, TRB, CJB, NPAIR>), grid, dim3(256), 0, ctx->stream, m, n, k, alpha, \
+#define OMX_ZL_RUN(CF, CY)                                                                                          \
+    hipLaunchKernelGGL((k_zgemm_dl<R, CF, TRA, CJA, TRB, CJB, NPAIR, CY>), grid, dim3(256), 0, ctx->stream, m, n, k, alpha, \
                        (const C2 *)A1, (const C2 *)A2, lda, (const C2 *)B1, (const C2 *)B2, ldb, beta0,             \
                        (const C2 *)C0, beta, (C2 *)C, ldc, sym, sps, partial, bat)
-    if (tile == 64)
-        OMX_ZL_RUN(Zl64);
-    else
-        OMX_ZL_RUN(Zl32);
+    constexpr bool single = sizeof(R) == 4;
+    if (tile == 64) {
+        if (single && allow_split)
+            OMX_ZL_RUN(Zl64, single);
+        else
+            OMX_ZL_RUN(Zl64, false);
+    } else {
+        if (single && allow_split)
+            OMX_ZL_RUN(Zl32, single);
+        else
+            OMX_ZL_RUN(Zl32, false);
+    }
 #undef OMX_ZL_RUN
     if (partial)
         hipLaunchKernelGGL((k_zl_reduce<R>), dim3((unsigned)std::min<int64_t>(((int64_t)m * n + 255) / 256, 8192)),
