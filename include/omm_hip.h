@@ -277,6 +277,15 @@ int omx_omm_coeff(omx_ctx ctx, int dt, int n, int64_t ld, const void *HW, const 
                   const void *SWd, const void *HWdd, const void *SWdd, double *coeff);
 
 /*
+ * The products of a line search along D: HWd = HC D^T, SWd = SC D^T, and the symmetric HWdd = HG D^T and
+ * SWdd = SG D^T with HG = D H, SG = D S (n x n; operands n x k; libOMM/src/omm.F90:448-464), dt OMX_F64 or
+ * OMX_F32.  One launch where that is faster than one by one.
+ */
+int omx_omm_search(omx_ctx ctx, int prec, int dt, int n, int k, const void *HC, const void *SC, const void *HG,
+                   const void *SG, int64_t ldx, const void *D, int64_t ldd, void *HWd, void *SWd, void *HWdd, void *SWdd,
+                   int64_t ldw);
+
+/*
  * G := 4*HC - 2*SW*HC - 2*HW*SC in one MFMA product with a K = 2n contraction
  * (calc_G, libOMM/src/omm_ops.F90:17-39).  HW, SW: n x n; HC, SC, G: n x m.
  */

@@ -105,6 +105,10 @@ __device__ inline int64_t dl_left(int extent, int k, int i0, int64_t ld) {
 // (elements; single products only, no split of K).
 struct DlBatch {
     int64_t sA = 0, sB = 0, sC = 0;
+    // with `four`: the line-search products A[y] B^T into C[y], the last two of them symmetric
+    int four = 0;
+    const void *A[4] = {nullptr, nullptr, nullptr, nullptr};
+    void *C[4] = {nullptr, nullptr, nullptr, nullptr};
 };
 
 // EXACT: m, n are multiples of the tile and k of the slice, so nothing needs the descriptors' end, a
@@ -129,9 +133,19 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
     static_assert(LPW * NW == INS && BM == BN && NW % 2 == 0, "each wave loads one operand");
     __shared__ __align__(16) R smem[NST * STAGE];
     if (mask && !*mask) return;  // system masked off (grouped solver; whole workgroup, before any barrier)
-    A1 += blockIdx.y * bat.sA;
-    B1 += blockIdx.y * bat.sB;
-    C += blockIdx.y * bat.sC;
+    if (bat.four) {
+        const int T = (m + BM - 1) / BM;
+        A1 = (const R *)bat.A[blockIdx.y];
+        C = (R *)bat.C[blockIdx.y];
+        if (blockIdx.y < 2)
+            sym = 0;
+        else if ((int)blockIdx.x >= T * (T + 1) / 2)
+            return;  // the tiles above the diagonal
+    } else {
+        A1 += blockIdx.y * bat.sA;
+        B1 += blockIdx.y * bat.sB;
+        C += blockIdx.y * bat.sC;
+    }
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int wm = wave / CF::WGN, wn = wave % CF::WGN;
     // tile w of the launch's tile order and the part z of K it takes
@@ -360,23 +374,31 @@ static int dl_tail_parts(omx_ctx ctx, int m, int tiles, bool sym, int nsl) {
     return parts;
 }
 static const int kDlEdge[3] = {128, 64, 32};
-static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int splits, int nbatch, int es) {
+// units workgroups of tile q and sps slices each
+static double dl_time(omx_ctx ctx, int q, int64_t units, int sps) {
     const double slice[3] = {1.90, 0.515, 0.172};  // a CU's time for one 16-wide slice of a tile
     const double alone[3] = {2.15, 0.69, 0.172};   // the same with a single workgroup on the CU
+    const int64_t rounds = (units + ctx->num_cus - 1) / ctx->num_cus;
+    // 64: three workgroups share a CU, so a last one alone costs more; with many rounds the CUs drift apart
+    // and the last is half empty on average.
+    double per = std::max(slice[q] * rounds, alone[q]);
+    if (q == 1 && rounds % 3 == 1 && rounds < 6) per = slice[q] * (rounds - 1) + alone[q];
+    if (q == 1 && rounds >= 6) per = slice[q] * 0.5 * (rounds + (double)units / ctx->num_cus);
+    return 4.5 + 0.55 * rounds + per * sps;
+}
+static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int splits, int nbatch, int es) {
     const int units = tiles_of(m, n, kDlEdge[q], sym) * splits * nbatch, rounds = (units + ctx->num_cus - 1) / ctx->num_cus;
     const int sps = (nsl + splits - 1) / splits;
     const int tail = dl_tail_parts(ctx, q == 0 && splits == 1 && nbatch == 1 && es == 8 ? m : 1, units, sym, nsl);
     if (tail > 1) {
         const int whole = units / (2 * ctx->num_cus) * 2;  // two workgroups of every round share a CU
-        return 9.8 + 0.55 * whole + slice[q] * (whole * sps + 2.0 * sps / tail);
+        return 9.8 + 0.55 * whole + 1.90 * (whole * sps + 2.0 * sps / tail);
     }
-    // 64: three workgroups share a CU, so a last one alone costs more; with many rounds the CUs drift apart
-    // and the last is half empty on average.  128: two share a CU, and the parts of most of a third round land in pairs.
-    double per = std::max(slice[q] * rounds, alone[q]);
-    if (q == 1 && rounds % 3 == 1 && rounds < 6) per = slice[q] * (rounds - 1) + alone[q];
-    if (q == 1 && rounds >= 6) per = slice[q] * 0.5 * (rounds + (double)units / ctx->num_cus);
-    if (q == 0 && splits > 1 && rounds == 3 && 2 * units > 5 * ctx->num_cus && units < 3 * ctx->num_cus) per *= 1.1;
-    return 4.5 + 0.55 * rounds + per * sps + (splits > 1 ? 5.3 + 1e-6 * es * (splits + 1) * m * n / 4.9 : 0.0);
+    double t = dl_time(ctx, q, units, sps);
+    // 128: two workgroups share a CU, and the parts of most of a third round land in pairs.
+    if (q == 0 && splits > 1 && rounds == 3 && 2 * units > 5 * ctx->num_cus && units < 3 * ctx->num_cus)
+        t += 0.1 * 1.90 * 3 * sps;
+    return t + (splits > 1 ? 5.3 + 1e-6 * es * (splits + 1) * m * n / 4.9 : 0.0);
 }
 static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, int es, double *cost = nullptr) {
     int best = 0;
@@ -498,6 +520,67 @@ static int launch_dl(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, i
     if (trA && !trB) return OMX_DL_OPS(true, false, 1);
     return OMX_DL_OPS(true, true, 1);
 #undef OMX_DL_OPS
+}
+
+// The line-search products of one CG step in one launch (see DlBatch), where the model finds that faster than
+// one by one: small results leave most of the chip idle each, larger ones are split along K to fill it
+// (twelve steps of omm() at 54 x 108 1.65 -> 1.33 ms, four at 1458 x 2916 6.48 -> 6.26 ms).
+template <typename R>
+static int run_search(omx_ctx ctx, int n, int k, const R *const A[4], int64_t lda, const R *B, int64_t ldb, R *const C[4],
+                      int64_t ldc) {
+    if (n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20)) return OMX_ERR_UNSUPPORTED;
+    const int nsl = (k + DlT<R>::DK - 1) / DlT<R>::DK, splits = dgemm_k_splits(ctx, n, n, nsl, sizeof(R));
+    int tile = 0;
+    double best = 0.0, full = 0.0, lower = 0.0;
+    for (int q = 0; q < 3; ++q) {
+        const double t = dl_time(ctx, q, 2LL * (tiles_of(n, n, kDlEdge[q], false) + tiles_of(n, n, kDlEdge[q], true)), nsl);
+        if (!q || t < best) {
+            tile = q;
+            best = t;
+        }
+    }
+    dl_tile(ctx, false, n, n, nsl, splits, 1, sizeof(R), &full);
+    dl_tile(ctx, true, n, n, nsl, splits, 1, sizeof(R), &lower);
+    if (best >= 2.0 * (full + lower)) return OMX_ERR_UNSUPPORTED;
+    DlBatch bat;
+    bat.four = 1;
+    for (int q = 0; q < 4; ++q) {
+        bat.A[q] = A[q];
+        bat.C[q] = C[q];
+    }
+    hipEvent_t ev;
+    prof_begin(ctx, OMX_K_GEMM, &ev);
+    prof_work(ctx, OMX_K_GEMM, 4.0 * ((double)n * n + sym_area(n, kDlEdge[tile])) * k,
+              sizeof(R) * (5.0 * n * k + 4.0 * (double)n * n));
+    const dim3 grid(tiles_of(n, n, kDlEdge[tile], false), 4);
+#define OMX_DL_FOUR(CF, EX)                                                                                                \
+    hipLaunchKernelGGL((k_dgemm_dl<R, CF, false, true, 1, EX>), grid, dim3(CF::NT), 0, ctx->stream, n, n, k, 1.0, A[0], A[0], \
+                       lda, B, B, ldb, 0.0, (const R *)nullptr, (int64_t)0, 0.0, C[0], ldc, 2, 0, 1, nsl, (R *)nullptr,     \
+                       ctx->launch_mask, bat)
+    if (tile == 0 && n % 128 == 0 && k % DlT<R>::DK == 0)
+        OMX_DL_FOUR(Dl128, true);
+    else if (tile == 0)
+        OMX_DL_FOUR(Dl128, false);
+    else if (tile == 1)
+        OMX_DL_FOUR(Dl64, false);
+    else
+        OMX_DL_FOUR(Dl32, false);
+#undef OMX_DL_FOUR
+    prof_end(ctx, OMX_K_GEMM, ev);
+    OMX_CHECK_HIP(hipGetLastError());
+    return OMX_OK;
+}
+
+int launch_search(omx_ctx ctx, int dt, int n, int k, const void *const A[4], int64_t lda, const void *B, int64_t ldb,
+                  void *const C[4], int64_t ldc) {
+    if (dt == OMX_F64) {
+        const double *const a[4] = {(const double *)A[0], (const double *)A[1], (const double *)A[2], (const double *)A[3]};
+        double *const c[4] = {(double *)C[0], (double *)C[1], (double *)C[2], (double *)C[3]};
+        return run_search(ctx, n, k, a, lda, (const double *)B, ldb, c, ldc);
+    }
+    const float *const a[4] = {(const float *)A[0], (const float *)A[1], (const float *)A[2], (const float *)A[3]};
+    float *const c[4] = {(float *)C[0], (float *)C[1], (float *)C[2], (float *)C[3]};
+    return run_search(ctx, n, k, a, lda, (const float *)B, ldb, c, ldc);
 }
 
 int launch_dgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const double *A1,

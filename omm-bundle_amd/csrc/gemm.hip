@@ -1192,6 +1192,29 @@ extern "C" int omx_gemm(omx_ctx ctx, int prec, int dt, char opA, char opB, int m
     return launch_gemm(ctx, prec, dt, trA, trB, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
 }
 
+extern "C" int omx_omm_search(omx_ctx ctx, int prec, int dt, int n, int k, const void *HC, const void *SC, const void *HG,
+                              const void *SG, int64_t ldx, const void *D, int64_t ldd, void *HWd, void *SWd, void *HWdd,
+                              void *SWdd, int64_t ldw) {
+    OMX_REQUIRE(ctx && n >= 0 && k >= 0, "omx_omm_search: bad arguments");
+    OMX_REQUIRE(ldx >= std::max(1, n) && ldd >= std::max(1, n) && ldw >= std::max(1, n),
+                "omx_omm_search: leading dimension too small");
+    OMX_REQUIRE(dt == OMX_F64 || dt == OMX_F32, "omx_omm_search: unsupported element type %d", dt);
+    if (n == 0) return OMX_OK;
+    OMX_REQUIRE(HC && SC && HG && SG && D && HWd && SWd && HWdd && SWdd, "omx_omm_search: null operand");
+    const void *const A[4] = {HC, SC, HG, SG};
+    void *const C[4] = {HWd, SWd, HWdd, SWdd};
+    if (prec == (dt == OMX_F64 ? OMX_PREC_F64 : OMX_PREC_F32) && (ctx->gemm_cfg < 0 || ctx->gemm_cfg == 7) && !ctx->autotune) {
+        const int rc = launch_search(ctx, dt, n, k, A, ldx, D, ldd, C, ldw);
+        if (rc != OMX_ERR_UNSUPPORTED) return rc;
+    }
+    for (int q = 0; q < 4; ++q) {
+        const int rc = q < 2 ? omx_gemm(ctx, prec, dt, 'n', 't', n, n, k, 1.0, A[q], ldx, D, ldd, 0.0, C[q], ldw)
+                             : omx_gemm_sym(ctx, prec, dt, n, k, 1.0, A[q], ldx, D, ldd, C[q], ldw);
+        if (rc) return rc;
+    }
+    return OMX_OK;
+}
+
 extern "C" int omx_gemm_sym(omx_ctx ctx, int prec, int dt, int n, int k, double alpha, const void *A, int64_t lda,
                             const void *B, int64_t ldb, void *C, int64_t ldc) {
     OMX_REQUIRE(ctx, "omx_gemm_sym: null context");

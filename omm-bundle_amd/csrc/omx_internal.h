@@ -238,6 +238,10 @@ int launch_dgemm_batched(omx_ctx ctx, int m, int n, int k, double alpha, const d
 int launch_sgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k, double alpha, const float *A1,
                  const float *A2, int64_t lda, const float *B1, const float *B2, int64_t ldb, double beta0, const float *C0,
                  double beta, float *C, int64_t ldc);
+// C_q := A_q B^T (n x n, k columns; q = 2, 3 symmetric) in one launch, dt OMX_F64 or OMX_F32 for operands and
+// products; OMX_ERR_UNSUPPORTED (nothing launched) where single products are faster.
+int launch_search(omx_ctx ctx, int dt, int n, int k, const void *const A[4], int64_t lda, const void *B, int64_t ldb,
+                  void *const C[4], int64_t ldc);
 // Parts K is split into for such a product of nsl slices of 128 bytes (es: element size); a function of the
 // shape alone, so that every tile configuration and the symmetric form add in the same order.
 int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es);

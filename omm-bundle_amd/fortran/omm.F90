@@ -347,15 +347,11 @@ contains
     else
       if (std_form) then
         call mm_multiply(pC, 'n', G, 'c', SWd, 1.0_dp, 0.0_dp, lab)
-      else
-        call mm_multiply(pSC, 'n', G, 'c', SWd, 1.0_dp, 0.0_dp, lab)
-      end if
-      call mm_multiply(HC, 'n', G, 'c', pHWd, 1.0_dp, 0.0_dp, lab)
-      call calc_AW(H, G, pHWdd, HG, lab)
-      if (std_form) then
+        call mm_multiply(HC, 'n', G, 'c', pHWd, 1.0_dp, 0.0_dp, lab)
+        call calc_AW(H, G, pHWdd, HG, lab)
         call mm_multiply(G, 'n', G, 'c', SWdd, 1.0_dp, 0.0_dp, lab)
       else
-        call calc_AW(S, G, SWdd, pSG, lab)
+        call search_products(H, S, G, HC, pSC, HG, pSG, pHWd, SWd, pHWdd, SWdd, lab)
       end if
     end if
     call calc_coeff(pHW, pSW, pHWd, SWd, pHWdd, SWdd, work1, coeff, lab)
@@ -418,17 +414,13 @@ contains
         e_min_old = e_min
         ! after the first step of a phase, line-search data along the new direction (omm.F90:448-464)
         if (steps > 0) then
-          call mm_multiply(HC, 'n', D, 'c', pHWd, 1.0_dp, 0.0_dp, lab)
           if (std_form) then
+            call mm_multiply(HC, 'n', D, 'c', pHWd, 1.0_dp, 0.0_dp, lab)
             call mm_multiply(pC, 'n', D, 'c', SWd, 1.0_dp, 0.0_dp, lab)
-          else
-            call mm_multiply(pSC, 'n', D, 'c', SWd, 1.0_dp, 0.0_dp, lab)
-          end if
-          call calc_AW(H, D, pHWdd, HG, lab)
-          if (std_form) then
+            call calc_AW(H, D, pHWdd, HG, lab)
             call mm_multiply(D, 'n', D, 'c', SWdd, 1.0_dp, 0.0_dp, lab)
           else
-            call calc_AW(S, D, SWdd, pSG, lab)
+            call search_products(H, S, D, HC, pSC, HG, pSG, pHWd, SWd, pHWdd, SWdd, lab)
           end if
           call calc_coeff(pHW, pSW, pHWd, SWd, pHWdd, SWdd, work1, coeff, lab)
         end if

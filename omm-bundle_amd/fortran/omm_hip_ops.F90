@@ -110,6 +110,34 @@ contains
     call mm_multiply(AC, 'n', C, 'c', AW, 1.0_dp, 0.0_dp, m_operation)
   end subroutine calc_AW
 
+  !> HG := D*H, SG := D*S, HWd := HC*D^T, SWd := SC*D^T, HWdd := HG*D^T, SWdd := SG*D^T: a line search's
+  !> products along D (omm.F90:448-464), the four of them in one call on device storage.
+  subroutine search_products(H, S, D, HC, SC, HG, SG, HWd, SWd, HWdd, SWdd, m_operation)
+    character(3), intent(in) :: m_operation
+    type(matrix), intent(in) :: H, S, D, HC, SC
+    type(matrix), intent(inout) :: HG, SG, HWd, SWd, HWdd, SWdd
+    integer(c_int) :: rc
+    if (opt_fused .and. on_device(D) .and. on_device(HC) .and. on_device(SC) .and. on_device(HG) .and. on_device(SG) &
+        .and. on_device(HWd) .and. on_device(SWd) .and. on_device(HWdd) .and. on_device(SWdd) &
+        .and. all([HC%dtype, SC%dtype, HG%dtype, SG%dtype, HWd%dtype, SWd%dtype, HWdd%dtype, SWdd%dtype] == D%dtype) &
+        .and. all([SC%ld, HG%ld, SG%ld] == HC%ld) .and. all([SWd%ld, HWdd%ld, SWdd%ld] == HWd%ld) &
+        .and. (D%dtype == OMX_F64 .or. D%dtype == OMX_F32) .and. &
+        (opt_sym_gram == 2 .or. ((opt_sym_gram == 1 .or. opt_sym_gram == 3) .and. m_operation == 'hip') .or. &
+         (opt_sym_gram == 3 .and. m_operation == 'h32'))) then
+      call mm_multiply(D, 'n', H, 'n', HG, 1.0_dp, 0.0_dp, m_operation)
+      call mm_multiply(D, 'n', S, 'n', SG, 1.0_dp, 0.0_dp, m_operation)
+      rc = omx_omm_search(ms_hip_ctx(), ms_label_prec(m_operation), D%dtype, int(HWd%dim1, c_int), int(D%dim2, c_int), &
+                          HC%dptr, SC%dptr, HG%dptr, SG%dptr, HC%ld, D%dptr, D%ld, HWd%dptr, SWd%dptr, HWdd%dptr, &
+                          SWdd%dptr, HWd%ld)
+      if (rc /= 0) call die('search_products: '//omx_error_string())
+      return
+    end if
+    call mm_multiply(HC, 'n', D, 'c', HWd, 1.0_dp, 0.0_dp, m_operation)
+    call mm_multiply(SC, 'n', D, 'c', SWd, 1.0_dp, 0.0_dp, m_operation)
+    call calc_AW(H, D, HWdd, HG, m_operation)
+    call calc_AW(S, D, SWdd, SG, m_operation)
+  end subroutine search_products
+
   !> CAW := AW*C1; A := C1^T*CAW  (omm_ops.F90:104-124)
   subroutine calc_A(AW, C1, A, CAW, m_operation)
     character(3), intent(in) :: m_operation

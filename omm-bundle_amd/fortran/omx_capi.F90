@@ -248,6 +248,13 @@ module omx_capi
       integer(c_int64_t), value :: ld
       real(c_double), intent(out) :: coeff(5)
     end function
+    integer(c_int) function omx_omm_search(ctx, prec, dt, n, k, HC, SC, HG, SG, ldx, D, ldd, HWd, SWd, HWdd, SWdd, &
+        ldw) bind(c, name='omx_omm_search')
+      import :: c_int, c_ptr, c_int64_t
+      type(c_ptr), value :: ctx, HC, SC, HG, SG, D, HWd, SWd, HWdd, SWdd
+      integer(c_int), value :: prec, dt, n, k
+      integer(c_int64_t), value :: ldx, ldd, ldw
+    end function
     integer(c_int) function omx_omm_calc_G(ctx, prec, dt, n, m, HW, SW, ldw, HC, SC, G, ldc) &
         bind(c, name='omx_omm_calc_G')
       import :: c_int, c_ptr, c_int64_t
