@@ -58,10 +58,10 @@ extern "C" int omx_bsr_param_grad(omx_ctx ctx, omx_bsr Dp, int nparam, const int
     hipEvent_t ev;
     prof_begin(ctx, OMX_K_DOT, &ev);
     hipLaunchKernelGGL(k_param_grad, dim3(nparam), dim3(PG_NT), 0, ctx->stream, nparam, seg, ent, coef, Dp->d_val,
-                       16 * Dp->nnzb, ctx->d_scalars);
+                       16 * Dp->nnzb, ctx->r_scalars);
     prof_end(ctx, OMX_K_DOT, ev);
     OMX_CHECK_HIP(hipGetLastError());
-    int rc = read_scalars(ctx, nparam);
+    int rc = read_scalars(ctx);
     if (rc) return rc;
     for (int p = 0; p < nparam; ++p) grad[p] = ctx->h_scalars[p];
     return OMX_OK;

@@ -193,9 +193,7 @@ void prof_end(omx_ctx ctx, int kclass, hipEvent_t ev_start) {
     if (ctx->prof_pending.size() > 4096) prof_drain(ctx);
 }
 
-int read_scalars(omx_ctx ctx, int n) {
-    OMX_CHECK_HIP(hipMemcpyAsync(ctx->h_scalars, ctx->d_scalars, sizeof(double) * n, hipMemcpyDeviceToHost,
-                                 ctx->stream));
+int read_scalars(omx_ctx ctx) {
     OMX_CHECK_HIP(hipStreamSynchronize(ctx->stream));
     return OMX_OK;
 }
@@ -324,7 +322,8 @@ int omx_init(int device, omx_ctx *out) {
         return OMX_ERR_HIP;
     }
     if (hipMalloc(&ctx->d_scalars, sizeof(double) * kScalarSlots) != hipSuccess ||
-        hipHostMalloc(&ctx->h_scalars, sizeof(double) * kScalarSlots, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc(&ctx->h_scalars, sizeof(double) * kScalarSlots, hipHostMallocMapped) != hipSuccess ||
+        hipHostGetDevicePointer((void **)&ctx->r_scalars, ctx->h_scalars, 0) != hipSuccess) {
         set_error("omx_init: scalar buffer allocation failed");
         return OMX_ERR_NOMEM;
     }
@@ -780,23 +779,23 @@ int omx_get_element(omx_ctx ctx, int dt, const void *C, int64_t ldc, int i, int 
     int64_t off = (int64_t)(i - 1) + (int64_t)(j - 1) * ldc;
     if (dt == OMX_F64)
         hipLaunchKernelGGL(k_get_element<double>, dim3(1), dim3(1), 0, ctx->stream, (const double *)C, off,
-                           ctx->d_scalars);
+                           ctx->r_scalars);
     else if (dt == OMX_F32)
         hipLaunchKernelGGL(k_get_element<float>, dim3(1), dim3(1), 0, ctx->stream, (const float *)C, off,
-                           ctx->d_scalars);
+                           ctx->r_scalars);
     else if (dt == OMX_C128)
         hipLaunchKernelGGL(k_get_element_z<double>, dim3(1), dim3(1), 0, ctx->stream, (const double *)C, off,
-                           ctx->d_scalars);
+                           ctx->r_scalars);
     else if (dt == OMX_C64)
         hipLaunchKernelGGL(k_get_element_z<float>, dim3(1), dim3(1), 0, ctx->stream, (const float *)C, off,
-                           ctx->d_scalars);
+                           ctx->r_scalars);
     else {
         set_error("omx_get_element: unsupported type %d", dt);
         return OMX_ERR_UNSUPPORTED;
     }
     OMX_CHECK_HIP(hipGetLastError());
     const bool z = (dt == OMX_C128 || dt == OMX_C64);
-    int rc = read_scalars(ctx, z ? 2 : 1);
+    int rc = read_scalars(ctx);
     if (rc) return rc;
     out[0] = ctx->h_scalars[0];
     if (z) out[1] = ctx->h_scalars[1];

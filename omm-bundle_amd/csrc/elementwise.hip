@@ -372,9 +372,9 @@ inline int grid_for(int64_t total) { return (int)std::max<int64_t>(1, std::min<i
 // Two-stage sum: partial kernel already launched with `blocks` workgroups and NV values each.
 template <int NV>
 static int finish_reduce(omx_ctx ctx, int blocks, double *partial) {
-    hipLaunchKernelGGL((k_reduce_partials<NV>), dim3(1), dim3(EW_NT), 0, ctx->stream, blocks, partial, ctx->d_scalars);
+    hipLaunchKernelGGL((k_reduce_partials<NV>), dim3(1), dim3(EW_NT), 0, ctx->stream, blocks, partial, ctx->r_scalars);
     OMX_CHECK_HIP(hipGetLastError());
-    return read_scalars(ctx, NV);
+    return read_scalars(ctx);
 }
 
 // ---- scratch of the allocation-free Polak-Ribiere dots (omx_omm_pr_dots_noalloc) ---------------
@@ -571,10 +571,10 @@ int omx_omm_coeff(omx_ctx ctx, int dt, int n, int64_t ldm, const void *HW, const
         set_error("omx_omm_coeff: unsupported element type %d", dt);
         return OMX_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(k_coeff_final, dim3(1), dim3(EW_NT), 0, ctx->stream, (int)blocks, partial, ctx->d_scalars);
+    hipLaunchKernelGGL(k_coeff_final, dim3(1), dim3(EW_NT), 0, ctx->stream, (int)blocks, partial, ctx->r_scalars);
     prof_end(ctx, OMX_K_COEFF, ev);
     OMX_CHECK_HIP(hipGetLastError());
-    rc = read_scalars(ctx, 18);
+    rc = read_scalars(ctx);
     if (rc) return rc;
     for (int q = 0; q < 5; ++q) coeff[q] = ctx->h_scalars[q];
     return OMX_OK;

