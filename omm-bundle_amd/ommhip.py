@@ -91,6 +91,7 @@ SIGNATURES = {
     "omx_set_element": (_i, [_vp, _i, _vp, _i64, _i, _i, _d, _d]),
     "omx_get_element": (_i, [_vp, _i, _vp, _i64, _i, _i, _pd]),
     "omx_omm_coeff": (_i, [_vp, _i, _i, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "omx_omm_search": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _i64]),
     "omx_omm_calc_G": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _i64, _vp, _vp, _vp, _i64]),
     "omx_omm_pr_dots": (_i, [_vp, _i, _i, _i, _vp, _vp, _i64, _vp]),
     "omx_spmm_stencil": (_i, [_vp, _i]),
@@ -543,6 +544,12 @@ def omm_coeff(ctx, HW, SW, HWd, SWd, HWdd, SWdd) -> np.ndarray:
     check(lib().omx_omm_coeff(ctx.h, HW.dt, HW.rows, HW.ld, HW.p, SW.p, HWd.p, SWd.p, HWdd.p, SWdd.p, _ptr(out)),
           "omx_omm_coeff")
     return out
+
+
+def omm_search(ctx, HC, SC, HG, SG, D, HWd, SWd, HWdd, SWdd, prec=PREC_F64):
+    """HWd = HC D^T, SWd = SC D^T and the symmetric HWdd = HG D^T, SWdd = SG D^T (one ld for each group)."""
+    check(lib().omx_omm_search(ctx.h, prec, D.dt, D.rows, D.cols, HC.p, SC.p, HG.p, SG.p, HC.ld, D.p, D.ld, HWd.p, SWd.p,
+                               HWdd.p, SWdd.p, HWd.ld), "omx_omm_search")
 
 
 def omm_calc_G(ctx, HW, SW, HC, SC, G, prec=PREC_F64):
