@@ -327,6 +327,11 @@ int omx_init(int device, omx_ctx *out) {
         set_error("omx_init: scalar buffer allocation failed");
         return OMX_ERR_NOMEM;
     }
+    // (the tickets of the reductions start at 0)
+    if (hipMemset(ctx->d_scalars, 0, sizeof(double) * kScalarSlots) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+        set_error("omx_init: clearing the scalar buffer failed");
+        return OMX_ERR_HIP;
+    }
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->num_cus = prop.multiProcessorCount;
     const int rc = noalloc_setup(device);

@@ -182,7 +182,8 @@ template <typename T>
 __global__ __launch_bounds__(EW_NT) void k_pr_partial(int64_t total_m, int m, const T *__restrict__ G,
                                                       const T *__restrict__ Gp, int64_t ld,
                                                       double *__restrict__ partial, int64_t sG = 0,
-                                                      const int *__restrict__ mask = nullptr) {
+                                                      const int *__restrict__ mask = nullptr,
+                                                      unsigned *ticket = nullptr, double *__restrict__ out = nullptr) {
     typedef El<T> E;
     if (mask && !mask[blockIdx.y]) return;
     // batched use: blockIdx.y selects the system
@@ -206,6 +207,7 @@ __global__ __launch_bounds__(EW_NT) void k_pr_partial(int64_t total_m, int m, co
         }
     }
     block_reduce_store<2>(v, partial + 2 * (int64_t)blockIdx.x);
+    if (ticket && last_workgroup(ticket)) reduce_partials<2>((int)gridDim.x, partial, out);
 }
 
 // ---- fused line-search coefficients (calc_coeff, libOMM/src/omm_ops.F90:156-219) --------------
@@ -226,7 +228,8 @@ __global__ __launch_bounds__(EW_NT) void k_coeff_partial(int n, int64_t ldm, con
                                                          const T *__restrict__ SW, const T *__restrict__ HWd,
                                                          const T *__restrict__ SWd, const T *__restrict__ HWdd,
                                                          const T *__restrict__ SWdd, double *__restrict__ partial,
-                                                         int64_t sW = 0, const int *__restrict__ mask = nullptr) {
+                                                         int64_t sW = 0, const int *__restrict__ mask = nullptr,
+                                                         unsigned *ticket = nullptr, double *__restrict__ out = nullptr) {
     typedef El<T> E;
     if (mask && !mask[blockIdx.y]) return;  // whole workgroup, before the barrier
     // batched use: blockIdx.y selects the system (all six matrices offset by sW elements)
@@ -283,6 +286,7 @@ __global__ __launch_bounds__(EW_NT) void k_coeff_partial(int n, int64_t ldm, con
         v[12] += cdot(hwdd, swdd);
     }
     block_reduce_store<13>(v, partial + 13 * (int64_t)blockIdx.x);
+    if (ticket && last_workgroup(ticket)) coeff_final((int)gridDim.x, partial, out);
 }
 
 __global__ __launch_bounds__(EW_NT) void k_coeff_final(int nblocks, const double *__restrict__ partial,
@@ -368,6 +372,13 @@ inline bool with_type(int dt, F &&f) {
 }
 
 inline int grid_for(int64_t total) { return (int)std::max<int64_t>(1, std::min<int64_t>((total + EW_NT - 1) / EW_NT, 65536)); }
+
+// The ticket of a reduction whose last workgroup adds the parts itself: up to 64 workgroups, where a second
+// launch costs more than their fences (twelve steps of omm() at 54 x 108, which wait for two reductions each:
+// 1.21 -> 1.11 ms); null for more.
+static unsigned *one_launch(omx_ctx ctx, int64_t blocks) {
+    return blocks <= 64 ? (unsigned *)(ctx->d_scalars + (kScalarSlots - 2)) : nullptr;
+}
 
 // Two-stage sum: partial kernel already launched with `blocks` workgroups and NV values each.
 template <int NV>
@@ -556,6 +567,7 @@ int omx_omm_coeff(omx_ctx ctx, int dt, int n, int64_t ldm, const void *HW, const
     int rc = ensure_ws(ctx, sizeof(double) * 13 * blocks);
     if (rc) return rc;
     double *partial = (double *)ctx->ws;
+    unsigned *const ticket = one_launch(ctx, blocks);
     hipEvent_t ev;
     prof_begin(ctx, OMX_K_COEFF, &ev);
     prof_work(ctx, OMX_K_COEFF, (is_complex_dt(dt) ? 4.0 : 1.0) * 26.0 * n * (double)n,
@@ -564,14 +576,15 @@ int omx_omm_coeff(omx_ctx ctx, int dt, int n, int64_t ldm, const void *HW, const
         typedef decltype(tag) T;
         hipLaunchKernelGGL(k_coeff_partial<T>, dim3((unsigned)blocks), dim3(EW_NT), 0, ctx->stream, n, ldm,
                            (const T *)HW, (const T *)SW, (const T *)HWd, (const T *)SWd, (const T *)HWdd,
-                           (const T *)SWdd, partial);
+                           (const T *)SWdd, partial, (int64_t)0, (const int *)nullptr, ticket, ctx->r_scalars);
     });
     if (!ok) {
         prof_end(ctx, OMX_K_COEFF, ev);
         set_error("omx_omm_coeff: unsupported element type %d", dt);
         return OMX_ERR_UNSUPPORTED;
     }
-    hipLaunchKernelGGL(k_coeff_final, dim3(1), dim3(EW_NT), 0, ctx->stream, (int)blocks, partial, ctx->r_scalars);
+    if (!ticket)
+        hipLaunchKernelGGL(k_coeff_final, dim3(1), dim3(EW_NT), 0, ctx->stream, (int)blocks, partial, ctx->r_scalars);
     prof_end(ctx, OMX_K_COEFF, ev);
     OMX_CHECK_HIP(hipGetLastError());
     rc = read_scalars(ctx);
@@ -587,12 +600,13 @@ int omx_omm_pr_dots(omx_ctx ctx, int dt, int n, int m, const void *G, const void
     int rc = ensure_ws(ctx, sizeof(double) * 2 * blocks);
     if (rc) return rc;
     double *partial = (double *)ctx->ws;
+    unsigned *const ticket = one_launch(ctx, blocks);
     hipEvent_t ev;
     prof_begin(ctx, OMX_K_DOT, &ev);
     const bool ok = with_type(dt, [&](auto tag) {
         typedef decltype(tag) T;
         hipLaunchKernelGGL(k_pr_partial<T>, dim3(blocks), dim3(EW_NT), 0, ctx->stream, total, n, (const T *)G,
-                           (const T *)G_p, ld, partial);
+                           (const T *)G_p, ld, partial, (int64_t)0, (const int *)nullptr, ticket, ctx->r_scalars);
     });
     prof_end(ctx, OMX_K_DOT, ev);
     if (!ok) {
@@ -600,7 +614,7 @@ int omx_omm_pr_dots(omx_ctx ctx, int dt, int n, int m, const void *G, const void
         return OMX_ERR_UNSUPPORTED;
     }
     OMX_CHECK_HIP(hipGetLastError());
-    rc = finish_reduce<2>(ctx, blocks, partial);
+    rc = ticket ? read_scalars(ctx) : finish_reduce<2>(ctx, blocks, partial);
     if (rc) return rc;
     out[0] = ctx->h_scalars[0];
     out[1] = ctx->h_scalars[1];

@@ -67,6 +67,22 @@ __device__ inline void reduce_partials(int nblocks, const double *__restrict__ p
     block_reduce_store<NV>(v, out);
 }
 
+// True in every thread of the last of the launch's workgroups to get here, once the others' global stores from
+// before their calls are visible to it; the ticket is back at 0 then.  (A workgroup's values are stored by
+// threads that fence; the release and acquire at device scope cover the L2s of the other XCDs.)
+__device__ inline bool last_workgroup(unsigned *ticket) {
+    __shared__ bool last;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+        if (last) atomicExch(ticket, 0u);
+    }
+    __syncthreads();
+    __threadfence();
+    return last;
+}
+
 // The line-search coefficients and then their thirteen sums (k_coeff_partial's order) into out[0..17]:
 // deterministic per-term sums, then the closed forms, written by thread 0.
 __device__ inline void coeff_final(int nblocks, const double *__restrict__ partial, double *__restrict__ out) {
