@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256) void k_spmm_bsr4(int no, int nb, int nbc, doub
 // halo) instead of 7 times.  The 7 blocks of a column are taken in stored order with the FMA
 // sequence of k_spmm_bsr4, so the results are the same bits.
 // Measured at n = 16384 (FP64): 1.2x the algorithmic HBM bytes (2.6 GB per launch against 4.4 GB
-// for k_spmm_bsr4), but 0.89 ms against 0.83 ms in the same run (FP32: 0.57 against 0.47 ms): one
+// for k_spmm_bsr4), but 0.89 ms against 0.59 ms (FP32: 0.57 against 0.30 ms): one
 // workgroup per CU (128 KB of LDS) and a barrier per plane.  The block values come through the
 // scalar cache (broadcast with v_readlane they cost 2.6x the VALU instructions of k_spmm_bsr4 and
 // the kernel 1.08 ms).  It is therefore opt-in (omx_spmm_stencil).
