@@ -817,7 +817,7 @@ __global__ __launch_bounds__(64 * WPG) void k_spmm_bsr4_z(int no, int nb, int nb
         }
         band = w / jgroups;
         jg = w % jgroups;
-    } else {  // as in k_spmm_bsr4, mode 1
+    } else {  // as in k_spmm_bsr4, mode 1 (spmm_z_grid launches what each map needs)
         const int xcd = w & 7, local = w >> 3, whole = (nbands >> 3) * jgroups, eighth = (jgroups + 7) >> 3;
         if (local < whole) {
             band = (local / jgroups) * 8 + xcd;
@@ -921,13 +921,20 @@ __global__ __launch_bounds__(64 * WPG) void k_spmm_bsr4_z(int no, int nb, int nb
         }
 }
 
+// Workgroups of k_spmm_bsr4_z's map: a batch's systems one after another; a single system (of an operator
+// or of a batch of one) in the eight-XCD map, whose left-over bands end in whole eighths.
+static int64_t spmm_z_grid(int nbands, int jgroups, int nbatch) {
+    if (nbatch > 1) return (int64_t)nbands * jgroups * nbatch;
+    return 8 * ((int64_t)(nbands >> 3) * jgroups + (int64_t)(nbands & 7) * ((jgroups + 7) >> 3));
+}
+
 template <typename R, int VEC>
 static int run_spmm_z(omx_ctx ctx, int no, int nb, double alpha, const R *X, int64_t ldx, omx_bsr A, double beta,
                       R *Y, int64_t ldy) {
     constexpr int ROWS = 64 * VEC, WPG = 4;
     const int nbands = (no + ROWS - 1) / ROWS;
     const int jgroups = (A->nbc + WPG - 1) / WPG;
-    const int64_t total = 8 * ((int64_t)(nbands >> 3) * jgroups + (nbands & 7) * ((jgroups + 7) >> 3));
+    const int64_t total = spmm_z_grid(nbands, jgroups, 1);
     OMX_REQUIRE(total < (1LL << 31), "omx_spmm: grid too large");
     hipEvent_t ev;
     prof_begin(ctx, OMX_K_SPMM, &ev);
@@ -949,7 +956,7 @@ static int run_spmm_z_batched(omx_ctx ctx, int no, int nb, int nbc, const int *c
                               int64_t ldy, int64_t sY, int nbatch, const int *active) {
     constexpr int ROWS = 64 * VEC, WPG = 4;
     const int nbands = (no + ROWS - 1) / ROWS, jgroups = (nbc + WPG - 1) / WPG;
-    const int64_t total = (int64_t)nbands * jgroups * nbatch;
+    const int64_t total = spmm_z_grid(nbands, jgroups, nbatch);
     OMX_REQUIRE(total < (1LL << 31), "batched spmm: grid too large");
     hipLaunchKernelGGL((k_spmm_bsr4_z<R, VEC, WPG, true>), dim3((unsigned)total), dim3(64 * WPG), 0, ctx->stream, no, nb, nbc,
                        1.0, (const R *)X, ldx, colptr, rowidx, val, 0.0, (R *)Y, ldy, nbands, jgroups, 0, 2 * sX, 2 * sY, sV,
