@@ -12,7 +12,8 @@ constexpr int EW_NT = 256;
 // The workgroup's sums of v into out[0..NV-1].  Many values are summed over a wave by recursive halving: at
 // offset 32 a lane keeps half of the (sixteen) values and adds its partner's copies of that half, then at 16,
 // 8 and 4; two more steps add the four lanes that share a value: 17 shuffles instead of 6 per value (the
-// coefficient kernel at 54 x 54 7.5 -> 5.5 us, at 1458 x 1458 33 -> 28).
+// coefficient kernel at 54 x 54 7.5 -> 5.5 us, at 1458 x 1458 33 -> 28).  Few or many, a wave's values are added
+// in one order, lanes 32 apart first, then 16, 8, 4, 2 and 1: a CG trajectory hangs on the last bit of these sums.
 template <int NV>
 __device__ inline void block_reduce_store(double (&v)[NV], double *__restrict__ out) {
     static_assert(NV <= 16, "sixteen values at most");
@@ -33,8 +34,8 @@ __device__ inline void block_reduce_store(double (&v)[NV], double *__restrict__ 
             }
         }
         double s = w[0];
-        s += __shfl_xor(s, 1, 64);
         s += __shfl_xor(s, 2, 64);
+        s += __shfl_xor(s, 1, 64);
         const int q = lane >> 2;  // the value this lane holds
         if ((lane & 3) == 0 && q < NV) red[q][wave] = s;
     } else {
