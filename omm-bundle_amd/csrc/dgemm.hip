@@ -23,7 +23,8 @@
 // loaded this way: 54 x 54 x 108 21 us (now 5.8), 250 x 250 x 500 30 (6.2), 1458 x 1458 x 2916 242 (124;
 // symmetric 252, now 75; pair 512, now 237), 4394 x 4394 x 8788 4.14 ms (2.70; symmetric 2.61, now 1.37), pair
 // of 4394 x 8788 8.64 ms (5.17), 4096 x 4096 x 8192 1.90 (1.91).  Errors against FP64 (relative, Gram): 250 x
-// 500 2.4e-7 (2.1e-7), 1458 x 2916 4.9e-7 (2.1e-7), 4096 x 8192 1.6e-6 (2.5e-7); the carry costs 2 %.
+// 500 2.4e-7 (2.1e-7), 1458 x 2916 4.9e-7 (2.1e-7), as before where K is one chain (see f32_carries); the carry
+// costs 2 %.
 //
 // Tiles.  Three tile sizes with the same K chain per element (K in order, so the results do not depend
 // on the tile): 128x128 (8 waves of 32x64, two stages), 64x64 (4 waves of 32x32, three stages) and 32x32
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
                                                                int64_t ldc0, double beta, R *__restrict__ C,
                                                                int64_t ldc, int sym, int tbase, int nsplit, int sps,
                                                                R *__restrict__ partial,
-                                                               const int *__restrict__ mask, DlBatch bat) {
+                                                               const int *__restrict__ mask, int carry, DlBatch bat) {
     constexpr int BM = CF::BM, BN = CF::BN, NST = CF::NST, NW = CF::WGM * CF::WGN;
     constexpr int DK = DlT<R>::DK, LD = 1024 / sizeof(R);  // K slice, elements of a wave load
     constexpr int INS = DK * (BM + BN) / LD, LPW = INS / NW, U = CF::U;
@@ -266,7 +267,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
                 if (decltype(work)::value) {
                     slice(As, Bs);
                     if constexpr (CARRY) {
-                        if (sl % 4 == 3 || (NPAIR == 2 && sl + 1 == sw)) f32_carry(acc, tot);
+                        if (carry && (sl % 4 == 3 || (NPAIR == 2 && sl + 1 == sw))) f32_carry(acc, tot);
                     }
                 }
             }
@@ -417,7 +418,7 @@ static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int
 // The number of parts with the least time; for a square result that of the full and the symmetric form
 // together, so that both add the same parts.
 int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es) {
-    if (ctx->launch_mask) return 1;
+    if (ctx->launch_mask || (es == 4 && !f32_carries(ctx, m, n))) return 1;
     int best = 1;
     double cost = 0.0;
     for (int s : {1, 2, 3, 4, 5, 6, 8, 12}) {
@@ -451,15 +452,16 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
         whole = tiles - rest;
         sps = nsl / rsplit;
     }
+    const int carry = f32_carries(ctx, m, n);
     auto launch = [&](int grid, int tbase, int parts, int per, R *partial, const int *mask) {
         if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
             hipLaunchKernelGGL((k_dgemm_dl<R, CF, TRA, TRB, NPAIR, CF::BM == 128>), dim3(grid, nbatch), dim3(CF::NT), 0,
                                ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
-                               tbase, parts, per, partial, mask, bat);
+                               tbase, parts, per, partial, mask, carry, bat);
         else
             hipLaunchKernelGGL((k_dgemm_dl<R, CF, TRA, TRB, NPAIR, false>), dim3(grid, nbatch), dim3(CF::NT), 0,
                                ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
-                               tbase, parts, per, partial, mask, bat);
+                               tbase, parts, per, partial, mask, carry, bat);
     };
     if (whole) launch(whole, 0, 1, nsl, nullptr, ctx->launch_mask);
     if (rest) {
@@ -556,7 +558,7 @@ static int run_search(omx_ctx ctx, int n, int k, const R *const A[4], int64_t ld
 #define OMX_DL_FOUR(CF, EX)                                                                                                \
     hipLaunchKernelGGL((k_dgemm_dl<R, CF, false, true, 1, EX>), grid, dim3(CF::NT), 0, ctx->stream, n, n, k, 1.0, A[0], A[0], \
                        lda, B, B, ldb, 0.0, (const R *)nullptr, (int64_t)0, 0.0, C[0], ldc, 2, 0, 1, nsl, (R *)nullptr,     \
-                       ctx->launch_mask, bat)
+                       ctx->launch_mask, (int)f32_carries(ctx, n, n), bat)
     if (tile == 0 && n % 128 == 0 && k % DlT<R>::DK == 0)
         OMX_DL_FOUR(Dl128, true);
     else if (tile == 0)

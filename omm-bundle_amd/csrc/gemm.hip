@@ -276,7 +276,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_gemm(int m, int n, int k, 
                                                  const TS *__restrict__ C0, double beta, TS *__restrict__ C,
                                                  int64_t ldc, int k_per_split, int vec_a, int vec_b, int sym,
                                                  typename Prec<PREC>::acc_t *__restrict__ partial,
-                                                 const int *__restrict__ mask) {
+                                                 const int *__restrict__ mask, int carry) {
     typedef typename Prec<PREC>::lds_t LT;
     typedef typename Prec<PREC>::acc_t AT;
     typedef typename Prec<PREC>::accv AV;
@@ -307,8 +307,9 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_gemm(int m, int n, int k, 
 #pragma unroll
         for (int b = 0; b < CF::FBN; ++b) acc[a][b] = AV{0, 0, 0, 0};
 
-    AV tot[CF::FBM][CF::FBN];  // FP32 only (see f32_carry)
-    if constexpr (PREC == OMX_PREC_F32) {
+    constexpr bool CARRY = PREC == OMX_PREC_F32 && sizeof(TS) == 4;
+    AV tot[CARRY ? CF::FBM : 1][CARRY ? CF::FBN : 1];  // (see f32_carry)
+    if constexpr (CARRY) {
 #pragma unroll
         for (int a = 0; a < CF::FBM; ++a)
 #pragma unroll
@@ -348,8 +349,8 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_gemm(int m, int n, int k, 
             const bool more = (s + 1 < nslices);
             if (more) fetch(kb + (s + 1) * BK);
             mma_slice<PREC, CF>(Ac, Bc, acc, wm, wn, lane);
-            if constexpr (PREC == OMX_PREC_F32) {
-                if (s % 4 == 3 || (NPAIR == 2 && kb + (s + 1) * BK == k)) f32_carry(acc, tot);
+            if constexpr (CARRY) {
+                if (carry && (s % 4 == 3 || (NPAIR == 2 && kb + (s + 1) * BK == k))) f32_carry(acc, tot);
             }
             if (more) {
                 sa.store(An, t);
@@ -359,7 +360,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_gemm(int m, int n, int k, 
         }
     }
 
-    if constexpr (PREC == OMX_PREC_F32) {
+    if constexpr (CARRY) {
 #pragma unroll
         for (int a = 0; a < CF::FBM; ++a)
 #pragma unroll
@@ -452,7 +453,7 @@ static int run_cfg(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1,
                             (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
     hipLaunchKernelGGL((k_gemm<TS, PREC, TRA, TRB, NPAIR, CF>), dim3(grid, 1, splits), dim3(CF::NT), 0, ctx->stream,
                        m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, kps, vec_a, vec_b, (int)sym,
-                       partial, ctx->launch_mask);
+                       partial, ctx->launch_mask, (int)f32_carries(ctx, m, n));
     if (splits > 1) {
         int64_t total = (int64_t)m * n;
         int grid = (int)std::min<int64_t>((total + 255) / 256, 8192);

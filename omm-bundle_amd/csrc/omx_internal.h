@@ -244,6 +244,14 @@ int launch_sgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k
 // products; OMX_ERR_UNSUPPORTED (nothing launched) where single products are faster.
 int launch_search(omx_ctx ctx, int dt, int n, int k, const void *const A[4], int64_t lda, const void *B, int64_t ldb,
                   void *const C[4], int64_t ldc);
+// Whether an m x n FP32 product on FP32 storage may split K and carries its sums (f32_carry): results of fewer
+// than two 128 tiles per CU.  Larger ones are one FP32 chain over K, element by element: with carried sums (1.6e-6
+// -> 2.5e-7 off FP64 at 8192 x 8192 x 16384) the mixed solve at n = 16384 took 670 to 950 low-precision steps
+// and 22.8 to 29.9 s from six starts, against 555 to 665 steps and 18.4 to 22.3 s, and ended higher in energy:
+// its stop and the FP32 recomputation of its state go by the rounding of these products.
+inline bool f32_carries(omx_ctx ctx, int m, int n) {
+    return (int64_t)((m + 127) / 128) * ((n + 127) / 128) < 2 * ctx->num_cus;
+}
 // Parts K is split into for such a product of nsl slices of 128 bytes (es: element size); a function of the
 // shape alone, so that every tile configuration and the symmetric form add in the same order.
 int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es);
