@@ -26,8 +26,8 @@ void clear_error() { g_err[0] = 0; }
 // frees 17 matrices, which for 1458 x 2916 was 4.4 of its 11.1 ms (6.8 without).  A freed block therefore stays mapped
 // until an allocation of up to an eighth less asks for it, it is the oldest of too many (64 blocks, 1/64 of
 // the device's memory), an allocation fails, or a context ends.  Shared by all contexts and threads: a block
-// becomes idle only after a device synchronisation, as with hipFree, so whichever stream takes it next
-// finds no work left on it, and omx_malloc clears it like a new one.
+// becomes idle only after a wait for the whole device, as in hipFree (device_wait), so whichever stream takes it
+// next finds no work left on it, and omx_malloc clears it like a new one.
 class DevPool {
   public:
     // An idle block of at least `bytes` on the current device, or null.
@@ -133,6 +133,16 @@ hipError_t dev_malloc(void **p, size_t bytes) {
 }
 
 bool dev_release() { return dev_pool().release(); }
+
+// Waits for all work on the current device by hipFree's implicit synchronisation, on a block of 256 bytes (1.4 us
+// with its allocation when the device is idle).  hipDeviceSynchronize (0.2 us) would end the graph capture of any
+// stream of the process; this does what freeing a matrix would: it disturbs neither a relaxed capture nor a
+// thread-local one of another thread.
+static hipError_t device_wait() {
+    void *p = nullptr;
+    const hipError_t e = hipMalloc(&p, 256);
+    return e == hipSuccess ? hipFree(p) : e;
+}
 
 int ensure_ws(omx_ctx ctx, size_t bytes) {
     if (ctx->ws_bytes >= bytes) return OMX_OK;
@@ -327,8 +337,10 @@ int omx_init(int device, omx_ctx *out) {
         set_error("omx_init: scalar buffer allocation failed");
         return OMX_ERR_NOMEM;
     }
-    // (the tickets of the reductions start at 0)
-    if (hipMemset(ctx->d_scalars, 0, sizeof(double) * kScalarSlots) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
+    // the tickets of the reductions start at 0 (on the context's stream: a wait for the device would end the
+    // graph captures of other streams)
+    if (hipMemsetAsync(ctx->d_scalars, 0, sizeof(double) * kScalarSlots, ctx->stream) != hipSuccess ||
+        hipStreamSynchronize(ctx->stream) != hipSuccess) {
         set_error("omx_init: clearing the scalar buffer failed");
         return OMX_ERR_HIP;
     }
@@ -417,11 +429,10 @@ int omx_free(omx_ctx ctx, void *dptr) {
     // work of any stream on the block ends here, as in hipFree
     hipError_t e = hipGetDevice(&cur);
     if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
-    if (e == hipSuccess) e = hipDeviceSynchronize();
+    if (e == hipSuccess) e = device_wait();
     if (cur != dev) (void)hipSetDevice(cur);
     try {
-        if (e == hipSuccess) e = dev_pool().put(dptr, bytes, dev);
-        else dev_pool().note(dptr, bytes);
+        e = e == hipSuccess ? dev_pool().put(dptr, bytes, dev) : hipFree(dptr);
     } catch (const std::exception &) {
         e = hipFree(dptr);
     }
