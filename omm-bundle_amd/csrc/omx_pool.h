@@ -12,7 +12,7 @@ namespace omx {
 // hipFree unmaps (0.2 ms for a 34 MB matrix) and hipMalloc maps again (0.06 ms); an omm() call makes and
 // frees 17 matrices, which for 1458 x 2916 was 4.4 of its 11.1 ms (6.8 without).  A freed block therefore stays mapped
 // until an allocation of up to an eighth less asks for it, it is the oldest of too many (64 blocks, 1/64 of
-// the device's memory), an allocation fails, or a context ends.  Shared by all contexts and threads: a block
+// the device's memory: a block beyond that is freed at once), an allocation fails, or a context ends.  Shared by all contexts and threads: a block
 // becomes idle only after a wait for the whole device, as in hipFree (device_wait), so whichever stream takes it
 // next finds no work left on it, and omx_malloc clears it like a new one.
 class DevPool {
@@ -62,12 +62,14 @@ class DevPool {
             std::lock_guard<std::mutex> lock(mu_);
             out.reserve(idle_.size() + 1);
             idle_.reserve(idle_.size() + 1);
-            if (!limit_) {
-                size_t avail = 0, total = 0;
-                limit_ = hipMemGetInfo(&avail, &total) == hipSuccess ? total / 64 + 1 : 1;
+            size_t avail = 0, total = 0;
+            if (!limit_ && hipMemGetInfo(&avail, &total) == hipSuccess) limit_ = total / 64 + 1;
+            if (bytes > limit_) {
+                out.push_back(Block{p, bytes, dev});  // it alone: the smaller idle ones stay
+            } else {
+                idle_.push_back(Block{p, bytes, dev});
+                held_ += bytes;
             }
-            idle_.push_back(Block{p, bytes, dev});
-            held_ += bytes;
             while (held_ > limit_ || idle_.size() > 64) {
                 out.push_back(idle_.front());
                 held_ -= idle_.front().bytes;

@@ -1,6 +1,7 @@
 """The pool of freed device blocks on the host, with the HIP calls it makes replaced by ones that keep count.
 
-What it holds and what it frees when host memory runs out at any point of taking a block in."""
+What it holds and what it frees when host memory runs out at any point of taking a block in, and when a block is
+larger than all it may hold."""
 import os
 import subprocess
 
@@ -80,8 +81,23 @@ static void out_of_host_memory() {
     if (whole < 6) printf("put needs too many allocations\n");
 }
 
+static void large_blocks() {
+    device_bytes = 64 * 1000;  // 1001 bytes are kept
+    DevPool pool;
+    for (int q = 0; q < 3; ++q) put(pool, q, 300);
+    put(pool, 3, 5000);
+    for (int q = 0; q < 3; ++q)
+        if (!idle(pool, q)) printf("block %d gone\n", q);
+    if (idle(pool, 3) || freed != std::set<void *>{at(3)}) printf("the large block stays\n");
+    put(pool, 4, 300);
+    if (idle(pool, 0) || !idle(pool, 1) || !idle(pool, 2) || !idle(pool, 4)) printf("the oldest did not go\n");
+    put(pool, 5, 1001);
+    if (!idle(pool, 5) || idle(pool, 1) || idle(pool, 2) || idle(pool, 4)) printf("a block of the whole room\n");
+}
+
 int main(int, char **argv) {
     if (argv[1][0] == 'm') out_of_host_memory();
+    if (argv[1][0] == 'l') large_blocks();
     printf("done\n");
 }
 """
@@ -103,3 +119,7 @@ def _run(program, what):
 
 def test_host_memory_runs_out(program):
     _run(program, "memory")
+
+
+def test_large_block_leaves_the_others(program):
+    _run(program, "large")
