@@ -369,7 +369,7 @@ static int tiles_of(int m, int n, int b, bool sym) {
 // that are multiples of 128; elsewhere the symmetric form adds exactly as the full product does.
 static int dl_tail_parts(omx_ctx ctx, int m, int tiles, bool sym, int nsl) {
     const int slots = 2 * ctx->num_cus, rest = tiles % slots;
-    if (!sym || m % 128 || ctx->launch_mask || tiles < slots || !rest) return 1;
+    if (!sym || m % 128 || ctx->launch_mask || ctx->one_part || tiles < slots || !rest) return 1;
     int parts = std::max(1, std::min(16, slots / rest));
     while (parts > 1 && nsl % parts) --parts;
     return parts;
@@ -418,7 +418,7 @@ static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int
 // The number of parts with the least time; for a square result that of the full and the symmetric form
 // together, so that both add the same parts.
 int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es) {
-    if (ctx->launch_mask || (es == 4 && !f32_carries(ctx, m, n))) return 1;
+    if (ctx->launch_mask || ctx->one_part || (es == 4 && !f32_carries(ctx, m, n))) return 1;
     int best = 1;
     double cost = 0.0;
     for (int s : {1, 2, 3, 4, 5, 6, 8, 12}) {
@@ -527,23 +527,33 @@ static int launch_dl(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, i
 // The line-search products of one CG step in one launch (see DlBatch), where the model finds that faster than
 // one by one: small results leave most of the chip idle each, larger ones are split along K to fill it
 // (twelve steps of omm() at 54 x 108 1.65 -> 1.33 ms, four at 1458 x 2916 6.48 -> 6.26 ms).
+static int search_tile(omx_ctx ctx, int n, int nsl, double &time) {
+    int tile = 0;
+    for (int q = 0; q < 3; ++q) {
+        const double t = dl_time(ctx, q, 2LL * (tiles_of(n, n, kDlEdge[q], false) + tiles_of(n, n, kDlEdge[q], true)), nsl);
+        if (!q || t < time) {
+            tile = q;
+            time = t;
+        }
+    }
+    return tile;
+}
+bool search_in_one(omx_ctx ctx, int dt, int n, int k, int64_t lda, int64_t ldb) {
+    if (n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20)) return false;
+    const int es = dt == OMX_F64 ? 8 : 4, dk = 128 / es, nsl = (k + dk - 1) / dk, splits = dgemm_k_splits(ctx, n, n, nsl, es);
+    double four = 0.0, full = 0.0, lower = 0.0;
+    search_tile(ctx, n, nsl, four);
+    dl_tile(ctx, false, n, n, nsl, splits, 1, es, &full);
+    dl_tile(ctx, true, n, n, nsl, splits, 1, es, &lower);
+    return four < 2.0 * (full + lower);
+}
+
 template <typename R>
 static int run_search(omx_ctx ctx, int n, int k, const R *const A[4], int64_t lda, const R *B, int64_t ldb, R *const C[4],
                       int64_t ldc) {
-    if (n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20)) return OMX_ERR_UNSUPPORTED;
-    const int nsl = (k + DlT<R>::DK - 1) / DlT<R>::DK, splits = dgemm_k_splits(ctx, n, n, nsl, sizeof(R));
-    int tile = 0;
-    double best = 0.0, full = 0.0, lower = 0.0;
-    for (int q = 0; q < 3; ++q) {
-        const double t = dl_time(ctx, q, 2LL * (tiles_of(n, n, kDlEdge[q], false) + tiles_of(n, n, kDlEdge[q], true)), nsl);
-        if (!q || t < best) {
-            tile = q;
-            best = t;
-        }
-    }
-    dl_tile(ctx, false, n, n, nsl, splits, 1, sizeof(R), &full);
-    dl_tile(ctx, true, n, n, nsl, splits, 1, sizeof(R), &lower);
-    if (best >= 2.0 * (full + lower)) return OMX_ERR_UNSUPPORTED;
+    const int nsl = (k + DlT<R>::DK - 1) / DlT<R>::DK;
+    double time = 0.0;
+    const int tile = search_tile(ctx, n, nsl, time);
     DlBatch bat;
     bat.four = 1;
     for (int q = 0; q < 4; ++q) {

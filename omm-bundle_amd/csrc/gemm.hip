@@ -1204,16 +1204,17 @@ extern "C" int omx_omm_search(omx_ctx ctx, int prec, int dt, int n, int k, const
     OMX_REQUIRE(HC && SC && HG && SG && D && HWd && SWd && HWdd && SWdd, "omx_omm_search: null operand");
     const void *const A[4] = {HC, SC, HG, SG};
     void *const C[4] = {HWd, SWd, HWdd, SWdd};
-    if (prec == (dt == OMX_F64 ? OMX_PREC_F64 : OMX_PREC_F32) && (ctx->gemm_cfg < 0 || ctx->gemm_cfg == 7) && !ctx->autotune) {
-        const int rc = launch_search(ctx, dt, n, k, A, ldx, D, ldd, C, ldw);
-        if (rc != OMX_ERR_UNSUPPORTED) return rc;
-    }
-    for (int q = 0; q < 4; ++q) {
-        const int rc = q < 2 ? omx_gemm(ctx, prec, dt, 'n', 't', n, n, k, 1.0, A[q], ldx, D, ldd, 0.0, C[q], ldw)
-                             : omx_gemm_sym(ctx, prec, dt, n, k, 1.0, A[q], ldx, D, ldd, C[q], ldw);
-        if (rc) return rc;
-    }
-    return OMX_OK;
+    // The tuner has no say in it, and a forced tile gets the one launch's order of adding, so that neither
+    // changes a bit.
+    const bool one = prec == (dt == OMX_F64 ? OMX_PREC_F64 : OMX_PREC_F32) && search_in_one(ctx, dt, n, k, ldx, ldd);
+    if (one && (ctx->gemm_cfg < 0 || ctx->gemm_cfg == 7)) return launch_search(ctx, dt, n, k, A, ldx, D, ldd, C, ldw);
+    int rc = OMX_OK;
+    ctx->one_part = one;
+    for (int q = 0; q < 4 && !rc; ++q)
+        rc = q < 2 ? omx_gemm(ctx, prec, dt, 'n', 't', n, n, k, 1.0, A[q], ldx, D, ldd, 0.0, C[q], ldw)
+                   : omx_gemm_sym(ctx, prec, dt, n, k, 1.0, A[q], ldx, D, ldd, C[q], ldw);
+    ctx->one_part = false;
+    return rc;
 }
 
 extern "C" int omx_gemm_sym(omx_ctx ctx, int prec, int dt, int n, int k, double alpha, const void *A, int64_t lda,

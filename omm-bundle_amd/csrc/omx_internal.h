@@ -79,6 +79,7 @@ struct omx_ctx_s {
     // Set around a product known to be symmetric: 1 = only the lower triangle is wanted, 2 = both
     // triangles.  A kernel that writes both sets 3 (no mirror pass needed).
     int gemm_sym = 0;
+    bool one_part = false;  // set around products whose K is not to be split
     omx_spmm_shape_s spmm_shape;  // forced SpMM launch shape (when spmm_forced)
     bool spmm_forced = false;
     bool spmm_stencil = false;  // lattice operators use the 2.5-D stencil SpMM (omx_spmm_stencil)
@@ -241,7 +242,9 @@ int launch_sgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k
                  const float *A2, int64_t lda, const float *B1, const float *B2, int64_t ldb, double beta0, const float *C0,
                  double beta, float *C, int64_t ldc);
 // C_q := A_q B^T (n x n, k columns; q = 2, 3 symmetric) in one launch, dt OMX_F64 or OMX_F32 for operands and
-// products; OMX_ERR_UNSUPPORTED (nothing launched) where single products are faster.
+// products, where search_in_one finds that faster than single products.  K is not split then: the bits are
+// those of single products with ctx->one_part.
+bool search_in_one(omx_ctx ctx, int dt, int n, int k, int64_t lda, int64_t ldb);
 int launch_search(omx_ctx ctx, int dt, int n, int k, const void *const A[4], int64_t lda, const void *B, int64_t ldb,
                   void *const C[4], int64_t ldc);
 // Whether an m x n FP32 product on FP32 storage may split K and carries its sums (f32_carry): results of fewer
