@@ -232,7 +232,8 @@ int omx_bsr_set_walk_groups(omx_bsr A, const int *order, int group);
  * 32x32 tiles by shape, the default there).  A configuration that does not apply to
  * a product falls back to 0.  Used by the tile autotuner; results do not depend on it, except that
  * 7 splits K for the last tiles of symmetric FP64 products of whole 128 x 128 tiles that fill the
- * chip (rounding of those tiles). */
+ * chip, and makes gradients whose order the K slice (FP64 16, FP32 32) does not divide in one
+ * product instead of three passes (rounding, both). */
 int omx_gemm_set_tile(omx_ctx ctx, int cfg);
 /* Autotuner (project-written; no counterpart in the reference): with enable != 0, the first
  * product or SpMM of each shape on this context times every applicable tile configuration / SpMM

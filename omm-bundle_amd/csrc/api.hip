@@ -28,9 +28,10 @@ static DevPool &dev_pool() {
 
 hipError_t dev_malloc(void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess && dev_pool().release()) {
-        (void)hipGetLastError();
-        e = hipMalloc(p, bytes);
+    if (e != hipSuccess && dev_pool().release()) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // the caller's to report: not the next launch's
+        *p = nullptr;
     }
     return e;
 }

@@ -452,6 +452,16 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
         whole = tiles - rest;
         sps = nsl / rsplit;
     }
+    if (rest) {
+        const int rc = ensure_ws(ctx, sizeof(R) * (size_t)rest * rsplit * CF::BM * CF::BN);
+        if (rc == OMX_ERR_NOMEM) {  // no room for the parts: K whole, which needs none
+            clear_error();
+            whole = tiles;
+            rest = 0;
+        } else if (rc) {
+            return rc;
+        }
+    }
     const int carry = f32_carries(ctx, m, n);
     auto launch = [&](int grid, int tbase, int parts, int per, R *partial, const int *mask) {
         if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
@@ -465,8 +475,6 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
     };
     if (whole) launch(whole, 0, 1, nsl, nullptr, ctx->launch_mask);
     if (rest) {
-        int rc = ensure_ws(ctx, sizeof(R) * (size_t)rest * rsplit * CF::BM * CF::BN);
-        if (rc) return rc;
         launch(rest * rsplit, whole, rsplit, sps, (R *)ctx->ws, nullptr);
         hipLaunchKernelGGL((k_dl_split_reduce<R, CF::BM, CF::BN>), dim3(rest, CF::BM * CF::BN / 1024), dim3(256), 0,
                            ctx->stream, m, n, sym, whole, rsplit, (const R *)ctx->ws, alpha, beta0, C0,

@@ -972,6 +972,10 @@ static int bgemm_panels(omx_ctx ctx, int m, int n, int k, int nterm, const BgTer
     splits = ((int)(K / BK) + kps - 1) / kps;
     const size_t panels = (bytes_a + 255) / 256 * 256 + (bytes_b + 255) / 256 * 256;
     int rc = ensure_ws(ctx, panels + (splits > 1 ? sizeof(float) * (size_t)splits * m * n : 0));
+    if (rc == OMX_ERR_NOMEM && nsplit == 1) {  // no room for the panels: the staged kernel
+        clear_error();
+        return OMX_ERR_UNSUPPORTED;
+    }
     if (rc) return rc;
     float *partial = splits > 1 ? (float *)((char *)ctx->ws + panels) : nullptr;
     __bf16 *At = (__bf16 *)ctx->ws;

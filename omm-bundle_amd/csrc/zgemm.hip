@@ -657,13 +657,20 @@ static int run_zgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const vo
     // batched launches never split K: no workspace, so the launch can be graph-captured
     const bool lower = sym && !bat.nsys;  // a grid of lower-triangle tiles
     zl_shape(ctx, m, n, nsl, lower, bat.nsys ? (nbatch + bat.herm) / 2 : nbatch, allow_split && nbatch == 1, tile, splits);
-    const int sps = (nsl + splits - 1) / splits;
+    int sps = (nsl + splits - 1) / splits;
     splits = (nsl + sps - 1) / sps;
     C2 *partial = nullptr;
     if (splits > 1) {
-        int rc = ensure_ws(ctx, sizeof(C2) * (size_t)splits * m * n);
-        if (rc) return rc;
-        partial = (C2 *)ctx->ws;
+        const int rc = ensure_ws(ctx, sizeof(C2) * (size_t)splits * m * n);
+        if (rc == OMX_ERR_NOMEM) {  // no room for the parts: K whole, which needs none
+            clear_error();
+            splits = 1;
+            sps = nsl;
+        } else if (rc) {
+            return rc;
+        } else {
+            partial = (C2 *)ctx->ws;
+        }
     }
     const int64_t tiles = zl_tiles(m, n, tile, lower);
     OMX_REQUIRE(tiles < (1LL << 31), "complex product: grid too large");
