@@ -115,7 +115,8 @@ struct DlBatch {
 // EXACT: m, n are multiples of the tile and k of the slice, so nothing needs the descriptors' end, a
 // cleared tail or guarded stores; the 128x128 tile is faster without them (8192 x 8192 x 16384 Gram 29.8
 // against 29.9 ms, gradient 60.4 against 61.6 ms).
-template <typename R, class CF, bool TRA, bool TRB, int NPAIR, bool EXACT>
+// CY: the sums are carried where `carry` says so (FP32 products, and the FP64 ones of a factorisation).
+template <typename R, class CF, bool TRA, bool TRB, int NPAIR, bool EXACT, bool CY>
 __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int k, double alpha,
                                                                const R *__restrict__ A1,
                                                                const R *__restrict__ A2, int64_t lda,
@@ -167,9 +168,8 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
     for (int a = 0; a < CF::FBM; ++a)
 #pragma unroll
         for (int b = 0; b < CF::FBN; ++b) acc[a][b] = typename DlT<R>::acc{0, 0, 0, 0};
-    constexpr bool CARRY = sizeof(R) == 4;
-    typename DlT<R>::acc tot[CARRY ? CF::FBM : 1][CARRY ? CF::FBN : 1];  // FP32 (see f32_carry)
-    if constexpr (CARRY) {
+    typename DlT<R>::acc tot[CY ? CF::FBM : 1][CY ? CF::FBN : 1];  // (see carry_sums)
+    if constexpr (CY) {
 #pragma unroll
         for (int a = 0; a < CF::FBM; ++a)
 #pragma unroll
@@ -266,8 +266,8 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
                 }
                 if (decltype(work)::value) {
                     slice(As, Bs);
-                    if constexpr (CARRY) {
-                        if (carry && (sl % 4 == 3 || (NPAIR == 2 && sl + 1 == sw))) f32_carry(acc, tot);
+                    if constexpr (CY) {
+                        if (carry && (sl % 4 == 3 || (NPAIR == 2 && sl + 1 == sw))) carry_sums(acc, tot);
                     }
                 }
             }
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
         return;
     }
     march(std::true_type{});
-    if constexpr (CARRY) {
+    if constexpr (CY) {
 #pragma unroll
         for (int a = 0; a < CF::FBM; ++a)
 #pragma unroll
@@ -404,9 +404,10 @@ static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int s
 static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, int es, double *cost = nullptr) {
     int best = 0;
     double c = 0.0;
-    for (int q = 0; q < 3; ++q) {
+    const int first = ctx->carry64 && es == 8;  // no 128 tiles: no registers for the carried sums
+    for (int q = first; q < 3; ++q) {
         const double t = dl_cost(ctx, q, sym, m, n, nsl, splits, nbatch, es);
-        if (!q || t < c) {
+        if (q == first || t < c) {
             best = q;
             c = t;
         }
@@ -462,16 +463,26 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
             return rc;
         }
     }
-    const int carry = f32_carries(ctx, m, n);
+    constexpr bool single = sizeof(R) == 4;
     auto launch = [&](int grid, int tbase, int parts, int per, R *partial, const int *mask) {
-        if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
-            hipLaunchKernelGGL((k_dgemm_dl<R, CF, TRA, TRB, NPAIR, CF::BM == 128>), dim3(grid, nbatch), dim3(CF::NT), 0,
-                               ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
-                               tbase, parts, per, partial, mask, carry, bat);
-        else
-            hipLaunchKernelGGL((k_dgemm_dl<R, CF, TRA, TRB, NPAIR, false>), dim3(grid, nbatch), dim3(CF::NT), 0,
-                               ctx->stream, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym,
-                               tbase, parts, per, partial, mask, carry, bat);
+#define OMX_DL_LAUNCH(EX, CY, CARRY)                                                                                       \
+    hipLaunchKernelGGL((k_dgemm_dl<R, CF, TRA, TRB, NPAIR, EX, CY>), dim3(grid, nbatch), dim3(CF::NT), 0, ctx->stream, m, n, k, \
+                       alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym, tbase, parts, per, partial, mask, \
+                       CARRY, bat)
+        if constexpr (single) {
+            const int carry = f32_carries(ctx, m, n);
+            if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
+                OMX_DL_LAUNCH(CF::BM == 128, true, carry);
+            else
+                OMX_DL_LAUNCH(false, true, carry);
+        } else if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0) {
+            OMX_DL_LAUNCH(CF::BM == 128, false, 0);
+        } else if (CF::BM != 128 && NPAIR == 1 && ctx->carry64) {
+            OMX_DL_LAUNCH(false, CF::BM != 128 && NPAIR == 1, 1);
+        } else {
+            OMX_DL_LAUNCH(false, false, 0);
+        }
+#undef OMX_DL_LAUNCH
     };
     if (whole) launch(whole, 0, 1, nsl, nullptr, ctx->launch_mask);
     if (rest) {
@@ -574,7 +585,7 @@ static int run_search(omx_ctx ctx, int n, int k, const R *const A[4], int64_t ld
               sizeof(R) * (5.0 * n * k + 4.0 * (double)n * n));
     const dim3 grid(tiles_of(n, n, kDlEdge[tile], false), 4);
 #define OMX_DL_FOUR(CF, EX)                                                                                                \
-    hipLaunchKernelGGL((k_dgemm_dl<R, CF, false, true, 1, EX>), grid, dim3(CF::NT), 0, ctx->stream, n, n, k, 1.0, A[0], A[0], \
+    hipLaunchKernelGGL((k_dgemm_dl<R, CF, false, true, 1, EX, sizeof(R) == 4>), grid, dim3(CF::NT), 0, ctx->stream, n, n, k, 1.0, A[0], A[0], \
                        lda, B, B, ldb, 0.0, (const R *)nullptr, (int64_t)0, 0.0, C[0], ldc, 2, 0, 1, nsl, (R *)nullptr,     \
                        ctx->launch_mask, (int)f32_carries(ctx, n, n), bat)
     if (tile == 0 && n % 128 == 0 && k % DlT<R>::DK == 0)

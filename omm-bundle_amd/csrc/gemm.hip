@@ -308,7 +308,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_gemm(int m, int n, int k, 
         for (int b = 0; b < CF::FBN; ++b) acc[a][b] = AV{0, 0, 0, 0};
 
     constexpr bool CARRY = PREC == OMX_PREC_F32 && sizeof(TS) == 4;
-    AV tot[CARRY ? CF::FBM : 1][CARRY ? CF::FBN : 1];  // (see f32_carry)
+    AV tot[CARRY ? CF::FBM : 1][CARRY ? CF::FBN : 1];  // (see carry_sums)
     if constexpr (CARRY) {
 #pragma unroll
         for (int a = 0; a < CF::FBM; ++a)
@@ -350,7 +350,7 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_gemm(int m, int n, int k, 
             if (more) fetch(kb + (s + 1) * BK);
             mma_slice<PREC, CF>(Ac, Bc, acc, wm, wn, lane);
             if constexpr (CARRY) {
-                if (carry && (s % 4 == 3 || (NPAIR == 2 && kb + (s + 1) * BK == k))) f32_carry(acc, tot);
+                if (carry && (s % 4 == 3 || (NPAIR == 2 && kb + (s + 1) * BK == k))) carry_sums(acc, tot);
             }
             if (more) {
                 sa.store(An, t);

@@ -80,6 +80,7 @@ struct omx_ctx_s {
     // triangles.  A kernel that writes both sets 3 (no mirror pass needed).
     int gemm_sym = 0;
     bool one_part = false;  // set around products whose K is not to be split
+    bool carry64 = false;   // set around FP64 products that carry their sums (carry_sums)
     omx_spmm_shape_s spmm_shape;  // forced SpMM launch shape (when spmm_forced)
     bool spmm_forced = false;
     bool spmm_stencil = false;  // lattice operators use the 2.5-D stencil SpMM (omx_spmm_stencil)
@@ -247,7 +248,7 @@ int launch_sgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k
 bool search_in_one(omx_ctx ctx, int dt, int n, int k, int64_t lda, int64_t ldb);
 int launch_search(omx_ctx ctx, int dt, int n, int k, const void *const A[4], int64_t lda, const void *B, int64_t ldb,
                   void *const C[4], int64_t ldc);
-// Whether an m x n FP32 product on FP32 storage may split K and carries its sums (f32_carry): results of fewer
+// Whether an m x n FP32 product on FP32 storage may split K and carries its sums (carry_sums): results of fewer
 // than two 128 tiles per CU.  Larger ones are one FP32 chain over K, element by element: with carried sums (1.6e-6
 // -> 2.5e-7 off FP64 at 8192 x 8192 x 16384) the mixed solve at n = 16384 took 670 to 950 low-precision steps
 // and 22.8 to 29.9 s from six starts, against 555 to 665 steps and 18.4 to 22.3 s, and ended higher in energy:

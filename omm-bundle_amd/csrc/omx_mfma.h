@@ -35,11 +35,12 @@ __device__ inline void wg_barrier() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// FP32 products whose K is split (f32_carries) accumulate 128 values of K at a time and add these sums up apart
-// (restarting at a pair's second product too): one FP32 chain over all of K would be three times less accurate
-// at 700 x 700 x 1500 than the parts of about 160 that such a product used to be split into.
+// Carried sums: 512 bytes of a k-contiguous row's values (128 FP32, 64 FP64) are accumulated at a time and these sums
+// added up apart (restarting at a pair's second product too).  FP32 products whose K is split (f32_carries) do: one
+// FP32 chain over all of K would be three times less accurate at 700 x 700 x 1500 than the parts of about 160 that
+// such a product used to be split into.  So do the FP64 products of the factorisations (dense_la.hip).
 template <typename AV, int FM, int FN>
-__device__ inline void f32_carry(AV (&acc)[FM][FN], AV (&tot)[FM][FN]) {
+__device__ inline void carry_sums(AV (&acc)[FM][FN], AV (&tot)[FM][FN]) {
 #pragma unroll
     for (int a = 0; a < FM; ++a)
 #pragma unroll

@@ -355,7 +355,7 @@ struct ZlCfg {
 typedef ZlCfg<64, 2, 1> Zl64;
 typedef ZlCfg<32, 2, 4> Zl32;
 
-// CARRY (complex64, single products): sums of 32 values of K are added up apart (see f32_carry), which keeps
+// CARRY (complex64, single products): sums of 32 values of K are added up apart (see carry_sums), which keeps
 // the error at or below that of the many parts K used to be split into (Gram 54 x 108: 1.6e-7 -> 1.4e-7, 2000 x
 // 4000: 1.6e-6 -> 2.5e-7; with one chain 900 x 2916 1.3e-6) for 3 %.  Batched products keep one chain: their
 // roundings are part of a k-point solve's trajectory.
@@ -524,8 +524,8 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double
                     slice(As, Bs);
                     if constexpr (CARRY) {
                         if (sl % 2 == 1 || (NPAIR == 2 && sl + 1 == sw)) {
-                            f32_carry(are, tre);
-                            f32_carry(aim, tim);
+                            carry_sums(are, tre);
+                            carry_sums(aim, tim);
                         }
                     }
                 }
