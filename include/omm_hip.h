@@ -229,7 +229,8 @@ int omx_bsr_set_walk_groups(omx_bsr A, const int *order, int group);
  * 128x128 with 8 waves of 64x32 (FP64 products); 4 = 256x256 with 8 waves (BF16 products on
  * FP32 storage); 7 = the operands loaded straight into LDS (every FP64 product on FP64 storage
  * and every FP32 product on FP32 storage with leading dimensions up to 2^20, in 128x128, 64x64 or
- * 32x32 tiles by shape, the default there).  A configuration that does not apply to
+ * 32x32 tiles by shape, the default there; taken whatever is forced for FP64 results of fewer than
+ * two 128x128 tiles per CU, which carry their sums).  A configuration that does not apply to
  * a product falls back to 0.  Used by the tile autotuner; results do not depend on it, except that
  * 7 splits K for the last tiles of symmetric FP64 products of whole 128 x 128 tiles that fill the
  * chip, and makes gradients whose order the K slice (FP64 16, FP32 32) does not divide in one

@@ -23,7 +23,7 @@
 // loaded this way: 54 x 54 x 108 21 us (now 5.8), 250 x 250 x 500 30 (6.2), 1458 x 1458 x 2916 242 (124;
 // symmetric 252, now 75; pair 512, now 237), 4394 x 4394 x 8788 4.14 ms (2.70; symmetric 2.61, now 1.37), pair
 // of 4394 x 8788 8.64 ms (5.17), 4096 x 4096 x 8192 1.90 (1.91).  Errors against FP64 (relative, Gram): 250 x
-// 500 2.4e-7 (2.1e-7), 1458 x 2916 4.9e-7 (2.1e-7), as before where K is one chain (see f32_carries); the carry
+// 500 2.4e-7 (2.1e-7), 1458 x 2916 4.9e-7 (2.1e-7), as before where K is one chain (see carries); the carry
 // costs 2 %.
 //
 // Tiles.  Three tile sizes with the same K chain per element (K in order, so the results do not depend
@@ -115,7 +115,8 @@ struct DlBatch {
 // EXACT: m, n are multiples of the tile and k of the slice, so nothing needs the descriptors' end, a
 // cleared tail or guarded stores; the 128x128 tile is faster without them (8192 x 8192 x 16384 Gram 29.8
 // against 29.9 ms, gradient 60.4 against 61.6 ms).
-// CY: the sums are carried where `carry` says so (FP32 products, and the FP64 ones of a factorisation).
+// CY: the sums are carried every `carry` slices, not at all for 0 (FP32 products, and the FP64 ones of carries64, which take the 64 and
+// 32 tiles: the 128 tile has no registers for a second set of sums).
 template <typename R, class CF, bool TRA, bool TRB, int NPAIR, bool EXACT, bool CY>
 __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int k, double alpha,
                                                                const R *__restrict__ A1,
@@ -267,7 +268,9 @@ __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int
                 if (decltype(work)::value) {
                     slice(As, Bs);
                     if constexpr (CY) {
-                        if (carry && (sl % 4 == 3 || (NPAIR == 2 && sl + 1 == sw))) carry_sums(acc, tot);
+                        // (a period of 4 slices or more ends with a stage of 4)
+                        if (carry && ((u == U - 1 && (sl & (carry - 1)) == carry - 1) || (NPAIR == 2 && sl + 1 == sw)))
+                            carry_sums(acc, tot);
                     }
                 }
             }
@@ -404,7 +407,7 @@ static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int s
 static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, int es, double *cost = nullptr) {
     int best = 0;
     double c = 0.0;
-    const int first = ctx->carry64 && es == 8;  // no 128 tiles: no registers for the carried sums
+    const int first = es == 8 && carries64(ctx, m, n);
     for (int q = first; q < 3; ++q) {
         const double t = dl_cost(ctx, q, sym, m, n, nsl, splits, nbatch, es);
         if (q == first || t < c) {
@@ -419,7 +422,7 @@ static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int
 // The number of parts with the least time; for a square result that of the full and the symmetric form
 // together, so that both add the same parts.
 int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es) {
-    if (ctx->launch_mask || ctx->one_part || (es == 4 && !f32_carries(ctx, m, n))) return 1;
+    if (ctx->launch_mask || ctx->one_part || (es == 4 && !carries(ctx, m, n))) return 1;
     int best = 1;
     double cost = 0.0;
     for (int s : {1, 2, 3, 4, 5, 6, 8, 12}) {
@@ -433,6 +436,14 @@ int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es) {
         }
     }
     return best;
+}
+
+// Carry period of an FP64 product: by the parts that 128 tiles were split into, two workgroups per CU, 64 values at
+// the least.
+static int dl_period(omx_ctx ctx, int m, int n, int nsl) {
+    if (ctx->carry64) return 4;
+    const int64_t tiles = tiles_of(m, n, 128, false);
+    return carry_period(nsl, std::min<int64_t>((2 * ctx->num_cus + tiles - 1) / tiles, nsl / 4));
 }
 
 template <typename R, class CF, bool TRA, bool TRB, int NPAIR>
@@ -470,15 +481,15 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
                        alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym, tbase, parts, per, partial, mask, \
                        CARRY, bat)
         if constexpr (single) {
-            const int carry = f32_carries(ctx, m, n);
+            const int carry = carries(ctx, m, n) ? 4 : 0;
             if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
                 OMX_DL_LAUNCH(CF::BM == 128, true, carry);
             else
                 OMX_DL_LAUNCH(false, true, carry);
         } else if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0) {
             OMX_DL_LAUNCH(CF::BM == 128, false, 0);
-        } else if (CF::BM != 128 && NPAIR == 1 && ctx->carry64) {
-            OMX_DL_LAUNCH(false, CF::BM != 128 && NPAIR == 1, 1);
+        } else if (CF::BM != 128 && carries64(ctx, m, n)) {
+            OMX_DL_LAUNCH(false, CF::BM != 128, dl_period(ctx, m, n, nsl));
         } else {
             OMX_DL_LAUNCH(false, false, 0);
         }
@@ -546,11 +557,12 @@ static int launch_dl(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, i
 // The line-search products of one CG step in one launch (see DlBatch), where the model finds that faster than
 // one by one: small results leave most of the chip idle each, larger ones are split along K to fill it
 // (twelve steps of omm() at 54 x 108 1.65 -> 1.33 ms, four at 1458 x 2916 6.48 -> 6.26 ms).
-static int search_tile(omx_ctx ctx, int n, int nsl, double &time) {
-    int tile = 0;
-    for (int q = 0; q < 3; ++q) {
+static int search_tile(omx_ctx ctx, int n, int nsl, int es, double &time) {
+    const int first = es == 8 && carries64(ctx, n, n);
+    int tile = first;
+    for (int q = first; q < 3; ++q) {
         const double t = dl_time(ctx, q, 2LL * (tiles_of(n, n, kDlEdge[q], false) + tiles_of(n, n, kDlEdge[q], true)), nsl);
-        if (!q || t < time) {
+        if (q == first || t < time) {
             tile = q;
             time = t;
         }
@@ -561,7 +573,7 @@ bool search_in_one(omx_ctx ctx, int dt, int n, int k, int64_t lda, int64_t ldb) 
     if (n <= 0 || k <= 0 || lda > (1 << 20) || ldb > (1 << 20)) return false;
     const int es = dt == OMX_F64 ? 8 : 4, dk = 128 / es, nsl = (k + dk - 1) / dk, splits = dgemm_k_splits(ctx, n, n, nsl, es);
     double four = 0.0, full = 0.0, lower = 0.0;
-    search_tile(ctx, n, nsl, four);
+    search_tile(ctx, n, nsl, es, four);
     dl_tile(ctx, false, n, n, nsl, splits, 1, es, &full);
     dl_tile(ctx, true, n, n, nsl, splits, 1, es, &lower);
     return four < 2.0 * (full + lower);
@@ -572,7 +584,7 @@ static int run_search(omx_ctx ctx, int n, int k, const R *const A[4], int64_t ld
                       int64_t ldc) {
     const int nsl = (k + DlT<R>::DK - 1) / DlT<R>::DK;
     double time = 0.0;
-    const int tile = search_tile(ctx, n, nsl, time);
+    const int tile = search_tile(ctx, n, nsl, sizeof(R), time);
     DlBatch bat;
     bat.four = 1;
     for (int q = 0; q < 4; ++q) {
@@ -584,18 +596,24 @@ static int run_search(omx_ctx ctx, int n, int k, const R *const A[4], int64_t ld
     prof_work(ctx, OMX_K_GEMM, 4.0 * ((double)n * n + sym_area(n, kDlEdge[tile])) * k,
               sizeof(R) * (5.0 * n * k + 4.0 * (double)n * n));
     const dim3 grid(tiles_of(n, n, kDlEdge[tile], false), 4);
-#define OMX_DL_FOUR(CF, EX)                                                                                                \
-    hipLaunchKernelGGL((k_dgemm_dl<R, CF, false, true, 1, EX, sizeof(R) == 4>), grid, dim3(CF::NT), 0, ctx->stream, n, n, k, 1.0, A[0], A[0], \
-                       lda, B, B, ldb, 0.0, (const R *)nullptr, (int64_t)0, 0.0, C[0], ldc, 2, 0, 1, nsl, (R *)nullptr,     \
-                       ctx->launch_mask, (int)f32_carries(ctx, n, n), bat)
+    const int carry = sizeof(R) == 4 ? (carries(ctx, n, n) ? 4 : 0) : carries64(ctx, n, n) ? dl_period(ctx, n, n, nsl) : 0;
+#define OMX_DL_FOUR(CF, EX, CY)                                                                                            \
+    hipLaunchKernelGGL((k_dgemm_dl<R, CF, false, true, 1, EX, CY>), grid, dim3(CF::NT), 0, ctx->stream, n, n, k, 1.0, A[0], \
+                       A[0], lda, B, B, ldb, 0.0, (const R *)nullptr, (int64_t)0, 0.0, C[0], ldc, 2, 0, 1, nsl,             \
+                       (R *)nullptr, ctx->launch_mask, carry, bat)
+    constexpr bool single = sizeof(R) == 4;
     if (tile == 0 && n % 128 == 0 && k % DlT<R>::DK == 0)
-        OMX_DL_FOUR(Dl128, true);
+        OMX_DL_FOUR(Dl128, true, single);
     else if (tile == 0)
-        OMX_DL_FOUR(Dl128, false);
+        OMX_DL_FOUR(Dl128, false, single);
+    else if (tile == 1 && carry)
+        OMX_DL_FOUR(Dl64, false, true);
     else if (tile == 1)
-        OMX_DL_FOUR(Dl64, false);
+        OMX_DL_FOUR(Dl64, false, single);
+    else if (carry)
+        OMX_DL_FOUR(Dl32, false, true);
     else
-        OMX_DL_FOUR(Dl32, false);
+        OMX_DL_FOUR(Dl32, false, single);
 #undef OMX_DL_FOUR
     prof_end(ctx, OMX_K_GEMM, ev);
     OMX_CHECK_HIP(hipGetLastError());

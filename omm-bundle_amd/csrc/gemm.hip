@@ -418,11 +418,13 @@ static int run_cfg(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1,
     constexpr int VEC = 16 / sizeof(TS);
     const int tiles = ((m + CF::BM - 1) / CF::BM) * ((n + CF::BN - 1) / CF::BN);
     const int ktot = NPAIR * k;
-    // Split K when the tile count cannot fill the chip (aim for >= 2 workgroups per CU).
+    // Split K when the tile count cannot fill the chip (aim for >= 2 workgroups per CU), or as the direct-to-LDS
+    // kernel splits where that adds in the same way (FP64 small results reach this kernel only by leading dimensions
+    // beyond 2^20).
     int splits = 1;
     const int target = 2 * ctx->num_cus;
-    if constexpr (PREC == OMX_PREC_F64 || (PREC == OMX_PREC_F32 && sizeof(TS) == 4)) {
-        // as the direct-to-LDS kernel splits
+    constexpr bool f64 = PREC == OMX_PREC_F64 && sizeof(TS) == 8, f32 = PREC == OMX_PREC_F32 && sizeof(TS) == 4;
+    if ((f64 && !carries64(ctx, m, n)) || f32) {
         splits = dgemm_k_splits(ctx, m, n, (ktot + BK - 1) / BK, PREC == OMX_PREC_F64 ? 8 : 4);
     } else if (tiles < target && !ctx->launch_mask) {
         int max_splits = std::max(1, ktot / (4 * BK));
@@ -453,7 +455,7 @@ static int run_cfg(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1,
                             (double)m * n * (1 + (C0 ? 1 : 0) + (beta != 0.0 ? 1 : 0))));
     hipLaunchKernelGGL((k_gemm<TS, PREC, TRA, TRB, NPAIR, CF>), dim3(grid, 1, splits), dim3(CF::NT), 0, ctx->stream,
                        m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta, C, ldc, kps, vec_a, vec_b, (int)sym,
-                       partial, ctx->launch_mask, (int)f32_carries(ctx, m, n));
+                       partial, ctx->launch_mask, (int)carries(ctx, m, n));
     if (splits > 1) {
         int64_t total = (int64_t)m * n;
         int grid = (int)std::min<int64_t>((total + 255) / 256, 8192);
@@ -550,7 +552,8 @@ static int tuned_cfg(omx_ctx ctx, int m, int n, int k, const TS *A1, const TS *A
         out = it->second.first;
         return OMX_OK;
     }
-    const std::vector<int> ids = CS::ids();
+    std::vector<int> ids = CS::ids();
+    if (CS::dl && carries64(ctx, m, n)) ids = {7};
     if (ids.size() == 1) {
         ctx->tune_gemm[key] = {ids[0], 0.0};
         out = ids[0];
@@ -603,7 +606,9 @@ static int run_gemm(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1
     typedef CfgSet<TS, PREC, TRA, TRB, NPAIR> CS;
     int id = (CS::dl || CS::sdl) ? 7 : 0;
     if (ctx->gemm_cfg >= 0) {
-        id = ctx->gemm_cfg;  // forced (omx_gemm_set_tile); a configuration that does not apply falls back to 0
+        // forced (omx_gemm_set_tile); a configuration that does not apply falls back to 0, and 7 alone carries its
+        // sums in FP64
+        if (!(CS::dl && carries64(ctx, m, n))) id = ctx->gemm_cfg;
     } else if (ctx->autotune) {
         int rc = tuned_cfg<TS, PREC, TRA, TRB, NPAIR>(ctx, m, n, k, A1, A2, lda, B1, B2, ldb, id);
         if (rc) return rc;
@@ -1095,7 +1100,7 @@ int launch_gemm_pair(omx_ctx ctx, int prec, int dt, int m, int n, int k, double 
     // The pair boundary must fall on a K-slice boundary of the staged kernels (the direct-to-LDS FP64 and
     // FP32 kernels pad each product's last slice); otherwise the caller runs separate passes.
     if (k % bk != 0) {
-        if (dt == OMX_F64 && prec == OMX_PREC_F64 && (ctx->gemm_cfg < 0 || ctx->gemm_cfg == 7))
+        if (dt == OMX_F64 && prec == OMX_PREC_F64 && (ctx->gemm_cfg < 0 || ctx->gemm_cfg == 7 || carries64(ctx, m, n)))
             return launch_dgemm(ctx, false, false, 2, m, n, k, alpha, (const double *)A1, (const double *)A2, lda,
                                 (const double *)B1, (const double *)B2, ldb, beta0, (const double *)C0, ldc, beta,
                                 (double *)C, ldc);

@@ -80,7 +80,7 @@ struct omx_ctx_s {
     // triangles.  A kernel that writes both sets 3 (no mirror pass needed).
     int gemm_sym = 0;
     bool one_part = false;  // set around products whose K is not to be split
-    bool carry64 = false;   // set around FP64 products that carry their sums (carry_sums)
+    bool carry64 = false;   // set around FP64 products that carry their sums whatever their size
     omx_spmm_shape_s spmm_shape;  // forced SpMM launch shape (when spmm_forced)
     bool spmm_forced = false;
     bool spmm_stencil = false;  // lattice operators use the 2.5-D stencil SpMM (omx_spmm_stencil)
@@ -248,13 +248,23 @@ int launch_sgemm(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, int k
 bool search_in_one(omx_ctx ctx, int dt, int n, int k, int64_t lda, int64_t ldb);
 int launch_search(omx_ctx ctx, int dt, int n, int k, const void *const A[4], int64_t lda, const void *B, int64_t ldb,
                   void *const C[4], int64_t ldc);
-// Whether an m x n FP32 product on FP32 storage may split K and carries its sums (carry_sums): results of fewer
-// than two 128 tiles per CU.  Larger ones are one FP32 chain over K, element by element: with carried sums (1.6e-6
-// -> 2.5e-7 off FP64 at 8192 x 8192 x 16384) the mixed solve at n = 16384 took 670 to 950 low-precision steps
-// and 22.8 to 29.9 s from six starts, against 555 to 665 steps and 18.4 to 22.3 s, and ended higher in energy:
-// its stop and the FP32 recomputation of its state go by the rounding of these products.
-inline bool f32_carries(omx_ctx ctx, int m, int n) {
+// Results of fewer than two 128 tiles per CU carry their sums over K (carry_sums), FP64 products on FP64 storage
+// (carries64) and FP32 ones on FP32 storage: in 128 tiles K was split for these to fill the chip, and parts of a
+// few hundred values are rounded less than one chain (FP64 Grams against 80 bits, such parts, one chain, now: 250 x 500
+// 3.1e-16, 7.5e-16, 2.9e-16; 700 x 1400 3.5e-16, 1.2e-15, 3.1e-16; 2662 x 5324 1.7e-15, 1.2e-15, 5.5e-16).  Larger FP32 products are one FP32 chain over K,
+// unsplit: with carried sums (1.6e-6 -> 2.5e-7 off FP64 at 8192 x 8192 x 16384) the mixed solve at n = 16384 took 670 to
+// 950 low-precision steps and 22.8 to 29.9 s from six starts, against 555 to 665 steps and 18.4 to 22.3 s, and
+// ended higher in energy: its stop and the FP32 recomputation of its state go by the rounding of these products.
+inline bool carries(omx_ctx ctx, int m, int n) {
     return (int64_t)((m + 127) / 128) * ((n + 127) / 128) < 2 * ctx->num_cus;
+}
+// (a masked launch, of the grouped solver, never split K)
+inline bool carries64(omx_ctx ctx, int m, int n) { return !ctx->launch_mask && (ctx->carry64 || carries(ctx, m, n)); }
+// Slices of K (of nsl) between two carries, a power of two: 4 for the shortest parts that `parts` of K made, up to
+// 16 for longer ones (carrying costs 1 to 3 % at 4).
+inline int carry_period(int nsl, int64_t parts) {
+    const int64_t len = nsl / std::max<int64_t>(1, parts);
+    return len >= 32 ? 16 : len >= 16 ? 8 : 4;
 }
 // Parts K is split into for such a product of nsl slices of 128 bytes (es: element size); a function of the
 // shape alone, so that every tile configuration and the symmetric form add in the same order.

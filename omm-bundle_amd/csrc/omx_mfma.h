@@ -35,8 +35,8 @@ __device__ inline void wg_barrier() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// Carried sums: 512 bytes of a k-contiguous row's values (128 FP32, 64 FP64) are accumulated at a time and these sums
-// added up apart (restarting at a pair's second product too).  FP32 products whose K is split (f32_carries) do: one
+// Carried sums: a few slices of K (FP32 128 values, FP64 64 to 256) are accumulated at a time and these sums added up
+// apart (restarting at a pair's second product too).  FP32 and FP64 products of small results do (carries): one
 // FP32 chain over all of K would be three times less accurate at 700 x 700 x 1500 than the parts of about 160 that
 // such a product used to be split into.  So do the FP64 products of the factorisations (dense_la.hip).
 template <typename AV, int FM, int FN>

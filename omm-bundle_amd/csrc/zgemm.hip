@@ -355,10 +355,10 @@ struct ZlCfg {
 typedef ZlCfg<64, 2, 1> Zl64;
 typedef ZlCfg<32, 2, 4> Zl32;
 
-// CARRY (complex64, single products): sums of 32 values of K are added up apart (see carry_sums), which keeps
-// the error at or below that of the many parts K used to be split into (Gram 54 x 108: 1.6e-7 -> 1.4e-7, 2000 x
-// 4000: 1.6e-6 -> 2.5e-7; with one chain 900 x 2916 1.3e-6) for 3 %.  Batched products keep one chain: their
-// roundings are part of a k-point solve's trajectory.
+// CARRY (single products: complex64, every 32 values of K, and the complex128 ones of zl_carry): sums of `carry` slices are
+// added up apart (see carry_sums), which keeps the error at or below that of the many parts K used to be split into (complex64 Gram
+// 54 x 108: 1.6e-7 -> 1.4e-7, 2000 x 4000: 1.6e-6 -> 2.5e-7; with one chain 900 x 2916 1.3e-6) for 3 %.  Batched
+// products keep one chain: their roundings are part of a k-point solve's trajectory.
 template <typename R, class CF, bool TRA, bool CJA, bool TRB, bool CJB, int NPAIR, bool CARRY>
 __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double alpha,
                                                     const typename ZPrec<R>::cplx *__restrict__ A1,
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double
                                                     double beta0, const typename ZPrec<R>::cplx *__restrict__ C0,
                                                     double beta, typename ZPrec<R>::cplx *__restrict__ C, int64_t ldc,
                                                     int sym, int sps, typename ZPrec<R>::cplx *__restrict__ partial,
-                                                    ZBatch bat) {
+                                                    int carry, ZBatch bat) {
     typedef ZGeo<R> G;
     typedef typename ZPrec<R>::cplx C2;
     typedef typename ZPrec<R>::accv AV;
@@ -523,7 +523,8 @@ __global__ __launch_bounds__(256, 2) void k_zgemm_dl(int m, int n, int k, double
                 if (decltype(work)::value) {
                     slice(As, Bs);
                     if constexpr (CARRY) {
-                        if (sl % 2 == 1 || (NPAIR == 2 && sl + 1 == sw)) {
+                        const bool end = sizeof(R) == 4 ? sl % 2 == 1 : u == U - 1 && (sl & (carry - 1)) == carry - 1;
+                        if (end || (NPAIR == 2 && sl + 1 == sw)) {
                             carry_sums(are, tre);
                             carry_sums(aim, tim);
                         }
@@ -640,6 +641,18 @@ static void zl_shape(omx_ctx ctx, int m, int n, int nsl, bool sym, int nbatch, b
         }
 }
 
+// Slices of K (of nsl) between the carries of a complex128 product, 0 for none: carried where its parts of K (sps
+// slices) are a quarter longer than those that 64x128 tiles were split into to fill the chip (up to four for the
+// lower triangle of a Hermitian product).  Against 80 bits, with those parts, without and with carried sums: Gram
+// 250 x 500 2.8e-16, 4.6e-16, 2.4e-16, 700 x 1400 5.3e-16, 1.7e-15, 3.5e-16; Hermitian 2000 x 4000 1.15e-15, 2.8e-15,
+// 3.7e-16 (1.14 -> 1.17 ms).
+static int zl_carry(omx_ctx ctx, int m, int n, bool lower, int nsl, int sps) {
+    const int64_t tm = (m + ZBM - 1) / ZBM, tn = (n + ZBN - 1) / ZBN, tiles = lower ? (tm * tn + tm) / 2 : tm * tn;
+    const int64_t fill = tiles < 2 * ctx->num_cus ? (2 * ctx->num_cus + tiles - 1) / tiles : 1;
+    const int64_t parts = std::min<int64_t>(std::min<int64_t>(fill, lower ? 4 : 64), std::max(1, nsl / 4));
+    return 4 * sps * parts > 5 * (int64_t)nsl ? carry_period(nsl, parts) : 0;
+}
+
 // Launches the direct-to-LDS product; OMX_ERR_UNSUPPORTED for leading dimensions beyond 2^20.
 template <typename R, bool TRA, bool CJA, bool TRB, bool CJB, int NPAIR>
 static int run_zgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const void *A1, const void *A2, int64_t lda,
@@ -684,19 +697,16 @@ static int run_zgemm_dl(omx_ctx ctx, int m, int n, int k, double alpha, const vo
 #define OMX_ZL_RUN(CF, CY)                                                                                          \
     hipLaunchKernelGGL((k_zgemm_dl<R, CF, TRA, CJA, TRB, CJB, NPAIR, CY>), grid, dim3(256), 0, ctx->stream, m, n, k, alpha, \
                        (const C2 *)A1, (const C2 *)A2, lda, (const C2 *)B1, (const C2 *)B2, ldb, beta0,             \
-                       (const C2 *)C0, beta, (C2 *)C, ldc, sym, sps, partial, bat)
-    constexpr bool single = sizeof(R) == 4;
-    if (tile == 64) {
-        if (single && allow_split)
-            OMX_ZL_RUN(Zl64, single);
-        else
-            OMX_ZL_RUN(Zl64, false);
-    } else {
-        if (single && allow_split)
-            OMX_ZL_RUN(Zl32, single);
-        else
-            OMX_ZL_RUN(Zl32, false);
-    }
+                       (const C2 *)C0, beta, (C2 *)C, ldc, sym, sps, partial, carry, bat)
+    const int carry = !allow_split ? 0 : sizeof(R) == 4 ? 2 : zl_carry(ctx, m, n, lower, nsl, sps);
+    if (tile == 64 && carry)
+        OMX_ZL_RUN(Zl64, true);
+    else if (tile == 64)
+        OMX_ZL_RUN(Zl64, false);
+    else if (carry)
+        OMX_ZL_RUN(Zl32, true);
+    else
+        OMX_ZL_RUN(Zl32, false);
 #undef OMX_ZL_RUN
     if (partial)
         hipLaunchKernelGGL((k_zl_reduce<R>), dim3((unsigned)std::min<int64_t>(((int64_t)m * n + 255) / 256, 8192)),
