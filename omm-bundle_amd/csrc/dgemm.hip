@@ -16,13 +16,13 @@
 // What bounds it: the FP64 matrix core (64 cycles per 16x16x4 step and SIMD), except where the result has
 // fewer tiles than the chip has CUs; there it is the serial chain of slices of one tile, and below that
 // the launch.  Before, only m, n % 128 == 0 with k % 16 == 0 took this path and everything else was staged
-// through registers in 128x128 tiles: 54 x 54 x 108 22 us (now 5.5), 432 x 432 x 864 about 35 us (16),
-// 1458 x 1458 x 2916 340 us (236), 4394 x 4394 x 8788 5.84 ms (5.17), gradient of 2662 x 5324 2.96 ms (2.32).
+// through registers in 128x128 tiles: 54 x 54 x 108 22 us (now 4.3), 432 x 432 x 864 about 35 us (14),
+// 1458 x 1458 x 2916 340 us (225), 4394 x 4394 x 8788 5.84 ms (5.14), gradient of 2662 x 5324 2.96 ms (2.30).
 // FP32: an FP32 step takes half the time of an FP64 one, so a slice of 32 takes as long as an FP64 slice of
 // 16 and the same tiles and model serve.  Before, only Grams of whole 128 tiles that fill the chip were
-// loaded this way: 54 x 54 x 108 21 us (now 5.8), 250 x 250 x 500 30 (6.2), 1458 x 1458 x 2916 242 (124;
-// symmetric 252, now 75; pair 512, now 237), 4394 x 4394 x 8788 4.14 ms (2.70; symmetric 2.61, now 1.37), pair
-// of 4394 x 8788 8.64 ms (5.17), 4096 x 4096 x 8192 1.90 (1.91).  Errors against FP64 (relative, Gram): 250 x
+// loaded this way: 54 x 54 x 108 21 us (now 4.2), 250 x 250 x 500 30 (6.1), 1458 x 1458 x 2916 242 (124;
+// symmetric 252, now 76; pair 512, now 239), 4394 x 4394 x 8788 4.14 ms (2.93; symmetric 2.61, now 1.35), pair
+// of 4394 x 8788 8.64 ms (5.24), 4096 x 4096 x 8192 1.90 (1.86).  Errors against FP64 (relative, Gram): 250 x
 // 500 2.4e-7 (2.1e-7), 1458 x 2916 4.9e-7 (2.1e-7), as before where K is one chain (see carries); the carry
 // costs 2 %.
 //
@@ -360,14 +360,13 @@ static int tiles_of(int m, int n, int b, bool sym) {
     return sym ? tm * (tm + 1) / 2 : tm * tn;
 }
 
-// Time of a product by tile and by the parts K is split into, in microseconds: rounds of workgroups over
+// dl_time, dl_cost: time of a product by tile and by the parts K is split into, in microseconds: rounds of workgroups over
 // the CUs (workgroups that share a CU share its matrix cores) times the slices of a part, plus what a launch,
 // a round and the reduction of the parts cost.  The constants are a least-squares fit to 60 shapes (54 x 54
 // x 108 to 4394 x 4394 x 8788, Grams, symmetric Grams and pairs; every tile and 1 to 12 parts): 11 % rms, and
-// the choices they lead to are within 1.6 % of the fastest of all on average.  How the last rounds fill the
-// CUs is modelled apart (1458 x 1458 x 2916: 64 tiles, 4 parts 240 us instead of 128, 5 parts 267; the pair
-// 1700 x 3456 x 1700: 64 tiles 644 us instead of 128, 2 parts 740).
-// A symmetric product in 128x128 tiles whose last round of resident workgroups (two per CU) is not full:
+// the choices they lead to are within 1.6 % of the fastest of all on average.
+//
+// dl_tail_parts: a symmetric product in 128x128 tiles whose last round of resident workgroups (two per CU) is not full:
 // the parts along K that each tile of that round is split into (1: it is not split).  Only for orders
 // that are multiples of 128; elsewhere the symmetric form adds exactly as the full product does.
 static int dl_tail_parts(omx_ctx ctx, int m, int tiles, bool sym, int nsl) {
@@ -399,7 +398,9 @@ static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int s
         return 9.8 + 0.55 * whole + 1.90 * (whole * sps + 2.0 * sps / tail);
     }
     double t = dl_time(ctx, q, units, sps);
-    // 128: two workgroups share a CU, and the parts of most of a third round land in pairs.
+    // 128: two workgroups share a CU, and the parts of most of a third round land in pairs.  (Reached by FP32 products;
+    // FP32 Grams of 1410 to 1440 states 123 us instead of 146, 1474 to 1520 130 to 133 instead of 135, 2114 to 2176 335
+    // to 340 instead of 340 to 350, gradients of 1058 to 1088 states 110 instead of 123: all that it changes.)
     if (q == 0 && splits > 1 && rounds == 3 && 2 * units > 5 * ctx->num_cus && units < 3 * ctx->num_cus)
         t += 0.1 * 1.90 * 3 * sps;
     return t + (splits > 1 ? 5.3 + 1e-6 * es * (splits + 1) * m * n / 4.9 : 0.0);
@@ -556,7 +557,8 @@ static int launch_dl(omx_ctx ctx, bool trA, bool trB, int npair, int m, int n, i
 
 // The line-search products of one CG step in one launch (see DlBatch), where the model finds that faster than
 // one by one: small results leave most of the chip idle each, larger ones are split along K to fill it
-// (twelve steps of omm() at 54 x 108 1.65 -> 1.33 ms, four at 1458 x 2916 6.48 -> 6.26 ms).
+// (twelve steps of omm() at 54 x 108 1.65 -> 1.33 ms, four at 1458 x 2916 6.48 -> 6.26 ms).  search_tile: its tile and
+// time; search_in_one: whether it is taken.
 static int search_tile(omx_ctx ctx, int n, int nsl, int es, double &time) {
     const int first = es == 8 && carries64(ctx, n, n);
     int tile = first;

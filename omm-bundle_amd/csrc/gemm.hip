@@ -600,9 +600,8 @@ template <typename TS, int PREC, bool TRA, bool TRB, int NPAIR>
 static int run_gemm(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1, const TS *A2, int64_t lda,
                     const TS *B1, const TS *B2, int64_t ldb, double beta0, const TS *C0, double beta, TS *C,
                     int64_t ldc) {
-    // default: 128x128 with 8 waves and two workgroups per CU for the FP64 Gram and gradient products
-    // (3-4 % ahead of the 4-wave tile at n=16384, bitwise the same result), with direct-to-LDS
-    // staging where it applies (bitwise the same), as for FP32 products on FP32 storage; 0 otherwise
+    // default: the direct-to-LDS kernel for FP64 products on FP64 storage and FP32 ones on FP32 storage (past leading
+    // dimensions of 2^20 it hands over to the staged 8-wave tile 5, or 0), 0 otherwise
     typedef CfgSet<TS, PREC, TRA, TRB, NPAIR> CS;
     int id = (CS::dl || CS::sdl) ? 7 : 0;
     if (ctx->gemm_cfg >= 0) {

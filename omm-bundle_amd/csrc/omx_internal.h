@@ -149,11 +149,11 @@ struct El<double2> {
     __device__ static inline double2 make(double r, double i) { return make_double2(r, i); }
 };
 
-// Ensure ctx->ws holds at least `bytes`.  Returns OMX_OK or an error.
 // hipMalloc that gives back omx_malloc's idle blocks before it fails
 hipError_t dev_malloc(void **p, size_t bytes);
 // Gives them back; false if there are none.
 bool dev_release();
+// Ensure ctx->ws holds at least `bytes`.  Returns OMX_OK or an error.
 int ensure_ws(omx_ctx ctx, size_t bytes);
 
 // Look up this device's copy of the static scratch of omx_omm_pr_dots_noalloc (once per device,

@@ -23,7 +23,7 @@
 //           single chunk.
 // Of the chunks left over (their number mod 8) every XCD walks an eighth of the block columns.
 //
-// What bounds it is how often a basis column crosses from memory into an L2: a column is gathered by
+// What mattered is how often a basis column crosses from memory into an L2: a column is gathered by
 // seven block columns (a lattice operator), up to two lattice planes apart.  The default is therefore
 // the narrowest chunk (WPG = 1: 1 KB per basis column, so three planes of 256 sites are 3 MB of a 4 MB
 // L2) in mode 1, with large results stored past the L2 (spmm_nt); no load is predicated, and any number
@@ -32,7 +32,10 @@
 // access unless everything divides and aligns):
 //   FP64  8192 x 16384  797 -> 590    4394 x 8788  332 -> 182    2611 x 5280  128 -> 62   54 x 108  6.5 -> 4.9
 //   FP32  8192 x 16384  427 -> 300    4394 x 8788  179 -> 107    2611 x 5280   72 -> 39   250 x 500 5.1 -> 5.0
-// The copy rate of the card allows 419 and 209 us at the largest size.
+// The copy rate of the card allows 419 and 209 us at the largest size.  There, FP64, 2.8 GB cross
+// the L2s' memory side (1.3 times X and Y; 4.4 GB with 512-state chunks) at 4.6 TB/s, a copy at 5.9, and 9.4 GB are
+// requested of the L2s.  Which of the two binds is not established: a band of +-3 block columns takes the same time
+// with 13 % more of the one and 9 % less of the other.
 // A zero entry stored inside a block contributes an exact zero, so the per-element sum equals
 // the reference's CSC sum over its stored entries.
 #include <algorithm>
@@ -244,7 +247,7 @@ __global__ __launch_bounds__(256) void k_spmm_bsr4(int no, int nb, int nbc, doub
 // the in-plane neighbours are read.  Each basis column then crosses from L2 about twice (own +
 // halo) instead of 7 times.  The 7 blocks of a column are taken in stored order with the FMA
 // sequence of k_spmm_bsr4, so the results are the same bits.
-// Measured at n = 16384 (FP64): 1.2x the algorithmic HBM bytes (2.6 GB per launch against 4.4 GB
+// Measured at n = 16384 (FP64): 1.2x the algorithmic HBM bytes (2.6 GB per launch against 2.8 GB
 // for k_spmm_bsr4), but 0.89 ms against 0.59 ms (FP32: 0.57 against 0.30 ms): one
 // workgroup per CU (128 KB of LDS) and a barrier per plane.  The block values come through the
 // scalar cache (broadcast with v_readlane they cost 2.6x the VALU instructions of k_spmm_bsr4 and
@@ -500,8 +503,8 @@ static bool stencil_applies(const omx_ctx ctx, const omx_bsr A, int no, const T 
 typedef omx_spmm_shape_s SpmmShape;
 
 // Results go past the caches where they are more than the memory-side cache holds (256 MB), so that the
-// L2s keep the basis columns that later block columns gather (FP64, 8192 x 16384: 566 us against 535,
-// 4394 x 8788: 195 and 171); smaller results stay for the product that reads them next (complex128,
+// L2s keep the basis columns that later block columns gather (FP64, same run, 8192 x 16384: 535 us instead of 566
+// with results kept in the caches, 4394 x 8788: 171 instead of 195); smaller results stay for the product that reads them next (complex128,
 // 2000 x 4000, SpMM and Gram: 1168 us against 1200).
 static int spmm_nt(double bytes) { return bytes > 256e6; }
 
@@ -1092,8 +1095,9 @@ extern "C" int omx_spmm(omx_ctx ctx, int dt, int no, int nb, double alpha, const
 // The block's partial result goes to the workspace, and a second kernel adds the chunks in order
 // (deterministic).  The id -> (chunk, block columns) map is that of k_spmm_bsr4, mode 1.
 //
-// Bound by gathers through the L2s, like the SpMM: 2.14 GB come from memory, all there is.  Measured, us,
-// before (a thread per state, 17 shuffles per block, wave and chunk) and after:
+// Bound by what crosses the L2s' memory side: 4.5 GB are read there per launch at 8192 x 16384, twice the operands
+// (probably the waves that gather one basis column run apart and miss each other's lines), at 6.8 TB/s; the matrix cores are busy
+// 14 % of the time, and no LDS read conflicts.  Measured, us, before (a thread per state, 17 shuffles per block, wave and chunk) and after:
 //   FP64  8192 x 16384   976 -> 660   4394 x 8788  337 -> 244   1458 x 2916  34 -> 30   54 x 108  15 -> 8
 //   FP32  8192 x 16384  1610 -> 357   4394 x 8788  548 -> 121    250 x 500  20 ->  8
 // =============================================================================================

@@ -319,7 +319,7 @@ __global__ void k_zsplitk_reduce(int m, int n, int splits, const R *__restrict__
 // What bounds it: the matrix cores (a 64x64 complex tile moves as few bytes per operation as a real
 // 128x128 one), or, where the tiles do not fill the chip, the serial chain of slices of one tile.  The
 // register-staged kernel below ran 64x128 tiles only: the 2000 x 2000 x 4000 complex128 Hermitian Gram
-// took 1.60 ms (now 1.09), the full Gram 2.24 (1.85, 69 TF/s), 16 Grams of 128 x 128 x 256 on 32 workgroups
+// took 1.60 ms (now 1.14), the full Gram 2.24 (1.85, 69 TF/s), 16 Grams of 128 x 128 x 256 on 32 workgroups
 // 92 us (now 19).
 // ---------------------------------------------------------------------------------------------
 template <typename R>
@@ -645,7 +645,7 @@ static void zl_shape(omx_ctx ctx, int m, int n, int nsl, bool sym, int nbatch, b
 // slices) are a quarter longer than those that 64x128 tiles were split into to fill the chip (up to four for the
 // lower triangle of a Hermitian product).  Against 80 bits, with those parts, without and with carried sums: Gram
 // 250 x 500 2.8e-16, 4.6e-16, 2.4e-16, 700 x 1400 5.3e-16, 1.7e-15, 3.5e-16; Hermitian 2000 x 4000 1.15e-15, 2.8e-15,
-// 3.7e-16 (1.14 -> 1.17 ms).
+// 3.7e-16 (1.09 -> 1.14 ms).
 static int zl_carry(omx_ctx ctx, int m, int n, bool lower, int nsl, int sps) {
     const int64_t tm = (m + ZBM - 1) / ZBM, tn = (n + ZBN - 1) / ZBN, tiles = lower ? (tm * tn + tm) / 2 : tm * tn;
     const int64_t fill = tiles < 2 * ctx->num_cus ? (2 * ctx->num_cus + tiles - 1) / tiles : 1;
