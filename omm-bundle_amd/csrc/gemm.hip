@@ -605,13 +605,13 @@ static int run_gemm(omx_ctx ctx, int m, int n, int k, double alpha, const TS *A1
     typedef CfgSet<TS, PREC, TRA, TRB, NPAIR> CS;
     int id = (CS::dl || CS::sdl) ? 7 : 0;
     if (ctx->gemm_cfg >= 0) {
-        // forced (omx_gemm_set_tile); a configuration that does not apply falls back to 0, and 7 alone carries its
-        // sums in FP64
-        if (!(CS::dl && carries64(ctx, m, n))) id = ctx->gemm_cfg;
+        id = ctx->gemm_cfg;  // forced (omx_gemm_set_tile); a configuration that does not apply falls back to 0
     } else if (ctx->autotune) {
         int rc = tuned_cfg<TS, PREC, TRA, TRB, NPAIR>(ctx, m, n, k, A1, A2, lda, B1, B2, ldb, id);
         if (rc) return rc;
     }
+    // 7 alone carries its sums in FP64 (a masked launch may have left another choice for the shape)
+    if (CS::dl && carries64(ctx, m, n)) id = 7;
     return run_cfg_id<TS, PREC, TRA, TRB, NPAIR>(id, ctx, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, beta,
                                                  C, ldc);
 }
