@@ -1092,14 +1092,20 @@ extern "C" int omx_spmm(omx_ctx ctx, int dt, int no, int nb, double alpha, const
 // 64 cycles per load: 0.92 ms instead of 0.66 at 8192 x 16384).  The tiles' 16-byte vectors are swizzled
 // by column (no bank conflicts), and a wave has only one set of them: with 8 KB per wave 20 waves fit on a
 // CU and hide each other's waits (two sets, 8 waves: 0.70 ms; three: 1.02).
-// The block's partial result goes to the workspace, and a second kernel adds the chunks in order
-// (deterministic).  The id -> (chunk, block columns) map is that of k_spmm_bsr4, mode 1.
+// Sums are kept short: a block's two accumulators take turns and are added up apart every two steps, the parts of the
+// chunks in four sums.  Against 80 bits, FP64, 1458 and 8192 states 1.75e-16 and 2.2e-16 off, as with sums by thread and
+// wave (1.74e-16, 2.2e-16); in one chain per chunk and over the chunks 2.4e-16 and 3.4e-16, at the same time (FP32
+// 359 us instead of 375).  A block's vectors are read right before their products: all of them at once take the
+// registers of a fifth workgroup per CU.
+// The block's partial result goes to the workspace, and a second kernel adds the chunks in a
+// fixed order.  The id -> (chunk, block columns) map is that of k_spmm_bsr4, mode 1.
 //
 // Bound by what crosses the L2s' memory side: 4.5 GB are read there per launch at 8192 x 16384, twice the operands
-// (probably the waves that gather one basis column run apart and miss each other's lines), at 6.8 TB/s; the matrix cores are busy
-// 14 % of the time, and no LDS read conflicts.  Measured, us, before (a thread per state, 17 shuffles per block, wave and chunk) and after:
-//   FP64  8192 x 16384   976 -> 660   4394 x 8788  337 -> 244   1458 x 2916  34 -> 30   54 x 108  15 -> 8
-//   FP32  8192 x 16384  1610 -> 357   4394 x 8788  548 -> 121    250 x 500  20 ->  8
+// (probably the waves that gather one basis column run apart and miss each other's lines), at 6.8 TB/s; the matrix cores
+// are busy 14 % of the time, and no LDS read conflicts.  Measured, us, before (a thread per state, 17 shuffles per
+// block, wave and chunk) and after:
+//   FP64  8192 x 16384   976 -> 654   4394 x 8788  337 -> 244   1458 x 2916  34 -> 31   54 x 108  15 -> 9
+//   FP32  8192 x 16384  1610 -> 375   4394 x 8788  548 -> 127    250 x 500  20 -> 10
 // =============================================================================================
 namespace omx {
 
@@ -1107,7 +1113,7 @@ constexpr int SD_NBK = 7;           // stored blocks taken together (a lattice c
 constexpr int64_t SD_LD = 1 << 26;  // leading dimensions whose block columns 32-bit offsets reach
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_sddmm_bsr4_partial(int no, int nb, int nbc, const T *__restrict__ A, int64_t lda,
+__global__ __launch_bounds__(256, 5) void k_sddmm_bsr4_partial(int no, int nb, int nbc, const T *__restrict__ A, int64_t lda,
                                                           const T *__restrict__ B, int64_t ldb,
                                                           const int *__restrict__ colptr, const int *__restrict__ rowidx,
                                                           int chunk, int nrc, int njg, int64_t nnzb,
@@ -1142,12 +1148,12 @@ __global__ __launch_bounds__(256) void k_sddmm_bsr4_partial(int no, int nb, int 
         const int nblk = min(SD_NBK, le - l0);
         int I[SD_NBK];
         int oa[SD_NBK];
-        double acc[SD_NBK];
+        double acc[SD_NBK][2], tot[SD_NBK];
 #pragma unroll
         for (int b = 0; b < SD_NBK; ++b) {
             I[b] = rowidx[l0 + min(b, nblk - 1)];
             oa[b] = (min(lc, nb - 1 - 4 * I[b]) * (int)lda + lv) * (int)sizeof(T);
-            acc[b] = 0.0;
+            acc[b][0] = acc[b][1] = tot[b] = 0.0;
         }
         // products of one step: xb and the xa(b) are this lane's vectors of B and of A's block b
         auto products = [&](T (&xb)[VEC], auto xa) {
@@ -1155,21 +1161,26 @@ __global__ __launch_bounds__(256) void k_sddmm_bsr4_partial(int no, int nb, int 
 #pragma unroll
                 for (int q = 0; q < VEC; ++q) xb[q] = jin ? xb[q] : (T)0;
             }
-            T x[SD_NBK][VEC];
-#pragma unroll
-            for (int b = 0; b < SD_NBK; ++b)
-                if (b < nblk) xa(b, x[b]);
 #pragma unroll
             for (int b = 0; b < SD_NBK; ++b)
                 if (b < nblk) {
+                    T x[VEC];
+                    xa(b, x);
                     if (4 * I[b] + 4 > nb) {
 #pragma unroll
-                        for (int q = 0; q < VEC; ++q) x[b][q] = 4 * I[b] + col < nb ? x[b][q] : (T)0;
+                        for (int q = 0; q < VEC; ++q) x[q] = 4 * I[b] + col < nb ? x[q] : (T)0;
                     }
 #pragma unroll
                     for (int q = 0; q < VEC; ++q)
-                        acc[b] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x[b][q], (double)xb[q], acc[b], 0, 0, 0);
+                        acc[b][q & 1] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)x[q], (double)xb[q], acc[b][q & 1], 0, 0, 0);
                 }
+        };
+        auto carry = [&]() {
+#pragma unroll
+            for (int b = 0; b < SD_NBK; ++b) {
+                tot[b] += acc[b][0] + acc[b][1];
+                acc[b][0] = acc[b][1] = 0.0;
+            }
         };
         auto load = [&](const T *p, T *to, int o) {
             const __amdgpu_buffer_rsrc_t r = raw_rsrc(p);
@@ -1187,7 +1198,9 @@ __global__ __launch_bounds__(256) void k_sddmm_bsr4_partial(int no, int nb, int 
             T xb[VEC];
             uload<T, VEC>(tb + at, xb);
             products(xb, [&](int b, T (&x)[VEC]) { uload<T, VEC>(ta + b * TILE + at, x); });
+            if (st & 1) carry();
         }
+        carry();
         for (int st = nfull; st * SV < len; ++st) {  // the last states
             const int s = st * SV + rv * VEC;
             auto tail = [&](const T *p, T (&x)[VEC]) {
@@ -1201,7 +1214,7 @@ __global__ __launch_bounds__(256) void k_sddmm_bsr4_partial(int no, int nb, int 
 #pragma unroll
         for (int b = 0; b < SD_NBK; ++b)
             if (b < nblk) {  // lane j + 4 g + 16 i holds entry (i, j) of product g
-                double t = acc[b];
+                double t = tot[b] + (acc[b][0] + acc[b][1]);
                 t += __shfl_xor(t, 4, 64);
                 t += __shfl_xor(t, 8, 64);
                 if ((lane & 12) == 0) partial[((int64_t)rc * nnzb + l0 + b) * 16 + (lane >> 4) + 4 * col] = t;
@@ -1213,8 +1226,15 @@ __global__ void k_sddmm_bsr4_final(int64_t nnzb, int nparts, const double *__res
                                    double beta, double *__restrict__ vals) {
     const int64_t total = nnzb * 16;
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-        double s = 0.0;
-        for (int p = 0; p < nparts; ++p) s += partial[(int64_t)p * total + q];
+        double t[4] = {0.0, 0.0, 0.0, 0.0};  // every fourth part, then the four: shorter chains
+        int p = 0;
+        for (; p + 4 <= nparts; p += 4)
+#pragma unroll
+            for (int h = 0; h < 4; ++h) t[h] += partial[(int64_t)(p + h) * total + q];
+#pragma unroll
+        for (int h = 0; h < 3; ++h)
+            if (p + h < nparts) t[h] += partial[(int64_t)(p + h) * total + q];
+        const double s = (t[0] + t[1]) + (t[2] + t[3]);
         vals[q] = (beta == 0.0) ? alpha * s : alpha * s + beta * vals[q];
     }
 }
