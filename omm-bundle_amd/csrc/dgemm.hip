@@ -115,8 +115,8 @@ struct DlBatch {
 // EXACT: m, n are multiples of the tile and k of the slice, so nothing needs the descriptors' end, a
 // cleared tail or guarded stores; the 128x128 tile is faster without them (8192 x 8192 x 16384 Gram 29.8
 // against 29.9 ms, gradient 60.4 against 61.6 ms).
-// CY: the sums are carried every `carry` slices, not at all for 0 (FP32 products, and the FP64 ones of carries64, which take the 64 and
-// 32 tiles: the 128 tile has no registers for a second set of sums).
+// CY: the sums are carried every `carry` slices, not at all for 0 (FP32 products, the FP64 ones of carries64 and masked
+// pairs (see seam); the FP64 ones take the 64 and 32 tiles: the 128 tile has no registers for a second set of sums).
 template <typename R, class CF, bool TRA, bool TRB, int NPAIR, bool EXACT, bool CY>
 __global__ __launch_bounds__(CF::NT, CF::MINW) void k_dgemm_dl(int m, int n, int k, double alpha,
                                                                const R *__restrict__ A1,
@@ -405,10 +405,11 @@ static double dl_cost(omx_ctx ctx, int q, bool sym, int m, int n, int nsl, int s
         t += 0.1 * 1.90 * 3 * sps;
     return t + (splits > 1 ? 5.3 + 1e-6 * es * (splits + 1) * m * n / 4.9 : 0.0);
 }
-static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, int es, double *cost = nullptr) {
+static int dl_tile(omx_ctx ctx, bool sym, int m, int n, int nsl, int splits, int nbatch, int es, double *cost = nullptr,
+                   bool carried = false) {
     int best = 0;
     double c = 0.0;
-    const int first = es == 8 && carries64(ctx, m, n);
+    const int first = es == 8 && (carried || carries64(ctx, m, n));
     for (int q = first; q < 3; ++q) {
         const double t = dl_cost(ctx, q, sym, m, n, nsl, splits, nbatch, es);
         if (q == first || t < c) {
@@ -439,6 +440,7 @@ int dgemm_k_splits(omx_ctx ctx, int m, int n, int nsl, int es) {
     return best;
 }
 
+constexpr int kSeam = 1 << 30;  // a carry period that no product reaches: carried at a pair's seam only
 // Carry period of an FP64 product: by the parts that 128 tiles were split into, two workgroups per CU, 64 values at
 // the least.
 static int dl_period(omx_ctx ctx, int m, int n, int nsl) {
@@ -451,7 +453,7 @@ template <typename R, class CF, bool TRA, bool TRB, int NPAIR>
 static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int k, double alpha, const R *A1,
                     const R *A2, int64_t lda, const R *B1, const R *B2, int64_t ldb, double beta0,
                     const R *C0, int64_t ldc0, double beta, R *C, int64_t ldc, int nbatch,
-                    const DlBatch &bat) {
+                    const DlBatch &bat, bool seam) {
     constexpr int DK = DlT<R>::DK;
     const int tiles = tiles_of(m, n, CF::BM, sym != 0);
     const int nsl = NPAIR * ((k + DK - 1) / DK);
@@ -482,15 +484,15 @@ static int run_tile(omx_ctx ctx, int sym, int splits, int sps, int m, int n, int
                        alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, sym, tbase, parts, per, partial, mask, \
                        CARRY, bat)
         if constexpr (single) {
-            const int carry = carries(ctx, m, n) ? 4 : 0;
+            const int carry = carries(ctx, m, n) ? 4 : seam ? kSeam : 0;
             if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0)
                 OMX_DL_LAUNCH(CF::BM == 128, true, carry);
             else
                 OMX_DL_LAUNCH(false, true, carry);
         } else if (CF::BM == 128 && m % 128 == 0 && n % 128 == 0 && k % DK == 0) {
             OMX_DL_LAUNCH(CF::BM == 128, false, 0);
-        } else if (CF::BM != 128 && carries64(ctx, m, n)) {
-            OMX_DL_LAUNCH(false, CF::BM != 128, dl_period(ctx, m, n, nsl));
+        } else if (CF::BM != 128 && (seam || carries64(ctx, m, n))) {
+            OMX_DL_LAUNCH(false, CF::BM != 128, seam ? kSeam : dl_period(ctx, m, n, nsl));
         } else {
             OMX_DL_LAUNCH(false, false, 0);
         }
@@ -514,10 +516,20 @@ static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const R *A1, 
     const int sym = (m == n && NPAIR == 1 && !TRA && TRB) ? ctx->gemm_sym : 0;
     const int nsl = NPAIR * ((k + DlT<R>::DK - 1) / DlT<R>::DK);
     int splits = nbatch > 1 ? 1 : dgemm_k_splits(ctx, m, n, nsl, sizeof(R));
+    // The two products of a pair whose K is no multiple of the slice used to be made in separate passes, and in one chain
+    // over both they are rounded 1.4 times as much.  Their sums are kept apart: carried at the seam (FP32, and
+    // masked launches, in 64 and 32 tiles), or in two parts of K where the model splits none (pairs against 80 bits,
+    // separate passes, one chain, now: FP64 2001 states 1.42e-15, 2.01e-15, 1.42e-15, 1.15 -> 1.21 ms, 4001 2.23e-15,
+    // 2.90e-15, 2.23e-15, 7.78 -> 8.01 ms; FP32 2662 9.2e-7, 1.31e-6, 9.2e-7).
+    bool seam = NPAIR == 2 && k % DlT<R>::DK != 0 && !(sizeof(R) == 4 ? carries(ctx, m, n) : carries64(ctx, m, n));
+    if (seam && sizeof(R) == 8 && !ctx->launch_mask) {
+        splits = std::max(splits, 2);
+        seam = false;
+    }
     const int sps = (nsl + splits - 1) / splits;
     splits = (nsl + sps - 1) / sps;
     const int cls = NPAIR == 2 ? OMX_K_GEMM_PAIR : OMX_K_GEMM;
-    const int tile = dl_tile(ctx, sym != 0, m, n, nsl, splits, nbatch, sizeof(R));
+    const int tile = dl_tile(ctx, sym != 0, m, n, nsl, splits, nbatch, sizeof(R), nullptr, seam);
     hipEvent_t ev;
     prof_begin(ctx, cls, &ev);
     prof_work(ctx, cls, 2.0 * (sym ? sym_area(m, kDlEdge[tile]) : (double)m * n) * (double)NPAIR * k,
@@ -526,7 +538,7 @@ static int run_ops(omx_ctx ctx, int m, int n, int k, double alpha, const R *A1, 
     int rc;
 #define OMX_DL_RUN(CF) \
     run_tile<R, CF, TRA, TRB, NPAIR>(ctx, sym, splits, sps, m, n, k, alpha, A1, A2, lda, B1, B2, ldb, beta0, C0, ldc0, beta, C, ldc, \
-                                  nbatch, bat)
+                                  nbatch, bat, seam)
     if (tile == 0)
         rc = OMX_DL_RUN(Dl128);
     else if (tile == 1)
